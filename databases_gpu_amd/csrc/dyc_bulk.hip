@@ -112,7 +112,7 @@ __device__ inline void fill_chunk(const SubRef &S, uint32_t b0, uint32_t len,
     __shared__ uint32_t wred[THREADS / kWave];
     __shared__ unsigned long long obase;
     __shared__ uint32_t onext;
-    uint64_t *const sub = S.keys;
+    uint64_t *const sub = as_global(S.keys);
     const uint4 *const src = reinterpret_cast<const uint4 *>(sub + (uint64_t)b0 * kSlots);
     constexpr uint32_t kParts = kChunkBuckets * kSlots / 2;  // 16-byte parts of the chunk
     if constexpr (DENSE) {

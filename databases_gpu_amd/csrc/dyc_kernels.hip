@@ -905,7 +905,7 @@ __global__ __launch_bounds__(256, W) void group_probe_kernel(const Desc *__restr
          it += waves) {
         const GroupItem item = items[it];
         if (item.len == 0) continue;  // wave-uniform: an empty slot of a layout by XCD
-        const Desc D = dir[item.table];
+        const Desc D = as_global(dir[item.table]);
         const uint64_t end = item.begin + item.len;
         unsigned long long nd = 0;
         for (uint64_t base = item.begin; base < end; base += kWave) {
@@ -940,7 +940,7 @@ __global__ __launch_bounds__(256, W) void group_insert_kernel(const Desc *__rest
          it += waves) {
         const GroupItem item = items[it];
         if (item.len == 0) continue;  // wave-uniform: a block the bulk fill's rounds emptied
-        const Desc D = dir[item.table];
+        const Desc D = as_global(dir[item.table]);
         uint64_t next = item.begin;
         const uint64_t end = item.begin + item.len;
         const unsigned long long rej0 = tally.rejected;
@@ -1069,8 +1069,8 @@ __global__ __launch_bounds__(256) void serve_probe_kernel(const Desc *__restrict
     WaveTotal del;
     for (uint32_t it = wave_uniform(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave); it < n_items;
          it += waves) {
-        const ServeItem item = items[it];
-        const Desc D = dir[item.table];
+        const ServeItem item = as_global(items[it]);
+        const Desc D = as_global(dir[item.table]);
         unsigned long long nd = serve_probe_item<G, ERASE>(D, item, pool, np);
         if constexpr (ERASE) del.add(del_total, item.table, wave_sum(nd));
     }
@@ -1090,8 +1090,8 @@ __global__ __launch_bounds__(256) void serve_insert_kernel(const Desc *__restric
     const uint32_t waves = gridDim.x * (blockDim.x / kWave);
     for (uint32_t it = wave_uniform(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave); it < n_items;
          it += waves) {
-        const ServeItem item = items[it];
-        ins.add(ins_total, item.table, serve_insert_item<G>(dir[item.table], item, c, P, C, sink, tally));
+        const ServeItem item = as_global(items[it]);
+        ins.add(ins_total, item.table, serve_insert_item<G>(as_global(dir[item.table]), item, c, P, C, sink, tally));
     }
     ins.flush(ins_total);
     wave_tally(C, &C->kicks, tally.kicks);
@@ -1128,7 +1128,8 @@ __global__ __launch_bounds__(256) void serve_tick_kernel(const Desc *__restrict_
         if (__lane_id() == 0) it = (uint32_t)atomicAdd(cursor, 1ull);
         it = wave_uniform(it);
         if (it >= n_items) break;
-        const TickItem ti = items[it];
+        TickItem ti = items[it];
+        ti.item = as_global(ti.item);
         if (ti.wait) {
             uint32_t ok = 1;
             if (__lane_id() == 0) {
@@ -1145,7 +1146,7 @@ __global__ __launch_bounds__(256) void serve_tick_kernel(const Desc *__restrict_
             }
             if (!wave_uniform(ok)) ++stalls;
         }
-        const Desc D = dir[ti.item.table];
+        const Desc D = as_global(dir[ti.item.table]);
         if (ti.op == 0) {
             ins.add(ins_total, ti.item.table, serve_insert_item<GI>(D, ti.item, c, P, C, sink, tally));
         } else {
@@ -1328,10 +1329,11 @@ __global__ __launch_bounds__(256) void serve_loop_kernel(LoopArgs A, InsertPolic
             }
             break;
         }
+        it.item = as_global(it.item);
         const uint32_t table = it.item.table;
         // the descriptor can be read before the wait: a table is resized only while none of its
         // requests is in flight, and the host writes the directory before it publishes items
-        const Desc D = load_desc_coherent(A.dir + table);
+        const Desc D = as_global(load_desc_coherent(A.dir + table));
         uint32_t stalled = 0;
         if (it.need) {
             uint32_t back = 1, spins = 0;

@@ -45,6 +45,44 @@ __device__ inline uint32_t wave_slot()
     return __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave);
 }
 
+// A wave-uniform pointer as one the compiler knows to be in global memory. A pointer in a kernel
+// argument is taken to be global; one read from memory (a directory's descriptor, a chunk record,
+// a work item) is generic, and accesses through it become flat ones, which count on the LDS
+// counter too: the bucket loads of a group's tile then waited for the shuffles that hand out
+// their addresses, one after the other. The empty asm keeps the round trip through the global
+// address space from being folded away.
+template <typename T>
+__device__ inline T *as_global(T *p)
+{
+    auto q = (__attribute__((address_space(1))) T *)p;
+    asm("" : "+s"(q));
+    return (T *)q;
+}
+
+__device__ inline Desc as_global(Desc D)
+{
+#pragma unroll
+    for (int t = 0; t < kMaxSubtables; ++t) D.sub[t] = as_global(D.sub[t]);
+    return D;
+}
+
+__device__ inline WideDesc as_global(WideDesc W)
+{
+    W.D = as_global(W.D);
+#pragma unroll
+    for (int t = 0; t < kMaxSubtables; ++t) W.val[t] = as_global(W.val[t]);
+    return W;
+}
+
+__device__ inline ServeItem as_global(ServeItem x)
+{
+    x.keys = as_global(x.keys);
+    x.vals = as_global(x.vals);
+    x.out_vals = as_global(x.out_vals);
+    x.flags = as_global(x.flags);
+    return x;
+}
+
 // Add v (from one lane) to the tally `field` (a member of *C) in the stripe of wave slot `slot`.
 __device__ inline void tally_add(Counters *C, unsigned long long *field, unsigned long long v, uint32_t slot)
 {

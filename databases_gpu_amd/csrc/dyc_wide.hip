@@ -402,7 +402,7 @@ __global__ __launch_bounds__(256) void wide_group_probe_kernel(const WideDesc *_
          it < n_items; it += waves) {
         const GroupItem item = items[it];
         if (item.len == 0) continue;  // wave-uniform: an empty slot of a layout by XCD
-        const WideDesc W = dir[item.table];
+        const WideDesc W = as_global(dir[item.table]);
         WideStash st = stash;
         st.table = item.table;
         const uint64_t end = item.begin + item.len;
@@ -433,7 +433,7 @@ __global__ __launch_bounds__(256) void wide_group_insert_kernel(const WideDesc *
          it < n_items; it += waves) {
         const GroupItem item = items[it];
         if (item.len == 0) continue;  // wave-uniform: a block the bulk fill's rounds emptied
-        const WideDesc W = dir[item.table];
+        const WideDesc W = as_global(dir[item.table]);
         const uint64_t end = item.begin + item.len;
         uint64_t next = item.begin + __lane_id();
         unsigned long long rej = 0;
@@ -642,8 +642,8 @@ __device__ inline void wide_fill_chunk(const SubRef &S, uint32_t b0, uint32_t le
     __shared__ uint32_t wred[THREADS / kWave];
     __shared__ unsigned long long obase;
     __shared__ uint32_t onext;
-    uint64_t *const ksub = S.keys;
-    uint64_t *const vsub = S.vals;
+    uint64_t *const ksub = as_global(S.keys);
+    uint64_t *const vsub = as_global(S.vals);
     const uint4 *const ksrc = reinterpret_cast<const uint4 *>(ksub + (uint64_t)b0 * kSlots);
     constexpr uint32_t kParts = kChunkBuckets * kSlots / 2;  // 16-byte parts of a chunk's lines
     if constexpr (DENSE) {
