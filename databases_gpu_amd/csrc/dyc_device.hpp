@@ -86,7 +86,8 @@ __host__ __device__ inline uint32_t h5(uint32_t a)
 // masks anyway.
 __host__ __device__ inline uint32_t hash_t(uint32_t k, uint32_t t)
 {
-    const uint32_t a = h1(k), b = h2(k), c = h3(k), d = h4(k);
+    // h3 without its own reduction: the one below is the same
+    const uint32_t a = h1(k), b = h2(k), c = (k ^ 59064253u) + 72355969u, d = h4(k);
     const uint32_t u = t & 3u;
     const uint32_t x = u == 0 ? a : (u == 1 ? b : (u == 2 ? c : d));
     return x % kPrime;

@@ -624,7 +624,7 @@ int dyc_group_find(dyc_group *g, const uint32_t *keys, const uint64_t *offsets, 
                                           : upload_items(g, offsets, s, &n_items);
     if (rc) return rc;
     Pool sp;
-    HIP_TRY(launch_group_find(g->ddir, g->ditems, n_items, keys, vals, hit, (int)g->launch.find_lanes,
+    HIP_TRY(launch_group_find(g->ddir, g->ditems, n_items, keys, vals, hit,
                               (int)g->launch.find_blocks, s, g->stash(sp), (int)g->launch.find_waves_per_eu));
     return DYC_OK;
 }
@@ -643,7 +643,7 @@ int dyc_group_erase(dyc_group *g, const uint32_t *keys, const uint64_t *offsets,
     rc = zero_and_run_prologue(g, s);
     if (rc) return rc;
     Pool sp;
-    HIP_TRY(launch_group_erase(g->ddir, g->ditems, n_items, keys, deleted, g->tcounts, (int)g->launch.find_lanes,
+    HIP_TRY(launch_group_erase(g->ddir, g->ditems, n_items, keys, deleted, g->tcounts,
                                (int)g->launch.find_blocks, s, g->stash(sp), (int)g->launch.find_waves_per_eu));
     rc = read_back(g, s);
     if (rc) return rc;
@@ -697,7 +697,7 @@ int dyc_group_find_per_table(dyc_group *g, const uint32_t *keys, const uint64_t 
         if (!m) continue;
         Pool sp;
         HIP_TRY(launch_find(g->hdir[i], keys + offsets[i], vals ? vals + offsets[i] : nullptr,
-                            hit ? hit + offsets[i] : nullptr, m, (int)g->launch.find_lanes, sh, s, g->stash(sp), i));
+                            hit ? hit + offsets[i] : nullptr, m, sh, s, g->stash(sp), i));
     }
     return DYC_OK;
 }
@@ -893,8 +893,7 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
                                     (int)g->launch.insert_waves_per_eu);
         }
         if (k == hipSuccess)
-            k = launch_group_find(g->ddir, p->d_items + p->n_ins, p->n_find, lookups, vals_out, hit,
-                                  (int)g->launch.find_lanes, (int)g->launch.find_blocks, cs, &stash,
+            k = launch_group_find(g->ddir, p->d_items + p->n_ins, p->n_find, lookups, vals_out, hit, (int)g->launch.find_blocks, cs, &stash,
                                   (int)g->launch.find_waves_per_eu);
         if (k == hipSuccess)
             k = launch_copy(g->ctr, g->hctr, kCounterWords, g->tcounts, g->htcounts, g->n, cs);

@@ -1,16 +1,9 @@
 // dyc_kernels.hip -- gfx950 kernels of the DyCuckoo hot path.
 //
-// Wave64 mapping shared by find and erase ("probe" kernels):
-//   * a wave owns a tile of 64 consecutive keys; lane i loads key i (one coalesced 256 B read)
-//     and hashes it (pair, both subtables, both bucket addresses) -- no lane hashes twice;
-//   * the wave splits into 64/G groups of G lanes; group g probes keys g*G .. g*G+G-1 of the
-//     tile, each lane reading 128/G bytes of every bucket (G = 8: one dwordx4 per lane, so a
-//     group reads a whole 128-byte bucket in one coalesced line). All G pos1 probes of a group
-//     are issued before the first compare, so a lane keeps G bucket loads in flight;
-//   * a 64-bit __ballot per probe gives every group its match mask; the group's answer is
-//     broadcast to its lanes, and lane g*G+s keeps the answer of key g*G+s -- the lane that
-//     loaded that key -- so results are stored with one coalesced write per tile.
-// pos2 is read only for keys pos1 did not resolve, in the reference order (cuckoo.cu:482-497).
+// Wave64 mapping shared by find, erase and update ("probe" kernels): a wave owns a tile of 64
+// consecutive keys; lane i loads key i (one coalesced 256 B read) and hashes it, and each quad of
+// lanes reads its four keys' buckets (probe_tile). pos2 is read only for keys pos1 did not
+// resolve, in the reference order (cuckoo.cu:482-497).
 //
 // Insert: each group of G lanes carries one entry through the eviction chain with 64-bit CAS
 // on the victim slot. Groups are independent: a group that finishes takes its next key while
@@ -19,22 +12,12 @@
 #include "dyc_wave.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace dyc {
 
 namespace {
 
-
-// A bucket location packed in 32 bits: subtable in the top 3 bits, bucket index below (bucket
-// counts are capped at 2^29). Shuffling this instead of a 64-bit address halves the cross-lane
-// traffic, and rebuilding the pointer from the descriptor keeps the loads in the global
-// address space (a pointer rebuilt from a shuffled integer would become a flat access, whose
-// completion the compiler can only track together with the shuffles).
-__device__ inline uint32_t pack_loc(uint32_t t, uint32_t bucket) { return (t << 29) | bucket; }
-__device__ inline uint64_t *loc_ptr(const Desc &D, uint32_t l)
-{
-    return selt(l >> 29, D.sub) + (uint64_t)(l & 0x1fffffffu) * kSlots;
-}
 
 // Plain (non-atomic) read of SPL consecutive slots, 16-byte vector loads where possible.
 template <int SPL>
@@ -51,25 +34,6 @@ __device__ inline void load_slots(const uint64_t *p, uint64_t (&e)[SPL])
             e[j + 1] = ((uint64_t)v.w << 32) | v.z;
         }
     }
-}
-
-// Device-coherent read of SPL slots (agent-scope relaxed atomic loads, which skip lines another
-// XCD's writes may have left stale in this XCD's L2). For reads that must see exchanges made
-// earlier in the same launch by other waves.
-template <int SPL>
-__device__ inline void load_slots_coherent(const uint64_t *p, uint64_t (&e)[SPL])
-{
-#pragma unroll
-    for (int j = 0; j < SPL; ++j) e[j] = __hip_atomic_load(p + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-template <int SPL, bool COH>
-__device__ inline void read_slots(const uint64_t *p, uint64_t (&e)[SPL])
-{
-    if constexpr (COH)
-        load_slots_coherent<SPL>(p, e);
-    else
-        load_slots<SPL>(p, e);
 }
 
 // An input word (key or value). COH: read device-coherently, for a launch that outlives the
@@ -103,235 +67,222 @@ __device__ inline void publish_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "m
 
 
 // ---------------------------------------------------------------- find / erase / update
+// The probe tile: 64 keys a wave, four lanes a bucket (32 bytes each). Small probes are a chain of
+// latencies and probes of lines in the caches come near the rate at which the SIMDs issue, so the
+// tile is built to need few instructions:
+//   * each lane finds its own key's two bucket addresses once; the quad's lanes take them, and
+//     the key, by quad permutes (DPP), which ride on the instruction that uses the result, where a
+//     wider group needs an LDS permute with an address of its own;
+//   * hit masks are wave masks in scalar registers: which quads have resolved key kk, which lane
+//     answers, and the flags are scalar arithmetic;
+//   * the values of the quad's four keys are combined by an OR over the quad that leaves key kk's
+//     in lane kk (a matching lane holds the value, the others 0), nine instructions for all four.
+// Against the same probe with 8 lanes a bucket, LDS permutes and vector hit masks (1178 vector
+// instructions a tile, 411 here), a find of 2^10 keys takes 3.5 us (5.9), of 2^17 keys in a table
+// of 2^23 5.2 us (7.6), of 2^23 keys 252 us (258: bound by the rate of random lines, 54 G/s), and
+// with 16 lanes 8.9, 10.8 and 316 us; so every probe takes this tile, whatever lanes per key the
+// caller set.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+#define DYC_GLOBAL __attribute__((address_space(1)))
 
-// Erase and update write-back of one probe phase. Bit kk * SPL + j of mm says that this lane's slot
-// j of key kk's bucket slice holds key kk; each such slot is CAS'd from what was read to `rep` (0
-// for erase, the key with its new value for update). Returns bit kk set where one of this lane's
-// CASes on key kk succeeded. Up to kCasInFlight CASes are issued before any result is compared, so
-// a wave waits about once per phase instead of once per key of its groups; a lane with more matches
-// (a duplicated key, or several of its group's keys in its slice) takes the rest one at a time.
-constexpr int kCasInFlight = 3;
-
-template <int G, int SPL, bool UPDATE>
-__device__ inline void pick_match(const Desc &D, int b, const uint64_t (&e)[G][SPL], const uint32_t (&loc)[G],
-                                  const uint32_t (&key)[G], const uint32_t *nv, int s, uint64_t *&ptr,
-                                  uint64_t &exp, uint64_t &rep, uint32_t &kk_out)
+// x of lane KK of each quad, in all of its lanes.
+template <int KK>
+__device__ inline uint32_t quad_bcast(uint32_t x)
 {
-    const int kk = b / SPL, j = b % SPL;
-    uint64_t x = 0;
-    uint32_t l = 0, k = 0, v = 0;
-#pragma unroll
-    for (int q = 0; q < G; ++q) {
-        if (q == kk) {
-            l = loc[q];
-            k = key[q];
-            if constexpr (UPDATE) v = nv[q];
-        }
-#pragma unroll
-        for (int r = 0; r < SPL; ++r)
-            if (q * SPL + r == b) x = e[q][r];
-    }
-    ptr = loc_ptr(D, l) + s * SPL + j;
-    exp = x;
-    rep = UPDATE ? pack(k, v) : 0ull;
-    kk_out = (uint32_t)kk;
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, KK * 0x55, 0xf, 0xf, true);
+}
+// x of the quad lane whose number differs in bit 0 (XOR = 1) or bit 1 (XOR = 2).
+template <int XOR>
+__device__ inline uint32_t quad_swap(uint32_t x)
+{
+    static_assert(XOR == 1 || XOR == 2, "a quad permute");
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, XOR == 1 ? 0xb1 : 0x4e, 0xf, 0xf, true);
 }
 
-template <int G, int SPL, bool UPDATE>
-__device__ inline uint32_t write_matches(const Desc &D, uint32_t mm, const uint64_t (&e)[G][SPL],
-                                         const uint32_t (&loc)[G], const uint32_t (&key)[G], const uint32_t *nv,
-                                         int s)
+constexpr uint64_t kQuadLow = 0x1111111111111111ull;  // lane 0 of every quad
+// Every lane of each quad that has a lane in m.
+__device__ inline uint64_t quad_any(uint64_t m)
 {
-    uint64_t found[kCasInFlight];
-    int bit[kCasInFlight];  // the match each in-flight CAS serves (-1: none)
-#pragma unroll
-    for (int q = 0; q < kCasInFlight; ++q) {
-        found[q] = 0;
-        bit[q] = -1;
-        if (mm) {
-            bit[q] = __builtin_ctz(mm);
-            mm &= mm - 1u;
-            uint64_t *ptr, x, rep;
-            uint32_t kk;
-            pick_match<G, SPL, UPDATE>(D, bit[q], e, loc, key, nv, s, ptr, x, rep, kk);
-            found[q] = cas_old(ptr, x, rep);
-        }
-    }
-    // The compiler would otherwise turn found == expected into the CAS's own success flag and
-    // test it (waiting for the CAS) before the next one issues; an empty asm hides the relation.
-#pragma unroll
-    for (int q = 0; q < kCasInFlight; ++q) asm volatile("" : "+v"(found[q]));
-    uint32_t ok = 0;
-#pragma unroll
-    for (int q = 0; q < kCasInFlight; ++q) {
-        if (bit[q] < 0) continue;
-        uint64_t x = 0;  // the expected value, selected again rather than held across the wait
-#pragma unroll
-        for (int kk = 0; kk < G; ++kk)
-#pragma unroll
-            for (int j = 0; j < SPL; ++j)
-                if (kk * SPL + j == bit[q]) x = e[kk][j];
-        if (found[q] == x) ok |= 1u << (bit[q] / SPL);
-    }
-    while (mm) {
-        const int b = __builtin_ctz(mm);
-        mm &= mm - 1u;
-        uint64_t *ptr, x, rep;
-        uint32_t kk;
-        pick_match<G, SPL, UPDATE>(D, b, e, loc, key, nv, s, ptr, x, rep, kk);
-        if (cas_old(ptr, x, rep) == x) ok |= 1u << kk;
-    }
-    return ok;
+    m |= m >> 1;
+    m = (m | m >> 2) & kQuadLow;
+    return (m << 4) - m;
 }
+
+template <typename F>
+__device__ inline void each_of_quad(F f)
+{
+    f(std::integral_constant<int, 0>{});
+    f(std::integral_constant<int, 1>{});
+    f(std::integral_constant<int, 2>{});
+    f(std::integral_constant<int, 3>{});
+}
+
+// A lane's four slots (32 bytes) of a bucket. COH: read device-coherently (agent-scope relaxed
+// atomic loads, which skip lines another XCD's writes may have left stale in this XCD's L2), for
+// reads that must see exchanges made earlier in the same launch by other waves.
+struct QuadSlots {
+    u32x4 a, b;
+};
+template <bool COH>
+__device__ inline QuadSlots load_quad_slots(uint32_t lo, uint32_t hi)
+{
+    const uint64_t at = (uint64_t)hi << 32 | lo;
+    QuadSlots e;
+    if constexpr (COH) {
+        const DYC_GLOBAL uint64_t *p = (const DYC_GLOBAL uint64_t *)at;
+        uint64_t x[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = __hip_atomic_load(p + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        e.a = u32x4{(uint32_t)x[0], (uint32_t)(x[0] >> 32), (uint32_t)x[1], (uint32_t)(x[1] >> 32)};
+        e.b = u32x4{(uint32_t)x[2], (uint32_t)(x[2] >> 32), (uint32_t)x[3], (uint32_t)(x[3] >> 32)};
+    } else {
+        const DYC_GLOBAL u32x4 *p = (const DYC_GLOBAL u32x4 *)at;
+        e.a = p[0];
+        e.b = p[1];
+    }
+    return e;
+}
+__device__ inline bool slots_hold(const QuadSlots &e, uint32_t k)
+{
+    return (e.a.y == k) | (e.a.w == k) | (e.b.y == k) | (e.b.w == k);
+}
+// The value of the first of the lane's slots that holds k, or 0.
+__device__ inline uint32_t slots_value(const QuadSlots &e, uint32_t k)
+{
+    uint32_t v = e.b.w == k ? e.b.z : 0u;
+    v = e.b.y == k ? e.b.x : v;
+    v = e.a.w == k ? e.a.z : v;
+    return e.a.y == k ? e.a.x : v;
+}
+
+// Byte offset in the lane's part of the first of its slots that holds k (the last one if none).
+__device__ inline uint32_t slots_at(const QuadSlots &e, uint32_t k)
+{
+    uint32_t o = e.b.y == k ? 16u : 24u;
+    o = e.a.w == k ? 8u : o;
+    return e.a.y == k ? 0u : o;
+}
+// Whether two or more of the lane's slots hold k (copies of one key).
+__device__ inline bool slots_hold_two(const QuadSlots &e, uint32_t k)
+{
+    const bool a = e.a.y == k, b = e.a.w == k, c = e.b.y == k, d = e.b.w == k;
+    return (a & b) | (c & d) | ((a | b) & (c | d));
+}
+
 // One wave probes the 64 keys keys[base, base + 64) clipped to n, in table D. Returns this
 // lane's flag for its own key (hit, deleted or updated); all 64 lanes must call it together.
-// MODE 0 find: vals (optional) receives the value. MODE 1 erase: every copy of the key in the
-// first bucket (pos1, then pos2) that holds it is CAS'd to empty. MODE 2 update: those copies
-// are CAS'd to the new value vals[i] (an input). COH: read the buckets and the inputs
-// device-coherently and write the results with system-scope stores (load_slots_coherent,
-// load_in, store_out).
-template <int G, int MODE, bool COH = false>
-__device__ inline uint32_t probe_tile_m(const Desc &D, const uint32_t *__restrict__ keys, uint32_t *__restrict__ vals,
-                                        uint8_t *__restrict__ flags, uint64_t base, uint64_t n)
-{
-    constexpr bool ERASE = MODE != 0;  // erase and update both rewrite the matching slots
-    constexpr bool UPDATE = MODE == 2;
-    constexpr int SPL = kSlots / G;  // slots each lane reads per bucket
-    constexpr uint64_t GMASK = (G >= 64) ? ~0ull : ((1ull << G) - 1ull);
-    const int lane = __lane_id();
-    const int g = lane / G, s = lane % G;
-    {
-        const uint64_t i = base + lane;
-        const bool inb = i < n;
-        const uint32_t k = inb ? load_in<COH>(keys + i) : 0u;  // past the end: key 0, which is reserved
-        const uint32_t nv = (UPDATE && inb) ? load_in<COH>(vals + i) : 0u;
-        const uint32_t p = pair_of(D, k);
-        const uint32_t t1 = pos1(D, p), t2 = pos2(D, p);
-        const uint32_t loc1 = pack_loc(t1, bucket_of(D, k, t1));
-        const uint32_t loc2 = pack_loc(t2, bucket_of(D, k, t2));
-
-        uint64_t e[G][SPL];
-        uint32_t kk_key[G];
-        uint32_t kk_new[UPDATE ? G : 1];  // update: the new value of key kk
-        bool kk_valid[G];
-        uint32_t kk_loc[ERASE ? G : 1];  // erase writes back to the bucket it matched in
-        // phase 1: pos1 buckets of the group's G keys, all loads in flight together
-#pragma unroll
-        for (int kk = 0; kk < G; ++kk) {
-            const int src = g * G + kk;
-            kk_key[kk] = __shfl(k, src);
-            if constexpr (UPDATE) kk_new[kk] = __shfl(nv, src);
-            kk_valid[kk] = !reserved_key(kk_key[kk]);
-            const uint32_t l = __shfl(loc1, src);
-            if constexpr (ERASE) kk_loc[kk] = l;
-#pragma unroll
-            for (int j = 0; j < SPL; ++j) e[kk][j] = 0;
-            if (kk_valid[kk]) read_slots<SPL, COH>(loc_ptr(D, l) + s * SPL, e[kk]);
-        }
-
-        uint32_t my_val = 0, my_flag = 0;
-        uint32_t done = 0;  // bit kk: key kk resolved in pos1
-        uint32_t mm = 0;    // erase/update: this lane's matching slots (write_matches)
-#pragma unroll
-        for (int kk = 0; kk < G; ++kk) {
-            int first = -1;
-#pragma unroll
-            for (int j = SPL - 1; j >= 0; --j)
-                if (key_of(e[kk][j]) == kk_key[kk]) first = j;
-            const uint32_t gm = (uint32_t)((__ballot(first >= 0 && kk_valid[kk]) >> (g * G)) & GMASK);
-            if (gm) {
-                done |= 1u << kk;
-                if constexpr (ERASE) {
-#pragma unroll
-                    for (int j = 0; j < SPL; ++j)
-                        if (kk_valid[kk] && key_of(e[kk][j]) == kk_key[kk]) mm |= 1u << (kk * SPL + j);
-                } else {
-                    const int w = __builtin_ctz(gm);
-                    uint32_t v = 0;
-#pragma unroll
-                    for (int j = 0; j < SPL; ++j)
-                        if (j == first) v = val_of(e[kk][j]);
-                    v = __shfl(v, g * G + w);
-                    if (kk == s) {
-                        my_val = v;
-                        my_flag = 1;
-                    }
-                }
-            }
-        }
-
-        if constexpr (ERASE) {
-            const uint32_t ok = write_matches<G, SPL, UPDATE>(D, mm, e, kk_loc, kk_key, kk_new, s);
-#pragma unroll
-            for (int kk = 0; kk < G; ++kk) {
-                if (!(done & (1u << kk))) continue;  // group-uniform
-                const uint32_t okm = (uint32_t)((__ballot((ok >> kk) & 1u) >> (g * G)) & GMASK);
-                if (kk == s) my_flag = okm != 0;
-            }
-            mm = 0;
-        }
-
-        // phase 2: pos2 buckets of the keys pos1 did not resolve
-        [[maybe_unused]] uint32_t done2 = 0;  // erase/update: bit kk: key kk found in pos2
-#pragma unroll
-        for (int kk = 0; kk < G; ++kk) {
-            const uint32_t l = __shfl(loc2, g * G + kk);
-            if constexpr (ERASE) kk_loc[kk] = l;
-            if (kk_valid[kk] && !(done & (1u << kk))) read_slots<SPL, COH>(loc_ptr(D, l) + s * SPL, e[kk]);
-        }
-        // Straight-line over every key (a key pos1 resolved is masked out, not skipped), so the
-        // wait for the pos2 slots falls on every path before write_matches issues its CASes.
-#pragma unroll
-        for (int kk = 0; kk < G; ++kk) {
-            const bool todo = kk_valid[kk] && !(done & (1u << kk));
-            int first = -1;
-#pragma unroll
-            for (int j = SPL - 1; j >= 0; --j)
-                if (key_of(e[kk][j]) == kk_key[kk]) first = j;
-            const uint32_t gm = (uint32_t)((__ballot(first >= 0 && todo) >> (g * G)) & GMASK);
-            if constexpr (ERASE) {
-                done2 |= (gm != 0 ? 1u : 0u) << kk;
-#pragma unroll
-                for (int j = 0; j < SPL; ++j)
-                    mm |= (todo && key_of(e[kk][j]) == kk_key[kk] ? 1u : 0u) << (kk * SPL + j);
-            } else {
-                if (!gm) continue;
-                const int w = __builtin_ctz(gm);
-                uint32_t v = 0;
-#pragma unroll
-                for (int j = 0; j < SPL; ++j)
-                    if (j == first) v = val_of(e[kk][j]);
-                v = __shfl(v, g * G + w);
-                if (kk == s) {
-                    my_val = v;
-                    my_flag = 1;
-                }
-            }
-        }
-
-        if constexpr (ERASE) {
-            const uint32_t ok = write_matches<G, SPL, UPDATE>(D, mm, e, kk_loc, kk_key, kk_new, s);
-#pragma unroll
-            for (int kk = 0; kk < G; ++kk) {
-                if (!(done2 & (1u << kk))) continue;  // group-uniform
-                const uint32_t okm = (uint32_t)((__ballot((ok >> kk) & 1u) >> (g * G)) & GMASK);
-                if (kk == s) my_flag = okm != 0;
-            }
-        }
-
-        if (inb) {
-            if (!ERASE && vals) store_out<COH>(vals + i, my_val);
-            if (flags) store_out<COH>(flags + i, (uint8_t)my_flag);
-        }
-        return my_flag;
-    }
-}
-
-template <int G, bool ERASE, bool COH = false>
+// The first bucket (pos1, then pos2) that holds a key answers. MODE 0 find: vals (optional)
+// receives the value of its first matching slot. MODE 1 erase: every copy in that bucket is CAS'd
+// to empty, so one of two identical requests deletes a copy. MODE 2 update: those copies are
+// CAS'd to the new value vals[i] (an input). The bucket is known once both reads are back, so
+// erase and update issue the CASes of all four keys together, after them. COH: read the buckets
+// and the inputs device-coherently and write the results with system-scope stores
+// (load_quad_slots, load_in, store_out).
+template <int MODE, bool COH = false>
 __device__ inline uint32_t probe_tile(const Desc &D, const uint32_t *__restrict__ keys, uint32_t *__restrict__ vals,
                                       uint8_t *__restrict__ flags, uint64_t base, uint64_t n)
 {
-    return probe_tile_m<G, ERASE ? 1 : 0, COH>(D, keys, vals, flags, base, n);
+    constexpr bool UPDATE = MODE == 2;
+    const uint32_t lane = __lane_id(), s = lane & 3u;
+    const uint64_t i = base + lane;
+    const bool inb = i < n;
+    const uint32_t k = inb ? load_in<COH>(keys + i) : 0u;  // past the end: key 0, which is reserved
+    const uint32_t nv = (UPDATE && inb) ? load_in<COH>(vals + i) : 0u;
+    const uint32_t p = pair_of(D, k);
+    const uint64_t a1 = (uint64_t)bucket_ptr(D, k, pos1(D, p)), a2 = (uint64_t)bucket_ptr(D, k, pos2(D, p));
+    // reserved keys read the buckets their hash names like any other and are masked out here
+    const uint64_t valid = __ballot(inb && !reserved_key(k));
+    const uint32_t off = s * 32u;  // buckets are 128-byte aligned: the lane's part is an OR away
+    uint32_t key[4];
+    QuadSlots e[4];
+    each_of_quad([&](auto q) {
+        constexpr int kk = decltype(q)::value;
+        key[kk] = quad_bcast<kk>(k);
+        e[kk] = load_quad_slots<COH>(quad_bcast<kk>((uint32_t)a1) | off, quad_bcast<kk>((uint32_t)(a1 >> 32)));
+    });
+    uint64_t done[4];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) done[kk] = quad_any(__ballot(slots_hold(e[kk], key[kk])));
+    // pos2 of the keys pos1 did not resolve; the others keep what they matched
+    each_of_quad([&](auto q) {
+        constexpr int kk = decltype(q)::value;
+        const uint32_t lo = quad_bcast<kk>((uint32_t)a2) | off, hi = quad_bcast<kk>((uint32_t)(a2 >> 32));
+        if (!__builtin_amdgcn_inverse_ballot_w64(done[kk])) e[kk] = load_quad_slots<COH>(lo, hi);
+    });
+    uint32_t v[4];
+    uint64_t found = 0;
+    if constexpr (MODE == 0) {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            v[kk] = slots_value(e[kk], key[kk]);
+            const uint64_t m = __ballot(slots_hold(e[kk], key[kk]));
+            const uint64_t any = quad_any(m);
+            // copies of one key in slots of several lanes: the lowest lane answers (uniform, rare)
+            if (__popcll(m) * 4 != __popcll(any)) {
+                const uint64_t later = ((m << 1) & ~kQuadLow) | ((m << 2) & (kQuadLow * 0xc)) | ((m << 3) & (kQuadLow * 8));
+                if (__builtin_amdgcn_inverse_ballot_w64(later)) v[kk] = 0;
+            }
+            found |= any & (kQuadLow << kk);
+        }
+    } else {
+        uint64_t got[4];
+        uint64_t m[4];
+        each_of_quad([&](auto q) {
+            constexpr int kk = decltype(q)::value;
+            const bool first = __builtin_amdgcn_inverse_ballot_w64(done[kk]);
+            v[kk] = slots_value(e[kk], key[kk]);
+            const uint32_t lo1 = quad_bcast<kk>((uint32_t)a1), hi1 = quad_bcast<kk>((uint32_t)(a1 >> 32));
+            const uint32_t lo2 = quad_bcast<kk>((uint32_t)a2), hi2 = quad_bcast<kk>((uint32_t)(a2 >> 32));
+            const uint32_t new_v = UPDATE ? quad_bcast<kk>(nv) : 0u;
+            m[kk] = __ballot(slots_hold(e[kk], key[kk])) & ((((valid >> kk) & kQuadLow) << 4) - ((valid >> kk) & kQuadLow));
+            const uint64_t at = (uint64_t)(first ? hi1 : hi2) << 32 | ((first ? lo1 : lo2) | off | slots_at(e[kk], key[kk]));
+            got[kk] = 0;
+            if (__builtin_amdgcn_inverse_ballot_w64(m[kk]))
+                got[kk] = cas_old((DYC_GLOBAL uint64_t *)at, pack(key[kk], v[kk]), UPDATE ? pack(key[kk], new_v) : 0ull);
+        });
+        // The compiler would otherwise turn got == expected into the CAS's own success flag and
+        // test it (waiting for the CAS) before the next one issues; an empty asm hides the relation.
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) asm volatile("" : "+v"(got[kk]));
+        each_of_quad([&](auto q) {
+            constexpr int kk = decltype(q)::value;
+            uint64_t ok = __ballot(got[kk] == pack(key[kk], v[kk])) & m[kk];
+            // copies of one key in several of a lane's slots: the rest, one at a time (uniform, rare)
+            if (__ballot(slots_hold_two(e[kk], key[kk])) & m[kk]) {
+                const bool first = __builtin_amdgcn_inverse_ballot_w64(done[kk]);
+                const uint32_t lo1 = quad_bcast<kk>((uint32_t)a1), hi1 = quad_bcast<kk>((uint32_t)(a1 >> 32));
+                const uint32_t lo2 = quad_bcast<kk>((uint32_t)a2), hi2 = quad_bcast<kk>((uint32_t)(a2 >> 32));
+                const uint32_t new_v = UPDATE ? quad_bcast<kk>(nv) : 0u;
+                const uint64_t at = (uint64_t)(first ? hi1 : hi2) << 32 | ((first ? lo1 : lo2) | off);
+                const uint32_t sk[4] = {e[kk].a.y, e[kk].a.w, e[kk].b.y, e[kk].b.w};
+                const uint32_t sv[4] = {e[kk].a.x, e[kk].a.z, e[kk].b.x, e[kk].b.z};
+                bool more = false, seen = false;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (sk[j] != key[kk] || !__builtin_amdgcn_inverse_ballot_w64(m[kk])) continue;
+                    if (seen) {
+                        const uint64_t x = pack(sk[j], sv[j]);
+                        more |= cas_old((DYC_GLOBAL uint64_t *)(at + 8 * j), x, UPDATE ? pack(key[kk], new_v) : 0ull) == x;
+                    }
+                    seen = true;
+                }
+                ok |= __ballot(more);
+            }
+            found |= quad_any(ok) & (kQuadLow << kk);
+        });
+    }
+    found &= valid;
+    const bool hit = __builtin_amdgcn_inverse_ballot_w64(found);
+    if constexpr (MODE == 0) {
+        // OR over the quad, key kk's value in lane kk
+        const bool odd = s & 1u, high = s & 2u;
+        const uint32_t v01 = (odd ? v[1] : v[0]) | quad_swap<1>(odd ? v[0] : v[1]);
+        const uint32_t v23 = (odd ? v[3] : v[2]) | quad_swap<1>(odd ? v[2] : v[3]);
+        const uint32_t my = (high ? v23 : v01) | quad_swap<2>(high ? v01 : v23);
+        if (inb && vals) store_out<COH>(vals + i, hit ? my : 0u);
+    }
+    if (inb && flags) store_out<COH>(flags + i, (uint8_t)hit);
+    return hit;
 }
 
 template <int MODE, bool COH = false>
@@ -346,50 +297,24 @@ __device__ inline uint64_t pool_size(const Pool &pool)
     return pc < pool.cap ? pc : pool.cap;
 }
 
-// Waves per SIMD the find / erase kernels are held to (the occupancy their register use gives
-// with a four-subtable selection; the six-way one would otherwise cost a wave at G = 8). Erase
-// keeps up to three CASes per lane in flight (write_matches), which costs G = 4 its sixth wave.
-template <int G, bool ERASE>
-constexpr int probe_waves()
-{
-    return G == 4 ? (ERASE ? 5 : 7) : (G == 8 ? (ERASE ? 5 : 7) : (ERASE ? 4 : 5));
-}
-
 // Misses also look in the pool's entries of `table` (a serving table's overflow pool, a single
 // table's stash); an empty pool costs nothing.
-template <int G, bool ERASE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(probe_waves<G, ERASE>()))) void probe_kernel(Desc D, const uint32_t *__restrict__ keys,
+template <int MODE>
+__global__ __launch_bounds__(256) void probe_kernel(Desc D, const uint32_t *__restrict__ keys,
                                                     uint32_t *__restrict__ vals, uint8_t *__restrict__ flags,
                                                     uint64_t n, Counters *__restrict__ C, Pool pool, uint32_t table)
 {
     const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x / kWave);
     const uint64_t np = pool_size(pool);
-    unsigned long long ndel = 0;
+    unsigned long long nhit = 0;
     const uint32_t slot = wave_slot();
     for (uint64_t base = (uint64_t)slot * kWave; base < n; base += waves * kWave) {
-        uint32_t f = probe_tile<G, ERASE>(D, keys, vals, flags, base, n);
-        if (np) f |= pool_probe_at<ERASE ? 1 : 0>(pool, np, keys, vals, flags, n, table, base, f);
-        ndel += f;
+        uint32_t f = probe_tile<MODE>(D, keys, vals, flags, base, n);
+        if (np) f |= pool_probe_at<MODE>(pool, np, keys, vals, flags, n, table, base, f);
+        nhit += f;
     }
-    if constexpr (ERASE) wave_tally(C, &C->deleted, ndel, slot);
-}
-
-// Upsert's first pass: rewrite the value of keys already stored (probe_tile_m mode 2).
-template <int G>
-__global__ __launch_bounds__(256) void update_kernel(Desc D, const uint32_t *__restrict__ keys,
-                                                     uint32_t *__restrict__ vals, uint8_t *__restrict__ updated,
-                                                     uint64_t n, Counters *__restrict__ C, Pool pool)
-{
-    const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x / kWave);
-    const uint64_t np = pool_size(pool);
-    unsigned long long nu = 0;
-    const uint32_t slot = wave_slot();
-    for (uint64_t base = (uint64_t)slot * kWave; base < n; base += waves * kWave) {
-        uint32_t f = probe_tile_m<G, 2>(D, keys, vals, updated, base, n);
-        if (np) f |= pool_probe_at<2>(pool, np, keys, vals, updated, n, 0, base, f);
-        nu += f;
-    }
-    wave_tally(C, &C->updated, nu, slot);
+    if constexpr (MODE == 1) wave_tally(C, &C->deleted, nhit, slot);
+    if constexpr (MODE == 2) wave_tally(C, &C->updated, nhit, slot);
 }
 
 // ------------------------------------------------------------------------------- insert
@@ -892,7 +817,7 @@ __device__ inline uint32_t wave_uniform(uint32_t v) { return __builtin_amdgcn_re
 
 // W: the least waves per SIMD the compiler must leave room for (1: its own choice); the group
 // launches take it as an occupancy knob, chosen by measurement.
-template <int G, bool ERASE, int W>
+template <bool ERASE, int W>
 __global__ __launch_bounds__(256, W) void group_probe_kernel(const Desc *__restrict__ dir,
                                                           const GroupItem *__restrict__ items, uint32_t n_items,
                                                           const uint32_t *__restrict__ keys,
@@ -909,7 +834,7 @@ __global__ __launch_bounds__(256, W) void group_probe_kernel(const Desc *__restr
         const uint64_t end = item.begin + item.len;
         unsigned long long nd = 0;
         for (uint64_t base = item.begin; base < end; base += kWave) {
-            uint32_t f = probe_tile<G, ERASE>(D, keys, vals, flags, base, end);
+            uint32_t f = probe_tile<ERASE ? 1 : 0>(D, keys, vals, flags, base, end);
             if (np) f |= pool_probe_at<ERASE ? 1 : 0>(pool, np, keys, vals, flags, end, item.table, base, f);
             nd += f;
         }
@@ -1003,14 +928,14 @@ __device__ inline uint32_t pool_probe(const Pool &pool, uint64_t np, const Serve
 }
 
 // One item of finds or erases; returns this lane's count of hits (erase: deletions).
-template <int G, bool ERASE, bool COH = false>
+template <bool ERASE, bool COH = false>
 __device__ inline unsigned long long serve_probe_item(const Desc &D, const ServeItem &item, const Pool &pool,
                                                       uint64_t np)
 {
     unsigned long long nd = 0;
     for (uint64_t base = 0; base < item.len; base += kWave) {
-        uint32_t f = probe_tile<G, ERASE, COH>(D, item.keys, ERASE ? nullptr : item.out_vals, item.flags, base,
-                                               item.len);
+        uint32_t f = probe_tile<ERASE ? 1 : 0, COH>(D, item.keys, ERASE ? nullptr : item.out_vals, item.flags, base,
+                                                    item.len);
         if (np) f |= pool_probe<ERASE, COH>(pool, np, item, base, f);
         nd += f;
     }
@@ -1059,7 +984,7 @@ struct WaveTotal {
 };
 
 
-template <int G, bool ERASE>
+template <bool ERASE>
 __global__ __launch_bounds__(256) void serve_probe_kernel(const Desc *__restrict__ dir,
                                                           const ServeItem *__restrict__ items, uint32_t n_items,
                                                           Pool pool, unsigned long long *__restrict__ del_total)
@@ -1071,7 +996,7 @@ __global__ __launch_bounds__(256) void serve_probe_kernel(const Desc *__restrict
          it += waves) {
         const ServeItem item = as_global(items[it]);
         const Desc D = as_global(dir[item.table]);
-        unsigned long long nd = serve_probe_item<G, ERASE>(D, item, pool, np);
+        unsigned long long nd = serve_probe_item<ERASE>(D, item, pool, np);
         if constexpr (ERASE) del.add(del_total, item.table, wave_sum(nd));
     }
     if constexpr (ERASE) del.flush(del_total);
@@ -1109,7 +1034,7 @@ __global__ __launch_bounds__(256) void serve_insert_kernel(const Desc *__restric
 // running waves, so the earliest unfinished item never waits and the launch always drains. The
 // wait is bounded all the same: past spin_cap polls the wave records a stall and goes on (the
 // host reports the tick failed).
-template <int GI, int GF>
+template <int GI>
 __global__ __launch_bounds__(256) void serve_tick_kernel(const Desc *__restrict__ dir, const TickItem *__restrict__ items,
                                                          uint32_t n_items, unsigned long long *__restrict__ cursor,
                                                          TickStages stages, InsertPolicy P, Counters *__restrict__ C,
@@ -1155,11 +1080,11 @@ __global__ __launch_bounds__(256) void serve_tick_kernel(const Desc *__restrict_
             unsigned long long nd;
             const uint64_t np = pool_size(pool);
             if (ti.op == 1)
-                nd = ti.wait ? serve_probe_item<GF, false, true>(D, ti.item, pool, np)
-                             : serve_probe_item<GF, false, false>(D, ti.item, pool, np);
+                nd = ti.wait ? serve_probe_item<false, true>(D, ti.item, pool, np)
+                             : serve_probe_item<false, false>(D, ti.item, pool, np);
             else
-                nd = ti.wait ? serve_probe_item<GF, true, true>(D, ti.item, pool, np)
-                             : serve_probe_item<GF, true, false>(D, ti.item, pool, np);
+                nd = ti.wait ? serve_probe_item<true, true>(D, ti.item, pool, np)
+                             : serve_probe_item<true, false>(D, ti.item, pool, np);
             if (ti.op == 2) del.add(del_total, ti.item.table, wave_sum(nd));
         }
         if (__lane_id() == 0) {
@@ -1276,7 +1201,7 @@ __device__ inline void loop_front(const LoopArgs &A)
     if (__lane_id() == 0) __hip_atomic_store(A.words + kLoopQuit, 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int GI, int GF>
+template <int GI>
 __global__ __launch_bounds__(256) void serve_loop_kernel(LoopArgs A, InsertPolicy P, Counters *__restrict__ C,
                                                          PendSink sink, Pool pool,
                                                          unsigned long long *__restrict__ ins_total,
@@ -1353,9 +1278,9 @@ __global__ __launch_bounds__(256) void serve_loop_kernel(LoopArgs A, InsertPolic
         } else {
             const uint64_t np = pool_size(pool);
             if (it.op == 1) {
-                acc = wave_sum(serve_probe_item<GF, false, true>(D, it.item, pool, np));
+                acc = wave_sum(serve_probe_item<false, true>(D, it.item, pool, np));
             } else {
-                acc = wave_sum(serve_probe_item<GF, true, true>(D, it.item, pool, np));
+                acc = wave_sum(serve_probe_item<true, true>(D, it.item, pool, np));
                 del.add(del_total, table, acc);
             }
         }
@@ -1466,31 +1391,23 @@ inline uint64_t insert_default_cap(uint64_t work_waves, LaunchShape sh)
 
 }  // namespace
 
-hipError_t launch_find(const Desc &D, const uint32_t *keys, uint32_t *vals, uint8_t *hit, uint64_t n, int lanes,
-                       LaunchShape sh, hipStream_t st, const Pool *pool, uint32_t table)
+hipError_t launch_find(const Desc &D, const uint32_t *keys, uint32_t *vals, uint8_t *hit, uint64_t n, LaunchShape sh,
+                       hipStream_t st, const Pool *pool, uint32_t table)
 {
     if (n == 0) return hipSuccess;
     const int grid = grid_for((n + kWave - 1) / kWave, sh);
     const Pool p = pool ? *pool : Pool{};
-    switch (lanes) {
-    case 4: probe_kernel<4, false><<<grid, sh.block_threads, 0, st>>>(D, keys, vals, hit, n, nullptr, p, table); break;
-    case 16: probe_kernel<16, false><<<grid, sh.block_threads, 0, st>>>(D, keys, vals, hit, n, nullptr, p, table); break;
-    default: probe_kernel<8, false><<<grid, sh.block_threads, 0, st>>>(D, keys, vals, hit, n, nullptr, p, table); break;
-    }
+    probe_kernel<0><<<grid, sh.block_threads, 0, st>>>(D, keys, vals, hit, n, nullptr, p, table);
     return hipGetLastError();
 }
 
-hipError_t launch_erase(const Desc &D, const uint32_t *keys, uint8_t *deleted, uint64_t n, int lanes, LaunchShape sh,
+hipError_t launch_erase(const Desc &D, const uint32_t *keys, uint8_t *deleted, uint64_t n, LaunchShape sh,
                         Counters *C, hipStream_t st, const Pool *pool, uint32_t table)
 {
     if (n == 0) return hipSuccess;
     const int grid = grid_for((n + kWave - 1) / kWave, sh);
     const Pool p = pool ? *pool : Pool{};
-    switch (lanes) {
-    case 4: probe_kernel<4, true><<<grid, sh.block_threads, 0, st>>>(D, keys, nullptr, deleted, n, C, p, table); break;
-    case 16: probe_kernel<16, true><<<grid, sh.block_threads, 0, st>>>(D, keys, nullptr, deleted, n, C, p, table); break;
-    default: probe_kernel<8, true><<<grid, sh.block_threads, 0, st>>>(D, keys, nullptr, deleted, n, C, p, table); break;
-    }
+    probe_kernel<1><<<grid, sh.block_threads, 0, st>>>(D, keys, nullptr, deleted, n, C, p, table);
     return hipGetLastError();
 }
 
@@ -1537,17 +1454,13 @@ hipError_t launch_insert(const Desc &D, const uint32_t *keys, const uint32_t *va
 }
 
 hipError_t launch_update(const Desc &D, const uint32_t *keys, const uint32_t *vals, uint8_t *updated, uint64_t n,
-                         int lanes, LaunchShape sh, Counters *C, hipStream_t st, const Pool *pool)
+                         LaunchShape sh, Counters *C, hipStream_t st, const Pool *pool)
 {
     if (n == 0) return hipSuccess;
     const int grid = grid_for((n + kWave - 1) / kWave, sh);
     uint32_t *v = const_cast<uint32_t *>(vals);  // read-only in update mode
     const Pool p = pool ? *pool : Pool{};
-    switch (lanes) {
-    case 4: update_kernel<4><<<grid, sh.block_threads, 0, st>>>(D, keys, v, updated, n, C, p); break;
-    case 16: update_kernel<16><<<grid, sh.block_threads, 0, st>>>(D, keys, v, updated, n, C, p); break;
-    default: update_kernel<8><<<grid, sh.block_threads, 0, st>>>(D, keys, v, updated, n, C, p); break;
-    }
+    probe_kernel<2><<<grid, sh.block_threads, 0, st>>>(D, keys, v, updated, n, C, p, 0);
     return hipGetLastError();
 }
 
@@ -1593,57 +1506,43 @@ hipError_t launch_downsize(const uint64_t *old, uint32_t new_nb, uint64_t *dst, 
 
 constexpr int kGroupDefaultBlocks = 2048;  // 8192 waves: 256 CUs x 32 resident waves
 
-template <int G, bool ERASE>
+template <bool ERASE>
 static void group_probe_w(int wpe, int grid, hipStream_t st, const Desc *dir, const GroupItem *items, uint32_t n_items,
                           const uint32_t *keys, uint32_t *vals, uint8_t *flags, unsigned long long *table_counts,
                           const Pool &p)
 {
     switch (wpe) {
     case 6:
-        group_probe_kernel<G, ERASE, 6><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, flags, table_counts, p);
+        group_probe_kernel<ERASE, 6><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, flags, table_counts, p);
         break;
     case 8:
-        group_probe_kernel<G, ERASE, 8><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, flags, table_counts, p);
+        group_probe_kernel<ERASE, 8><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, flags, table_counts, p);
         break;
     default:
-        group_probe_kernel<G, ERASE, 1><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, flags, table_counts, p);
+        group_probe_kernel<ERASE, 1><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, flags, table_counts, p);
         break;
     }
 }
 
 hipError_t launch_group_find(const Desc *dir, const GroupItem *items, uint32_t n_items, const uint32_t *keys,
-                             uint32_t *vals, uint8_t *hit, int lanes, int blocks, hipStream_t st, const Pool *pool,
+                             uint32_t *vals, uint8_t *hit, int blocks, hipStream_t st, const Pool *pool,
                              int waves_per_eu)
 {
     const Pool p = pool ? *pool : Pool{};
     if (n_items == 0) return hipSuccess;
     const int grid = blocks > 0 ? blocks : std::min<int>(kGroupDefaultBlocks, (int)((n_items + 3) / 4));
-    switch (lanes) {
-    case 4: group_probe_w<4, false>(waves_per_eu, grid, st, dir, items, n_items, keys, vals, hit, nullptr, p); break;
-    case 16: group_probe_w<16, false>(waves_per_eu, grid, st, dir, items, n_items, keys, vals, hit, nullptr, p); break;
-    default: group_probe_w<8, false>(waves_per_eu, grid, st, dir, items, n_items, keys, vals, hit, nullptr, p); break;
-    }
+    group_probe_w<false>(waves_per_eu, grid, st, dir, items, n_items, keys, vals, hit, nullptr, p);
     return hipGetLastError();
 }
 
 hipError_t launch_group_erase(const Desc *dir, const GroupItem *items, uint32_t n_items, const uint32_t *keys,
-                              uint8_t *deleted, unsigned long long *table_counts, int lanes, int blocks,
+                              uint8_t *deleted, unsigned long long *table_counts, int blocks,
                               hipStream_t st, const Pool *pool, int waves_per_eu)
 {
     const Pool p = pool ? *pool : Pool{};
     if (n_items == 0) return hipSuccess;
     const int grid = blocks > 0 ? blocks : std::min<int>(kGroupDefaultBlocks, (int)((n_items + 3) / 4));
-    switch (lanes) {
-    case 4:
-        group_probe_w<4, true>(waves_per_eu, grid, st, dir, items, n_items, keys, nullptr, deleted, table_counts, p);
-        break;
-    case 16:
-        group_probe_w<16, true>(waves_per_eu, grid, st, dir, items, n_items, keys, nullptr, deleted, table_counts, p);
-        break;
-    default:
-        group_probe_w<8, true>(waves_per_eu, grid, st, dir, items, n_items, keys, nullptr, deleted, table_counts, p);
-        break;
-    }
+    group_probe_w<true>(waves_per_eu, grid, st, dir, items, n_items, keys, nullptr, deleted, table_counts, p);
     return hipGetLastError();
 }
 
@@ -1707,29 +1606,21 @@ static int serve_grid(uint32_t n_items, int blocks)
     return blocks > 0 ? blocks : std::min<int>(kGroupDefaultBlocks, (int)((n_items + 3) / 4));
 }
 
-hipError_t launch_serve_find(const Desc *dir, const ServeItem *items, uint32_t n_items, Pool pool, int lanes,
-                             int blocks, hipStream_t st)
+hipError_t launch_serve_find(const Desc *dir, const ServeItem *items, uint32_t n_items, Pool pool, int blocks,
+                             hipStream_t st)
 {
     if (n_items == 0) return hipSuccess;
     const int grid = serve_grid(n_items, blocks);
-    switch (lanes) {
-    case 4: serve_probe_kernel<4, false><<<grid, 256, 0, st>>>(dir, items, n_items, pool, nullptr); break;
-    case 16: serve_probe_kernel<16, false><<<grid, 256, 0, st>>>(dir, items, n_items, pool, nullptr); break;
-    default: serve_probe_kernel<8, false><<<grid, 256, 0, st>>>(dir, items, n_items, pool, nullptr); break;
-    }
+    serve_probe_kernel<false><<<grid, 256, 0, st>>>(dir, items, n_items, pool, nullptr);
     return hipGetLastError();
 }
 
 hipError_t launch_serve_erase(const Desc *dir, const ServeItem *items, uint32_t n_items, Pool pool,
-                              unsigned long long *del_total, int lanes, int blocks, hipStream_t st)
+                              unsigned long long *del_total, int blocks, hipStream_t st)
 {
     if (n_items == 0) return hipSuccess;
     const int grid = serve_grid(n_items, blocks);
-    switch (lanes) {
-    case 4: serve_probe_kernel<4, true><<<grid, 256, 0, st>>>(dir, items, n_items, pool, del_total); break;
-    case 16: serve_probe_kernel<16, true><<<grid, 256, 0, st>>>(dir, items, n_items, pool, del_total); break;
-    default: serve_probe_kernel<8, true><<<grid, 256, 0, st>>>(dir, items, n_items, pool, del_total); break;
-    }
+    serve_probe_kernel<true><<<grid, 256, 0, st>>>(dir, items, n_items, pool, del_total);
     return hipGetLastError();
 }
 
@@ -1744,30 +1635,6 @@ hipError_t launch_serve_insert(const Desc *dir, const ServeItem *items, uint32_t
     case 8: serve_insert_kernel<8><<<grid, 256, 0, st>>>(dir, items, n_items, pol, C, sink, ins_total); break;
     case 16: serve_insert_kernel<16><<<grid, 256, 0, st>>>(dir, items, n_items, pol, C, sink, ins_total); break;
     default: serve_insert_kernel<1><<<grid, 256, 0, st>>>(dir, items, n_items, pol, C, sink, ins_total); break;
-    }
-    return hipGetLastError();
-}
-
-template <int GI>
-static hipError_t tick_by_find_lanes(int grid, int find_lanes, const Desc *dir, const TickItem *items,
-                                     uint32_t n_items, unsigned long long *cursor, TickStages done,
-                                     InsertPolicy pol, Counters *C, PendSink sink, Pool pool,
-                                     unsigned long long *ins_total, unsigned long long *del_total, uint32_t spin_cap,
-                                     uint32_t max_back, hipStream_t st)
-{
-    switch (find_lanes) {
-    case 4:
-        serve_tick_kernel<GI, 4><<<grid, 256, 0, st>>>(dir, items, n_items, cursor, done, pol, C, sink, pool, ins_total,
-                                                       del_total, spin_cap, max_back);
-        break;
-    case 16:
-        serve_tick_kernel<GI, 16><<<grid, 256, 0, st>>>(dir, items, n_items, cursor, done, pol, C, sink, pool, ins_total,
-                                                        del_total, spin_cap, max_back);
-        break;
-    default:
-        serve_tick_kernel<GI, 8><<<grid, 256, 0, st>>>(dir, items, n_items, cursor, done, pol, C, sink, pool, ins_total,
-                                                       del_total, spin_cap, max_back);
-        break;
     }
     return hipGetLastError();
 }
@@ -1789,26 +1656,17 @@ hipError_t launch_serve_tick(const Desc *dir, const TickItem *items, uint32_t n_
     const int grid = serve_grid(n_items, blocks);
     switch (insert_lanes) {
     case 2:
-        return tick_by_find_lanes<2>(grid, find_lanes, dir, items, n_items, cursor, done, pol, C, sink, pool, ins_total,
-                                     del_total, spin_cap, max_back, st);
+        serve_tick_kernel<2><<<grid, 256, 0, st>>>(dir, items, n_items, cursor, done, pol, C, sink, pool, ins_total,
+                                                   del_total, spin_cap, max_back);
+        break;
     case 4:
-        return tick_by_find_lanes<4>(grid, find_lanes, dir, items, n_items, cursor, done, pol, C, sink, pool, ins_total,
-                                     del_total, spin_cap, max_back, st);
+        serve_tick_kernel<4><<<grid, 256, 0, st>>>(dir, items, n_items, cursor, done, pol, C, sink, pool, ins_total,
+                                                   del_total, spin_cap, max_back);
+        break;
     default:
-        return tick_by_find_lanes<1>(grid, find_lanes, dir, items, n_items, cursor, done, pol, C, sink, pool, ins_total,
-                                     del_total, spin_cap, max_back, st);
-    }
-}
-
-template <int GI>
-static hipError_t loop_by_find_lanes(int grid, int find_lanes, const LoopArgs &A, InsertPolicy pol, Counters *C,
-                                     PendSink sink, Pool pool, unsigned long long *ins_total,
-                                     unsigned long long *del_total, hipStream_t st)
-{
-    switch (find_lanes) {
-    case 4: serve_loop_kernel<GI, 4><<<grid, 256, 0, st>>>(A, pol, C, sink, pool, ins_total, del_total); break;
-    case 16: serve_loop_kernel<GI, 16><<<grid, 256, 0, st>>>(A, pol, C, sink, pool, ins_total, del_total); break;
-    default: serve_loop_kernel<GI, 8><<<grid, 256, 0, st>>>(A, pol, C, sink, pool, ins_total, del_total); break;
+        serve_tick_kernel<1><<<grid, 256, 0, st>>>(dir, items, n_items, cursor, done, pol, C, sink, pool, ins_total,
+                                                   del_total, spin_cap, max_back);
+        break;
     }
     return hipGetLastError();
 }
@@ -1819,10 +1677,11 @@ hipError_t launch_serve_loop(const LoopArgs &A, InsertPolicy pol, int insert_lan
 {
     if (!serve_tick_supported(insert_lanes, find_lanes) || blocks < 2) return hipErrorInvalidValue;
     switch (insert_lanes) {
-    case 2: return loop_by_find_lanes<2>(blocks, find_lanes, A, pol, C, sink, pool, ins_total, del_total, st);
-    case 4: return loop_by_find_lanes<4>(blocks, find_lanes, A, pol, C, sink, pool, ins_total, del_total, st);
-    default: return loop_by_find_lanes<1>(blocks, find_lanes, A, pol, C, sink, pool, ins_total, del_total, st);
+    case 2: serve_loop_kernel<2><<<blocks, 256, 0, st>>>(A, pol, C, sink, pool, ins_total, del_total); break;
+    case 4: serve_loop_kernel<4><<<blocks, 256, 0, st>>>(A, pol, C, sink, pool, ins_total, del_total); break;
+    default: serve_loop_kernel<1><<<blocks, 256, 0, st>>>(A, pol, C, sink, pool, ins_total, del_total); break;
     }
+    return hipGetLastError();
 }
 
 hipError_t launch_loop_reset(unsigned long long *words, hipStream_t st)
@@ -1831,25 +1690,15 @@ hipError_t launch_loop_reset(unsigned long long *words, hipStream_t st)
     return hipGetLastError();
 }
 
-template <int GI, int GF>
+template <int GI>
 static int loop_blocks_per_cu()
 {
     int per = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, serve_loop_kernel<GI, GF>, 256, 0) != hipSuccess) {
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, serve_loop_kernel<GI>, 256, 0) != hipSuccess) {
         (void)hipGetLastError();
         return 0;
     }
     return per;
-}
-
-template <int GI>
-static int loop_blocks_by_find_lanes(int find_lanes)
-{
-    switch (find_lanes) {
-    case 4: return loop_blocks_per_cu<GI, 4>();
-    case 16: return loop_blocks_per_cu<GI, 16>();
-    default: return loop_blocks_per_cu<GI, 8>();
-    }
 }
 
 int serve_loop_capacity(int insert_lanes, int find_lanes)
@@ -1862,9 +1711,9 @@ int serve_loop_capacity(int insert_lanes, int find_lanes)
     }
     int per = 0;
     switch (insert_lanes) {
-    case 2: per = loop_blocks_by_find_lanes<2>(find_lanes); break;
-    case 4: per = loop_blocks_by_find_lanes<4>(find_lanes); break;
-    default: per = loop_blocks_by_find_lanes<1>(find_lanes); break;
+    case 2: per = loop_blocks_per_cu<2>(); break;
+    case 4: per = loop_blocks_per_cu<4>(); break;
+    default: per = loop_blocks_per_cu<1>(); break;
     }
     return per * cus;
 }

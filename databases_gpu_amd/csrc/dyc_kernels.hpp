@@ -78,12 +78,11 @@ struct InsertPolicy {
 };
 
 struct Pool;
-// find: vals/hit may be null. lanes in {4, 8, 16}. pool (optional): misses also look in the
-// pool's entries of `table`.
-hipError_t launch_find(const Desc &D, const uint32_t *keys, uint32_t *vals, uint8_t *hit, uint64_t n, int lanes,
-                       LaunchShape sh, hipStream_t st, const Pool *pool = nullptr, uint32_t table = 0);
+// find: vals/hit may be null. pool (optional): misses also look in the pool's entries of `table`.
+hipError_t launch_find(const Desc &D, const uint32_t *keys, uint32_t *vals, uint8_t *hit, uint64_t n, LaunchShape sh,
+                       hipStream_t st, const Pool *pool = nullptr, uint32_t table = 0);
 // erase: deleted may be null; counts into C->deleted.
-hipError_t launch_erase(const Desc &D, const uint32_t *keys, uint8_t *deleted, uint64_t n, int lanes, LaunchShape sh,
+hipError_t launch_erase(const Desc &D, const uint32_t *keys, uint8_t *deleted, uint64_t n, LaunchShape sh,
                         Counters *C, hipStream_t st, const Pool *pool = nullptr, uint32_t table = 0);
 // insert keys/vals (start rule of cuckoo.cu:336-341) or packed entries with a fixed previous
 // table `pre` (kNoTable = use the key-parity start rule).
@@ -95,7 +94,7 @@ hipError_t launch_insert(const Desc &D, const uint32_t *keys, const uint32_t *va
 // takes the value vals[i] (with a pool: failing that, every copy in the pool); updated[i] = 1 if
 // there was one; the count goes to C->updated.
 hipError_t launch_update(const Desc &D, const uint32_t *keys, const uint32_t *vals, uint8_t *updated, uint64_t n,
-                         int lanes, LaunchShape sh, Counters *C, hipStream_t st, const Pool *pool = nullptr);
+                         LaunchShape sh, Counters *C, hipStream_t st, const Pool *pool = nullptr);
 // A zero entry is an empty place (an erased pending entry, a slot without a residual): skipped,
 // and counted neither as rejected nor as placed. live (optional, a slot-addressed residual list's
 // tile flags from launch_downsize): entries of a tile whose byte is 0 are empty and not read.
@@ -175,10 +174,10 @@ struct GroupItem {
 // waves_per_eu: 6 or 8 builds the kernel for at least that many waves per SIMD (fewer
 // registers); anything else leaves the register budget to the compiler.
 hipError_t launch_group_find(const Desc *dir, const GroupItem *items, uint32_t n_items, const uint32_t *keys,
-                             uint32_t *vals, uint8_t *hit, int lanes, int blocks, hipStream_t st,
+                             uint32_t *vals, uint8_t *hit, int blocks, hipStream_t st,
                              const Pool *pool = nullptr, int waves_per_eu = 0);
 hipError_t launch_group_erase(const Desc *dir, const GroupItem *items, uint32_t n_items, const uint32_t *keys,
-                              uint8_t *deleted, unsigned long long *table_counts, int lanes, int blocks,
+                              uint8_t *deleted, unsigned long long *table_counts, int blocks,
                               hipStream_t st, const Pool *pool = nullptr, int waves_per_eu = 0);
 // insert: failures go to sink.pend with their table index in sink.tags; per-table inserted
 // counts (placed or pended, reserved keys excluded) are added to table_counts.
@@ -314,10 +313,10 @@ hipError_t launch_serve_tick(const Desc *dir, const TickItem *items, uint32_t n_
                              unsigned long long *del_total, uint32_t spin_cap, uint32_t max_back, hipStream_t st);
 hipError_t launch_serve_insert(const Desc *dir, const ServeItem *items, uint32_t n_items, InsertPolicy pol, int lanes,
                                int blocks, Counters *C, PendSink sink, unsigned long long *ins_total, hipStream_t st);
-hipError_t launch_serve_find(const Desc *dir, const ServeItem *items, uint32_t n_items, Pool pool, int lanes,
-                             int blocks, hipStream_t st);
+hipError_t launch_serve_find(const Desc *dir, const ServeItem *items, uint32_t n_items, Pool pool, int blocks,
+                             hipStream_t st);
 hipError_t launch_serve_erase(const Desc *dir, const ServeItem *items, uint32_t n_items, Pool pool,
-                              unsigned long long *del_total, int lanes, int blocks, hipStream_t st);
+                              unsigned long long *del_total, int blocks, hipStream_t st);
 
 // ---- device-resident serving loop
 // One launch that keeps running and takes work items from a ring in host memory as the host

@@ -686,10 +686,10 @@ int build_tick(dyc_server *s, bool *launched, bool *stuck)
             HIP_TRY(launch_insert(T.D, q.keys, q.vals, q.n, (int)s->cfg.insert_lanes, s->policy(), s->insert_shape(),
                                   s->pc(), s->sink(q.table, true), s->st));
         else if (q.op == DYC_OP_FIND)
-            HIP_TRY(launch_find(T.D, q.keys, q.out_vals, q.out_flags, q.n, (int)s->cfg.find_lanes, s->shape(), s->st,
+            HIP_TRY(launch_find(T.D, q.keys, q.out_vals, q.out_flags, q.n, s->shape(), s->st,
                                 &pool, q.table));
         else
-            HIP_TRY(launch_erase(T.D, q.keys, q.out_flags, q.n, (int)s->cfg.find_lanes, s->shape(), s->pc(), s->st,
+            HIP_TRY(launch_erase(T.D, q.keys, q.out_flags, q.n, s->shape(), s->pc(), s->st,
                                  &pool, q.table));
         s->ss.rounds += 1;
         return finish_launch(s, k, launched);
@@ -776,10 +776,9 @@ int build_tick(dyc_server *s, bool *launched, bool *stuck)
             HIP_TRY(launch_serve_insert(s->d_dir, items + at, (uint32_t)ni, s->policy(), (int)s->cfg.insert_lanes, 0,
                                         s->pc(), s->sink(0), s->ins_total(), s->st));
             at += ni;
-            HIP_TRY(launch_serve_find(s->d_dir, items + at, (uint32_t)nf, s->pool(), (int)s->cfg.find_lanes, 0, s->st));
+            HIP_TRY(launch_serve_find(s->d_dir, items + at, (uint32_t)nf, s->pool(), 0, s->st));
             at += nf;
-            HIP_TRY(launch_serve_erase(s->d_dir, items + at, (uint32_t)ne, s->pool(), s->del_total(),
-                                       (int)s->cfg.find_lanes, 0, s->st));
+            HIP_TRY(launch_serve_erase(s->d_dir, items + at, (uint32_t)ne, s->pool(), s->del_total(), 0, s->st));
             at += ne;
         }
     }
@@ -871,14 +870,14 @@ int run_sync(dyc_server *s, uint64_t tk)
     } else if (r.op == DYC_OP_FIND) {
         // a find changes nothing: launch, wait, done
         const Pool pool = s->pool();
-        HIP_TRY(launch_find(T.D, r.keys, r.out_vals, r.out_flags, r.n, (int)s->cfg.find_lanes, s->shape(), s->st,
+        HIP_TRY(launch_find(T.D, r.keys, r.out_vals, r.out_flags, r.n, s->shape(), s->st,
                             &pool, r.table));
         HIP_TRY(hipStreamSynchronize(s->st));
         finish(s, tk, status);
         return DYC_OK;
     } else {
         const Pool pool = s->pool();
-        HIP_TRY(launch_erase(T.D, r.keys, r.out_flags, r.n, (int)s->cfg.find_lanes, s->shape(), s->pc(), s->st,
+        HIP_TRY(launch_erase(T.D, r.keys, r.out_flags, r.n, s->shape(), s->pc(), s->st,
                              &pool, r.table));
     }
     int rc = read_stats_sync(s, snap);

@@ -1287,7 +1287,7 @@ int dyc_upsert(dyc_table *t, const uint32_t *keys, const uint32_t *vals, uint64_
     rc = zero_counters(t, s);
     if (rc) return rc;
     Pool sp;
-    HIP_TRY(launch_update(t->D, keys, vals, flags, n, (int)t->cfg.find_lanes, t->shape(), t->ctr, s, stash_of(t, sp)));
+    HIP_TRY(launch_update(t->D, keys, vals, flags, n, t->shape(), t->ctr, s, stash_of(t, sp)));
     HIP_TRY(launch_insert(t->D, keys, vals, n, (int)t->cfg.insert_lanes, t->policy(), t->insert_shape(), t->ctr,
                           sink_at(t, t->pend_n), s, flags));
     rc = read_counters(t, s);
@@ -1309,7 +1309,7 @@ int dyc_find(dyc_table *t, const uint32_t *keys, uint32_t *vals, uint8_t *hit, u
     DeviceGuard dg(t->device);
     SETTLE(t);
     Pool sp;
-    HIP_TRY(launch_find(t->D, keys, vals, hit, n, (int)t->cfg.find_lanes, t->shape(), (hipStream_t)stream,
+    HIP_TRY(launch_find(t->D, keys, vals, hit, n, t->shape(), (hipStream_t)stream,
                         stash_of(t, sp)));
     return DYC_OK;
 }
@@ -1325,7 +1325,7 @@ int dyc_erase(dyc_table *t, const uint32_t *keys, uint8_t *deleted, uint64_t n, 
     int rc = zero_counters(t, s);
     if (rc) return rc;
     Pool sp;
-    HIP_TRY(launch_erase(t->D, keys, deleted, n, (int)t->cfg.find_lanes, t->shape(), t->ctr, s, stash_of(t, sp)));
+    HIP_TRY(launch_erase(t->D, keys, deleted, n, t->shape(), t->ctr, s, stash_of(t, sp)));
     rc = read_counters(t, s);
     if (rc) return rc;
     t->count -= std::min<uint64_t>(t->count, t->hctr->deleted);
@@ -1588,11 +1588,10 @@ int probe_host(dyc_table *t, const uint32_t *keys, uint32_t *vals, uint8_t *flag
         HIP_TRY(hipStreamWaitEvent(s, S->in_ready[b], 0));
         Pool sp;
         if (erase)
-            HIP_TRY(launch_erase(t->D, S->dk[b], flags ? S->df[b] : nullptr, m, (int)t->cfg.find_lanes, t->shape(),
+            HIP_TRY(launch_erase(t->D, S->dk[b], flags ? S->df[b] : nullptr, m, t->shape(),
                                  t->ctr, s, stash_of(t, sp)));
         else
-            HIP_TRY(launch_find(t->D, S->dk[b], vals ? S->dv[b] : nullptr, flags ? S->df[b] : nullptr, m,
-                                (int)t->cfg.find_lanes, t->shape(), s, stash_of(t, sp)));
+            HIP_TRY(launch_find(t->D, S->dk[b], vals ? S->dv[b] : nullptr, flags ? S->df[b] : nullptr, m, t->shape(), s, stash_of(t, sp)));
         HIP_TRY(hipEventRecord(S->done[b], s));
         HIP_TRY(hipStreamWaitEvent(S->d2h, S->done[b], 0));
         if (vals && !erase) HIP_TRY(hipMemcpyAsync(S->hv[b], S->dv[b], m * 4, hipMemcpyDeviceToHost, S->d2h));

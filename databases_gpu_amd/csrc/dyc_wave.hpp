@@ -25,7 +25,8 @@ __device__ inline bool cas_slot(uint64_t *p, uint64_t &expected, uint64_t desire
 
 // 64-bit compare-and-swap at agent scope that returns the value it found (== expected on
 // success). Nothing waits for the result until the caller compares it, so several can be in flight.
-__device__ inline uint64_t cas_old(uint64_t *p, uint64_t expected, uint64_t desired)
+template <typename Ptr>
+__device__ inline uint64_t cas_old(Ptr p, uint64_t expected, uint64_t desired)
 {
     __hip_atomic_compare_exchange_strong(p, &expected, desired, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT);
