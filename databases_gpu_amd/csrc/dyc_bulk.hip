@@ -13,13 +13,16 @@
 //   4. fill: one workgroup per chunk owns its buckets for the launch. It takes the buckets'
 //      free-slot masks into LDS, counts the entries per bucket, reserves one range of the
 //      overflow list for the chunk's excess, then gives each entry the next free slot of its
-//      bucket (an LDS counter) or appends it to the overflow list. A dense round fills a copy
-//      of the chunk in LDS and writes it back whole; a sparse one stores each entry directly;
-//   5. the overflow is packed again for the key's other table (round 2) and filled the same way;
-//   6. what still overflows goes through the eviction insert (launch_insert_entries).
-// The placement rules that define a key's buckets are unchanged; only the order in which free
-// slots are taken differs, and the slot layout after a parallel insert is not deterministic
-// anyway. A placement by fill counts as one exchange in the kick tally.
+//      bucket (an LDS counter) or appends it to the overflow list, in a copy of the chunk in LDS
+//      that it writes back whole;
+//   5. the overflow goes to the other bucket of its pair by the eviction insert
+//      (launch_insert_overflow), which finds a free slot there for about half of it. A second
+//      round of partition and fill for that half saved its atomics and cost more than they do
+//      (2^28 keys: 850 + 1020 us for the round and its rest, 1495 us without it).
+// Each stage's work is known on the device, so the whole insert is one launch sequence with one
+// wait at its end. The placement rules that define a key's buckets are unchanged; only the order
+// in which free slots are taken differs, and the slot layout after a parallel insert is not
+// deterministic anyway. A placement by fill counts as one exchange in the kick tally.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <string.h>
@@ -33,24 +36,22 @@ namespace dyc {
 namespace {
 
 // Chunk ids of the batch in input order, and each block's counts of digit P (the partition's
-// first pass). Round 1 (IN_ENTRIES false): keys, target = fill_target (pos1, the bucket a find
-// reads first, for as many keys as equal subtable shares allow); reserved keys go to chunk 0 and
-// are rejected by its fill. Round 2 (IN_ENTRIES true): overflow entries, target = the other
-// bucket of the pair.
-template <bool IN_ENTRIES, typename CidT>
+// first pass). A key's target is its fill_target bucket (pos1, the bucket a find reads first, for
+// as many keys as equal subtable shares allow); reserved keys go to chunk 0 and are rejected by
+// its fill.
+template <typename CidT>
 __global__ __launch_bounds__(kCountThreads) void bulk_pack_kernel(Desc D, Chunks Ch, const uint32_t *__restrict__ keys,
-                                                                  const uint64_t *__restrict__ in, PartGrid G,
-                                                                  RadixPass P, CidT *__restrict__ cid,
+                                                                  PartGrid G, RadixPass P, CidT *__restrict__ cid,
                                                                   uint32_t *__restrict__ partial)
 {
     __shared__ uint32_t h[kMaxRadix];
     // per subtable: buckets, FastDiv multiplier and shifts, first chunk -- one LDS read per key
     // in place of a selection chain over the descriptor's arrays for each of them
     __shared__ uint4 sub_tab[kMaxSubtables];
-    __shared__ uint32_t tsel[32];  // the round's subtable by key parity and pair (fill_round_sub)
+    __shared__ uint32_t tsel[32];  // the target subtable by key parity and pair (fill_sub)
     const uint32_t R = 1u << P.bits;
     for (uint32_t d = threadIdx.x; d < R; d += kCountThreads) h[d] = 0;
-    if (threadIdx.x < 32) tsel[threadIdx.x] = fill_round_sub(D, threadIdx.x, IN_ENTRIES);
+    if (threadIdx.x < 32) tsel[threadIdx.x] = fill_sub(D, threadIdx.x);
     if (threadIdx.x < kMaxSubtables) {
         const uint32_t t = threadIdx.x;
         sub_tab[t] = make_uint4(selt(t, D.nb), selt(t, D.m), selt(t, D.sh), chunk_base(Ch, t));
@@ -63,17 +64,14 @@ __global__ __launch_bounds__(kCountThreads) void bulk_pack_kernel(Desc D, Chunks
 #pragma unroll
         for (int u = 0; u < kCountItems; ++u) {
             const uint64_t i = i0 + (uint64_t)u * kCountThreads;
-            if (i < hi) {
-                if constexpr (IN_ENTRIES) k[u] = key_of(in[i]);
-                else k[u] = keys[i];
-            }
+            if (i < hi) k[u] = keys[i];
         }
 #pragma unroll
         for (int u = 0; u < kCountItems; ++u) {
             const uint64_t i = i0 + (uint64_t)u * kCountThreads;
             if (i >= hi) continue;
             uint32_t c = 0;
-            if (IN_ENTRIES || !reserved_key(k[u])) {
+            if (!reserved_key(k[u])) {
                 const uint32_t p = pair_of(D, k[u]);
                 const uint32_t t = tsel[((k[u] & 1u) << 4) | p];
                 const uint4 q = sub_tab[t];
@@ -88,25 +86,21 @@ __global__ __launch_bounds__(kCountThreads) void bulk_pack_kernel(Desc D, Chunks
 }
 
 // One workgroup per chunk. Buckets of the chunk are written only by this workgroup during the
-// launch (every entry of the chunk targets one of them), so slots are taken with LDS counters.
-// DENSE (a round with at least two entries per bucket): the chunk's 512 buckets are copied into
-// LDS, filled there and written back whole, so every global access is a coalesced 16-byte
-// load or store. Otherwise the entries are counted first, the free-slot masks of the buckets
-// that received any are read coalesced (8 lanes per bucket, folded by ballot), and each placed
-// entry is one store into its slot.
+// launch (every entry of the chunk targets one of them), so slots are taken with LDS counters. The
+// chunk's 512 buckets are copied into LDS, filled there and written back whole, so every global
+// access is a coalesced 16-byte load or store.
 // The fill of one chunk by the whole workgroup: buckets [b0, b0 + len) of subtable S,
 // entries ent[lo, hi) (every one targets S). Entries that do not fit are appended to
 // ovf[0, ovf_cap) at the index *ovf_n hands out (one atomic for the chunk's whole excess).
 // Placements and rejected reserved keys are added to this lane's `placed` and `rejected`.
 // Every thread of the workgroup calls it with the same arguments.
-template <bool DENSE, int THREADS>
+template <int THREADS>
 __device__ inline void fill_chunk(const SubRef &S, uint32_t b0, uint32_t len,
                                   const uint64_t *__restrict__ ent, uint32_t lo, uint32_t hi,
                                   uint64_t *__restrict__ ovf, uint64_t ovf_cap, unsigned long long *__restrict__ ovf_n,
                                   bool zeroed, unsigned long long &placed, unsigned long long &rejected)
 {
-    constexpr uint32_t kImg = DENSE ? kChunkBuckets * kSlots : 2;
-    __shared__ uint64_t img[kImg];           // DENSE: the chunk's buckets
+    __shared__ uint64_t img[kChunkBuckets * kSlots];  // the chunk's buckets
     __shared__ uint32_t fm[kChunkBuckets];   // free-slot mask of each bucket
     __shared__ uint32_t cnt[kChunkBuckets];  // entries per bucket, then slots taken
     __shared__ uint32_t wred[THREADS / kWave];
@@ -115,7 +109,7 @@ __device__ inline void fill_chunk(const SubRef &S, uint32_t b0, uint32_t len,
     uint64_t *const sub = as_global(S.keys);
     const uint4 *const src = reinterpret_cast<const uint4 *>(sub + (uint64_t)b0 * kSlots);
     constexpr uint32_t kParts = kChunkBuckets * kSlots / 2;  // 16-byte parts of the chunk
-    if constexpr (DENSE) {
+    {
         uint4 *const im = reinterpret_cast<uint4 *>(img);
         if (zeroed) {
             // every slot of the table is known to be zero (the caller's host state says so):
@@ -151,8 +145,6 @@ __device__ inline void fill_chunk(const SubRef &S, uint32_t b0, uint32_t len,
                 }
             }
         }
-    } else {
-        for (uint32_t j = threadIdx.x; j < kChunkBuckets; j += blockDim.x) cnt[j] = 0;
     }
     if (threadIdx.x == 0) onext = 0;
     __syncthreads();
@@ -162,7 +154,7 @@ __device__ inline void fill_chunk(const SubRef &S, uint32_t b0, uint32_t len,
     // most kHold batches per thread keeps them in registers for the placement, so each entry
     // is read from memory once.
     constexpr uint32_t kBatch = 8;
-    constexpr uint32_t kHold = DENSE && THREADS < 1024 ? 2 : 1;  // about 8K entries of a dense chunk
+    constexpr uint32_t kHold = THREADS < 1024 ? 2 : 1;  // about 8K entries of a chunk
     const bool held = hi - lo <= kHold * kBatch * THREADS;  // block-uniform
     uint64_t hb[kHold][kBatch];
     // held entries also keep their place from the count: the bucket (9 bits) and the rank
@@ -218,34 +210,6 @@ __device__ inline void fill_chunk(const SubRef &S, uint32_t b0, uint32_t len,
         }
     }
     __syncthreads();
-    if constexpr (!DENSE) {
-        // free masks of the buckets that received entries only (a bucket's 8 parts are read
-        // by 8 consecutive lanes and folded by ballot; the others read as full)
-        // lane l of a wave reads part l % 8 of bucket (q / 8); a bucket's 8 parts sit in 8
-        // consecutive lanes, whose two ballot bits per part make its 16-bit mask
-        constexpr uint32_t kPer = kParts / THREADS;  // parts per thread, all loaded before use
-        uint4 v[kPer];
-#pragma unroll
-        for (uint32_t u = 0; u < kPer; ++u) {
-            const uint32_t q = threadIdx.x + u * THREADS;
-            v[u] = q < len * (kSlots / 2) && cnt[q / 8] ? src[q] : make_uint4(1u, 1u, 1u, 1u);
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < kPer; ++u) {
-            const uint32_t q = threadIdx.x + u * THREADS;
-            const bool e0 = (v[u].x | v[u].y) == 0u, e1 = (v[u].z | v[u].w) == 0u;
-            const uint64_t m0 = __ballot(e0), m1 = __ballot(e1);
-            const uint32_t lane = __lane_id();
-            if ((lane & 7u) == 0) {
-                const uint32_t a = (uint32_t)(m0 >> lane) & 0xffu, b = (uint32_t)(m1 >> lane) & 0xffu;
-                uint32_t m = 0;
-#pragma unroll
-                for (int p = 0; p < 8; ++p) m |= (((a >> p) & 1u) << (2 * p)) | (((b >> p) & 1u) << (2 * p + 1));
-                fm[q / 8] = m;
-            }
-        }
-        __syncthreads();
-    }
     uint32_t excess = stray;
     for (uint32_t j = threadIdx.x; j < kChunkBuckets; j += blockDim.x) {
         const uint32_t f = (uint32_t)__builtin_popcount(fm[j]);
@@ -287,8 +251,7 @@ __device__ inline void fill_chunk(const SubRef &S, uint32_t b0, uint32_t len,
                 const uint32_t m = fm[j];
                 if (r < (uint32_t)__builtin_popcount(m)) {
                     const uint32_t slot = nth_set_bit16(m, r);
-                    if constexpr (DENSE) img[j * kSlots + slot] = e;
-                    else sub[(uint64_t)b * kSlots + slot] = e;
+                    img[j * kSlots + slot] = e;
                     fits = true;
                     ++placed;
                 }
@@ -312,8 +275,7 @@ __device__ inline void fill_chunk(const SubRef &S, uint32_t b0, uint32_t len,
                     const uint32_t m = fm[j];
                     if (r < (uint32_t)__builtin_popcount(m)) {
                         const uint32_t slot = nth_set_bit16(m, r);
-                        if constexpr (DENSE) img[j * kSlots + slot] = hb[h][u];
-                        else sub[(uint64_t)(b0 + j) * kSlots + slot] = hb[h][u];
+                        img[j * kSlots + slot] = hb[h][u];
                         ++placed;
                         continue;
                     }
@@ -328,21 +290,18 @@ __device__ inline void fill_chunk(const SubRef &S, uint32_t b0, uint32_t len,
             place_batch(i0, eb);
         }
     }
-    if constexpr (DENSE) {
-        __syncthreads();
-        uint4 *const dst = reinterpret_cast<uint4 *>(sub + (uint64_t)b0 * kSlots);
-        const uint4 *const im = reinterpret_cast<const uint4 *>(img);
-        for (uint32_t q = threadIdx.x; q < len * (kSlots / 2); q += blockDim.x) dst[q] = im[q];
-    }
+    __syncthreads();
+    uint4 *const dst = reinterpret_cast<uint4 *>(sub + (uint64_t)b0 * kSlots);
+    const uint4 *const im = reinterpret_cast<const uint4 *>(img);
+    for (uint32_t q = threadIdx.x; q < len * (kSlots / 2); q += blockDim.x) dst[q] = im[q];
 }
 
 // One workgroup per chunk of one table (chunks numbered subtable by subtable, Ch); the entries
 // of chunk c are ent[start[c], start[c + 1]).
-template <bool DENSE, int THREADS>
+template <int THREADS>
 __global__ __launch_bounds__(THREADS) void bulk_fill_kernel(Desc D, Chunks Ch, const uint32_t *__restrict__ start,
                                                         const uint64_t *__restrict__ ent, uint64_t n,
                                                         uint64_t *__restrict__ ovf, uint64_t ovf_cap,
-                                                        unsigned long long *__restrict__ ovf_n,
                                                         Counters *__restrict__ C, bool zeroed)
 {
     const uint32_t c = blockIdx.x;
@@ -356,8 +315,7 @@ __global__ __launch_bounds__(THREADS) void bulk_fill_kernel(Desc D, Chunks Ch, c
             if (Ch.base[q] <= c) t = q;
         const uint32_t b0 = (c - chunk_base(Ch, t)) << kChunkShift;
         const uint32_t len = min(kChunkBuckets, selt(t, D.nb) - b0);
-        fill_chunk<DENSE, THREADS>(sub_ref(D, t), b0, len, ent, lo, hi, ovf, ovf_cap, ovf_n, zeroed, placed,
-                                   rejected);
+        fill_chunk<THREADS>(sub_ref(D, t), b0, len, ent, lo, hi, ovf, ovf_cap, &C->overflow, zeroed, placed, rejected);
     }
     wave_tally(C, &C->kicks, placed);
     wave_tally(C, &C->rejected, rejected);
@@ -387,39 +345,32 @@ constexpr int kBulkSortThreads = 256;
 constexpr uint32_t kBulkSortTile = kBulkSortThreads * kSortItems;
 
 template <typename CidT>
-hipError_t bulk_partition(const Desc &D, const Chunks &Ch, const uint32_t *keys, const uint32_t *vals, int in,
-                          uint64_t n, const BulkSpace &ws, uint32_t max_blocks, hipStream_t st, int *out)
+hipError_t bulk_partition(const Desc &D, const Chunks &Ch, const uint32_t *keys, const uint32_t *vals, uint64_t n,
+                          const BulkSpace &ws, uint32_t max_blocks, hipStream_t st, int *out)
 {
     RadixPass P[kMaxRadixPasses];
     const uint32_t np = radix_passes(Ch.bits, P);
     const PartGrid G = part_grid(n, max_blocks, kBulkSortTile);
     CidT *const cid[2] = {static_cast<CidT *>(ws.cid[0]), static_cast<CidT *>(ws.cid[1])};
     uint64_t *const ent[2] = {static_cast<uint64_t *>(ws.ent[0]), static_cast<uint64_t *>(ws.ent[1])};
-    if (keys) {
-        bulk_pack_kernel<false, CidT><<<G.blocks * G.sub, kCountThreads, 0, st>>>(D, Ch, keys, nullptr, G, P[0], cid[0],
-                                                                          ws.partial);
-        return partition_passes<uint64_t, KeyValSource, CidT, kBulkSortThreads>(
-            KeyValSource{keys, vals}, 0, ent, cid, G, P, np, ws.partial, ws.total, ws.start, Ch.total, st, out);
-    }
-    bulk_pack_kernel<true, CidT><<<G.blocks * G.sub, kCountThreads, 0, st>>>(D, Ch, nullptr, ent[in], G, P[0], cid[0],
-                                                                     ws.partial);
-    return partition_passes<uint64_t, EntrySource<uint64_t>, CidT, kBulkSortThreads>(
-        EntrySource<uint64_t>{ent[in]}, 1 - in, ent, cid, G, P, np, ws.partial, ws.total, ws.start, Ch.total, st, out);
+    bulk_pack_kernel<CidT><<<G.blocks * G.sub, kCountThreads, 0, st>>>(D, Ch, keys, G, P[0], cid[0], ws.partial);
+    return partition_passes<uint64_t, KeyValSource, CidT, kBulkSortThreads>(
+        KeyValSource{keys, vals}, 0, ent, cid, G, P, np, ws.partial, ws.total, ws.start, Ch.total, st, out);
 }
 
 }  // namespace
 
 size_t bulk_cid_bytes(const Chunks &Ch) { return Ch.total <= 65536u ? 2 : 4; }
 
-hipError_t launch_bulk_partition(const Desc &D, const Chunks &Ch, const uint32_t *keys, const uint32_t *vals, int in,
+hipError_t launch_bulk_partition(const Desc &D, const Chunks &Ch, const uint32_t *keys, const uint32_t *vals,
                                  uint64_t n, const BulkSpace &ws, uint32_t max_blocks, hipStream_t st, int *out)
 {
-    *out = keys ? 0 : 1 - in;
+    *out = 0;
     if (n == 0) return hipSuccess;
     if (n >= (1ull << 32) || Ch.total == 0 || Ch.bits > kMaxRadixPasses * kMaxRadixBits) return hipErrorInvalidValue;
     if (bulk_cid_bytes(Ch) == 2)
-        return bulk_partition<uint16_t>(D, Ch, keys, vals, in, n, ws, max_blocks, st, out);
-    return bulk_partition<uint32_t>(D, Ch, keys, vals, in, n, ws, max_blocks, st, out);
+        return bulk_partition<uint16_t>(D, Ch, keys, vals, n, ws, max_blocks, st, out);
+    return bulk_partition<uint32_t>(D, Ch, keys, vals, n, ws, max_blocks, st, out);
 }
 
 // ------------------------------------------------------------------------------ many tables
@@ -431,27 +382,20 @@ namespace {
 
 __device__ inline uint32_t sub_chunks(uint32_t nb) { return (nb + kChunkBuckets - 1) >> kChunkShift; }
 
-template <bool IN_ENTRIES>
 __global__ __launch_bounds__(kCountThreads) void group_bulk_pack_kernel(const Desc *__restrict__ dir,
                                                                         const GroupItem *__restrict__ blocks,
                                                                         const uint32_t *__restrict__ keys,
-                                                                        const uint64_t *__restrict__ in,
                                                                         uint8_t *__restrict__ lcid,
                                                                         uint32_t *__restrict__ partial)
 {
     __shared__ uint32_t h[kGroupBulkChunks];
     // per subtable: buckets, FastDiv multiplier and shifts, the table's first local chunk of it
     __shared__ uint4 sub_tab[kMaxSubtables];
-    __shared__ uint32_t tsel[32];  // the round's subtable by key parity and pair (fill_round_sub)
+    __shared__ uint32_t tsel[32];  // the target subtable by key parity and pair (fill_sub)
     const GroupItem item = blocks[blockIdx.x];
-    if (item.len == 0) {  // block-uniform: a clipped block of round 2 counts nothing
-        for (uint32_t d = threadIdx.x; d < kGroupBulkChunks; d += kCountThreads)
-            partial[(uint64_t)blockIdx.x * kGroupBulkChunks + d] = 0;
-        return;
-    }
     const Desc D = dir[item.table];  // by value: loaded once, not per use through memory
     for (uint32_t d = threadIdx.x; d < kGroupBulkChunks; d += kCountThreads) h[d] = 0;
-    if (threadIdx.x < 32) tsel[threadIdx.x] = fill_round_sub(D, threadIdx.x, IN_ENTRIES);
+    if (threadIdx.x < 32) tsel[threadIdx.x] = fill_sub(D, threadIdx.x);
     if (threadIdx.x < kMaxSubtables) {
         const uint32_t t = threadIdx.x;
         uint32_t first = 0;
@@ -465,15 +409,14 @@ __global__ __launch_bounds__(kCountThreads) void group_bulk_pack_kernel(const De
 #pragma unroll
         for (int u = 0; u < kCountItems; ++u) {
             const uint64_t i = i0 + (uint64_t)u * kCountThreads;
-            if constexpr (IN_ENTRIES) k[u] = i < hi ? key_of(in[i]) : 0u;
-            else k[u] = i < hi ? keys[i] : 0u;
+            k[u] = i < hi ? keys[i] : 0u;
         }
 #pragma unroll
         for (int u = 0; u < kCountItems; ++u) {
             const uint64_t i = i0 + (uint64_t)u * kCountThreads;
             if (i >= hi) continue;
             uint32_t lc = 0;
-            if (IN_ENTRIES || !reserved_key(k[u])) {
+            if (!reserved_key(k[u])) {
                 const uint32_t p = pair_of(D, k[u]);
                 const uint32_t t = tsel[((k[u] & 1u) << 4) | p];
                 const uint4 q = sub_tab[t];
@@ -537,7 +480,7 @@ __global__ __launch_bounds__(kGroupBulkChunks) void group_bulk_scan_kernel(const
     }
 }
 
-template <bool DENSE, int THREADS>
+template <int THREADS>
 __global__ __launch_bounds__(THREADS) void group_bulk_fill_kernel(const GroupChunk *__restrict__ chunks,
                                                                   const uint64_t *__restrict__ ent,
                                                                   uint64_t *__restrict__ ovf,
@@ -548,55 +491,56 @@ __global__ __launch_bounds__(THREADS) void group_bulk_fill_kernel(const GroupChu
     const GroupChunk R = chunks[blockIdx.x];
     unsigned long long placed = 0, rejected = 0;
     if (R.cnt)  // block-uniform
-        fill_chunk<DENSE, THREADS>(R.S, R.b0, R.len, ent, R.lo, R.lo + R.cnt, ovf + R.ovf_off, R.ovf_cap, ovf_n + R.j,
-                                   zeroed, placed, rejected);
+        fill_chunk<THREADS>(R.S, R.b0, R.len, ent, R.lo, R.lo + R.cnt, ovf + R.ovf_off, R.ovf_cap, ovf_n + R.j, zeroed,
+                            placed, rejected);
     const unsigned long long wp = wave_sum(placed);
     if (__lane_id() == 0 && wp) atomicAdd(&table_counts[R.table], wp);
     wave_tally(C, &C->kicks, placed);
     wave_tally(C, &C->rejected, rejected);
 }
 
-__global__ __launch_bounds__(256) void group_bulk_clip_kernel(const GroupItem *__restrict__ blocks,
-                                                              const uint32_t *__restrict__ btab, uint32_t n_blocks,
-                                                              const BulkTable *__restrict__ tabs, uint32_t n_tabs,
-                                                              const unsigned long long *__restrict__ ovf_n,
-                                                              GroupItem *__restrict__ out, BulkTable *__restrict__ tabs_out)
+// One thread per table; a workgroup reserves its tables' items with one atomic.
+__global__ __launch_bounds__(256) void group_bulk_items_kernel(const BulkTable *__restrict__ tabs, uint32_t n_tabs,
+                                                               const unsigned long long *__restrict__ ovf_n,
+                                                               GroupItem *__restrict__ items, uint64_t cap,
+                                                               unsigned long long *__restrict__ n_items)
 {
+    __shared__ uint32_t tmp[kScanWaves];
+    __shared__ unsigned long long first;
     const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x < n_blocks) {
-        const GroupItem b = blocks[x];
-        const uint32_t j = btab[x];
-        const uint64_t lim = tabs[j].off + min(ovf_n[j], (unsigned long long)tabs[j].n);
-        const uint64_t len = b.begin < lim ? min((uint64_t)b.len, lim - b.begin) : 0ull;
-        out[x] = GroupItem{b.begin, (uint32_t)len, b.table};
+    BulkTable T{};
+    uint32_t m = 0;
+    if (x < n_tabs) {
+        T = tabs[x];
+        m = (uint32_t)min(ovf_n[x], (unsigned long long)T.n);
     }
-    if (tabs_out && x < n_tabs) {
-        BulkTable T = tabs[x];
-        T.n = (uint32_t)min(ovf_n[x], (unsigned long long)T.n);
-        tabs_out[x] = T;
+    const uint32_t k = (m + kOverflowItem - 1) / kOverflowItem;
+    uint32_t all;
+    const uint32_t before = block_exclusive_scan(k, tmp, &all);
+    if (threadIdx.x == 0) first = all ? atomicAdd(n_items, (unsigned long long)all) : 0ull;
+    __syncthreads();
+    for (uint32_t j = 0; j < k; ++j) {
+        const uint64_t at = first + before + j;
+        if (at < cap)
+            items[at] = GroupItem{T.off + (uint64_t)j * kOverflowItem, min(kOverflowItem, m - j * kOverflowItem), T.table};
     }
 }
 
 }  // namespace
 
-hipError_t launch_group_bulk_clip(const GroupItem *blocks, const uint32_t *btab, uint32_t n_blocks,
-                                  const BulkTable *tabs, uint32_t n_tabs, const unsigned long long *ovf_n,
-                                  GroupItem *out, BulkTable *tabs_out, hipStream_t st)
+hipError_t launch_group_bulk_items(const BulkTable *tabs, uint32_t n_tabs, const unsigned long long *ovf_n,
+                                   GroupItem *items, uint64_t cap, unsigned long long *n_items, hipStream_t st)
 {
-    const uint32_t n = std::max(n_blocks, tabs_out ? n_tabs : 0u);
-    if (n == 0) return hipSuccess;
-    group_bulk_clip_kernel<<<(n + 255) / 256, 256, 0, st>>>(blocks, btab, n_blocks, tabs, n_tabs, ovf_n, out, tabs_out);
+    if (n_tabs == 0) return hipSuccess;
+    group_bulk_items_kernel<<<(n_tabs + 255) / 256, 256, 0, st>>>(tabs, n_tabs, ovf_n, items, cap, n_items);
     return hipGetLastError();
 }
 
 hipError_t launch_group_bulk_pack(const Desc *dir, const GroupItem *blocks, uint32_t n_blocks, const uint32_t *keys,
-                                  const uint64_t *entries, uint8_t *lcid, uint32_t *partial, hipStream_t st)
+                                  uint8_t *lcid, uint32_t *partial, hipStream_t st)
 {
     if (n_blocks == 0) return hipSuccess;
-    if (entries)
-        group_bulk_pack_kernel<true><<<n_blocks, kCountThreads, 0, st>>>(dir, blocks, nullptr, entries, lcid, partial);
-    else
-        group_bulk_pack_kernel<false><<<n_blocks, kCountThreads, 0, st>>>(dir, blocks, keys, nullptr, lcid, partial);
+    group_bulk_pack_kernel<<<n_blocks, kCountThreads, 0, st>>>(dir, blocks, keys, lcid, partial);
     return hipGetLastError();
 }
 
@@ -622,51 +566,39 @@ hipError_t launch_group_bulk_scan(const WideDesc *dir, const BulkTable *tabs, ui
 }
 
 hipError_t launch_group_bulk_scatter(const GroupItem *blocks, uint32_t n_blocks, const uint32_t *keys,
-                                     const uint32_t *vals, const uint64_t *entries, const uint8_t *lcid,
-                                     const uint32_t *partial, uint64_t n, uint64_t *ent, hipStream_t st)
+                                     const uint32_t *vals, const uint8_t *lcid, const uint32_t *partial, uint64_t n,
+                                     uint64_t *ent, hipStream_t st)
 {
     if (n_blocks == 0) return hipSuccess;
     if (n >= (1ull << 32)) return hipErrorInvalidValue;
     const SegLayout lay{blocks, partial, n};
     uint8_t *const no_cid = nullptr;
-    if (entries)
-        part_scatter_kernel<uint64_t, EntrySource<uint64_t>, uint8_t, kBulkSortThreads, -1, SegLayout>
-            <<<n_blocks, kBulkSortThreads, 0, st>>>(EntrySource<uint64_t>{entries}, lcid, lay, RadixPass{0, 8}, ent,
-                                                    no_cid);
-    else
-        part_scatter_kernel<uint64_t, KeyValSource, uint8_t, kBulkSortThreads, -1, SegLayout>
-            <<<n_blocks, kBulkSortThreads, 0, st>>>(KeyValSource{keys, vals}, lcid, lay, RadixPass{0, 8}, ent, no_cid);
+    part_scatter_kernel<uint64_t, KeyValSource, uint8_t, kBulkSortThreads, -1, SegLayout>
+        <<<n_blocks, kBulkSortThreads, 0, st>>>(KeyValSource{keys, vals}, lcid, lay, RadixPass{0, 8}, ent, no_cid);
     return hipGetLastError();
 }
 
+// The fill's 68 KB of LDS allow two workgroups per CU, so they are 1024 threads wide (8 waves per
+// SIMD) to keep more loads in flight (7.50 -> 7.40 ms for the 2^28-key insert against 512 threads).
+constexpr int kFillThreads = 1024;
+
 hipError_t launch_group_bulk_fill(const GroupChunk *chunks, uint32_t n_chunks, const uint64_t *ent, uint64_t *ovf,
-                                  unsigned long long *ovf_n, unsigned long long *table_counts, Counters *C, bool dense,
-                                  bool zeroed, hipStream_t st)
+                                  unsigned long long *ovf_n, unsigned long long *table_counts, Counters *C, bool zeroed,
+                                  hipStream_t st)
 {
     if (n_chunks == 0) return hipSuccess;
-    if (dense)
-        group_bulk_fill_kernel<true, 1024>
-            <<<n_chunks, 1024, 0, st>>>(chunks, ent, ovf, ovf_n, table_counts, C, zeroed);
-    else
-        group_bulk_fill_kernel<false, 256><<<n_chunks, 256, 0, st>>>(chunks, ent, ovf, ovf_n, table_counts, C, false);
+    group_bulk_fill_kernel<kFillThreads>
+        <<<n_chunks, kFillThreads, 0, st>>>(chunks, ent, ovf, ovf_n, table_counts, C, zeroed);
     return hipGetLastError();
 }
 
 hipError_t launch_bulk_fill(const Desc &D, const Chunks &Ch, const uint32_t *start, const uint64_t *ent, uint64_t n,
-                            uint64_t *ovf, uint64_t ovf_cap, unsigned long long *ovf_n, Counters *C, bool zeroed,
-                            hipStream_t st)
+                            uint64_t *ovf, uint64_t ovf_cap, Counters *C, bool zeroed, hipStream_t st)
 {
     if (n == 0) return hipSuccess;
     if (n >= (1ull << 32) || Ch.total == 0) return hipErrorInvalidValue;
-    uint64_t buckets = 0;
-    for (uint32_t t = 0; t < D.d; ++t) buckets += D.nb[t];
-    // dense: copying every chunk through LDS costs less than scattered stores; its 68 KB of LDS
-    // allow two workgroups per CU, so they are 1024 threads wide (48 VGPRs: 8 waves per SIMD) to
-    // keep more loads in flight (7.50 -> 7.40 ms for the 2^28-key insert against 512 threads)
-    if (n >= 2 * buckets)
-        bulk_fill_kernel<true, 1024><<<Ch.total, 1024, 0, st>>>(D, Ch, start, ent, n, ovf, ovf_cap, ovf_n, C, zeroed);
-    else
-        bulk_fill_kernel<false, 256><<<Ch.total, 256, 0, st>>>(D, Ch, start, ent, n, ovf, ovf_cap, ovf_n, C, false);
+    bulk_fill_kernel<kFillThreads>
+        <<<Ch.total, kFillThreads, 0, st>>>(D, Ch, start, ent, n, ovf, ovf_cap, C, zeroed);
     return hipGetLastError();
 }
 

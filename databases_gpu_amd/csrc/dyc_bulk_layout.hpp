@@ -13,12 +13,11 @@
 namespace dyc {
 namespace host {
 
-// The participating tables, their partition blocks (at most kGroupBulkBlockKeys keys of one
-// table each) and each block's table index.
+// The participating tables and their partition blocks (at most kGroupBulkBlockKeys keys of one
+// table each).
 struct BulkLayout {
     std::vector<BulkTable> tabs;
     std::vector<GroupItem> blocks;
-    std::vector<uint32_t> btab;
     uint64_t total = 0;
     uint32_t chunks = 0;
 };
@@ -42,12 +41,9 @@ bool bulk_layout(uint32_t n_tables, const uint64_t *offsets, DescOf desc, BulkLa
             buckets += D.nb[t];
         }
         if (ch > kGroupBulkChunks) return false;
-        const uint32_t j = (uint32_t)L->tabs.size();
         BulkTable T{offsets[i], (uint32_t)n, i, (uint32_t)L->blocks.size(), 0, L->chunks, ch};
-        for (uint64_t b = offsets[i]; b < offsets[i + 1]; b += kGroupBulkBlockKeys) {
+        for (uint64_t b = offsets[i]; b < offsets[i + 1]; b += kGroupBulkBlockKeys)
             L->blocks.push_back(GroupItem{b, (uint32_t)std::min<uint64_t>(kGroupBulkBlockKeys, offsets[i + 1] - b), i});
-            L->btab.push_back(j);
-        }
         T.blocks = (uint32_t)L->blocks.size() - T.first_block;
         L->chunks += ch;
         L->tabs.push_back(T);

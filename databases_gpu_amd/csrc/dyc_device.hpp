@@ -22,6 +22,9 @@ constexpr int kSlots = 16;                     // dy_hash.h:34 ELEM_NUM_P_gpu = 
 constexpr int kBucketBytes = kSlots * 8;       // 128
 constexpr uint32_t kPrime = 294967291u;        // dy_hash.h:24 PRIME_uint
 constexpr uint32_t kNoTable = 100u;            // cuckoo.cu:336 initial pre_table_no
+constexpr uint32_t kOddStart = kNoTable + 1;   // a fresh odd key: starts in pos2 (cuckoo.cu:336-341)
+constexpr uint32_t kAfterFill = kNoTable + 2;  // an entry the bulk fill found no slot for: starts in the
+                                               // bucket of its pair that is not its fill_target
 constexpr uint32_t kDefaultKickBound = 15u;    // dy_hash.h:33 MAX_ITER
 
 __host__ __device__ inline uint32_t key_of(uint64_t e) { return (uint32_t)(e >> 32); }
@@ -344,15 +347,12 @@ __host__ __device__ inline uint32_t fill_target(const Desc &D, uint32_t k, uint3
     return (r == 2u || (r == 0u && (k & 1u))) ? pos2(D, p) : pos1(D, p);
 }
 
-// A fill round's subtable for keys of pair p = idx & 15 and parity idx >> 4 (the index of a
-// 32-entry table the pack kernels keep in LDS, so a key's subtable costs one LDS read): round 1
-// fill_target, round 2 the other bucket of the pair.
-__host__ __device__ inline uint32_t fill_round_sub(const Desc &D, uint32_t idx, bool round2)
+// fill_target for keys of pair p = idx & 15 and parity idx >> 4 (the index of a 32-entry table the
+// pack kernels keep in LDS, so a key's subtable costs one LDS read).
+__host__ __device__ inline uint32_t fill_sub(const Desc &D, uint32_t idx)
 {
     const uint32_t p = idx & 15u;
-    if (p >= D.np) return 0;
-    const uint32_t t = fill_target(D, idx >> 4, p);
-    return round2 ? other_pos(D, p, t) : t;
+    return p < D.np ? fill_target(D, idx >> 4, p) : 0u;
 }
 
 // Depth-first search for Desc::fr over the np pairs (3^np choices, pruned): each pair's keys go

@@ -46,23 +46,23 @@ struct dyc_group {
     bool zeroed = false;
     // bulk fill (cfg.insert_order 3), grown on demand and kept by the group. Shared by the eager
     // calls and the plans (a plan refuses to run once one of these moved): partitioned entries and
-    // the overflow (8 B per key each), local chunk ids (1 B per key), per-block chunk counts,
-    // per-chunk start / count / table, and the overflow counts of both rounds (2 per table). The
-    // eager calls' own block and table arrays (device, with pinned staging) and the read-back of
-    // the last round's overflow counts.
+    // the overflow (8 B per key each), local chunk ids (1 B per key), per-block chunk counts, chunk
+    // records, the overflow's work items, and the tables' overflow counts with the item count after
+    // them. The eager calls' own block and table arrays (device, with pinned staging).
     uint64_t *bk_ent = nullptr, *bk_ovf = nullptr;
     uint8_t *bk_lcid = nullptr;
     uint64_t bk_cap = 0;
     uint32_t *bk_partial = nullptr;
     uint64_t bk_partial_cap = 0;
-    GroupChunk *bk_chunks = nullptr;  // chunk records of a round
+    GroupChunk *bk_chunks = nullptr;
     uint64_t bk_chunk_cap = 0;
-    unsigned long long *bk_ovfn = nullptr, *bk_hovfn = nullptr;
+    GroupItem *bk_items = nullptr;
+    uint64_t bk_items_cap = 0;
+    unsigned long long *bk_ovfn = nullptr;
     uint32_t bk_tabs_cap = 0;
-    GroupItem *bk_blk = nullptr, *bk_hblk = nullptr;  // device: 3 per block (rounds 1, 2, eviction)
-    uint32_t *bk_btab = nullptr, *bk_hbtab = nullptr;
+    GroupItem *bk_blk = nullptr, *bk_hblk = nullptr;
     uint64_t bk_blk_cap = 0;
-    BulkTable *bk_tabs = nullptr, *bk_htabs = nullptr;  // device: 2 per table (rounds 1, 2)
+    BulkTable *bk_tabs = nullptr, *bk_htabs = nullptr;
 
     InsertPolicy policy() const { return InsertPolicy{launch.kick_bound, cfg.rescue_kicks, cfg.max_retries}; }
     // The pending list is the group's stash: entries tagged with their table, searched by finds
@@ -313,10 +313,8 @@ int reserve_group_bulk(dyc_group *g, uint64_t n, uint64_t blocks, uint64_t chunk
     }
     if (blocks > g->bk_blk_cap) {
         g->bk_blk_cap = 0;
-        regrow((void **)&g->bk_blk, 3 * blocks * sizeof(GroupItem), "blocks");
-        regrow((void **)&g->bk_btab, blocks * sizeof(uint32_t), "block tables");
+        regrow((void **)&g->bk_blk, blocks * sizeof(GroupItem), "blocks");
         regrow_pinned((void **)&g->bk_hblk, blocks * sizeof(GroupItem));
-        regrow_pinned((void **)&g->bk_hbtab, blocks * sizeof(uint32_t));
         if (rc) return rc;
         g->bk_blk_cap = blocks;
     }
@@ -326,60 +324,55 @@ int reserve_group_bulk(dyc_group *g, uint64_t n, uint64_t blocks, uint64_t chunk
         if (rc) return rc;
         g->bk_chunk_cap = chunks;
     }
+    const uint64_t items = overflow_items(n, tabs);
+    if (items > g->bk_items_cap) {
+        g->bk_items_cap = 0;
+        regrow((void **)&g->bk_items, items * sizeof(GroupItem), "overflow items");
+        if (rc) return rc;
+        g->bk_items_cap = items;
+    }
     if (tabs > g->bk_tabs_cap) {
         g->bk_tabs_cap = 0;
-        regrow((void **)&g->bk_tabs, 2 * tabs * sizeof(BulkTable), "table list");
-        regrow((void **)&g->bk_ovfn, 2 * tabs * sizeof(unsigned long long), "overflow counts");
+        regrow((void **)&g->bk_tabs, tabs * sizeof(BulkTable), "table list");
+        regrow((void **)&g->bk_ovfn, (tabs + 1ull) * sizeof(unsigned long long), "overflow counts");
         regrow_pinned((void **)&g->bk_htabs, tabs * sizeof(BulkTable));
-        regrow_pinned((void **)&g->bk_hovfn, tabs * sizeof(unsigned long long));
         if (rc) return rc;
         g->bk_tabs_cap = tabs;
     }
     return DYC_OK;
 }
 
-// Device arrays of one laid-out batch: blocks of round 1, 2 and the eviction insert (nb each),
-// each block's table index, and the tables of rounds 1 and 2 (j each).
+// Device arrays of one laid-out batch: its partition blocks (nb) and participating tables (j).
 struct BulkArrays {
     GroupItem *blk;
-    uint32_t *btab;
     BulkTable *tabs;
     uint32_t nb, j, chunks;
 };
 
 // The whole bulk fill of a laid-out batch, launched on s with no read-back in between, so a
-// graph can hold it: round 1 (keys/vals -> entries by each table's chunks -> chunk fill), round 2
-// (each table's overflow, for the other bucket of its pair), then the eviction insert of what
-// overflows that. Each round's next work comes from the overflow counts on the device (clip).
-// Counters and per-table counts accumulate (the caller zeroes them); the last round's overflow
-// counts are left in bk_ovfn + j. zeroed: every slot of every table is zero (round 1 then does
-// not read the tables).
+// graph can hold it: keys/vals -> entries by each table's chunks -> chunk fill, then the eviction
+// insert of each table's overflow in the other bucket of its pair, over items of kOverflowItem
+// entries made on the device from the overflow counts. (2048 tables, 77 M keys: a second round of
+// partition and fill for the overflow took 250 us and its rest, as one item a table, 480 us; the
+// whole overflow in small items takes 270 us.) Counters and
+// per-table counts accumulate (the caller zeroes them). zeroed: every slot of every table is zero
+// (the fill then does not read the tables).
 hipError_t enqueue_group_bulk(dyc_group *g, const BulkArrays &A, const uint32_t *keys, const uint32_t *vals,
                               uint64_t total, bool zeroed, PendSink sink, hipStream_t s)
 {
-    GroupItem *const blk1 = A.blk, *const blk2 = A.blk + A.nb, *const items = A.blk + 2 * A.nb;
-    BulkTable *const tabs1 = A.tabs, *const tabs2 = A.tabs + A.j;
-    unsigned long long *const ovf1 = g->bk_ovfn, *const ovf2 = g->bk_ovfn + A.j;
+    unsigned long long *const n_items = g->bk_ovfn + A.j;
     hipError_t e;
-    if ((e = launch_group_bulk_pack(g->ddir, blk1, A.nb, keys, nullptr, g->bk_lcid, g->bk_partial, s)) != hipSuccess ||
-        (e = launch_group_bulk_scan(g->ddir, tabs1, A.j, g->bk_partial, g->bk_chunks, s)) != hipSuccess ||
-        (e = launch_group_bulk_scatter(blk1, A.nb, keys, vals, nullptr, g->bk_lcid, g->bk_partial, total, g->bk_ent,
-                                       s)) != hipSuccess ||
-        (e = launch_zero(ovf1, 2 * (uint64_t)A.j, s)) != hipSuccess ||
-        (e = launch_group_bulk_fill(g->bk_chunks, A.chunks, g->bk_ent, g->bk_ovf, ovf1, g->tcounts, g->ctr, true,
-                                    zeroed, s)) != hipSuccess ||
-        (e = launch_group_bulk_clip(blk1, A.btab, A.nb, tabs1, A.j, ovf1, blk2, tabs2, s)) != hipSuccess ||
-        (e = launch_group_bulk_pack(g->ddir, blk2, A.nb, nullptr, g->bk_ovf, g->bk_lcid, g->bk_partial, s)) !=
+    if ((e = launch_group_bulk_pack(g->ddir, A.blk, A.nb, keys, g->bk_lcid, g->bk_partial, s)) != hipSuccess ||
+        (e = launch_group_bulk_scan(g->ddir, A.tabs, A.j, g->bk_partial, g->bk_chunks, s)) != hipSuccess ||
+        (e = launch_group_bulk_scatter(A.blk, A.nb, keys, vals, g->bk_lcid, g->bk_partial, total, g->bk_ent, s)) !=
             hipSuccess ||
-        (e = launch_group_bulk_scan(g->ddir, tabs2, A.j, g->bk_partial, g->bk_chunks, s)) != hipSuccess ||
-        (e = launch_group_bulk_scatter(blk2, A.nb, nullptr, nullptr, g->bk_ovf, g->bk_lcid, g->bk_partial, total,
-                                       g->bk_ent, s)) != hipSuccess ||
-        (e = launch_group_bulk_fill(g->bk_chunks, A.chunks, g->bk_ent, g->bk_ovf, ovf2, g->tcounts, g->ctr, false,
-                                    false, s)) != hipSuccess ||
-        (e = launch_group_bulk_clip(blk1, A.btab, A.nb, tabs1, A.j, ovf2, items, nullptr, s)) != hipSuccess)
+        (e = launch_zero(g->bk_ovfn, A.j + 1ull, s)) != hipSuccess ||
+        (e = launch_group_bulk_fill(g->bk_chunks, A.chunks, g->bk_ent, g->bk_ovf, g->bk_ovfn, g->tcounts, g->ctr,
+                                    zeroed, s)) != hipSuccess ||
+        (e = launch_group_bulk_items(A.tabs, A.j, g->bk_ovfn, g->bk_items, g->bk_items_cap, n_items, s)) != hipSuccess)
         return e;
-    return launch_group_insert(g->ddir, items, A.nb, nullptr, nullptr, g->policy(), (int)g->launch.insert_lanes,
-                               (int)g->launch.insert_blocks, g->ctr, sink, g->tcounts, s, 0, g->bk_ovf);
+    return launch_group_insert_overflow(g->ddir, g->bk_items, n_items, overflow_items(total, A.j), g->bk_ovf,
+                                        g->policy(), (int)g->launch.insert_blocks, g->ctr, sink, g->tcounts, s);
 }
 
 // Sizes the shared workspace for a layout (synchronizes s first); DYC_ERR_OOM leaves no message
@@ -391,17 +384,14 @@ int reserve_for(dyc_group *g, const BulkLayout &L, hipStream_t s)
 }
 
 // insert_order 3 for a group: each table's batch is partitioned by its own chunks in one pass
-// (the batch is grouped by table already) and every chunk is filled by one workgroup; what
-// overflows its first bucket (fill_target) gets a second round for the other bucket of its pair
-// (sparse: a few percent of the keys), and what
-// overflows that goes through the group's eviction insert. Declines (*n_tabs 0, nothing
-// launched) when bulk_layout does, or when the workspace cannot be allocated. Counters and
-// per-table counts are zeroed here and read by the caller, who also finds the overflow counts of
-// the last round (*n_tabs of them) in bk_hovfn after its wait.
+// (the batch is grouped by table already), every chunk is filled by one workgroup, and what
+// overflows its first bucket (fill_target) goes through the group's eviction insert. Declines
+// (*filled false, nothing launched) when bulk_layout does, or when the workspace cannot be
+// allocated. Counters and per-table counts are zeroed here and read by the caller.
 int group_bulk_insert(dyc_group *g, const uint32_t *keys, const uint32_t *vals, const uint64_t *offsets, bool zeroed,
-                      hipStream_t s, uint64_t room, uint32_t *n_tabs)
+                      hipStream_t s, uint64_t room, bool *filled)
 {
-    *n_tabs = 0;
+    *filled = false;
     BulkLayout L;
     if (!dyc::host::bulk_layout(g->n, offsets, [g](uint32_t i) -> const Desc & { return g->hdir[i]; }, &L))
         return DYC_OK;
@@ -417,25 +407,22 @@ int group_bulk_insert(dyc_group *g, const uint32_t *keys, const uint32_t *vals, 
     const uint32_t NB = (uint32_t)L.blocks.size(), J = (uint32_t)L.tabs.size();
     // the pinned staging is free: the previous call waited for its work before returning
     memcpy(g->bk_hblk, L.blocks.data(), NB * sizeof(GroupItem));
-    memcpy(g->bk_hbtab, L.btab.data(), NB * sizeof(uint32_t));
     memcpy(g->bk_htabs, L.tabs.data(), J * sizeof(BulkTable));
     HIP_TRY(hipMemcpyAsync(g->bk_blk, g->bk_hblk, NB * sizeof(GroupItem), hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(g->bk_btab, g->bk_hbtab, NB * sizeof(uint32_t), hipMemcpyHostToDevice, s));
     HIP_TRY(hipMemcpyAsync(g->bk_tabs, g->bk_htabs, J * sizeof(BulkTable), hipMemcpyHostToDevice, s));
     int rc = zero_and_run_prologue(g, s);
     if (rc) return rc;
-    const BulkArrays A{g->bk_blk, g->bk_btab, g->bk_tabs, NB, J, L.chunks};
+    const BulkArrays A{g->bk_blk, g->bk_tabs, NB, J, L.chunks};
     HIP_TRY(enqueue_group_bulk(g, A, keys, vals, L.total, zeroed,
                                PendSink{g->pend + g->pend_n, g->pend_tag + g->pend_n, room, 0, 0, nullptr}, s));
-    HIP_TRY(hipMemcpyAsync(g->bk_hovfn, g->bk_ovfn + J, J * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-    *n_tabs = J;
+    *filled = true;
     return DYC_OK;
 }
 
 // The group's shared bulk-fill buffers a plan's graph uses (any of them moving voids the plan).
 std::vector<const void *> bulk_workspace(const dyc_group *g)
 {
-    return {g->bk_ent, g->bk_ovf, g->bk_lcid, g->bk_partial, g->bk_chunks, g->bk_ovfn};
+    return {g->bk_ent, g->bk_ovf, g->bk_lcid, g->bk_partial, g->bk_chunks, g->bk_items, g->bk_ovfn};
 }
 
 }  // namespace
@@ -540,10 +527,10 @@ int dyc_group_destroy(dyc_group *g)
     if (g->hitems) (void)hipHostFree(g->hitems);
     if (g->items_free) (void)hipEventDestroy(g->items_free);
     for (void *p : {(void *)g->bk_ent, (void *)g->bk_ovf, (void *)g->bk_lcid, (void *)g->bk_partial,
-                    (void *)g->bk_chunks, (void *)g->bk_tabs,
-                    (void *)g->bk_ovfn, (void *)g->bk_blk, (void *)g->bk_btab})
+                    (void *)g->bk_chunks, (void *)g->bk_tabs, (void *)g->bk_items,
+                    (void *)g->bk_ovfn, (void *)g->bk_blk})
         if (p) (void)hipFree(p);
-    for (void *p : {(void *)g->bk_htabs, (void *)g->bk_hovfn, (void *)g->bk_hblk, (void *)g->bk_hbtab})
+    for (void *p : {(void *)g->bk_htabs, (void *)g->bk_hblk})
         if (p) (void)hipHostFree(p);
     delete g;
     return DYC_OK;
@@ -582,15 +569,13 @@ int dyc_group_insert(dyc_group *g, const uint32_t *keys, const uint32_t *vals, c
     if (rc) return rc;
     const uint64_t room = g->pend_cap - g->pend_n;
     if (g->cfg.insert_order == 3) {
-        uint32_t n_tabs = 0;
-        rc = group_bulk_insert(g, keys, vals, offsets, zeroed, s, room, &n_tabs);
+        bool filled = false;
+        rc = group_bulk_insert(g, keys, vals, offsets, zeroed, s, room, &filled);
         if (rc) return rc;
-        if (n_tabs) {
-            rc = read_back(g, s);  // waits: the overflow counts are in bk_hovfn too
+        if (filled) {
+            rc = read_back(g, s);
             if (rc) return rc;
-            uint64_t left = 0;
-            for (uint32_t j = 0; j < n_tabs; ++j) left += g->bk_hovfn[j];
-            g->st.last_filled = total - g->hctr->rejected - left;
+            g->st.last_filled = total - g->hctr->rejected - g->hctr->left;
             return finish_insert(g, room);
         }
     }
@@ -599,7 +584,7 @@ int dyc_group_insert(dyc_group *g, const uint32_t *keys, const uint32_t *vals, c
     if (rc) return rc;
     rc = zero_and_run_prologue(g, s);
     if (rc) return rc;
-    HIP_TRY(launch_group_insert(g->ddir, g->ditems, n_items, keys, vals, g->policy(), (int)g->launch.insert_lanes,
+    HIP_TRY(launch_group_insert(g->ddir, g->ditems, n_items, keys, vals, g->policy(),
                                 (int)g->launch.insert_blocks, g->ctr,
                                 PendSink{g->pend + g->pend_n, g->pend_tag + g->pend_n, room, 0, 0, nullptr}, g->tcounts,
                                 s, (int)g->launch.insert_waves_per_eu));
@@ -672,7 +657,7 @@ int dyc_group_insert_per_table(dyc_group *g, const uint32_t *keys, const uint32_
     for (uint32_t i = 0; i < g->n; ++i) {
         const uint64_t m = offsets[i + 1] - offsets[i];
         if (!m) continue;
-        HIP_TRY(launch_insert(g->hdir[i], keys + offsets[i], vals + offsets[i], m, (int)g->launch.insert_lanes,
+        HIP_TRY(launch_insert(g->hdir[i], keys + offsets[i], vals + offsets[i], m,
                               g->policy(), sh, g->ctr,
                               PendSink{g->pend + g->pend_n, g->pend_tag + g->pend_n, room, i, 0, g->tcounts + i}, s));
     }
@@ -755,16 +740,13 @@ struct dyc_group_plan {
     hipGraphExec_t exec = nullptr;
     uint64_t room = 0;  // pending entries the insert may append
     uint64_t *pend = nullptr;  // the pending list the graph writes (a larger eager insert may move it)
-    // insert_order 3: the batch's own bulk-fill arrays, the group's shared workspace the graph
-    // uses (an eager insert that grows it moves these), and the last round's overflow counts
-    // (pinned, written by the graph) for last_filled
+    // insert_order 3: the batch's own bulk-fill arrays, and the group's shared workspace the graph
+    // uses (an eager insert that grows it moves these)
     bool bulk = false;
     uint64_t total = 0;
     GroupItem *bk_blk = nullptr;
-    uint32_t *bk_btab = nullptr;
     BulkTable *bk_tabs = nullptr;
     uint32_t bk_j = 0;
-    unsigned long long *hovfn = nullptr;
     std::vector<const void *> shared;
 };
 
@@ -777,9 +759,8 @@ int dyc_group_plan_destroy(dyc_group_plan *p)
     if (p->exec) (void)hipGraphExecDestroy(p->exec);
     if (p->graph) (void)hipGraphDestroy(p->graph);
     if (p->d_items) (void)hipFree(p->d_items);
-    for (void *q : {(void *)p->bk_blk, (void *)p->bk_btab, (void *)p->bk_tabs})
+    for (void *q : {(void *)p->bk_blk, (void *)p->bk_tabs})
         if (q) (void)hipFree(q);
-    if (p->hovfn) (void)hipHostFree(p->hovfn);
     delete p;
     return DYC_OK;
 }
@@ -850,16 +831,13 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
             p->bulk = true;
             p->total = L.total;
             p->bk_j = J;
-            if (hipMalloc(&p->bk_blk, 3ull * NB * sizeof(GroupItem)) != hipSuccess ||
-                hipMalloc(&p->bk_btab, NB * sizeof(uint32_t)) != hipSuccess ||
-                hipMalloc(&p->bk_tabs, 2ull * J * sizeof(BulkTable)) != hipSuccess ||
-                hipHostMalloc((void **)&p->hovfn, J * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess) {
+            if (hipMalloc(&p->bk_blk, NB * sizeof(GroupItem)) != hipSuccess ||
+                hipMalloc(&p->bk_tabs, J * sizeof(BulkTable)) != hipSuccess) {
                 (void)hipGetLastError();
                 fail(DYC_ERR_OOM, "plan bulk-fill arrays failed");
                 return undo(DYC_ERR_OOM);
             }
             if (hipMemcpy(p->bk_blk, L.blocks.data(), NB * sizeof(GroupItem), hipMemcpyHostToDevice) != hipSuccess ||
-                hipMemcpy(p->bk_btab, L.btab.data(), NB * sizeof(uint32_t), hipMemcpyHostToDevice) != hipSuccess ||
                 hipMemcpy(p->bk_tabs, L.tabs.data(), J * sizeof(BulkTable), hipMemcpyHostToDevice) != hipSuccess) {
                 fail(DYC_ERR_HIP, "plan bulk-fill upload failed");
                 return undo(DYC_ERR_HIP);
@@ -884,11 +862,10 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
         const PendSink sink{g->pend, g->pend_tag, g->pend_cap, 0, 0, nullptr};
         if (k == hipSuccess && p->bulk) {
             // the graph clears every table first, so round 1 need not read them
-            const BulkArrays A{p->bk_blk, p->bk_btab, p->bk_tabs, (uint32_t)L.blocks.size(), p->bk_j, L.chunks};
+            const BulkArrays A{p->bk_blk, p->bk_tabs, (uint32_t)L.blocks.size(), p->bk_j, L.chunks};
             k = enqueue_group_bulk(g, A, keys, vals, p->total, true, sink, cs);
-            if (k == hipSuccess) k = launch_copy(g->bk_ovfn + p->bk_j, p->hovfn, p->bk_j, nullptr, nullptr, 0, cs);
         } else if (k == hipSuccess) {
-            k = launch_group_insert(g->ddir, p->d_items, p->n_ins, keys, vals, g->policy(), (int)g->launch.insert_lanes,
+            k = launch_group_insert(g->ddir, p->d_items, p->n_ins, keys, vals, g->policy(),
                                     (int)g->launch.insert_blocks, g->ctr, sink, g->tcounts, cs,
                                     (int)g->launch.insert_waves_per_eu);
         }
@@ -930,11 +907,7 @@ int dyc_group_plan_run(dyc_group_plan *p, dyc_stream stream)
     // the step cleared every table: counts and the pending list start again from zero
     std::fill(g->count.begin(), g->count.end(), 0);
     g->pend_n = 0;
-    if (p->bulk) {
-        uint64_t left = 0;
-        for (uint32_t j = 0; j < p->bk_j; ++j) left += p->hovfn[j];
-        g->st.last_filled = p->total - g->hctr->rejected - left;
-    }
+    if (p->bulk) g->st.last_filled = p->total - g->hctr->rejected - g->hctr->left;
     return finish_insert(g, p->room);
 }
 

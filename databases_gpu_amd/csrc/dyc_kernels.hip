@@ -5,9 +5,9 @@
 // lanes reads its four keys' buckets (probe_tile). pos2 is read only for keys pos1 did not
 // resolve, in the reference order (cuckoo.cu:482-497).
 //
-// Insert: each group of G lanes carries one entry through the eviction chain with 64-bit CAS
-// on the victim slot. Groups are independent: a group that finishes takes its next key while
-// the rest of the wave keeps kicking, so no lane idles behind a long chain.
+// Insert: each lane carries one entry through the eviction chain, its bucket read by the quad as
+// in a probe. Lanes are independent: one that finishes takes its next key while the rest of the
+// wave keeps kicking, so no lane idles behind a long chain.
 #include "dyc_kernels.hpp"
 #include "dyc_wave.hpp"
 
@@ -318,258 +318,330 @@ __global__ __launch_bounds__(256) void probe_kernel(Desc D, const uint32_t *__re
 }
 
 // ------------------------------------------------------------------------------- insert
-// One group of G lanes per in-hand entry. Per iteration (cuckoo.cu:377-421):
+// One lane per in-hand entry, four lanes per bucket read. Per iteration (cuckoo.cu:377-421):
 //   t = the other subtable of the entry's pair relative to the previous one; read the bucket;
-//   victim = first empty slot, else (first kick_bound iterations) the first slot whose resident
-//   pair index differs from t (cuckoo.cu:398-400), else slot (iteration & 15); after kick_bound
-//   iterations the victim is rescue_lane(). CAS the victim slot from the value read to the
-//   entry: on success carry the old value on (done if it was empty).
-// The bucket is read with plain vector loads. The view may be stale (another XCD's L2 may hold
-// a newer line), but only the CAS decides: a stale view can make a CAS fail, never lose or
-// duplicate an entry. A failed CAS returns the slot's current value, which replaces that slot in
-// the view; the group then chooses again without re-reading, so every retry learns one slot's
-// true value and at most max_retries races are spent on one entry before it is pended.
+//   an empty slot takes the entry by CAS; a full bucket gives up a victim: in the first kick_bound
+//   iterations the first slot whose resident's pair index differs from t (cuckoo.cu:398-400), else
+//   slot (iteration & 15); after them rescue_lane(). The entry is exchanged with the victim, which
+//   is carried on (the chain is done if the slot turned out empty).
+// With kick_bound 0 (no iteration follows the reference rule) a fresh key whose first bucket is
+// full tries the other bucket of its pair before it evicts: at fill 0.8 that saves 0.2 of 1.25
+// exchanges a key, and exchanges are what a large insert waits for (18-20 G/s).
+// The quad's lanes read the buckets of its four entries as the probe tile does (32 bytes each), so
+// a bucket costs two cache accesses a lane and a step about 250 vector instructions; one lane
+// reading its whole bucket took eight accesses, each a line of its own, and held its 16 slots in
+// registers.
+// The buckets are read with plain vector loads. The view may be stale (another XCD's L2 may hold
+// a newer line), but no entry is lost or doubled by it: an empty slot is taken by CAS, and a slot
+// lost to another entry is not tried again (Hand::from; the bucket is read again, and the view
+// may still show the slot empty), so a bucket costs at most 16 lost races and an entry at most
+// max_retries before it is pended; a victim is exchanged, which cannot fail.
 //
-// Input is taken in chunks of kChunk indexes: wave w owns chunks w, w + W, w + 2W, ... and
-// hands each chunk's indexes to its idle groups by ballot rank as they free up, so no group
-// waits for the slowest chain of its wave. Resident waves sweep the input front to back
-// together; when the batch was ordered by bucket region (launch_partition), the window they
+// Input is taken in chunks of 64 indexes: wave w owns chunks w, w + W, w + 2W, ..., loads the next
+// one ahead into a register a lane, and hands its entries to idle lanes by ballot rank as they free
+// up, so no lane waits for the slowest chain of its wave. Resident waves sweep the input front to
+// back together; when the batch was ordered by bucket region (launch_partition), the window they
 // work on touches one region's buckets at a time.
-// State of one group's in-hand entry (group-uniform except the view, which is per lane).
-template <int SPL>
-struct Carry {
-    uint64_t entry;
+struct Hand {
+    uint32_t k, v;
     uint64_t idx;  // input index of the key that started the chain
     uint32_t pre, kicks, retries;
-    uint64_t cur[SPL];  // this lane's SPL slots of the current bucket
-    bool fresh;         // the view must be (re)read
+    uint32_t from;  // the first slot of the current bucket still worth a CAS
+    bool fresh;     // not placed or carried yet: its other bucket is still to be tried
     bool active;
 };
 
+// A wave's tallies: the counts are wave-uniform, the longest chain is the lane's own.
 struct InsertTally {
     unsigned long long kicks = 0, rejected = 0, retries = 0;
     unsigned long long empty = 0;  // zero entries skipped by a from-entries insert
-    unsigned long long max_chain = 0;
+    unsigned long long direct = 0;  // chains that ended with their first exchange
+    uint32_t max_chain = 0;
 };
 
-// A chain ended after c.kicks exchanges (its entry placed or parked): tally it, and record it
-// for the input index that started it.
-template <int SPL>
-__device__ inline void chain_end(const Carry<SPL> &c, const PendSink &sink, int s, InsertTally &tally)
+// A chain ended (its entry placed or parked): record it for the input index that started it.
+__device__ inline void chain_end(Hand &h, const PendSink &sink, InsertTally &tally)
 {
-    if (s == 0) {
-        tally.kicks += c.kicks;
-        tally.max_chain = tally.max_chain > c.kicks ? tally.max_chain : c.kicks;
-        if (sink.chain) sink.chain[c.idx] = c.kicks;
-    }
+    tally.max_chain = tally.max_chain > h.kicks ? tally.max_chain : h.kicks;
+    if (sink.chain) sink.chain[h.idx] = h.kicks;
+    h.active = false;
 }
 
-// Take entry e (previous table pr, kNoTable for a fresh key) into the group's hand.
-template <int SPL>
-__device__ inline void carry_start(const Desc &D, Carry<SPL> &c, uint64_t e, uint32_t pr, int s, InsertTally &tally,
-                                   uint64_t idx = 0, uint32_t *chain = nullptr)
+// Park the in-hand entry on the pending list.
+__device__ inline void give_up(Hand &h, Counters *C, const PendSink &sink, uint32_t tag, InsertTally &tally)
 {
-    const uint32_t k = key_of(e);
-    if (reserved_key(k)) {
-        if (s == 0) {
-            ++tally.rejected;
-            if (chain) chain[idx] = 0;
-        }
-        return;
-    }
-    if (pr == kNoTable && (k & 1u)) pr = pos1(D, pair_of(D, k));  // odd keys start in pos2 (cuckoo.cu:336-341)
-    c.entry = e;
-    c.idx = idx;
-    c.pre = pr;
-    c.kicks = 0;
-    c.retries = 0;
-    c.fresh = true;
-    c.active = true;
-}
-
-// One eviction-chain iteration for an active group (see the comment above insert_kernel).
-template <int G>
-__device__ inline void kick_step(const Desc &D, Carry<kSlots / G> &c, const InsertPolicy &P, Counters *C,
-                                 const PendSink &sink, uint32_t tag, InsertTally &tally)
-{
-    constexpr int SPL = kSlots / G;
-    constexpr uint64_t GMASK = (G >= 64) ? ~0ull : ((1ull << G) - 1ull);
-    const int lane = __lane_id();
-    const int g = lane / G, s = lane % G;
-    const uint32_t total_kicks = P.kick_bound + P.rescue_kicks;
-
-    auto give_up = [&]() {  // park the in-hand entry on the pending list
-        if (s == 0) {
-            unsigned long long at = atomicAdd(&C->pending, 1ull);
-            if (at < sink.cap) {
-                sink.pend[at] = c.entry;
-                if (sink.tags) sink.tags[at] = tag;
-                // rare: publish the entry to every XCD (a serving tick's later finds read the pool
-                // within the same launch)
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            } else {
-                atomicAdd(&C->lost, 1ull);
-            }
-        }
-        c.active = false;
-    };
-
-    const uint32_t k = key_of(c.entry);
-    const uint32_t t = other_pos(D, pair_of(D, k), c.pre);
-    uint64_t *b = bucket_ptr(D, k, t);
-    if (c.fresh) load_slots<SPL>(b + s * SPL, c.cur);
-    c.fresh = false;
-
-    // victim slot (group-uniform)
-    int fe = -1;
-#pragma unroll
-    for (int j = SPL - 1; j >= 0; --j)
-        if (key_of(c.cur[j]) == 0u) fe = j;
-    uint32_t gm = (uint32_t)((__ballot(fe >= 0) >> (g * G)) & GMASK);
-    int slot;
-    if (gm) {
-        const int w = __builtin_ctz(gm);
-        slot = w * SPL + __shfl(fe, g * G + w);
-    } else if (c.kicks < P.kick_bound) {
-        int fo = -1;
-#pragma unroll
-        for (int j = SPL - 1; j >= 0; --j)
-            if (vote_victim(D, key_of(c.cur[j]), t)) fo = j;
-        gm = (uint32_t)((__ballot(fo >= 0) >> (g * G)) & GMASK);
-        if (gm) {
-            const int w = __builtin_ctz(gm);
-            slot = w * SPL + __shfl(fo, g * G + w);
-        } else {
-            slot = (int)(c.kicks & 15u);
-        }
+    chain_end(h, sink, tally);
+    const unsigned long long at = atomicAdd(&C->pending, 1ull);
+    if (at < sink.cap) {
+        sink.pend[at] = pack(h.k, h.v);
+        if (sink.tags) sink.tags[at] = tag;
+        // rare: publish the entry to every XCD (a serving tick's later finds read the pool
+        // within the same launch)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     } else {
-        slot = (int)rescue_lane(k, c.kicks);
+        atomicAdd(&C->lost, 1ull);
     }
-    const int owner = slot / SPL, sj = slot % SPL;
-    uint64_t mine = 0;
+}
+
+// The slot the reference vote gives up of a full bucket at `at` in subtable t: the first whose
+// resident's pair index differs from t. Its slots 0..3 are keys k4 (the quad's first lane read
+// them); five in six of them qualify at four subtables, so the others are rarely looked at.
+__device__ inline uint32_t vote_slot(const Desc &D, const uint32_t (&k4)[4], uint64_t at, uint32_t t, uint32_t kicks,
+                                     bool wanted)
+{
+    uint32_t slot = kSlots;
 #pragma unroll
-    for (int j = 0; j < SPL; ++j)
-        if (j == sj) mine = c.cur[j];
-    uint64_t expected = shfl64(mine, g * G + owner);
-    int won = 0;
-    if (s == owner) {
-        uint64_t exp = expected;
-        won = cas_slot(b + slot, exp, c.entry);
-        if (!won) {  // the slot's current value replaces the stale one in the view
-#pragma unroll
-            for (int j = 0; j < SPL; ++j)
-                if (j == sj) c.cur[j] = exp;
-        }
+    for (int j = 3; j >= 0; --j)
+        if (vote_victim(D, k4[j], t)) slot = (uint32_t)j;
+    const DYC_GLOBAL uint32_t *words = (const DYC_GLOBAL uint32_t *)at;
+    for (uint32_t j = 4; j < (uint32_t)kSlots; ++j) {
+        if (!__ballot(wanted && slot == (uint32_t)kSlots)) break;
+        if (wanted && slot == (uint32_t)kSlots && vote_victim(D, words[2 * j + 1], t)) slot = j;
     }
-    won = __shfl(won, g * G + owner);
-    if (won) {
-        ++c.kicks;
-        c.fresh = true;
-        if (expected == 0) {
-            chain_end(c, sink, s, tally);
-            c.active = false;
+    return slot < (uint32_t)kSlots ? slot : (kicks & 15u);
+}
+
+// One eviction-chain iteration of every active lane; all 64 lanes call it together.
+__device__ inline void insert_step(const Desc &D, Hand &h, const InsertPolicy &P, Counters *C, const PendSink &sink,
+                                   uint32_t tag, InsertTally &tally)
+{
+    const uint32_t s = __lane_id() & 3u;
+    const uint64_t act = __ballot(h.active);
+    const uint32_t p = pair_of(D, h.k), ta = pos1(D, p), tb = pos2(D, p);
+    const uint32_t t = h.pre == ta || h.pre == kOddStart ? tb : ta;
+    const uint64_t at = (uint64_t)bucket_ptr(D, h.k, t);
+    const uint32_t off = s * 32u;
+    QuadSlots e[4];
+    each_of_quad([&](auto q) {
+        constexpr int kk = decltype(q)::value;
+        const uint32_t lo = quad_bcast<kk>((uint32_t)at) | off, hi = quad_bcast<kk>((uint32_t)(at >> 32));
+        const uint64_t low = (act >> kk) & kQuadLow;
+        if (__builtin_amdgcn_inverse_ballot_w64((low << 4) - low)) e[kk] = load_quad_slots<false>(lo, hi);
+        else e[kk].a = e[kk].b = u32x4{0u, 0u, 0u, 0u};
+    });
+    // the first empty slot at or past h.from of the quad's four buckets, bucket kk's in lane kk
+    uint32_t c[4];
+    const bool some_from = __ballot(h.active && h.from) != 0;  // wave-uniform, rare
+    each_of_quad([&](auto q) {
+        constexpr int kk = decltype(q)::value;
+        const uint32_t b = s * 4u;
+        if (!some_from) {
+            c[kk] = e[kk].b.w == 0u ? b + 3u : 64u;
+            c[kk] = e[kk].b.y == 0u ? b + 2u : c[kk];
+            c[kk] = e[kk].a.w == 0u ? b + 1u : c[kk];
+            c[kk] = e[kk].a.y == 0u ? b : c[kk];
         } else {
-            c.entry = expected;
-            c.pre = t;
-            if (c.kicks >= total_kicks) {
-                chain_end(c, sink, s, tally);
-                give_up();
-            }
+            const uint32_t f = quad_bcast<kk>(h.from);
+            c[kk] = e[kk].b.w == 0u && b + 3u >= f ? b + 3u : 64u;
+            c[kk] = e[kk].b.y == 0u && b + 2u >= f ? b + 2u : c[kk];
+            c[kk] = e[kk].a.w == 0u && b + 1u >= f ? b + 1u : c[kk];
+            c[kk] = e[kk].a.y == 0u && b >= f ? b : c[kk];
         }
-    } else {
-        if (s == 0) ++tally.retries;
-        if (++c.retries > P.max_retries) {
-            chain_end(c, sink, s, tally);
-            give_up();
+    });
+    const bool odd = s & 1u, high = s & 2u;
+    const uint32_t c01 = min(odd ? c[1] : c[0], quad_swap<1>(odd ? c[0] : c[1]));
+    const uint32_t c23 = min(odd ? c[3] : c[2], quad_swap<1>(odd ? c[2] : c[3]));
+    uint32_t slot = min(high ? c23 : c01, quad_swap<2>(high ? c01 : c23));
+    const bool full = slot >= (uint32_t)kSlots;
+    const bool place = h.active && !full;
+    const bool swing = h.active && full && h.fresh && P.kick_bound == 0;
+    const bool evict = h.active && full && !swing;
+    if (__ballot(evict)) {
+        uint32_t victim = rescue_lane(h.k, h.kicks);
+        const bool vote = evict && h.kicks < P.kick_bound;
+        if (__ballot(vote)) {
+            uint32_t k4[4];
+            auto first_lane = [&](auto get) {  // bucket kk's word from the quad's lane 0, in lane kk
+                const uint32_t x0 = quad_bcast<0>(get(e[0])), x1 = quad_bcast<0>(get(e[1]));
+                const uint32_t x2 = quad_bcast<0>(get(e[2])), x3 = quad_bcast<0>(get(e[3]));
+                return high ? (odd ? x3 : x2) : (odd ? x1 : x0);
+            };
+            k4[0] = first_lane([](const QuadSlots &x) { return x.a.y; });
+            k4[1] = first_lane([](const QuadSlots &x) { return x.a.w; });
+            k4[2] = first_lane([](const QuadSlots &x) { return x.b.y; });
+            k4[3] = first_lane([](const QuadSlots &x) { return x.b.w; });
+            const uint32_t vs = vote_slot(D, k4, at, t, h.kicks, vote);
+            victim = vote ? vs : victim;
+        }
+        slot = evict ? victim : slot;
+    }
+    DYC_GLOBAL uint64_t *const dst = (DYC_GLOBAL uint64_t *)(at + 8u * (slot & 15u));
+    const uint64_t mine = pack(h.k, h.v);
+    uint64_t was = 0, out = 0;
+    if (place) was = cas_old(dst, 0ull, mine);
+    if (evict) out = __hip_atomic_exchange(dst, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool lost = place && was != 0;
+    const uint64_t won = __ballot((place && !lost) || evict);
+    tally.kicks += __popcll(won);
+    tally.direct += __popcll(won & __ballot(h.kicks == 0 && out == 0));
+    if (__builtin_amdgcn_inverse_ballot_w64(won)) {
+        ++h.kicks;
+        if (out == 0) {
+            chain_end(h, sink, tally);
+        } else {
+            h.k = key_of(out);
+            h.v = val_of(out);
+            h.pre = t;
+            h.fresh = false;
+            h.from = 0;
+            if (h.kicks >= P.kick_bound + P.rescue_kicks) give_up(h, C, sink, tag, tally);
+        }
+    }
+    if (swing) {  // its other bucket next, with nothing exchanged
+        h.pre = t;
+        h.fresh = false;
+        h.from = 0;
+    }
+    const uint64_t losers = __ballot(lost);
+    if (losers) {
+        tally.retries += __popcll(losers);
+        if (lost) {
+            h.from = slot + 1u;
+            if (++h.retries > P.max_retries) give_up(h, C, sink, tag, tally);
         }
     }
 }
 
-// Feed the wave's idle groups from input indexes [next, end), advancing next; returns when every
-// group is busy or the range is used up (some groups may then still be idle).
-template <int G, bool FROM_ENTRIES, bool COH = false>
-__device__ inline void refill(const Desc &D, Carry<kSlots / G> &c, uint64_t &next, uint64_t end, const uint32_t *__restrict__ keys,
-                              const uint32_t *__restrict__ vals, const uint64_t *__restrict__ entries,
-                              uint32_t pre_fixed, InsertTally &tally, uint64_t &taken,
-                              const uint8_t *__restrict__ skip = nullptr, uint32_t *chain = nullptr)
-{
-    const int lane = __lane_id();
-    const int g = lane / G, s = lane % G;
-    while (next < end) {
-        const uint64_t idle = __ballot(!c.active && s == 0);  // bit g*G for every idle group
-        if (!idle) return;
-        const uint64_t avail = end - next;
-        const uint32_t nidle = (uint32_t)__popcll(idle);
-        const uint32_t take = (uint32_t)(avail < nidle ? avail : nidle);
-        const uint32_t rank = (uint32_t)__popcll(idle & ((1ull << (g * G)) - 1ull));
-        if (!c.active && rank < take) {
-            const uint64_t idx = next + rank;
+// A wave's way through its input. Input is keys/vals[i], or packed entries[i] (FROM_ENTRIES; a zero
+// entry is an empty place). run() inserts the indexes of chunks first, first + stride, ... of 64
+// within [begin, end) and returns when every chain has ended; the lanes are idle before and after.
+// COH: read the inputs device-coherently (load_in).
+template <bool FROM_ENTRIES, bool COH = false>
+struct InsertRange {
+    const uint32_t *keys, *vals;
+    const uint64_t *entries;
+    const uint8_t *skip;  // keys: skip[i] != 0 leaves key i out. entries: tile flags (see insert_kernel)
+    uint32_t pre_fixed;   // entries: previous table of every entry, kNoTable (the start rule) or kAfterFill
+    unsigned long long taken = 0;  // indexes taken in (wave-uniform)
+
+    // input i of the lane (key 0 for an index left out)
+    __device__ void load(uint64_t i, bool in, uint32_t &k, uint32_t &v, bool &left_out) const
+    {
+        k = v = 0;
+        left_out = false;
+        if (!in) return;
+        if constexpr (FROM_ENTRIES) {
+            const uint64_t e = entries[i];
+            k = key_of(e);
+            v = val_of(e);
+            left_out = e == 0;
+        } else {
+            k = load_in<COH>(keys + i);
+            v = load_in<COH>(vals + i);
+            left_out = skip && skip[i];
+        }
+    }
+
+    __device__ void run(const Desc &D, uint64_t begin, uint64_t end, uint64_t first, uint64_t stride,
+                        const InsertPolicy &P, Counters *C, const PendSink &sink, uint32_t tag, InsertTally &tally)
+    {
+        const uint32_t lane = __lane_id();
+        Hand h{};
+        uint32_t bk = 0, bv = 0;        // the chunk being handed out
+        uint64_t base = 0;              // its first index
+        uint32_t pos = 0, len = 0;      // handed out up to pos of len
+        uint32_t nk = 0, nv = 0;        // the chunk loaded ahead
+        bool nleft = false;
+        uint64_t nbase = begin + first * kWave;
+        auto fetch = [&]() {
             if constexpr (FROM_ENTRIES) {
-                const uint64_t e = entries[idx];
-                if (e)
-                    carry_start(D, c, e, pre_fixed, s, tally, idx, chain);
-                else if (s == 0)
-                    ++tally.empty;
-            } else if (!skip || !skip[idx])
-                carry_start(D, c, pack(load_in<COH>(keys + idx), load_in<COH>(vals + idx)), kNoTable, s, tally, idx,
-                            chain);
-            else if (chain && s == 0)
-                chain[idx] = 0;
+                // a residual list's dead tiles (skip flag 0, a chunk lies inside one tile): find
+                // the next live chunk 64 at a time
+                while (skip && nbase < end) {
+                    const uint64_t b = nbase + (uint64_t)lane * stride * kWave;
+                    const uint64_t live = __ballot(b < end && skip[b / kResTileEntries]);
+                    if (live) {
+                        nbase += (uint64_t)__builtin_ctzll(live) * stride * kWave;
+                        break;
+                    }
+                    nbase += (uint64_t)kWave * stride * kWave;
+                }
+            }
+            load(nbase + lane, nbase + lane < end, nk, nv, nleft);
+        };
+        if (nbase < end) fetch();
+        while (true) {
+            while (true) {  // hand entries to idle lanes
+                if (pos == len) {
+                    if (nbase >= end) break;
+                    base = nbase;
+                    len = end - base < kWave ? (uint32_t)(end - base) : (uint32_t)kWave;
+                    pos = 0;
+                    taken += len;
+                    bk = nk;
+                    bv = nv;
+                    const uint64_t left = __ballot(lane < len && nleft);
+                    if constexpr (FROM_ENTRIES) tally.empty += __popcll(left);
+                    const bool bad = lane < len && !nleft && reserved_key(bk);
+                    tally.rejected += __popcll(__ballot(bad));
+                    if (sink.chain && lane < len && (nleft || bad)) sink.chain[base + lane] = 0;
+                    if (nleft || bad) bk = 0;
+                    nbase += stride * kWave;
+                    if (nbase < end) fetch();
+                }
+                const uint64_t idle = __ballot(!h.active);
+                if (!idle) break;
+                const uint32_t room = (uint32_t)__popcll(idle);
+                const uint32_t take = len - pos < room ? len - pos : room;
+                const uint32_t rank = (uint32_t)__popcll(idle & lanemask_lt());
+                const uint32_t src = (pos + rank) & 63u;
+                const uint32_t k = __shfl(bk, src), v = __shfl(bv, src);
+                if (!h.active && rank < take && k != 0u) {
+                    h.k = k;
+                    h.v = v;
+                    h.idx = base + src;
+                    h.pre = pre_fixed == kAfterFill ? fill_target(D, k, pair_of(D, k)) : pre_fixed;
+                    h.fresh = pre_fixed == kNoTable;
+                    if (h.fresh && (k & 1u)) h.pre = kOddStart;
+                    h.kicks = h.retries = h.from = 0;
+                    h.active = true;
+                }
+                pos += take;
+            }
+            if (!__ballot(h.active)) break;  // input used up and every lane idle
+            insert_step(D, h, P, C, sink, tag, tally);
         }
-        next += take;
-        taken += take;
+    }
+};
+
+// The wave's tallies into its stripe.
+__device__ inline void tally_out(Counters *C, const InsertTally &tally)
+{
+    const uint32_t slot = wave_slot();
+    if (__lane_id() == 0) {
+        if (tally.kicks) tally_add(C, &C->kicks, tally.kicks, slot);
+        if (tally.rejected) tally_add(C, &C->rejected, tally.rejected, slot);
+        if (tally.retries) tally_add(C, &C->retries, tally.retries, slot);
     }
 }
 
 // skip (optional): a keys insert leaves out key i where skip[i] != 0; an entries insert reads it
 // as the tile flags of a slot-addressed residual list (entries of a tile flagged 0 are empty).
-template <int G, bool FROM_ENTRIES>
+// n_dev (optional): the input ends at *n_dev if that is less than n.
+template <bool FROM_ENTRIES>
 __global__ __launch_bounds__(256) void insert_kernel(Desc D, const uint32_t *__restrict__ keys,
                                                      const uint32_t *__restrict__ vals,
                                                      const uint64_t *__restrict__ entries, uint64_t n,
                                                      uint32_t pre_fixed, InsertPolicy P, Counters *__restrict__ C,
-                                                     PendSink sink, const uint8_t *__restrict__ skip)
+                                                     PendSink sink, const uint8_t *__restrict__ skip,
+                                                     const unsigned long long *__restrict__ n_dev)
 {
-    constexpr int NG = kWave / G;
-    constexpr uint64_t kChunk = 2 * NG;  // indexes a wave takes at a time
-    static_assert(kResTileEntries % kChunk == 0, "a chunk lies inside one residual tile");
-    Carry<kSlots / G> c;
-    c.active = false;
+    static_assert(kResTileEntries % kWave == 0, "a chunk lies inside one residual tile");
     InsertTally tally;
-    const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x / kWave);
-    uint64_t next_chunk = (uint64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
-    uint64_t next = 0, end = 0;  // wave-uniform: the wave's current chunk
-    uint64_t taken = 0;          // wave-uniform: input indexes this wave took
-    while (true) {
-        refill<G, FROM_ENTRIES>(D, c, next, end, keys, vals, entries, pre_fixed, tally, taken, skip, sink.chain);
-        if (next == end) {
-            // chunks w, w + W, w + 2W, ... (W = waves in the grid)
-            const uint64_t base = next_chunk * kChunk;
-            if (base < n) {
-                next_chunk += waves;
-                // an entries insert reads skip as the tile flags of a slot-addressed list; a chunk
-                // lies inside one tile, and a tile flagged 0 holds no entry
-                if constexpr (FROM_ENTRIES)
-                    if (skip && !skip[base / kResTileEntries]) continue;
-                next = base;
-                end = base + kChunk < n ? base + kChunk : n;
-                continue;
-            }
-        }
-        if (!__ballot(c.active)) break;  // input exhausted and every group idle
-        if (c.active) kick_step<G>(D, c, P, C, sink, sink.tag, tally);
-    }
+    if (n_dev) n = min((unsigned long long)n, *n_dev);
+    InsertRange<FROM_ENTRIES> in{keys, vals, entries, skip, pre_fixed};
+    in.run(D, 0, n, wave_slot(), (uint64_t)gridDim.x * (blockDim.x / kWave), P, C, sink, sink.tag, tally);
+    if (FROM_ENTRIES && pre_fixed == kAfterFill && __lane_id() == 0 && in.taken > tally.direct)
+        tally_add(C, &C->left, in.taken - tally.direct, wave_slot());
     if (sink.count_placed || sink.rejected_at) {
-        const unsigned long long rej = wave_sum(tally.rejected);
-        const unsigned long long skipped = rej + wave_sum(tally.empty);
+        const unsigned long long skipped = tally.rejected + tally.empty;
         if (__lane_id() == 0) {
-            if (sink.count_placed && taken > skipped) tally_add(C, &C->placed, taken - skipped, wave_slot());
-            if (sink.rejected_at && rej) atomicAdd(sink.rejected_at, rej);
+            if (sink.count_placed && in.taken > skipped)
+                tally_add(C, &C->placed, in.taken - skipped, wave_slot());
+            if (sink.rejected_at && tally.rejected) atomicAdd(sink.rejected_at, tally.rejected);
         }
     }
-    wave_tally(C, &C->kicks, tally.kicks);
-    wave_tally(C, &C->rejected, tally.rejected);
-    wave_tally(C, &C->retries, tally.retries);
+    tally_out(C, tally);
     wave_tally_max(C, &C->max_chain, tally.max_chain);
 }
 
@@ -845,42 +917,36 @@ __global__ __launch_bounds__(256, W) void group_probe_kernel(const Desc *__restr
     }
 }
 
-// Groups of one wave share an item: they are fed from it until it is used up, and the wave
-// moves on only when all its groups have placed (or pended) their entries. FROM_ENTRIES: the
-// items index packed entries (a bulk fill's overflow) instead of keys/vals.
-template <int G, int W, bool FROM_ENTRIES = false>
+// A wave takes an item's entries in chunks and moves on only when all its lanes have placed (or
+// pended) theirs. FROM_ENTRIES: the items index a bulk fill's overflow (packed entries) instead of
+// keys/vals, and there are *n_dev of them if that is less than n_items.
+template <int W, bool FROM_ENTRIES = false>
 __global__ __launch_bounds__(256, W) void group_insert_kernel(const Desc *__restrict__ dir,
                                                            const GroupItem *__restrict__ items, uint32_t n_items,
                                                            const uint32_t *__restrict__ keys,
                                                            const uint32_t *__restrict__ vals, InsertPolicy P,
                                                            Counters *__restrict__ C, PendSink sink,
                                                            unsigned long long *__restrict__ table_counts,
-                                                           const uint64_t *__restrict__ entries = nullptr)
+                                                           const uint64_t *__restrict__ entries,
+                                                           const unsigned long long *__restrict__ n_dev)
 {
-    Carry<kSlots / G> c;
-    c.active = false;
     InsertTally tally;
+    unsigned long long taken = 0;
+    if constexpr (FROM_ENTRIES) n_items = (uint32_t)min((unsigned long long)n_items, *n_dev);
     const uint32_t waves = gridDim.x * (blockDim.x / kWave);
-    for (uint32_t it = wave_uniform(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave); it < n_items;
-         it += waves) {
+    for (uint32_t it = wave_slot(); it < n_items; it += waves) {
         const GroupItem item = items[it];
-        if (item.len == 0) continue;  // wave-uniform: a block the bulk fill's rounds emptied
         const Desc D = as_global(dir[item.table]);
-        uint64_t next = item.begin;
-        const uint64_t end = item.begin + item.len;
         const unsigned long long rej0 = tally.rejected;
-        uint64_t taken = 0;
-        while (true) {
-            refill<G, FROM_ENTRIES>(D, c, next, end, keys, vals, entries, kNoTable, tally, taken);
-            if (!__ballot(c.active)) break;  // item used up and every group idle
-            if (c.active) kick_step<G>(D, c, P, C, sink, item.table, tally);
-        }
-        const unsigned long long rej = wave_sum(tally.rejected - rej0);
+        InsertRange<FROM_ENTRIES> in{keys, vals, entries, nullptr, FROM_ENTRIES ? kAfterFill : kNoTable};
+        in.run(D, item.begin, item.begin + item.len, 0, 1, P, C, sink, item.table, tally);
+        taken += in.taken;
+        const unsigned long long rej = tally.rejected - rej0;
         if (__lane_id() == 0 && item.len > rej) atomicAdd(&table_counts[item.table], item.len - rej);
     }
-    wave_tally(C, &C->kicks, tally.kicks);
-    wave_tally(C, &C->rejected, tally.rejected);
-    wave_tally(C, &C->retries, tally.retries);
+    if (FROM_ENTRIES && __lane_id() == 0 && taken > tally.direct)
+        tally_add(C, &C->left, taken - tally.direct, wave_slot());
+    tally_out(C, tally);
 }
 
 // ------------------------------------------------------------------------------ serving
@@ -942,23 +1008,15 @@ __device__ inline unsigned long long serve_probe_item(const Desc &D, const Serve
     return nd;
 }
 
-// One item of inserts; the wave's groups are all idle on return. COH: read the inputs
-// device-coherently (load_in).
-template <int G, bool COH = false>
-__device__ inline unsigned long long serve_insert_item(const Desc &D, const ServeItem &item, Carry<kSlots / G> &c,
-                                                       const InsertPolicy &P, Counters *C, const PendSink &sink,
-                                                       InsertTally &tally)
+// One item of inserts. COH: read the inputs device-coherently (load_in).
+template <bool COH = false>
+__device__ inline unsigned long long serve_insert_item(const Desc &D, const ServeItem &item, const InsertPolicy &P,
+                                                       Counters *C, const PendSink &sink, InsertTally &tally)
 {
-    uint64_t next = 0;
-    const uint64_t end = item.len;
     const unsigned long long rej0 = tally.rejected;
-    uint64_t taken = 0;
-    while (true) {
-        refill<G, false, COH>(D, c, next, end, item.keys, item.vals, nullptr, kNoTable, tally, taken);
-        if (!__ballot(c.active)) break;
-        if (c.active) kick_step<G>(D, c, P, C, sink, item.table, tally);
-    }
-    const unsigned long long rej = wave_sum(tally.rejected - rej0);
+    InsertRange<false, COH> in{item.keys, item.vals, nullptr, nullptr, kNoTable};
+    in.run(D, 0, item.len, 0, 1, P, C, sink, item.table, tally);
+    const unsigned long long rej = tally.rejected - rej0;
     return item.len > rej ? item.len - rej : 0;  // entries the item took in (wave-uniform)
 }
 
@@ -1002,26 +1060,21 @@ __global__ __launch_bounds__(256) void serve_probe_kernel(const Desc *__restrict
     if constexpr (ERASE) del.flush(del_total);
 }
 
-template <int G>
 __global__ __launch_bounds__(256) void serve_insert_kernel(const Desc *__restrict__ dir,
                                                            const ServeItem *__restrict__ items, uint32_t n_items,
                                                            InsertPolicy P, Counters *__restrict__ C, PendSink sink,
                                                            unsigned long long *__restrict__ ins_total)
 {
-    Carry<kSlots / G> c;
-    c.active = false;
     InsertTally tally;
     WaveTotal ins;
     const uint32_t waves = gridDim.x * (blockDim.x / kWave);
     for (uint32_t it = wave_uniform(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave); it < n_items;
          it += waves) {
         const ServeItem item = as_global(items[it]);
-        ins.add(ins_total, item.table, serve_insert_item<G>(as_global(dir[item.table]), item, c, P, C, sink, tally));
+        ins.add(ins_total, item.table, serve_insert_item(as_global(dir[item.table]), item, P, C, sink, tally));
     }
     ins.flush(ins_total);
-    wave_tally(C, &C->kicks, tally.kicks);
-    wave_tally(C, &C->rejected, tally.rejected);
-    wave_tally(C, &C->retries, tally.retries);
+    tally_out(C, tally);
 }
 
 // A whole serving tick in one launch. Waves claim items in list order from a counter; an item
@@ -1034,7 +1087,6 @@ __global__ __launch_bounds__(256) void serve_insert_kernel(const Desc *__restric
 // running waves, so the earliest unfinished item never waits and the launch always drains. The
 // wait is bounded all the same: past spin_cap polls the wave records a stall and goes on (the
 // host reports the tick failed).
-template <int GI>
 __global__ __launch_bounds__(256) void serve_tick_kernel(const Desc *__restrict__ dir, const TickItem *__restrict__ items,
                                                          uint32_t n_items, unsigned long long *__restrict__ cursor,
                                                          TickStages stages, InsertPolicy P, Counters *__restrict__ C,
@@ -1043,8 +1095,6 @@ __global__ __launch_bounds__(256) void serve_tick_kernel(const Desc *__restrict_
                                                          unsigned long long *__restrict__ del_total, uint32_t spin_cap,
                                                          uint32_t max_back)
 {
-    Carry<kSlots / GI> c;
-    c.active = false;
     InsertTally tally;
     WaveTotal ins, del;
     unsigned long long stalls = 0;
@@ -1073,7 +1123,7 @@ __global__ __launch_bounds__(256) void serve_tick_kernel(const Desc *__restrict_
         }
         const Desc D = as_global(dir[ti.item.table]);
         if (ti.op == 0) {
-            ins.add(ins_total, ti.item.table, serve_insert_item<GI>(D, ti.item, c, P, C, sink, tally));
+            ins.add(ins_total, ti.item.table, serve_insert_item(D, ti.item, P, C, sink, tally));
         } else {
             // an item that waited reads what earlier stages of this launch wrote: coherently;
             // a table's first stage reads what earlier launches wrote: through the caches
@@ -1100,9 +1150,7 @@ __global__ __launch_bounds__(256) void serve_tick_kernel(const Desc *__restrict_
     }
     ins.flush(ins_total);
     del.flush(del_total);
-    wave_tally(C, &C->kicks, tally.kicks);
-    wave_tally(C, &C->rejected, tally.rejected);
-    wave_tally(C, &C->retries, tally.retries);
+    tally_out(C, tally);
     if (__lane_id() == 0 && stalls) tally_add(C, &C->stalls, stalls, wave_slot());
 }
 
@@ -1201,7 +1249,6 @@ __device__ inline void loop_front(const LoopArgs &A)
     if (__lane_id() == 0) __hip_atomic_store(A.words + kLoopQuit, 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int GI>
 __global__ __launch_bounds__(256) void serve_loop_kernel(LoopArgs A, InsertPolicy P, Counters *__restrict__ C,
                                                          PendSink sink, Pool pool,
                                                          unsigned long long *__restrict__ ins_total,
@@ -1211,8 +1258,6 @@ __global__ __launch_bounds__(256) void serve_loop_kernel(LoopArgs A, InsertPolic
         loop_front(A);
         return;
     }
-    Carry<kSlots / GI> c;
-    c.active = false;
     InsertTally tally;
     WaveTotal ins, del;
     const int lane = __lane_id();
@@ -1273,7 +1318,7 @@ __global__ __launch_bounds__(256) void serve_loop_kernel(LoopArgs A, InsertPolic
         }
         unsigned long long acc;
         if (it.op == 0) {
-            acc = serve_insert_item<GI, true>(D, it.item, c, P, C, sink, tally);
+            acc = serve_insert_item<true>(D, it.item, P, C, sink, tally);
             ins.add(ins_total, table, acc);
         } else {
             const uint64_t np = pool_size(pool);
@@ -1319,9 +1364,7 @@ __global__ __launch_bounds__(256) void serve_loop_kernel(LoopArgs A, InsertPolic
     }
     ins.flush(ins_total);
     del.flush(del_total);
-    wave_tally(C, &C->kicks, tally.kicks);
-    wave_tally(C, &C->rejected, tally.rejected);
-    wave_tally(C, &C->retries, tally.retries);
+    tally_out(C, tally);
 }
 
 __global__ void loop_reset_kernel(unsigned long long *words)
@@ -1413,44 +1456,21 @@ hipError_t launch_erase(const Desc &D, const uint32_t *keys, uint8_t *deleted, u
 
 template <bool FE>
 static hipError_t insert_common(const Desc &D, const uint32_t *keys, const uint32_t *vals, const uint64_t *entries,
-                                uint64_t n, uint32_t pre, int lanes,
-                                InsertPolicy pol, LaunchShape sh, Counters *C, PendSink sink, hipStream_t st,
-                                const uint8_t *skip = nullptr)
+                                uint64_t n, uint32_t pre, InsertPolicy pol, LaunchShape sh, Counters *C, PendSink sink,
+                                hipStream_t st, const uint8_t *skip, const unsigned long long *n_dev = nullptr)
 {
     if (n == 0) return hipSuccess;
-    const int per_wave = kWave / lanes;  // entries in flight per wave
-    const uint64_t work_waves = (n + per_wave - 1) / per_wave;
+    const uint64_t work_waves = (n + kWave - 1) / kWave;
     const int grid = grid_for(work_waves, sh, insert_default_cap(work_waves, sh));
-    switch (lanes) {
-    case 8:
-        insert_kernel<8, FE><<<grid, sh.block_threads, 0, st>>>(D, keys, vals, entries, n, pre, pol, C,
-                                                                      sink, skip);
-        break;
-    case 4:
-        insert_kernel<4, FE><<<grid, sh.block_threads, 0, st>>>(D, keys, vals, entries, n, pre, pol, C,
-                                                                      sink, skip);
-        break;
-    case 2:
-        insert_kernel<2, FE><<<grid, sh.block_threads, 0, st>>>(D, keys, vals, entries, n, pre, pol, C,
-                                                                      sink, skip);
-        break;
-    case 1:
-        insert_kernel<1, FE><<<grid, sh.block_threads, 0, st>>>(D, keys, vals, entries, n, pre, pol, C,
-                                                                      sink, skip);
-        break;
-    default:
-        insert_kernel<16, FE><<<grid, sh.block_threads, 0, st>>>(D, keys, vals, entries, n, pre, pol, C,
-                                                                      sink, skip);
-        break;
-    }
+    insert_kernel<FE><<<grid, sh.block_threads, 0, st>>>(D, keys, vals, entries, n, pre, pol, C, sink, skip, n_dev);
     return hipGetLastError();
 }
 
-hipError_t launch_insert(const Desc &D, const uint32_t *keys, const uint32_t *vals, uint64_t n, int lanes,
-                         InsertPolicy pol, LaunchShape sh, Counters *C, PendSink sink, hipStream_t st,
+hipError_t launch_insert(const Desc &D, const uint32_t *keys, const uint32_t *vals, uint64_t n, InsertPolicy pol,
+                         LaunchShape sh, Counters *C, PendSink sink, hipStream_t st,
                          const uint8_t *skip)
 {
-    return insert_common<false>(D, keys, vals, nullptr, n, kNoTable, lanes, pol, sh, C, sink, st, skip);
+    return insert_common<false>(D, keys, vals, nullptr, n, kNoTable, pol, sh, C, sink, st, skip);
 }
 
 hipError_t launch_update(const Desc &D, const uint32_t *keys, const uint32_t *vals, uint8_t *updated, uint64_t n,
@@ -1464,11 +1484,17 @@ hipError_t launch_update(const Desc &D, const uint32_t *keys, const uint32_t *va
     return hipGetLastError();
 }
 
-hipError_t launch_insert_entries(const Desc &D, const uint64_t *entries, uint64_t n, uint32_t pre, int lanes,
-                                 InsertPolicy pol, LaunchShape sh, Counters *C, PendSink sink, hipStream_t st,
+hipError_t launch_insert_entries(const Desc &D, const uint64_t *entries, uint64_t n, uint32_t pre, InsertPolicy pol,
+                                 LaunchShape sh, Counters *C, PendSink sink, hipStream_t st,
                                  const uint8_t *live)
 {
-    return insert_common<true>(D, nullptr, nullptr, entries, n, pre, lanes, pol, sh, C, sink, st, live);
+    return insert_common<true>(D, nullptr, nullptr, entries, n, pre, pol, sh, C, sink, st, live);
+}
+
+hipError_t launch_insert_overflow(const Desc &D, const uint64_t *ovf, uint64_t n, InsertPolicy pol, LaunchShape sh,
+                                  Counters *C, PendSink sink, hipStream_t st)
+{
+    return insert_common<true>(D, nullptr, nullptr, ovf, n, kAfterFill, pol, sh, C, sink, st, nullptr, &C->overflow);
 }
 
 hipError_t launch_partition(const Desc &D, const Regions &M, const uint32_t *keys, const uint32_t *vals, uint64_t n,
@@ -1546,45 +1572,38 @@ hipError_t launch_group_erase(const Desc *dir, const GroupItem *items, uint32_t 
     return hipGetLastError();
 }
 
-template <int G>
-static void group_insert_w(int wpe, int grid, hipStream_t st, const Desc *dir, const GroupItem *items,
-                           uint32_t n_items, const uint32_t *keys, const uint32_t *vals, InsertPolicy pol, Counters *C,
-                           PendSink sink, unsigned long long *table_counts, const uint64_t *entries)
-{
-    if (entries) {  // a bulk fill's overflow: the compiler's occupancy only
-        group_insert_kernel<G, 1, true>
-            <<<grid, 256, 0, st>>>(dir, items, n_items, nullptr, nullptr, pol, C, sink, table_counts, entries);
-        return;
-    }
-    switch (wpe) {
-    case 6:
-        group_insert_kernel<G, 6><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts);
-        break;
-    case 8:
-        group_insert_kernel<G, 8><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts);
-        break;
-    default:
-        group_insert_kernel<G, 1><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts);
-        break;
-    }
-}
-
 hipError_t launch_group_insert(const Desc *dir, const GroupItem *items, uint32_t n_items, const uint32_t *keys,
-                               const uint32_t *vals, InsertPolicy pol, int lanes, int blocks, Counters *C,
-                               PendSink sink, unsigned long long *table_counts, hipStream_t st, int waves_per_eu,
-                               const uint64_t *entries)
+                               const uint32_t *vals, InsertPolicy pol, int blocks, Counters *C, PendSink sink,
+                               unsigned long long *table_counts, hipStream_t st, int waves_per_eu)
 {
     if (n_items == 0) return hipSuccess;
     const int grid = blocks > 0 ? blocks : std::min<int>(kGroupDefaultBlocks, (int)((n_items + 3) / 4));
-    const int w = waves_per_eu;
-    const uint64_t *const e = entries;
-    switch (lanes) {
-    case 2: group_insert_w<2>(w, grid, st, dir, items, n_items, keys, vals, pol, C, sink, table_counts, e); break;
-    case 4: group_insert_w<4>(w, grid, st, dir, items, n_items, keys, vals, pol, C, sink, table_counts, e); break;
-    case 8: group_insert_w<8>(w, grid, st, dir, items, n_items, keys, vals, pol, C, sink, table_counts, e); break;
-    case 16: group_insert_w<16>(w, grid, st, dir, items, n_items, keys, vals, pol, C, sink, table_counts, e); break;
-    default: group_insert_w<1>(w, grid, st, dir, items, n_items, keys, vals, pol, C, sink, table_counts, e); break;
+    switch (waves_per_eu) {
+    case 6:
+        group_insert_kernel<6><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts,
+                                                       nullptr, nullptr);
+        break;
+    case 8:
+        group_insert_kernel<8><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts,
+                                                       nullptr, nullptr);
+        break;
+    default:
+        group_insert_kernel<1><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts,
+                                                       nullptr, nullptr);
+        break;
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_group_insert_overflow(const Desc *dir, const GroupItem *items, const unsigned long long *n_items,
+                                        uint64_t max_items, const uint64_t *ovf, InsertPolicy pol, int blocks,
+                                        Counters *C, PendSink sink, unsigned long long *table_counts, hipStream_t st)
+{
+    if (max_items == 0) return hipSuccess;
+    if (max_items > 0xffffffffull) return hipErrorInvalidValue;
+    const int grid = blocks > 0 ? blocks : (int)std::min<uint64_t>(kGroupDefaultBlocks, (max_items + 3) / 4);
+    group_insert_kernel<1, true><<<grid, 256, 0, st>>>(dir, items, (uint32_t)max_items, nullptr, nullptr, pol, C, sink,
+                                                       table_counts, ovf, n_items);
     return hipGetLastError();
 }
 
@@ -1624,18 +1643,12 @@ hipError_t launch_serve_erase(const Desc *dir, const ServeItem *items, uint32_t 
     return hipGetLastError();
 }
 
-hipError_t launch_serve_insert(const Desc *dir, const ServeItem *items, uint32_t n_items, InsertPolicy pol, int lanes,
-                               int blocks, Counters *C, PendSink sink, unsigned long long *ins_total, hipStream_t st)
+hipError_t launch_serve_insert(const Desc *dir, const ServeItem *items, uint32_t n_items, InsertPolicy pol, int blocks,
+                               Counters *C, PendSink sink, unsigned long long *ins_total, hipStream_t st)
 {
     if (n_items == 0) return hipSuccess;
     const int grid = serve_grid(n_items, blocks);
-    switch (lanes) {
-    case 2: serve_insert_kernel<2><<<grid, 256, 0, st>>>(dir, items, n_items, pol, C, sink, ins_total); break;
-    case 4: serve_insert_kernel<4><<<grid, 256, 0, st>>>(dir, items, n_items, pol, C, sink, ins_total); break;
-    case 8: serve_insert_kernel<8><<<grid, 256, 0, st>>>(dir, items, n_items, pol, C, sink, ins_total); break;
-    case 16: serve_insert_kernel<16><<<grid, 256, 0, st>>>(dir, items, n_items, pol, C, sink, ins_total); break;
-    default: serve_insert_kernel<1><<<grid, 256, 0, st>>>(dir, items, n_items, pol, C, sink, ins_total); break;
-    }
+    serve_insert_kernel<<<grid, 256, 0, st>>>(dir, items, n_items, pol, C, sink, ins_total);
     return hipGetLastError();
 }
 
@@ -1654,20 +1667,8 @@ hipError_t launch_serve_tick(const Desc *dir, const TickItem *items, uint32_t n_
     if (!serve_tick_supported(insert_lanes, find_lanes)) return hipErrorInvalidValue;
     if (max_back == 0) max_back = 1;
     const int grid = serve_grid(n_items, blocks);
-    switch (insert_lanes) {
-    case 2:
-        serve_tick_kernel<2><<<grid, 256, 0, st>>>(dir, items, n_items, cursor, done, pol, C, sink, pool, ins_total,
-                                                   del_total, spin_cap, max_back);
-        break;
-    case 4:
-        serve_tick_kernel<4><<<grid, 256, 0, st>>>(dir, items, n_items, cursor, done, pol, C, sink, pool, ins_total,
-                                                   del_total, spin_cap, max_back);
-        break;
-    default:
-        serve_tick_kernel<1><<<grid, 256, 0, st>>>(dir, items, n_items, cursor, done, pol, C, sink, pool, ins_total,
-                                                   del_total, spin_cap, max_back);
-        break;
-    }
+    serve_tick_kernel<<<grid, 256, 0, st>>>(dir, items, n_items, cursor, done, pol, C, sink, pool, ins_total, del_total,
+                                            spin_cap, max_back);
     return hipGetLastError();
 }
 
@@ -1676,11 +1677,7 @@ hipError_t launch_serve_loop(const LoopArgs &A, InsertPolicy pol, int insert_lan
                              unsigned long long *del_total, hipStream_t st)
 {
     if (!serve_tick_supported(insert_lanes, find_lanes) || blocks < 2) return hipErrorInvalidValue;
-    switch (insert_lanes) {
-    case 2: serve_loop_kernel<2><<<blocks, 256, 0, st>>>(A, pol, C, sink, pool, ins_total, del_total); break;
-    case 4: serve_loop_kernel<4><<<blocks, 256, 0, st>>>(A, pol, C, sink, pool, ins_total, del_total); break;
-    default: serve_loop_kernel<1><<<blocks, 256, 0, st>>>(A, pol, C, sink, pool, ins_total, del_total); break;
-    }
+    serve_loop_kernel<<<blocks, 256, 0, st>>>(A, pol, C, sink, pool, ins_total, del_total);
     return hipGetLastError();
 }
 
@@ -1690,30 +1687,15 @@ hipError_t launch_loop_reset(unsigned long long *words, hipStream_t st)
     return hipGetLastError();
 }
 
-template <int GI>
-static int loop_blocks_per_cu()
-{
-    int per = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, serve_loop_kernel<GI>, 256, 0) != hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
-    }
-    return per;
-}
-
 int serve_loop_capacity(int insert_lanes, int find_lanes)
 {
     if (!serve_tick_supported(insert_lanes, find_lanes)) return 0;
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+    int dev = 0, cus = 0, per = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, serve_loop_kernel, 256, 0) != hipSuccess) {
         (void)hipGetLastError();
         return 0;
-    }
-    int per = 0;
-    switch (insert_lanes) {
-    case 2: per = loop_blocks_per_cu<2>(); break;
-    case 4: per = loop_blocks_per_cu<4>(); break;
-    default: per = loop_blocks_per_cu<1>(); break;
     }
     return per * cus;
 }

@@ -27,7 +27,9 @@ struct Counters {
     unsigned long long residuals;  // downsize: entries of the upper half that did not stay
     unsigned long long placed;     // insert with PendSink::count_placed: entries taken in
     unsigned long long max_chain;  // insert: the longest eviction chain (exchanges); folded by max
-    unsigned long long pad[3];
+    unsigned long long overflow;   // bulk fill: entries appended to the overflow list (append index)
+    unsigned long long left;       // bulk fill: entries placed by evicting others, or parked
+    unsigned long long pad[1];
 };
 constexpr int kMaxChainWord = 12;  // index of max_chain: stripes fold into it by max, not by sum
 static_assert(offsetof(Counters, max_chain) == kMaxChainWord * sizeof(unsigned long long), "max_chain's word");
@@ -87,9 +89,8 @@ hipError_t launch_erase(const Desc &D, const uint32_t *keys, uint8_t *deleted, u
 // insert keys/vals (start rule of cuckoo.cu:336-341) or packed entries with a fixed previous
 // table `pre` (kNoTable = use the key-parity start rule).
 // skip (optional): skip[i] != 0 leaves keys[i] out (an upsert already updated it in place).
-hipError_t launch_insert(const Desc &D, const uint32_t *keys, const uint32_t *vals, uint64_t n, int lanes,
-                         InsertPolicy pol, LaunchShape sh, Counters *C, PendSink sink, hipStream_t st,
-                         const uint8_t *skip = nullptr);
+hipError_t launch_insert(const Desc &D, const uint32_t *keys, const uint32_t *vals, uint64_t n, InsertPolicy pol,
+                         LaunchShape sh, Counters *C, PendSink sink, hipStream_t st, const uint8_t *skip = nullptr);
 // update in place: every copy of keys[i] in the first bucket (pos1, then pos2) that holds it
 // takes the value vals[i] (with a pool: failing that, every copy in the pool); updated[i] = 1 if
 // there was one; the count goes to C->updated.
@@ -98,8 +99,8 @@ hipError_t launch_update(const Desc &D, const uint32_t *keys, const uint32_t *va
 // A zero entry is an empty place (an erased pending entry, a slot without a residual): skipped,
 // and counted neither as rejected nor as placed. live (optional, a slot-addressed residual list's
 // tile flags from launch_downsize): entries of a tile whose byte is 0 are empty and not read.
-hipError_t launch_insert_entries(const Desc &D, const uint64_t *entries, uint64_t n, uint32_t pre, int lanes,
-                                 InsertPolicy pol, LaunchShape sh, Counters *C, PendSink sink, hipStream_t st,
+hipError_t launch_insert_entries(const Desc &D, const uint64_t *entries, uint64_t n, uint32_t pre, InsertPolicy pol,
+                                 LaunchShape sh, Counters *C, PendSink sink, hipStream_t st,
                                  const uint8_t *live = nullptr);
 // ---- bulk insert by bucket fill (insert_order 3)
 // A chunk is kChunkBuckets consecutive buckets of one subtable; chunk ids of subtable t start
@@ -143,19 +144,22 @@ size_t bulk_cid_bytes(const Chunks &Ch);
 // (8192-entry tiles, or 4096) and three per CU measured slower.
 constexpr uint32_t kBulkSortBlocks = 512;
 constexpr uint32_t kWideSortBlocks = 512;
-// Group n entries by chunk (n < 2^32): round 1 from keys/vals for each key's fill_target bucket
-// (keys != nullptr; reserved keys go to chunk 0), round 2 from the entries in ws.ent[in] for the
-// other bucket of the pair. The sorted entries end in ws.ent[*out] (the round-2 input buffer is
-// reused), and ws.start receives the first index of every chunk.
-hipError_t launch_bulk_partition(const Desc &D, const Chunks &Ch, const uint32_t *keys, const uint32_t *vals, int in,
+// Group the n entries keys/vals (n < 2^32) by the chunk of each key's fill_target bucket (reserved
+// keys go to chunk 0). The sorted entries end in ws.ent[*out], and ws.start receives the first
+// index of every chunk.
+hipError_t launch_bulk_partition(const Desc &D, const Chunks &Ch, const uint32_t *keys, const uint32_t *vals,
                                  uint64_t n, const BulkSpace &ws, uint32_t max_blocks, hipStream_t st, int *out);
 // Fill free slots chunk by chunk from the partitioned entries (n < 2^32); start holds total + 1
-// words. Entries that do not fit are appended to ovf (*ovf_n, zeroed by the caller, counts them;
-// ovf_cap >= n). Placements go to the kick tally, reserved keys to the rejected tally. zeroed:
-// every slot of the table is zero (a fresh or cleared table), so a dense round need not read it.
+// words. Entries that do not fit are appended to ovf at C->overflow (ovf_cap >= n). Placements go
+// to the kick tally, reserved keys to the rejected tally. zeroed: every slot of the table is zero (a
+// fresh or cleared table), so the fill need not read it.
 hipError_t launch_bulk_fill(const Desc &D, const Chunks &Ch, const uint32_t *start, const uint64_t *ent, uint64_t n,
-                            uint64_t *ovf, uint64_t ovf_cap, unsigned long long *ovf_n, Counters *C, bool zeroed,
-                            hipStream_t st);
+                            uint64_t *ovf, uint64_t ovf_cap, Counters *C, bool zeroed, hipStream_t st);
+// The eviction insert of what a bulk fill of n entries left (ovf[0, C->overflow), read on the
+// device): each entry goes to the other bucket of its pair, evicting if that is full too. Those
+// that had to evict, or were parked, count in C->left.
+hipError_t launch_insert_overflow(const Desc &D, const uint64_t *ovf, uint64_t n, InsertPolicy pol, LaunchShape sh,
+                                  Counters *C, PendSink sink, hipStream_t st);
 // Order an insert batch by the region of its first bucket: out[0, n) receives the packed
 // entries, region by region. counts and cursors are R words each (counts zeroed by the caller).
 hipError_t launch_partition(const Desc &D, const Regions &M, const uint32_t *keys, const uint32_t *vals, uint64_t n,
@@ -181,11 +185,10 @@ hipError_t launch_group_erase(const Desc *dir, const GroupItem *items, uint32_t 
                               hipStream_t st, const Pool *pool = nullptr, int waves_per_eu = 0);
 // insert: failures go to sink.pend with their table index in sink.tags; per-table inserted
 // counts (placed or pended, reserved keys excluded) are added to table_counts.
-// insert: an item's entries are keys/vals[i], or entries[i] (packed) when entries is not null.
 hipError_t launch_group_insert(const Desc *dir, const GroupItem *items, uint32_t n_items, const uint32_t *keys,
-                               const uint32_t *vals, InsertPolicy pol, int lanes, int blocks, Counters *C,
+                               const uint32_t *vals, InsertPolicy pol, int blocks, Counters *C,
                                PendSink sink, unsigned long long *table_counts, hipStream_t st,
-                               int waves_per_eu = 0, const uint64_t *entries = nullptr);
+                               int waves_per_eu = 0);
 
 // ---- bulk fill of many tables (dyc_group.hip, insert_order 3)
 // The batch is grouped by table already (host offsets), so one pass partitions each table's
@@ -221,11 +224,10 @@ struct alignas(16) GroupChunk {
     uint32_t table;    // the table's index in the group (its live count)
 };
 // Per partition block (blocks[b]: one table's range): every key's local chunk into lcid, and the
-// block's count of each local chunk into partial[b * 256 + lc]. Round 1 (entries null): keys,
-// chunk of the fill_target bucket (reserved keys count as chunk 0, whose fill rejects them).
-// Round 2: packed entries (a fill's overflow), chunk of the other bucket of the pair.
+// block's count of each local chunk (of the fill_target bucket; reserved keys count as chunk 0,
+// whose fill rejects them) into partial[b * 256 + lc].
 hipError_t launch_group_bulk_pack(const Desc *dir, const GroupItem *blocks, uint32_t n_blocks, const uint32_t *keys,
-                                  const uint64_t *entries, uint8_t *lcid, uint32_t *partial, hipStream_t st);
+                                  uint8_t *lcid, uint32_t *partial, hipStream_t st);
 // Per table: partial[b * 256 + lc] becomes the place of block b's first entry of chunk lc in the
 // partitioned batch, and chunk c = chunk0 + lc of the call gets its record chunks[c] (subtable
 // from dir[table], entries, overflow region of the table's BulkTable).
@@ -233,26 +235,29 @@ hipError_t launch_group_bulk_scan(const Desc *dir, const BulkTable *tabs, uint32
                                   GroupChunk *chunks, hipStream_t st);
 hipError_t launch_group_bulk_scan(const WideDesc *dir, const BulkTable *tabs, uint32_t n_tabs, uint32_t *partial,
                                   GroupChunk *chunks, hipStream_t st);
-// The pass itself: keys/vals (or packed entries, when not null) of every block to ent[0, n) by
-// local chunk (no stable order).
+// The pass itself: keys/vals of every block to ent[0, n) by local chunk (no stable order).
 hipError_t launch_group_bulk_scatter(const GroupItem *blocks, uint32_t n_blocks, const uint32_t *keys,
-                                     const uint32_t *vals, const uint64_t *entries, const uint8_t *lcid,
-                                     const uint32_t *partial, uint64_t n, uint64_t *ent, hipStream_t st);
-// One workgroup per chunk record of the call (dense: the chunk's image in LDS; sparse: stores
-// into the free slots of the buckets that received entries). Entries that do not fit go to the
-// table's region of ovf, counted in ovf_n[j] (zeroed by the caller). Placements are added to
-// table_counts and to the kick tally, reserved keys to the rejected tally. zeroed (dense only):
-// every slot of every table is zero.
-// The next round's work from this round's overflow counts, on the device (no read-back): block b
-// of blocks (table tabs[btab[b]]) clipped to its table's overflow, out[b] = its part of
-// [off, off + ovf_n[j]); tabs_out (optional) = tabs with n = ovf_n[j]. Blocks past the overflow
-// become empty.
-hipError_t launch_group_bulk_clip(const GroupItem *blocks, const uint32_t *btab, uint32_t n_blocks,
-                                  const BulkTable *tabs, uint32_t n_tabs, const unsigned long long *ovf_n,
-                                  GroupItem *out, BulkTable *tabs_out, hipStream_t st);
+                                     const uint32_t *vals, const uint8_t *lcid, const uint32_t *partial, uint64_t n,
+                                     uint64_t *ent, hipStream_t st);
+// One workgroup per chunk record of the call (the chunk's image in LDS). Entries that do not fit go
+// to the table's region of ovf, counted in ovf_n[j] (zeroed by the caller). Placements are added
+// to table_counts and to the kick tally, reserved keys to the rejected tally. zeroed: every slot of
+// every table is zero.
 hipError_t launch_group_bulk_fill(const GroupChunk *chunks, uint32_t n_chunks, const uint64_t *ent, uint64_t *ovf,
-                                  unsigned long long *ovf_n, unsigned long long *table_counts, Counters *C, bool dense,
-                                  bool zeroed, hipStream_t st);
+                                  unsigned long long *ovf_n, unsigned long long *table_counts, Counters *C, bool zeroed,
+                                  hipStream_t st);
+// The overflow as work items, on the device (no read-back): table j's [off, off + ovf_n[j]) in
+// items of kOverflowItem entries, their number added to *n_items (zeroed by the caller). cap
+// (>= overflow_items) bounds the list.
+constexpr uint32_t kOverflowItem = 128;
+inline uint64_t overflow_items(uint64_t n, uint32_t n_tabs) { return n / kOverflowItem + n_tabs; }
+hipError_t launch_group_bulk_items(const BulkTable *tabs, uint32_t n_tabs, const unsigned long long *ovf_n,
+                                   GroupItem *items, uint64_t cap, unsigned long long *n_items, hipStream_t st);
+// The eviction insert of those items (at most max_items of them, *n_items read on the device), as
+// launch_insert_overflow does for one table.
+hipError_t launch_group_insert_overflow(const Desc *dir, const GroupItem *items, const unsigned long long *n_items,
+                                        uint64_t max_items, const uint64_t *ovf, InsertPolicy pol, int blocks,
+                                        Counters *C, PendSink sink, unsigned long long *table_counts, hipStream_t st);
 
 // ---- serving ticks
 // A work item of a serving tick: keys [0, len) of one request (pointers already offset to the
@@ -311,8 +316,8 @@ hipError_t launch_serve_tick(const Desc *dir, const TickItem *items, uint32_t n_
                              TickStages stages, InsertPolicy pol, int insert_lanes, int find_lanes, int blocks,
                              Counters *C, PendSink sink, Pool pool, unsigned long long *ins_total,
                              unsigned long long *del_total, uint32_t spin_cap, uint32_t max_back, hipStream_t st);
-hipError_t launch_serve_insert(const Desc *dir, const ServeItem *items, uint32_t n_items, InsertPolicy pol, int lanes,
-                               int blocks, Counters *C, PendSink sink, unsigned long long *ins_total, hipStream_t st);
+hipError_t launch_serve_insert(const Desc *dir, const ServeItem *items, uint32_t n_items, InsertPolicy pol, int blocks,
+                               Counters *C, PendSink sink, unsigned long long *ins_total, hipStream_t st);
 hipError_t launch_serve_find(const Desc *dir, const ServeItem *items, uint32_t n_items, Pool pool, int blocks,
                              hipStream_t st);
 hipError_t launch_serve_erase(const Desc *dir, const ServeItem *items, uint32_t n_items, Pool pool,

@@ -296,7 +296,7 @@ int downsize_now(dyc_server *s, uint32_t i, Counters *rctr, bool *done)
     s->dir_dirty = true;
     // residuals continue from the shrunk subtable into the other one of their pair
     // (cuckoo.cu:719), after the compaction; failures go to the pool
-    HIP_TRY(launch_insert_entries(T.D, res, res_n, sub, (int)s->cfg.insert_lanes, s->policy(), s->insert_shape(),
+    HIP_TRY(launch_insert_entries(T.D, res, res_n, sub, s->policy(), s->insert_shape(),
                                   s->pc(), s->sink(i), s->ms(), live));
     s->arena.release(old_off);
     s->arena.release(loff);
@@ -368,8 +368,7 @@ int resolve_pool(dyc_server *s, unsigned long long *scratch)
             bool ok = false;
             rc = upsize_now(s, sp.table, &ok);
             if (rc) return rc;
-            HIP_TRY(launch_insert_entries(s->t[sp.table].D, s->d_resolve + sp.begin, sp.len, kNoTable,
-                                          (int)s->cfg.insert_lanes, s->policy(), s->insert_shape(), s->pc(),
+            HIP_TRY(launch_insert_entries(s->t[sp.table].D, s->d_resolve + sp.begin, sp.len, kNoTable, s->policy(), s->insert_shape(), s->pc(),
                                           s->sink(sp.table), s->ms()));
         }
         HIP_TRY(hipStreamSynchronize(s->ms()));
@@ -683,7 +682,7 @@ int build_tick(dyc_server *s, bool *launched, bool *stuck)
         k.solo_table = q.table;
         if (dir_up) s->dir_dirty = true;  // the plain kernels take the descriptor by value
         if (q.op == DYC_OP_INSERT)
-            HIP_TRY(launch_insert(T.D, q.keys, q.vals, q.n, (int)s->cfg.insert_lanes, s->policy(), s->insert_shape(),
+            HIP_TRY(launch_insert(T.D, q.keys, q.vals, q.n, s->policy(), s->insert_shape(),
                                   s->pc(), s->sink(q.table, true), s->st));
         else if (q.op == DYC_OP_FIND)
             HIP_TRY(launch_find(T.D, q.keys, q.out_vals, q.out_flags, q.n, s->shape(), s->st,
@@ -773,7 +772,7 @@ int build_tick(dyc_server *s, bool *launched, bool *stuck)
         at = 0;
         for (uint32_t r = 0; r < rounds; ++r) {
             const uint64_t ni = s->items[r][0].size(), nf = s->items[r][1].size(), ne = s->items[r][2].size();
-            HIP_TRY(launch_serve_insert(s->d_dir, items + at, (uint32_t)ni, s->policy(), (int)s->cfg.insert_lanes, 0,
+            HIP_TRY(launch_serve_insert(s->d_dir, items + at, (uint32_t)ni, s->policy(), 0,
                                         s->pc(), s->sink(0), s->ins_total(), s->st));
             at += ni;
             HIP_TRY(launch_serve_find(s->d_dir, items + at, (uint32_t)nf, s->pool(), 0, s->st));
@@ -865,7 +864,7 @@ int run_sync(dyc_server *s, uint64_t tk)
             }
         }
         if (status == DYC_OK)
-            HIP_TRY(launch_insert(T.D, r.keys, r.vals, r.n, (int)s->cfg.insert_lanes, s->policy(), s->insert_shape(),
+            HIP_TRY(launch_insert(T.D, r.keys, r.vals, r.n, s->policy(), s->insert_shape(),
                                   s->pc(), s->sink(r.table, true), s->st));
     } else if (r.op == DYC_OP_FIND) {
         // a find changes nothing: launch, wait, done

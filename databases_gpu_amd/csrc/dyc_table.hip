@@ -107,8 +107,7 @@ struct dyc_table {
     uint64_t part_cap = 0;
     unsigned long long *part_counts = nullptr;   // kMaxRegions counts, then kMaxRegions cursors
     // bulk fill (insert_order 3): the partition's entry and chunk-id buffers (bk_cid_bytes per
-    // chunk id), its per-block counts and digit totals, the chunk starts and the overflow count
-    // (device, and a pinned read-back)
+    // chunk id), its per-block counts and digit totals, and the chunk starts
     void *bk_cid[2] = {};
     uint64_t *bk_ent[2] = {};
     uint64_t bk_cap = 0;
@@ -116,8 +115,6 @@ struct dyc_table {
     uint32_t *bk_start = nullptr;
     uint64_t bk_start_cap = 0;
     uint32_t *bk_partial = nullptr;  // kPartialWords, then 256 digit totals
-    unsigned long long *bk_ovf = nullptr;
-    unsigned long long *bk_hovf = nullptr;
     DycHostStage *stage = nullptr;
     uint8_t *upd = nullptr;  // upsert: per-key "updated in place" flags
     uint64_t upd_cap = 0;
@@ -380,7 +377,7 @@ int place_pending(dyc_table *t, hipStream_t s, uint64_t before)
         t->pend_n = 0;
         rc = zero_counters(t, s);
         if (!rc) {
-            hipError_t e = launch_insert_entries(t->D, src, m, kNoTable, (int)t->cfg.insert_lanes, t->policy(),
+            hipError_t e = launch_insert_entries(t->D, src, m, kNoTable, t->policy(),
                                                  t->insert_shape(), t->ctr, sink_at(t, 0), s);
             if (e != hipSuccess) rc = fail(DYC_ERR_HIP, "pending re-insert launch: %s", hipGetErrorString(e));
         }
@@ -454,7 +451,7 @@ int do_resize_down(dyc_table *t, hipStream_t s)
         if (!rc) rc = zero_counters(t, s);
         if (!rc) {
             // the slot-addressed list: its live tiles, zeros skipped
-            hipError_t e = launch_insert_entries(t->D, res, res_n, sub, (int)t->cfg.insert_lanes, t->policy(),
+            hipError_t e = launch_insert_entries(t->D, res, res_n, sub, t->policy(),
                                                  t->insert_shape(), t->ctr, sink_at(t, t->pend_n), s, t->live);
             if (e != hipSuccess) rc = fail(DYC_ERR_HIP, "residual insert launch: %s", hipGetErrorString(e));
         }
@@ -567,15 +564,6 @@ int reserve_bulk(dyc_table *t, uint64_t n, const Chunks &Ch, hipStream_t s)
         rc = bulk_alloc((void **)&t->bk_partial, (kPartialWords + kMaxRadixWords) * sizeof(uint32_t), "partition counts");
         if (rc) return rc;
     }
-    if (!t->bk_ovf) {
-        rc = bulk_alloc((void **)&t->bk_ovf, 256, "overflow count");
-        if (rc) return rc;
-    }
-    if (!t->bk_hovf && hipHostMalloc((void **)&t->bk_hovf, 64, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        t->bk_hovf = nullptr;
-        return fail(DYC_ERR_OOM, "hipHostMalloc of the bulk-fill read-back word failed");
-    }
     return DYC_OK;
 }
 
@@ -585,49 +573,23 @@ BulkSpace bulk_space(const dyc_table *t)
                      t->bk_partial + kPartialWords, t->bk_start};
 }
 
-// One fill round over n entries: round 1 from keys/vals (keys != nullptr), round 2 from the
-// entries in bk_ent[in]. Partition them by chunk, fill, and read back how many entries overflowed
-// into bk_ent[*out] (the buffer the partition did not end in).
-int bulk_round(dyc_table *t, const Chunks &Ch, const uint32_t *keys, const uint32_t *vals, int in, uint64_t n,
-               bool zeroed, hipStream_t s, int *out, uint64_t *overflow)
-{
-    int r = 0;
-    HIP_TRY(launch_bulk_partition(t->D, Ch, keys, vals, in, n, bulk_space(t), kBulkSortBlocks, s, &r));
-    HIP_TRY(launch_zero(t->bk_ovf, 1, s));
-    HIP_TRY(launch_bulk_fill(t->D, Ch, t->bk_start, t->bk_ent[r], n, t->bk_ent[1 - r], t->bk_cap, t->bk_ovf, t->ctr,
-                             zeroed, s));
-    HIP_TRY(hipMemcpyAsync(t->bk_hovf, t->bk_ovf, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    *overflow = *t->bk_hovf;
-    *out = 1 - r;
-    if (*overflow > n) return fail(DYC_ERR_CORRUPT, "bulk fill overflow count %llu exceeds the batch (%llu)",
-                                   (unsigned long long)*overflow, (unsigned long long)n);
-    return DYC_OK;
-}
-
 // insert_order 3: place keys by bucket fill in their fill_target bucket (pos1, the bucket a find
-// reads first, wherever equal subtable shares allow), then the overflow in the other bucket of
-// their pair, then the rest by the eviction insert. Counters are zeroed here
-// and read by the caller.
-int bulk_insert(dyc_table *t, const uint32_t *keys, const uint32_t *vals, uint64_t n, bool was_zeroed, hipStream_t s,
-                uint64_t *left)
+// reads first, wherever equal subtable shares allow), then the overflow, whose length stays on the
+// device, in the other bucket of its pair by the eviction insert. Counters are zeroed here and
+// read by the caller (Counters::left: the entries that had to evict, or were parked).
+int bulk_insert(dyc_table *t, const uint32_t *keys, const uint32_t *vals, uint64_t n, bool was_zeroed, hipStream_t s)
 {
-    *left = 0;
     const Chunks Ch = make_chunks(t->D);  // the workspace was reserved for it
     int rc = zero_counters(t, s);
     if (rc) return rc;
-    int ov = 0, ov2 = 0;
-    uint64_t m1 = 0, m2 = 0;
     // an empty table (count 0, nothing pending) that no call has stored into since it was
     // created or cleared holds zeros only
     const bool zeroed = was_zeroed && t->count == 0 && t->pend_n == 0;
-    rc = bulk_round(t, Ch, keys, vals, 0, n, zeroed, s, &ov, &m1);
-    if (rc || m1 == 0) return rc;
-    rc = bulk_round(t, Ch, nullptr, nullptr, ov, m1, false, s, &ov2, &m2);  // the overflow, in its other table
-    if (rc || m2 == 0) return rc;
-    *left = m2;
-    HIP_TRY(launch_insert_entries(t->D, t->bk_ent[ov2], m2, kNoTable, (int)t->cfg.insert_lanes, t->policy(),
-                                  t->insert_shape(), t->ctr, sink_at(t, t->pend_n), s));
+    int r = 0;
+    HIP_TRY(launch_bulk_partition(t->D, Ch, keys, vals, n, bulk_space(t), kBulkSortBlocks, s, &r));
+    uint64_t *const ovf = t->bk_ent[1 - r];  // the buffer the partition did not end in
+    HIP_TRY(launch_bulk_fill(t->D, Ch, t->bk_start, t->bk_ent[r], n, ovf, t->bk_cap, t->ctr, zeroed, s));
+    HIP_TRY(launch_insert_overflow(t->D, ovf, n, t->policy(), t->insert_shape(), t->ctr, sink_at(t, t->pend_n), s));
     return DYC_OK;
 }
 
@@ -1063,8 +1025,6 @@ int dyc_destroy(dyc_table *t)
     }
     if (t->bk_start) (void)hipFree(t->bk_start);
     if (t->bk_partial) (void)hipFree(t->bk_partial);
-    if (t->bk_ovf) (void)hipFree(t->bk_ovf);
-    if (t->bk_hovf) (void)hipHostFree(t->bk_hovf);
     if (t->hctr) (void)hipHostFree(t->hctr);
     if (t->hpost) (void)hipHostFree(t->hpost);
     if (t->upd) (void)hipFree(t->upd);
@@ -1117,9 +1077,8 @@ int dyc_insert_counted(dyc_table *t, const uint32_t *keys, const uint32_t *vals,
             return rc;
         }
     }
-    uint64_t left = 0;  // entries the bulk fill left to the eviction insert
     if (bulk) {
-        rc = bulk_insert(t, keys, vals, n, zeroed, s, &left);
+        rc = bulk_insert(t, keys, vals, n, zeroed, s);
         if (rc) return rc;
     } else if (R) {
         rc = reserve_partition(t, n, s);
@@ -1129,14 +1088,14 @@ int dyc_insert_counted(dyc_table *t, const uint32_t *keys, const uint32_t *vals,
                                  t->part_counts + kMaxRegions, t->part, s));
         rc = zero_counters(t, s);
         if (rc) return rc;
-        HIP_TRY(launch_insert_entries(t->D, t->part, n, kNoTable, (int)t->cfg.insert_lanes, t->policy(),
+        HIP_TRY(launch_insert_entries(t->D, t->part, n, kNoTable, t->policy(),
                                       t->insert_shape(), t->ctr, sink_at(t, t->pend_n), s));
     } else {
         rc = zero_counters(t, s);
         if (rc) return rc;
         PendSink sink = sink_at(t, t->pend_n);
         sink.chain = iter_count;
-        HIP_TRY(launch_insert(t->D, keys, vals, n, (int)t->cfg.insert_lanes, t->policy(), t->insert_shape(), t->ctr,
+        HIP_TRY(launch_insert(t->D, keys, vals, n, t->policy(), t->insert_shape(), t->ctr,
                               sink, s));
     }
     rc = read_counters(t, s);
@@ -1144,7 +1103,7 @@ int dyc_insert_counted(dyc_table *t, const uint32_t *keys, const uint32_t *vals,
     const uint64_t rejected = t->hctr->rejected;
     t->st.rejected += rejected;
     t->count += n - rejected;
-    if (bulk) t->st.last_filled = n - rejected - left;
+    if (bulk) t->st.last_filled = n - rejected - t->hctr->left;
     rc = absorb_insert_counters(t, room);
     t->st.pending = t->pend_n;
     if (rc) return rc;
@@ -1186,7 +1145,7 @@ int dyc_insert_async(dyc_table *t, const uint32_t *keys, const uint32_t *vals, u
     if (rc) return rc;
     if (t->async_keys == 0) t->st.last_kicks = t->st.last_max_chain = t->st.last_filled = 0;
     HIP_TRY(launch_zero(reinterpret_cast<unsigned long long *>(a->ctr), kCounterWords, s));
-    HIP_TRY(launch_insert(t->D, keys, vals, n, (int)t->cfg.insert_lanes, t->policy(), t->insert_shape(), a->ctr,
+    HIP_TRY(launch_insert(t->D, keys, vals, n, t->policy(), t->insert_shape(), a->ctr,
                           PendSink{a->pend, nullptr, a->cap, 0, 0, nullptr}, s));
     HIP_TRY(launch_fold_post(a->ctr, a->post, ++a->seq, s));
     a->busy = true;
@@ -1231,7 +1190,7 @@ int dyc_insert_noalloc(dyc_table *t, const uint32_t *keys, const uint32_t *vals,
     if (rc) return rc;
     // the block keeps the last call's contents (a call that failed may have left it dirty)
     HIP_TRY(launch_zero(reinterpret_cast<unsigned long long *>(C), kCounterWords, s));
-    HIP_TRY(launch_insert(t->D, keys, vals, n, (int)t->cfg.insert_lanes, t->policy(), t->insert_shape(), C,
+    HIP_TRY(launch_insert(t->D, keys, vals, n, t->policy(), t->insert_shape(), C,
                           sink_at(t, t->pend_n), s));
     // read back as read_counters does, from the static block (the fold also clears it)
     const unsigned long long seq = ++t->post_seq;
@@ -1288,7 +1247,7 @@ int dyc_upsert(dyc_table *t, const uint32_t *keys, const uint32_t *vals, uint64_
     if (rc) return rc;
     Pool sp;
     HIP_TRY(launch_update(t->D, keys, vals, flags, n, t->shape(), t->ctr, s, stash_of(t, sp)));
-    HIP_TRY(launch_insert(t->D, keys, vals, n, (int)t->cfg.insert_lanes, t->policy(), t->insert_shape(), t->ctr,
+    HIP_TRY(launch_insert(t->D, keys, vals, n, t->policy(), t->insert_shape(), t->ctr,
                           sink_at(t, t->pend_n), s, flags));
     rc = read_counters(t, s);
     if (rc) return rc;
@@ -1540,7 +1499,7 @@ int dyc_insert_host(dyc_table *t, const uint32_t *keys, const uint32_t *vals, ui
         HIP_TRY(hipMemcpyAsync(S->dv[b], S->hv[b], m * 4, hipMemcpyHostToDevice, S->h2d));
         HIP_TRY(hipEventRecord(S->in_ready[b], S->h2d));
         HIP_TRY(hipStreamWaitEvent(s, S->in_ready[b], 0));
-        HIP_TRY(launch_insert(t->D, S->dk[b], S->dv[b], m, (int)t->cfg.insert_lanes, t->policy(), t->insert_shape(),
+        HIP_TRY(launch_insert(t->D, S->dk[b], S->dv[b], m, t->policy(), t->insert_shape(),
                               t->ctr, sink_at(t, t->pend_n), s));
         HIP_TRY(hipEventRecord(S->done[b], s));
         used[b] = true;

@@ -219,11 +219,14 @@ __global__ __launch_bounds__(256) void wide_probe_kernel(WideDesc W, const uint6
 // grid-stride sequence, so it never waits behind a longer chain in its wave. The chain is the
 // narrow table's (victim = first empty slot; else, for kick_bound iterations, the first slot
 // whose resident's pair index differs from the table number; else slot iteration & 15; then
-// the rescue walk), over fold(k), with the three-step exchange described at the top.
+// the rescue walk), over fold(k), with the three-step exchange described at the top. With
+// kick_bound 0 a fresh key whose first bucket is full tries its other bucket before it evicts, as
+// in the narrow insert.
 struct WideCarry {
     uint64_t key, val;
     uint32_t pre, kicks, retries;
     bool active, fresh;
+    bool swing;  // a fresh key whose other bucket is still to be tried
     uint64_t cur[kSlots];  // the lane's view of the bucket it is about to write
 };
 
@@ -240,10 +243,13 @@ __device__ inline void wide_give_up(WideCarry &c, const WideSink &sink, Counters
     c.active = false;
 }
 
-// Take entry (k, v) into the lane's hand; pr is its previous table (kNoTable for a fresh key).
+// Take entry (k, v) into the lane's hand; pr is its previous table (kNoTable for a fresh key,
+// kAfterFill for one the bulk fill found no slot for).
 __device__ inline void wide_take(WideCarry &c, const Desc &D, uint64_t k, uint64_t v, uint32_t pr)
 {
-    if (pr == kNoTable && (k & 1u)) pr = pos1(D, pair_of(D, fold64(k)));  // odd keys start in pos2
+    c.swing = pr == kNoTable;
+    if (pr == kAfterFill) pr = fill_target(D, (uint32_t)k, pair_of(D, fold64(k)));
+    else if (pr == kNoTable && (k & 1u)) pr = pos1(D, pair_of(D, fold64(k)));  // odd keys start in pos2
     c.key = k;
     c.val = v;
     c.pre = pr;
@@ -257,7 +263,7 @@ __device__ inline void wide_take(WideCarry &c, const Desc &D, uint64_t k, uint64
 // add their exchanges to kicks.
 __device__ inline void wide_step(WideCarry &c, const WideDesc &W, const InsertPolicy &P, Counters *C,
                                  const WideSink &sink, uint32_t tag, unsigned long long &kicks,
-                                 unsigned long long &retries)
+                                 unsigned long long &retries, unsigned long long &direct)
 {
     const Desc &D = W.D;
     const uint32_t total_kicks = P.kick_bound + P.rescue_kicks;
@@ -281,6 +287,12 @@ __device__ inline void wide_step(WideCarry &c, const WideDesc &W, const InsertPo
     for (int j = kSlots - 1; j >= 0; --j)
         if (c.cur[j] == 0ull) slot = j;
     if (slot < 0) {
+        if (c.swing && P.kick_bound == 0) {  // nothing exchanged
+            c.pre = t;
+            c.swing = false;
+            c.fresh = true;
+            return;
+        }
         if (c.kicks < P.kick_bound) {
 #pragma unroll
             for (int j = kSlots - 1; j >= 0; --j)
@@ -327,11 +339,13 @@ __device__ inline void wide_step(WideCarry &c, const WideDesc &W, const InsertPo
     c.fresh = true;
     if (expected == 0ull) {
         kicks += c.kicks;
+        direct += c.kicks == 1u;
         c.active = false;
     } else {
         c.key = expected;
         c.val = old_val;
         c.pre = t;
+        c.swing = false;
         if (c.kicks >= total_kicks) {
             kicks += c.kicks;
             wide_give_up(c, sink, C, tag);
@@ -339,41 +353,51 @@ __device__ inline void wide_step(WideCarry &c, const WideDesc &W, const InsertPo
     }
 }
 
+// What a wide insert reads: the caller's key and value arrays, the arrays of a residual or pending
+// list (key 0: an empty place), or a bulk fill's overflow entries.
+enum WideSource { kWideBatch, kWideList, kWideOverflow };
+
 // skip (optional): a keys insert leaves out key i where skip[i] != 0 (an upsert updated it in
-// place); an entries insert reads it as the tile flags of a slot-addressed residual list.
-template <bool FROM_ENTRIES>
+// place); a list insert reads it as the tile flags of a slot-addressed residual list. n_dev
+// (optional): the input ends at *n_dev if that is less than n.
+template <WideSource SRC>
 __global__ __launch_bounds__(256) void wide_insert_kernel(WideDesc W, const uint64_t *__restrict__ keys,
-                                                          const uint64_t *__restrict__ vals, uint64_t n,
+                                                          const uint64_t *__restrict__ vals,
+                                                          const WideEntry *__restrict__ entries, uint64_t n,
                                                           uint32_t pre_fixed, InsertPolicy P, Counters *__restrict__ C,
-                                                          WideSink sink, const uint8_t *__restrict__ skip)
+                                                          WideSink sink, const uint8_t *__restrict__ skip,
+                                                          const unsigned long long *__restrict__ n_dev)
 {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     uint64_t next = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    unsigned long long kicks = 0, rejected = 0, retries = 0;
+    unsigned long long kicks = 0, rejected = 0, retries = 0, direct = 0, taken = 0;
+    if (n_dev) n = min((unsigned long long)n, *n_dev);
     WideCarry c;
     c.active = false;
     for (;;) {
         while (!c.active && next < n) {  // take the next entry
-            if (FROM_ENTRIES && skip && !skip[next / kResTileEntries]) {  // a residual tile with none
+            if (SRC == kWideList && skip && !skip[next / kResTileEntries]) {  // a residual tile with none
                 next += stride;
                 continue;
             }
-            if (!FROM_ENTRIES && skip && skip[next]) {  // updated in place
+            if (SRC == kWideBatch && skip && skip[next]) {  // updated in place
                 next += stride;
                 continue;
             }
-            const uint64_t k = keys[next];
-            const uint64_t v = vals[next];
+            WideEntry e;
+            if constexpr (SRC == kWideOverflow) e = entries[next];
+            else e = WideEntry{keys[next], vals[next]};
             next += stride;
-            if (FROM_ENTRIES && k == 0) continue;  // an empty place in a residual or pending list
-            if (wide_reserved(k)) {
+            if (SRC == kWideList && e.k == 0) continue;  // an empty place
+            if (wide_reserved(e.k)) {
                 ++rejected;
                 continue;
             }
-            wide_take(c, W.D, k, v, FROM_ENTRIES ? pre_fixed : kNoTable);
+            ++taken;
+            wide_take(c, W.D, e.k, e.v, pre_fixed);
         }
         if (!__any(c.active)) break;
-        if (c.active) wide_step(c, W, P, C, sink, sink.tag, kicks, retries);
+        if (c.active) wide_step(c, W, P, C, sink, sink.tag, kicks, retries, direct);
     }
     if (sink.rejected_at) {
         const unsigned long long rej = wave_sum(rejected);
@@ -382,6 +406,7 @@ __global__ __launch_bounds__(256) void wide_insert_kernel(WideDesc W, const uint
     wave_tally(C, &C->kicks, kicks);
     wave_tally(C, &C->rejected, rejected);
     wave_tally(C, &C->retries, retries);
+    if constexpr (SRC == kWideOverflow) wave_tally(C, &C->left, taken - direct);
 }
 
 // ------------------------------------------------------------------------------ many tables
@@ -417,39 +442,45 @@ __global__ __launch_bounds__(256) void wide_group_probe_kernel(const WideDesc *_
 }
 
 // Lanes of a wave take the item's entries one each (lane-per-chain, as wide_insert_kernel); the
-// wave moves to its next item when the item is used up and every lane's chain has ended.
+// wave moves to its next item when the item is used up and every lane's chain has ended. With
+// kWideOverflow there are *n_dev items if that is less than n_items.
+template <WideSource SRC>
 __global__ __launch_bounds__(256) void wide_group_insert_kernel(const WideDesc *__restrict__ dir,
                                                                 const GroupItem *__restrict__ items, uint32_t n_items,
                                                                 const uint64_t *__restrict__ keys,
-                                                                const uint64_t *__restrict__ vals, InsertPolicy P,
+                                                                const uint64_t *__restrict__ vals,
+                                                                const WideEntry *__restrict__ entries, InsertPolicy P,
                                                                 Counters *__restrict__ C, WideSink sink,
-                                                                unsigned long long *__restrict__ table_counts)
+                                                                unsigned long long *__restrict__ table_counts,
+                                                                const unsigned long long *__restrict__ n_dev)
 {
     const uint32_t waves = gridDim.x * (blockDim.x / kWave);
-    unsigned long long kicks = 0, rejected = 0, retries = 0;
+    unsigned long long kicks = 0, rejected = 0, retries = 0, direct = 0, taken = 0;
+    if constexpr (SRC == kWideOverflow) n_items = (uint32_t)min((unsigned long long)n_items, *n_dev);
     WideCarry c;
     c.active = false;
     for (uint32_t it = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave);
          it < n_items; it += waves) {
         const GroupItem item = items[it];
-        if (item.len == 0) continue;  // wave-uniform: a block the bulk fill's rounds emptied
         const WideDesc W = as_global(dir[item.table]);
         const uint64_t end = item.begin + item.len;
         uint64_t next = item.begin + __lane_id();
         unsigned long long rej = 0;
         for (;;) {
             while (!c.active && next < end) {
-                const uint64_t k = keys[next];
-                const uint64_t v = vals[next];
+                WideEntry e;
+                if constexpr (SRC == kWideOverflow) e = entries[next];
+                else e = WideEntry{keys[next], vals[next]};
                 next += kWave;
-                if (wide_reserved(k)) {
+                if (wide_reserved(e.k)) {
                     ++rej;
                     continue;
                 }
-                wide_take(c, W.D, k, v, kNoTable);
+                ++taken;
+                wide_take(c, W.D, e.k, e.v, SRC == kWideOverflow ? kAfterFill : kNoTable);
             }
             if (!__any(c.active)) break;
-            if (c.active) wide_step(c, W, P, C, sink, item.table, kicks, retries);
+            if (c.active) wide_step(c, W, P, C, sink, item.table, kicks, retries, direct);
         }
         rejected += rej;
         rej = wave_sum(rej);
@@ -458,6 +489,7 @@ __global__ __launch_bounds__(256) void wide_group_insert_kernel(const WideDesc *
     wave_tally(C, &C->kicks, kicks);
     wave_tally(C, &C->rejected, rejected);
     wave_tally(C, &C->retries, retries);
+    if constexpr (SRC == kWideOverflow) wave_tally(C, &C->left, taken - direct);
 }
 
 // ---------------------------------------------------------------------------------- resize
@@ -570,12 +602,11 @@ constexpr uint64_t kWideInsertBlocks = 16384;
 // eviction insert for the rest. The dense round keeps the chunk's key lines and value lines in
 // LDS (2 x 64 KB), so one 1024-thread workgroup runs per CU.
 // Chunk ids of the batch in input order and each block's counts of the partition's first digit
-// (dyc_part.hpp), over fold(k): round 1 from the keys (fill_target; reserved keys go to chunk 0,
-// whose fill rejects them), round 2 from overflow entries (the other bucket of the pair).
-template <bool IN_ENTRIES, typename CidT>
+// (dyc_part.hpp), over fold(k), of the fill_target bucket (reserved keys go to chunk 0, whose fill
+// rejects them).
+template <typename CidT>
 __global__ __launch_bounds__(kCountThreads) void wide_bulk_pack_kernel(WideDesc W, Chunks Ch,
-                                                                       const uint64_t *__restrict__ keys,
-                                                                       const WideEntry *__restrict__ in, PartGrid G,
+                                                                       const uint64_t *__restrict__ keys, PartGrid G,
                                                                        RadixPass P, CidT *__restrict__ cid,
                                                                        uint32_t *__restrict__ partial)
 {
@@ -584,10 +615,10 @@ __global__ __launch_bounds__(kCountThreads) void wide_bulk_pack_kernel(WideDesc 
     // per subtable: buckets, FastDiv multiplier and shifts, first chunk -- one LDS read per key
     // in place of a selection chain over the descriptor's arrays for each of them
     __shared__ uint4 sub_tab[kMaxSubtables];
-    __shared__ uint32_t tsel[32];  // the round's subtable by key parity and pair (fill_round_sub)
+    __shared__ uint32_t tsel[32];  // the target subtable by key parity and pair (fill_sub)
     const uint32_t R = 1u << P.bits;
     for (uint32_t d = threadIdx.x; d < R; d += kCountThreads) h[d] = 0;
-    if (threadIdx.x < 32) tsel[threadIdx.x] = fill_round_sub(D, threadIdx.x, IN_ENTRIES);
+    if (threadIdx.x < 32) tsel[threadIdx.x] = fill_sub(D, threadIdx.x);
     if (threadIdx.x < kMaxSubtables) {
         const uint32_t t = threadIdx.x;
         sub_tab[t] = make_uint4(selt(t, D.nb), selt(t, D.m), selt(t, D.sh), chunk_base(Ch, t));
@@ -600,17 +631,14 @@ __global__ __launch_bounds__(kCountThreads) void wide_bulk_pack_kernel(WideDesc 
 #pragma unroll
         for (int u = 0; u < kCountItems; ++u) {
             const uint64_t i = i0 + (uint64_t)u * kCountThreads;
-            if (i < hi) {
-                if constexpr (IN_ENTRIES) k[u] = in[i].k;
-                else k[u] = keys[i];
-            }
+            if (i < hi) k[u] = keys[i];
         }
 #pragma unroll
         for (int u = 0; u < kCountItems; ++u) {
             const uint64_t i = i0 + (uint64_t)u * kCountThreads;
             if (i >= hi) continue;
             uint32_t c = 0;
-            if (IN_ENTRIES || !wide_reserved(k[u])) {
+            if (!wide_reserved(k[u])) {
                 const uint32_t f = fold64(k[u]), p = pair_of(D, f);
                 const uint32_t t = tsel[(((uint32_t)k[u] & 1u) << 4) | p];
                 const uint4 q = sub_tab[t];
@@ -628,15 +656,14 @@ __global__ __launch_bounds__(kCountThreads) void wide_bulk_pack_kernel(WideDesc 
 // subtable S (key lines S.keys, value lines S.vals), entries ent[lo, hi) (all targeting S); entries that do not fit go to
 // ovf[0, ovf_cap) at the index *ovf_n hands out. Placements and rejected reserved keys are added
 // to this lane's `placed` and `rejected`. Every thread of the workgroup calls it alike.
-template <bool DENSE, int THREADS>
+template <int THREADS>
 __device__ inline void wide_fill_chunk(const SubRef &S, uint32_t b0, uint32_t len,
                                        const WideEntry *__restrict__ ent, uint32_t lo, uint32_t hi,
                                        WideEntry *__restrict__ ovf, uint64_t ovf_cap,
                                        unsigned long long *__restrict__ ovf_n, bool zeroed,
                                        unsigned long long &placed, unsigned long long &rejected)
 {
-    constexpr uint32_t kImg = DENSE ? kChunkBuckets * kSlots : 2;
-    __shared__ uint64_t kimg[kImg], vimg[kImg];  // DENSE: the chunk's key and value lines
+    __shared__ uint64_t kimg[kChunkBuckets * kSlots], vimg[kChunkBuckets * kSlots];  // the chunk's lines
     __shared__ uint32_t fm[kChunkBuckets];       // free-slot mask of each bucket
     __shared__ uint32_t cnt[kChunkBuckets];      // entries per bucket, then slots taken
     __shared__ uint32_t wred[THREADS / kWave];
@@ -646,7 +673,7 @@ __device__ inline void wide_fill_chunk(const SubRef &S, uint32_t b0, uint32_t le
     uint64_t *const vsub = as_global(S.vals);
     const uint4 *const ksrc = reinterpret_cast<const uint4 *>(ksub + (uint64_t)b0 * kSlots);
     constexpr uint32_t kParts = kChunkBuckets * kSlots / 2;  // 16-byte parts of a chunk's lines
-    if constexpr (DENSE) {
+    {
         const uint4 *const vsrc = reinterpret_cast<const uint4 *>(vsub + (uint64_t)b0 * kSlots);
         uint4 *const ki = reinterpret_cast<uint4 *>(kimg);
         uint4 *const vi = reinterpret_cast<uint4 *>(vimg);
@@ -681,8 +708,6 @@ __device__ inline void wide_fill_chunk(const SubRef &S, uint32_t b0, uint32_t le
                 cnt[q / 8] = 0;
             }
         }
-    } else {
-        for (uint32_t j = threadIdx.x; j < kChunkBuckets; j += blockDim.x) cnt[j] = 0;
     }
     if (threadIdx.x == 0) onext = 0;
     __syncthreads();
@@ -736,32 +761,6 @@ __device__ inline void wide_fill_chunk(const SubRef &S, uint32_t b0, uint32_t le
         }
     }
     __syncthreads();
-    if constexpr (!DENSE) {
-        // free masks of the buckets that received entries only (a bucket's 8 parts are read
-        // by 8 consecutive lanes and folded by ballot; the others read as full)
-        constexpr uint32_t kPer = kParts / THREADS;
-        uint4 v[kPer];
-#pragma unroll
-        for (uint32_t u = 0; u < kPer; ++u) {
-            const uint32_t q = threadIdx.x + u * THREADS;
-            v[u] = q < len * (kSlots / 2) && cnt[q / 8] ? ksrc[q] : make_uint4(1u, 1u, 1u, 1u);
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < kPer; ++u) {
-            const uint32_t q = threadIdx.x + u * THREADS;
-            const bool e0 = (v[u].x | v[u].y) == 0u, e1 = (v[u].z | v[u].w) == 0u;
-            const uint64_t m0 = __ballot(e0), m1 = __ballot(e1);
-            const uint32_t lane = __lane_id();
-            if ((lane & 7u) == 0) {
-                const uint32_t a = (uint32_t)(m0 >> lane) & 0xffu, b = (uint32_t)(m1 >> lane) & 0xffu;
-                uint32_t m = 0;
-#pragma unroll
-                for (int p = 0; p < 8; ++p) m |= (((a >> p) & 1u) << (2 * p)) | (((b >> p) & 1u) << (2 * p + 1));
-                fm[q / 8] = m;
-            }
-        }
-        __syncthreads();
-    }
     uint32_t excess = stray;
     for (uint32_t j = threadIdx.x; j < kChunkBuckets; j += THREADS) {
         const uint32_t f = (uint32_t)__builtin_popcount(fm[j]);
@@ -779,13 +778,8 @@ __device__ inline void wide_fill_chunk(const SubRef &S, uint32_t b0, uint32_t le
         for (uint32_t j = threadIdx.x; j < kChunkBuckets; j += THREADS) cnt[j] = 0;
     __syncthreads();
     auto put = [&](uint32_t j, uint32_t slot, const WideEntry &e) {
-        if constexpr (DENSE) {
-            kimg[j * kSlots + slot] = e.k;
-            vimg[j * kSlots + slot] = e.v;
-        } else {
-            ksub[(uint64_t)(b0 + j) * kSlots + slot] = e.k;
-            vsub[(uint64_t)(b0 + j) * kSlots + slot] = e.v;
-        }
+        kimg[j * kSlots + slot] = e.k;
+        vimg[j * kSlots + slot] = e.v;
     };
     auto overflow = [&](const WideEntry &e) {  // the counted excess reserved exactly these places
         const unsigned long long at = obase + atomicAdd(&onext, 1u);
@@ -842,26 +836,23 @@ __device__ inline void wide_fill_chunk(const SubRef &S, uint32_t b0, uint32_t le
             if (!fits) overflow(e);
         }
     }
-    if constexpr (DENSE) {
-        __syncthreads();
-        uint4 *const kd = reinterpret_cast<uint4 *>(ksub + (uint64_t)b0 * kSlots);
-        uint4 *const vd = reinterpret_cast<uint4 *>(vsub + (uint64_t)b0 * kSlots);
-        const uint4 *const ki = reinterpret_cast<const uint4 *>(kimg);
-        const uint4 *const vi = reinterpret_cast<const uint4 *>(vimg);
-        for (uint32_t q = threadIdx.x; q < len * (kSlots / 2); q += THREADS) {
-            kd[q] = ki[q];
-            vd[q] = vi[q];
-        }
+    __syncthreads();
+    uint4 *const kd = reinterpret_cast<uint4 *>(ksub + (uint64_t)b0 * kSlots);
+    uint4 *const vd = reinterpret_cast<uint4 *>(vsub + (uint64_t)b0 * kSlots);
+    const uint4 *const ki = reinterpret_cast<const uint4 *>(kimg);
+    const uint4 *const vi = reinterpret_cast<const uint4 *>(vimg);
+    for (uint32_t q = threadIdx.x; q < len * (kSlots / 2); q += THREADS) {
+        kd[q] = ki[q];
+        vd[q] = vi[q];
     }
 }
 
 // One workgroup per chunk of one wide table (chunks numbered subtable by subtable, Ch); the
 // entries of chunk c are ent[start[c], start[c + 1]).
-template <bool DENSE, int THREADS>
+template <int THREADS>
 __global__ __launch_bounds__(THREADS) void wide_bulk_fill_kernel(WideDesc W, Chunks Ch, const uint32_t *__restrict__ start,
                                                                  const WideEntry *__restrict__ ent, uint64_t n,
                                                                  WideEntry *__restrict__ ovf, uint64_t ovf_cap,
-                                                                 unsigned long long *__restrict__ ovf_n,
                                                                  Counters *__restrict__ C, bool zeroed)
 {
     const uint32_t c = blockIdx.x;
@@ -875,23 +866,11 @@ __global__ __launch_bounds__(THREADS) void wide_bulk_fill_kernel(WideDesc W, Chu
             if (Ch.base[q] <= c) t = q;
         const uint32_t b0 = (c - chunk_base(Ch, t)) << kChunkShift;
         const uint32_t len = min(kChunkBuckets, selt(t, W.D.nb) - b0);
-        wide_fill_chunk<DENSE, THREADS>(sub_ref(W.D, t, selt(t, W.val)), b0, len, ent, lo, hi, ovf, ovf_cap, ovf_n,
-                                        zeroed, placed, rejected);
+        wide_fill_chunk<THREADS>(sub_ref(W.D, t, selt(t, W.val)), b0, len, ent, lo, hi, ovf, ovf_cap, &C->overflow,
+                                 zeroed, placed, rejected);
     }
     wave_tally(C, &C->kicks, placed);
     wave_tally(C, &C->rejected, rejected);
-}
-
-// The last overflow list (entries) as the key and value arrays the eviction insert reads.
-__global__ __launch_bounds__(256) void wide_split_kernel(const WideEntry *__restrict__ in, uint64_t n,
-                                                         uint64_t *__restrict__ keys, uint64_t *__restrict__ vals)
-{
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const WideEntry e = in[i];
-        keys[i] = e.k;
-        vals[i] = e.v;
-    }
 }
 
 }  // namespace
@@ -900,26 +879,19 @@ __global__ __launch_bounds__(256) void wide_split_kernel(const WideEntry *__rest
 // The wide form of the group bulk fill (dyc_bulk.hip): keys fold to 32 bits for the pair and the
 // bucket (fold64), and entries are 16-byte key/value pairs.
 
-template <bool IN_ENTRIES>
 __global__ __launch_bounds__(kCountThreads) void wide_group_bulk_pack_kernel(const WideDesc *__restrict__ dir,
                                                                              const GroupItem *__restrict__ blocks,
                                                                              const uint64_t *__restrict__ keys,
-                                                                             const WideEntry *__restrict__ in,
                                                                              uint8_t *__restrict__ lcid,
                                                                              uint32_t *__restrict__ partial)
 {
     __shared__ uint32_t h[kGroupBulkChunks];
     __shared__ uint4 sub_tab[kMaxSubtables];  // per subtable: buckets, divider, the table's first local chunk of it
-    __shared__ uint32_t tsel[32];  // the round's subtable by key parity and pair (fill_round_sub)
+    __shared__ uint32_t tsel[32];  // the target subtable by key parity and pair (fill_sub)
     const GroupItem item = blocks[blockIdx.x];
-    if (item.len == 0) {  // block-uniform: a clipped block of round 2 counts nothing
-        for (uint32_t d = threadIdx.x; d < kGroupBulkChunks; d += kCountThreads)
-            partial[(uint64_t)blockIdx.x * kGroupBulkChunks + d] = 0;
-        return;
-    }
     const Desc D = dir[item.table].D;  // by value: loaded once, not per use through memory
     for (uint32_t d = threadIdx.x; d < kGroupBulkChunks; d += kCountThreads) h[d] = 0;
-    if (threadIdx.x < 32) tsel[threadIdx.x] = fill_round_sub(D, threadIdx.x, IN_ENTRIES);
+    if (threadIdx.x < 32) tsel[threadIdx.x] = fill_sub(D, threadIdx.x);
     if (threadIdx.x < kMaxSubtables) {
         const uint32_t t = threadIdx.x;
         uint32_t first = 0;
@@ -933,15 +905,14 @@ __global__ __launch_bounds__(kCountThreads) void wide_group_bulk_pack_kernel(con
 #pragma unroll
         for (int u = 0; u < kCountItems; ++u) {
             const uint64_t i = i0 + (uint64_t)u * kCountThreads;
-            if constexpr (IN_ENTRIES) k[u] = i < hi ? in[i].k : 0ull;
-            else k[u] = i < hi ? keys[i] : 0ull;
+            k[u] = i < hi ? keys[i] : 0ull;
         }
 #pragma unroll
         for (int u = 0; u < kCountItems; ++u) {
             const uint64_t i = i0 + (uint64_t)u * kCountThreads;
             if (i >= hi) continue;
             uint32_t lc = 0;
-            if (IN_ENTRIES || !wide_reserved(k[u])) {
+            if (!wide_reserved(k[u])) {
                 const uint32_t f = fold64(k[u]), p = pair_of(D, f);
                 const uint32_t t = tsel[(((uint32_t)k[u] & 1u) << 4) | p];
                 const uint4 q = sub_tab[t];
@@ -956,7 +927,7 @@ __global__ __launch_bounds__(kCountThreads) void wide_group_bulk_pack_kernel(con
         partial[(uint64_t)blockIdx.x * kGroupBulkChunks + d] = h[d];
 }
 
-template <bool DENSE, int THREADS>
+template <int THREADS>
 __global__ __launch_bounds__(THREADS) void wide_group_bulk_fill_kernel(const GroupChunk *__restrict__ chunks,
                                                                        const WideEntry *__restrict__ ent,
                                                                        WideEntry *__restrict__ ovf,
@@ -967,26 +938,12 @@ __global__ __launch_bounds__(THREADS) void wide_group_bulk_fill_kernel(const Gro
     const GroupChunk R = chunks[blockIdx.x];
     unsigned long long placed = 0, rejected = 0;
     if (R.cnt)  // block-uniform
-        wide_fill_chunk<DENSE, THREADS>(R.S, R.b0, R.len, ent, R.lo, R.lo + R.cnt, ovf + R.ovf_off, R.ovf_cap,
-                                        ovf_n + R.j, zeroed, placed, rejected);
+        wide_fill_chunk<THREADS>(R.S, R.b0, R.len, ent, R.lo, R.lo + R.cnt, ovf + R.ovf_off, R.ovf_cap, ovf_n + R.j,
+                                 zeroed, placed, rejected);
     const unsigned long long wp = wave_sum(placed);
     if (__lane_id() == 0 && wp) atomicAdd(&table_counts[R.table], wp);
     wave_tally(C, &C->kicks, placed);
     wave_tally(C, &C->rejected, rejected);
-}
-
-// The overflow entries of every item as the key and value arrays the group insert reads (same
-// indexes); one workgroup per item.
-__global__ __launch_bounds__(256) void wide_items_split_kernel(const GroupItem *__restrict__ items,
-                                                               const WideEntry *__restrict__ in,
-                                                               uint64_t *__restrict__ keys, uint64_t *__restrict__ vals)
-{
-    const GroupItem it = items[blockIdx.x];
-    for (uint64_t i = it.begin + threadIdx.x; i < it.begin + it.len; i += blockDim.x) {
-        const WideEntry e = in[i];
-        keys[i] = e.k;
-        vals[i] = e.v;
-    }
 }
 
 // ------------------------------------------------------------------------------ launchers
@@ -1021,10 +978,22 @@ hipError_t launch_wide_insert(const WideDesc &W, const uint64_t *keys, const uin
     if (n == 0) return hipSuccess;
     const int grid = grid_for((n + kWave - 1) / kWave, sh, kWideInsertBlocks);
     if (from_entries)
-        wide_insert_kernel<true><<<grid, sh.block_threads, 0, st>>>(W, keys, vals, n, pre_fixed, pol, C, sink, skip);
+        wide_insert_kernel<kWideList>
+            <<<grid, sh.block_threads, 0, st>>>(W, keys, vals, nullptr, n, pre_fixed, pol, C, sink, skip, nullptr);
     else
-        wide_insert_kernel<false><<<grid, sh.block_threads, 0, st>>>(W, keys, vals, n, kNoTable, pol, C, sink,
-                                                                     skip);
+        wide_insert_kernel<kWideBatch>
+            <<<grid, sh.block_threads, 0, st>>>(W, keys, vals, nullptr, n, kNoTable, pol, C, sink, skip, nullptr);
+    return hipGetLastError();
+}
+
+// As launch_insert_overflow, for a wide bulk fill of n entries (ovf[0, C->overflow)).
+hipError_t launch_wide_insert_overflow(const WideDesc &W, const WideEntry *ovf, uint64_t n, InsertPolicy pol,
+                                       LaunchShape sh, Counters *C, const WideSink &sink, hipStream_t st)
+{
+    if (n == 0) return hipSuccess;
+    const int grid = grid_for((n + kWave - 1) / kWave, sh, kWideInsertBlocks);
+    wide_insert_kernel<kWideOverflow><<<grid, sh.block_threads, 0, st>>>(W, nullptr, nullptr, ovf, n, kAfterFill, pol, C,
+                                                                        sink, nullptr, &C->overflow);
     return hipGetLastError();
 }
 
@@ -1050,7 +1019,22 @@ hipError_t launch_wide_group_insert(const WideDesc *dir, const GroupItem *items,
 {
     if (n_items == 0) return hipSuccess;
     const int grid = blocks > 0 ? blocks : std::min<int>(kWideGroupBlocks, (int)((n_items + 3) / 4));
-    wide_group_insert_kernel<<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts);
+    wide_group_insert_kernel<kWideBatch>
+        <<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, nullptr, pol, C, sink, table_counts, nullptr);
+    return hipGetLastError();
+}
+
+// As launch_group_insert_overflow.
+hipError_t launch_wide_group_insert_overflow(const WideDesc *dir, const GroupItem *items,
+                                             const unsigned long long *n_items, uint64_t max_items,
+                                             const WideEntry *ovf, InsertPolicy pol, int blocks, Counters *C,
+                                             const WideSink &sink, unsigned long long *table_counts, hipStream_t st)
+{
+    if (max_items == 0) return hipSuccess;
+    if (max_items > 0xffffffffull) return hipErrorInvalidValue;
+    const int grid = blocks > 0 ? blocks : (int)std::min<uint64_t>(kWideGroupBlocks, (max_items + 3) / 4);
+    wide_group_insert_kernel<kWideOverflow><<<grid, 256, 0, st>>>(dir, items, (uint32_t)max_items, nullptr, nullptr, ovf,
+                                                                  pol, C, sink, table_counts, n_items);
     return hipGetLastError();
 }
 
@@ -1059,60 +1043,37 @@ constexpr int kWideSortThreads = 256;
 constexpr uint32_t kWideSortTile = kWideSortThreads * kSortItems;
 
 template <typename CidT>
-hipError_t wide_partition(const WideDesc &W, const Chunks &Ch, const uint64_t *keys, const uint64_t *vals, int in,
-                          uint64_t n, const BulkSpace &ws, uint32_t max_blocks, hipStream_t st, int *out)
+hipError_t wide_partition(const WideDesc &W, const Chunks &Ch, const uint64_t *keys, const uint64_t *vals, uint64_t n,
+                          const BulkSpace &ws, uint32_t max_blocks, hipStream_t st, int *out)
 {
     RadixPass P[kMaxRadixPasses];
     const uint32_t np = radix_passes(Ch.bits, P);
     const PartGrid G = part_grid(n, max_blocks, kWideSortTile);
     CidT *const cid[2] = {static_cast<CidT *>(ws.cid[0]), static_cast<CidT *>(ws.cid[1])};
     WideEntry *const ent[2] = {static_cast<WideEntry *>(ws.ent[0]), static_cast<WideEntry *>(ws.ent[1])};
-    if (keys) {
-        wide_bulk_pack_kernel<false, CidT><<<G.blocks * G.sub, kCountThreads, 0, st>>>(W, Ch, keys, nullptr, G, P[0], cid[0],
-                                                                               ws.partial);
-        return partition_passes<WideEntry, WideKeyValSource, CidT, kWideSortThreads>(
-            WideKeyValSource{keys, vals}, 0, ent, cid, G, P, np, ws.partial, ws.total, ws.start, Ch.total, st, out);
-    }
-    wide_bulk_pack_kernel<true, CidT><<<G.blocks * G.sub, kCountThreads, 0, st>>>(W, Ch, nullptr, ent[in], G, P[0], cid[0],
-                                                                          ws.partial);
-    return partition_passes<WideEntry, EntrySource<WideEntry>, CidT, kWideSortThreads>(
-        EntrySource<WideEntry>{ent[in]}, 1 - in, ent, cid, G, P, np, ws.partial, ws.total, ws.start, Ch.total, st,
-        out);
+    wide_bulk_pack_kernel<CidT><<<G.blocks * G.sub, kCountThreads, 0, st>>>(W, Ch, keys, G, P[0], cid[0], ws.partial);
+    return partition_passes<WideEntry, WideKeyValSource, CidT, kWideSortThreads>(
+        WideKeyValSource{keys, vals}, 0, ent, cid, G, P, np, ws.partial, ws.total, ws.start, Ch.total, st, out);
 }
 
-// Group n wide entries by chunk, as launch_bulk_partition does for the 32-bit table (round 1
-// from keys/vals, round 2 from ws.ent[in]); the sorted entries end in ws.ent[*out].
+// Group n wide entries by chunk, as launch_bulk_partition does for the 32-bit table; the sorted
+// entries end in ws.ent[*out].
 hipError_t launch_wide_partition(const WideDesc &W, const Chunks &Ch, const uint64_t *keys, const uint64_t *vals,
-                                 int in, uint64_t n, const BulkSpace &ws, uint32_t max_blocks, hipStream_t st,
-                                 int *out)
+                                 uint64_t n, const BulkSpace &ws, uint32_t max_blocks, hipStream_t st, int *out)
 {
-    *out = keys ? 0 : 1 - in;
+    *out = 0;
     if (n == 0) return hipSuccess;
     if (n >= (1ull << 32) || Ch.total == 0 || Ch.bits > kMaxRadixPasses * kMaxRadixBits) return hipErrorInvalidValue;
-    if (bulk_cid_bytes(Ch) == 2) return wide_partition<uint16_t>(W, Ch, keys, vals, in, n, ws, max_blocks, st, out);
-    return wide_partition<uint32_t>(W, Ch, keys, vals, in, n, ws, max_blocks, st, out);
+    if (bulk_cid_bytes(Ch) == 2) return wide_partition<uint16_t>(W, Ch, keys, vals, n, ws, max_blocks, st, out);
+    return wide_partition<uint32_t>(W, Ch, keys, vals, n, ws, max_blocks, st, out);
 }
 
 hipError_t launch_wide_bulk_fill(const WideDesc &W, const Chunks &Ch, const uint32_t *start, const WideEntry *ent,
-                                 uint64_t n, WideEntry *ovf, uint64_t ovf_cap, unsigned long long *ovf_n, Counters *C,
-                                 bool zeroed, hipStream_t st)
+                                 uint64_t n, WideEntry *ovf, uint64_t ovf_cap, Counters *C, bool zeroed, hipStream_t st)
 {
     if (n == 0) return hipSuccess;
     if (n >= (1ull << 32) || Ch.total == 0) return hipErrorInvalidValue;
-    uint64_t buckets = 0;
-    for (uint32_t t = 0; t < W.D.d; ++t) buckets += W.D.nb[t];
-    if (n >= 2 * buckets)
-        wide_bulk_fill_kernel<true, 1024><<<Ch.total, 1024, 0, st>>>(W, Ch, start, ent, n, ovf, ovf_cap, ovf_n, C, zeroed);
-    else
-        wide_bulk_fill_kernel<false, 256><<<Ch.total, 256, 0, st>>>(W, Ch, start, ent, n, ovf, ovf_cap, ovf_n, C, false);
-    return hipGetLastError();
-}
-
-hipError_t launch_wide_split(const WideEntry *in, uint64_t n, uint64_t *keys, uint64_t *vals, hipStream_t st)
-{
-    if (n == 0) return hipSuccess;
-    const int grid = grid_for((n + kWave - 1) / kWave, LaunchShape{256, 0}, 16384);
-    wide_split_kernel<<<grid, 256, 0, st>>>(in, n, keys, vals);
+    wide_bulk_fill_kernel<1024><<<Ch.total, 1024, 0, st>>>(W, Ch, start, ent, n, ovf, ovf_cap, C, zeroed);
     return hipGetLastError();
 }
 
@@ -1174,7 +1135,7 @@ struct dyc_wide {
     uint8_t *upd = nullptr;  // upsert: per-key "updated in place" flags
     uint64_t upd_cap = 0;
     // bulk fill (insert_order 3): (chunk id, entry) pairs and their sort buffers, the chunk
-    // starts, the radix sort's scratch and the overflow count (device, and a pinned read-back)
+    // starts and the partition's counts
     void *bk_cid[2] = {};
     WideEntry *bk_ent[2] = {};
     uint64_t bk_cap = 0;
@@ -1182,8 +1143,6 @@ struct dyc_wide {
     uint32_t *bk_start = nullptr;
     uint64_t bk_start_cap = 0;
     uint32_t *bk_partial = nullptr;  // kPartialWords, then 256 digit totals
-    unsigned long long *bk_ovf = nullptr;
-    unsigned long long *bk_hovf = nullptr;
     Reclaimer reclaim;  // frees retired subtables off the calling thread
     dyc_stats st{};
 
@@ -1571,60 +1530,25 @@ int wreserve_bulk(dyc_wide *t, uint64_t n, const Chunks &Ch, hipStream_t s)
     if (!t->bk_partial &&
         (rc = walloc((void **)&t->bk_partial, (kPartialWords + kMaxRadixWords) * sizeof(uint32_t), "partition counts")))
         return rc;
-    if (!t->bk_ovf && (rc = walloc((void **)&t->bk_ovf, 256, "overflow count"))) return rc;
-    if (!t->bk_hovf && hipHostMalloc((void **)&t->bk_hovf, 64, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        t->bk_hovf = nullptr;
-        return fail(DYC_ERR_OOM, "hipHostMalloc of the bulk-fill read-back word failed");
-    }
     return DYC_OK;
 }
 
-// One fill round over n entries: round 1 from keys/vals (keys != nullptr), round 2 from the
-// entries in bk_ent[in]. Partition them by chunk, fill, and read back how many entries overflowed
-// into bk_ent[*out] (the buffer the partition did not end in).
-int wbulk_round(dyc_wide *t, const Chunks &Ch, const uint64_t *keys, const uint64_t *vals, int in, uint64_t n,
-                bool zeroed, hipStream_t s, int *out, uint64_t *overflow)
+// insert_order 3 for wide keys: fill each key's fill_target bucket, then the overflow, whose length
+// stays on the device, goes to the other bucket by the eviction insert (the narrow table's
+// bulk_insert over fold(k)).
+int wbulk_insert(dyc_wide *t, const uint64_t *keys, const uint64_t *vals, uint64_t n, bool was_zeroed, hipStream_t s)
 {
-    const BulkSpace ws{{t->bk_ent[0], t->bk_ent[1]}, {t->bk_cid[0], t->bk_cid[1]}, t->bk_partial,
-                       t->bk_partial + kPartialWords, t->bk_start};
-    int r = 0;
-    HIP_TRY(launch_wide_partition(t->W, Ch, keys, vals, in, n, ws, kWideSortBlocks, s, &r));
-    HIP_TRY(launch_zero(t->bk_ovf, 1, s));
-    HIP_TRY(launch_wide_bulk_fill(t->W, Ch, t->bk_start, t->bk_ent[r], n, t->bk_ent[1 - r], t->bk_cap, t->bk_ovf,
-                                  t->ctr, zeroed, s));
-    HIP_TRY(hipMemcpyAsync(t->bk_hovf, t->bk_ovf, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    *overflow = *t->bk_hovf;
-    *out = 1 - r;
-    if (*overflow > n)
-        return fail(DYC_ERR_CORRUPT, "bulk fill overflow count %llu exceeds the batch (%llu)",
-                    (unsigned long long)*overflow, (unsigned long long)n);
-    return DYC_OK;
-}
-
-// insert_order 3 for wide keys: fill each key's fill_target bucket, then the other bucket, then
-// the eviction insert for the rest (the narrow table's bulk_insert over fold(k)).
-int wbulk_insert(dyc_wide *t, const uint64_t *keys, const uint64_t *vals, uint64_t n, bool was_zeroed, hipStream_t s,
-                 uint64_t *left)
-{
-    *left = 0;
     const Chunks Ch = make_chunks(t->W.D);  // the workspace was reserved for it
-    int ov = 0, ov2 = 0;
-    uint64_t m1 = 0, m2 = 0;
     // an empty table (count 0, nothing pending) that no call has stored into since it was
     // created or cleared holds zeros only
     const bool zeroed = was_zeroed && t->count == 0 && t->pend_n == 0;
-    int rc = wbulk_round(t, Ch, keys, vals, 0, n, zeroed, s, &ov, &m1);
-    if (rc || m1 == 0) return rc;
-    rc = wbulk_round(t, Ch, nullptr, nullptr, ov, m1, false, s, &ov2, &m2);  // the overflow, in its other table
-    if (rc || m2 == 0) return rc;
-    *left = m2;
-    // the other entry buffer (16 B per key of capacity) holds m2 keys and then m2 values
-    uint64_t *const sk = reinterpret_cast<uint64_t *>(t->bk_ent[1 - ov2]);
-    HIP_TRY(launch_wide_split(t->bk_ent[ov2], m2, sk, sk + m2, s));
-    HIP_TRY(launch_wide_insert(t->W, sk, sk + m2, m2, kNoTable, true, t->policy(), t->insert_shape(), t->ctr,
-                               t->sink_at(t->pend_n), s));
+    const BulkSpace ws{{t->bk_ent[0], t->bk_ent[1]}, {t->bk_cid[0], t->bk_cid[1]}, t->bk_partial,
+                       t->bk_partial + kPartialWords, t->bk_start};
+    int r = 0;
+    HIP_TRY(launch_wide_partition(t->W, Ch, keys, vals, n, ws, kWideSortBlocks, s, &r));
+    WideEntry *const ovf = t->bk_ent[1 - r];  // the buffer the partition did not end in
+    HIP_TRY(launch_wide_bulk_fill(t->W, Ch, t->bk_start, t->bk_ent[r], n, ovf, t->bk_cap, t->ctr, zeroed, s));
+    HIP_TRY(launch_wide_insert_overflow(t->W, ovf, n, t->policy(), t->insert_shape(), t->ctr, t->sink_at(t->pend_n), s));
     return DYC_OK;
 }
 
@@ -1704,8 +1628,6 @@ int dyc_wide_destroy(dyc_wide *t)
     }
     if (t->bk_start) (void)hipFree(t->bk_start);
     if (t->bk_partial) (void)hipFree(t->bk_partial);
-    if (t->bk_ovf) (void)hipFree(t->bk_ovf);
-    if (t->bk_hovf) (void)hipHostFree(t->bk_hovf);
     delete t;
     return DYC_OK;
 }
@@ -1746,9 +1668,8 @@ int dyc_wide_insert(dyc_wide *t, const uint64_t *keys, const uint64_t *vals, uin
     }
     rc = wzero(t, s);
     if (rc) return rc;
-    uint64_t left = 0;  // entries the bulk fill left to the eviction insert
     if (bulk) {
-        rc = wbulk_insert(t, keys, vals, n, zeroed, s, &left);
+        rc = wbulk_insert(t, keys, vals, n, zeroed, s);
         if (rc) return rc;
     } else {
         HIP_TRY(launch_wide_insert(t->W, keys, vals, n, kNoTable, false, t->policy(), t->insert_shape(), t->ctr,
@@ -1759,7 +1680,7 @@ int dyc_wide_insert(dyc_wide *t, const uint64_t *keys, const uint64_t *vals, uin
     const uint64_t rejected = t->hctr->rejected;
     t->st.rejected += rejected;
     t->count += n - rejected;
-    if (bulk) t->st.last_filled = n - rejected - left;
+    if (bulk) t->st.last_filled = n - rejected - t->hctr->left;
     rc = wabsorb(t, room);
     t->st.pending = t->pend_n;
     if (rc) return rc;
@@ -1985,19 +1906,19 @@ struct dyc_wide_group {
     // insert
     bool zeroed = false;
     // bulk fill (cfg.insert_order 3), grown on demand: partitioned entries and the overflow (16 B
-    // per key each; the entry buffer also holds the last overflow split into keys and values),
-    // local chunk ids, per-block chunk counts, per-chunk start / count / table, overflow counts
-    // of both rounds, and the block and table arrays (device, with pinned staging)
+    // per key each), local chunk ids, per-block chunk counts, chunk records, overflow counts and
+    // items, and the block and table arrays (device, with pinned staging)
     WideEntry *bk_ent = nullptr, *bk_ovf = nullptr;
     uint8_t *bk_lcid = nullptr;
     uint64_t bk_cap = 0;
     uint32_t *bk_partial = nullptr;
     uint64_t bk_partial_cap = 0;
-    GroupChunk *bk_chunks = nullptr;  // chunk records of a round
+    GroupChunk *bk_chunks = nullptr;
     uint64_t bk_chunk_cap = 0;
-    unsigned long long *bk_ovfn = nullptr, *bk_hovfn = nullptr;
+    GroupItem *bk_items = nullptr;   // the overflow's work items
+    uint64_t bk_items_cap = 0;
+    unsigned long long *bk_ovfn = nullptr;  // the tables' overflow counts, then the item count
     GroupItem *bk_blk = nullptr, *bk_hblk = nullptr;
-    uint32_t *bk_btab = nullptr, *bk_hbtab = nullptr;
     uint64_t bk_blk_cap = 0;
     BulkTable *bk_tabs = nullptr, *bk_htabs = nullptr;
     uint32_t bk_tabs_cap = 0;
@@ -2187,10 +2108,8 @@ int wg_reserve_bulk(dyc_wide_group *g, const dyc::host::BulkLayout &L)
     }
     if (blocks > g->bk_blk_cap) {
         g->bk_blk_cap = 0;
-        regrow((void **)&g->bk_blk, 3 * blocks * sizeof(GroupItem), "blocks");
-        regrow((void **)&g->bk_btab, blocks * sizeof(uint32_t), "block tables");
+        regrow((void **)&g->bk_blk, blocks * sizeof(GroupItem), "blocks");
         regrow_pinned((void **)&g->bk_hblk, blocks * sizeof(GroupItem));
-        regrow_pinned((void **)&g->bk_hbtab, blocks * sizeof(uint32_t));
         if (rc) return rc;
         g->bk_blk_cap = blocks;
     }
@@ -2200,75 +2119,58 @@ int wg_reserve_bulk(dyc_wide_group *g, const dyc::host::BulkLayout &L)
         if (rc) return rc;
         g->bk_chunk_cap = chunks;
     }
+    const uint64_t items = overflow_items(n, tabs);
+    if (items > g->bk_items_cap) {
+        g->bk_items_cap = 0;
+        regrow((void **)&g->bk_items, items * sizeof(GroupItem), "overflow items");
+        if (rc) return rc;
+        g->bk_items_cap = items;
+    }
     if (tabs > g->bk_tabs_cap) {
         g->bk_tabs_cap = 0;
-        regrow((void **)&g->bk_tabs, 2 * tabs * sizeof(BulkTable), "table list");
-        regrow((void **)&g->bk_ovfn, 2 * tabs * sizeof(unsigned long long), "overflow counts");
+        regrow((void **)&g->bk_tabs, tabs * sizeof(BulkTable), "table list");
+        regrow((void **)&g->bk_ovfn, (tabs + 1ull) * sizeof(unsigned long long), "overflow counts");
         regrow_pinned((void **)&g->bk_htabs, tabs * sizeof(BulkTable));
-        regrow_pinned((void **)&g->bk_hovfn, tabs * sizeof(unsigned long long));
         if (rc) return rc;
         g->bk_tabs_cap = tabs;
     }
     return DYC_OK;
 }
 
-// The whole wide bulk fill of a laid-out batch on s, rounds chained on the device as in the
-// 32-bit group fill (dyc_group.hip): round 1, round 2 for the other bucket, then the eviction
-// insert of what overflows that (its entries split into key and value arrays first).
+// The whole wide bulk fill of a laid-out batch on s, as the 32-bit group's (enqueue_group_bulk in
+// dyc_group.hip).
 hipError_t wg_enqueue_bulk(dyc_wide_group *g, uint32_t NB, uint32_t J, uint32_t chunks, const uint64_t *keys,
                            const uint64_t *vals, uint64_t total, bool zeroed, const WideSink &sink, hipStream_t s)
 {
-    GroupItem *const blk1 = g->bk_blk, *const blk2 = g->bk_blk + NB, *const items = g->bk_blk + 2 * NB;
-    BulkTable *const tabs1 = g->bk_tabs, *const tabs2 = g->bk_tabs + J;
-    unsigned long long *const ovf1 = g->bk_ovfn, *const ovf2 = g->bk_ovfn + J;
+    unsigned long long *const n_items = g->bk_ovfn + J;
     uint8_t *const no_cid = nullptr;
-    const SegLayout lay1{blk1, g->bk_partial, total}, lay2{blk2, g->bk_partial, total};
+    const SegLayout lay{g->bk_blk, g->bk_partial, total};
     hipError_t e;
-    wide_group_bulk_pack_kernel<false><<<NB, kCountThreads, 0, s>>>(g->ddir, blk1, keys, nullptr, g->bk_lcid,
-                                                                    g->bk_partial);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = launch_group_bulk_scan(g->ddir, tabs1, J, g->bk_partial, g->bk_chunks, s)) != hipSuccess)
+    wide_group_bulk_pack_kernel<<<NB, kCountThreads, 0, s>>>(g->ddir, g->bk_blk, keys, g->bk_lcid, g->bk_partial);
+    if ((e = hipGetLastError()) != hipSuccess ||
+        (e = launch_group_bulk_scan(g->ddir, g->bk_tabs, J, g->bk_partial, g->bk_chunks, s)) != hipSuccess)
         return e;
     part_scatter_kernel<WideEntry, WideKeyValSource, uint8_t, kWideSortThreads, -1, SegLayout>
-        <<<NB, kWideSortThreads, 0, s>>>(WideKeyValSource{keys, vals}, g->bk_lcid, lay1, RadixPass{0, 8}, g->bk_ent,
+        <<<NB, kWideSortThreads, 0, s>>>(WideKeyValSource{keys, vals}, g->bk_lcid, lay, RadixPass{0, 8}, g->bk_ent,
                                          no_cid);
-    if ((e = hipGetLastError()) != hipSuccess || (e = launch_zero(ovf1, 2 * (uint64_t)J, s)) != hipSuccess) return e;
-    wide_group_bulk_fill_kernel<true, 1024><<<chunks, 1024, 0, s>>>(g->bk_chunks, g->bk_ent, g->bk_ovf, ovf1,
-                                                                   g->tcounts, g->ctr, zeroed);
+    if ((e = hipGetLastError()) != hipSuccess || (e = launch_zero(g->bk_ovfn, J + 1ull, s)) != hipSuccess) return e;
+    wide_group_bulk_fill_kernel<1024><<<chunks, 1024, 0, s>>>(g->bk_chunks, g->bk_ent, g->bk_ovf, g->bk_ovfn,
+                                                              g->tcounts, g->ctr, zeroed);
     if ((e = hipGetLastError()) != hipSuccess ||
-        (e = launch_group_bulk_clip(blk1, g->bk_btab, NB, tabs1, J, ovf1, blk2, tabs2, s)) != hipSuccess)
+        (e = launch_group_bulk_items(g->bk_tabs, J, g->bk_ovfn, g->bk_items, g->bk_items_cap, n_items, s)) !=
+            hipSuccess)
         return e;
-    wide_group_bulk_pack_kernel<true><<<NB, kCountThreads, 0, s>>>(g->ddir, blk2, nullptr, g->bk_ovf, g->bk_lcid,
-                                                                   g->bk_partial);
-    if ((e = hipGetLastError()) != hipSuccess ||
-        (e = launch_group_bulk_scan(g->ddir, tabs2, J, g->bk_partial, g->bk_chunks, s)) != hipSuccess)
-        return e;
-    part_scatter_kernel<WideEntry, EntrySource<WideEntry>, uint8_t, kWideSortThreads, -1, SegLayout>
-        <<<NB, kWideSortThreads, 0, s>>>(EntrySource<WideEntry>{g->bk_ovf}, g->bk_lcid, lay2, RadixPass{0, 8},
-                                         g->bk_ent, no_cid);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    wide_group_bulk_fill_kernel<false, 256><<<chunks, 256, 0, s>>>(g->bk_chunks, g->bk_ent, g->bk_ovf, ovf2,
-                                                                   g->tcounts, g->ctr, false);
-    if ((e = hipGetLastError()) != hipSuccess ||
-        (e = launch_group_bulk_clip(blk1, g->bk_btab, NB, tabs1, J, ovf2, items, nullptr, s)) != hipSuccess)
-        return e;
-    // the entry buffer (16 B per key) is free now: keys, then values, at the overflow's indexes
-    uint64_t *const sk = reinterpret_cast<uint64_t *>(g->bk_ent);
-    uint64_t *const sv = sk + total;
-    wide_items_split_kernel<<<NB, 256, 0, s>>>(items, g->bk_ovf, sk, sv);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    return launch_wide_group_insert(g->ddir, items, NB, sk, sv, g->policy(), (int)g->cfg.insert_blocks, g->ctr, sink,
-                                    g->tcounts, s);
+    return launch_wide_group_insert_overflow(g->ddir, g->bk_items, n_items, overflow_items(total, J), g->bk_ovf,
+                                             g->policy(), (int)g->cfg.insert_blocks, g->ctr, sink, g->tcounts, s);
 }
 
-// insert_order 3 for a wide group (see group_bulk_insert in dyc_group.hip). Declines (*n_tabs 0)
-// when the batch does not qualify or the workspace cannot be allocated; counters and per-table
-// counts are zeroed here; the last round's overflow counts (*n_tabs) are in bk_hovfn after the
-// caller's wait.
+// insert_order 3 for a wide group (see group_bulk_insert in dyc_group.hip). Declines (*filled
+// false) when the batch does not qualify or the workspace cannot be allocated; counters and
+// per-table counts are zeroed here.
 int wg_bulk_insert(dyc_wide_group *g, const uint64_t *keys, const uint64_t *vals, const uint64_t *offsets,
-                   bool zeroed, hipStream_t s, uint64_t room, uint32_t *n_tabs)
+                   bool zeroed, hipStream_t s, uint64_t room, bool *filled)
 {
-    *n_tabs = 0;
+    *filled = false;
     dyc::host::BulkLayout L;
     if (!dyc::host::bulk_layout(g->n, offsets, [g](uint32_t i) -> const Desc & { return g->hdir[i].D; }, &L))
         return DYC_OK;
@@ -2284,17 +2186,14 @@ int wg_bulk_insert(dyc_wide_group *g, const uint64_t *keys, const uint64_t *vals
     }
     const uint32_t NB = (uint32_t)L.blocks.size(), J = (uint32_t)L.tabs.size();
     memcpy(g->bk_hblk, L.blocks.data(), NB * sizeof(GroupItem));
-    memcpy(g->bk_hbtab, L.btab.data(), NB * sizeof(uint32_t));
     memcpy(g->bk_htabs, L.tabs.data(), J * sizeof(BulkTable));
     HIP_TRY(hipMemcpyAsync(g->bk_blk, g->bk_hblk, NB * sizeof(GroupItem), hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(g->bk_btab, g->bk_hbtab, NB * sizeof(uint32_t), hipMemcpyHostToDevice, s));
     HIP_TRY(hipMemcpyAsync(g->bk_tabs, g->bk_htabs, J * sizeof(BulkTable), hipMemcpyHostToDevice, s));
     const int rc = wg_prologue(g, s);
     if (rc) return rc;
     HIP_TRY(wg_enqueue_bulk(g, NB, J, L.chunks, keys, vals, L.total, zeroed,
                             WideSink{g->pk + g->pend_n, g->pv + g->pend_n, room, g->ptag + g->pend_n}, s));
-    HIP_TRY(hipMemcpyAsync(g->bk_hovfn, g->bk_ovfn + J, J * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-    *n_tabs = J;
+    *filled = true;
     return DYC_OK;
 }
 
@@ -2320,10 +2219,10 @@ int dyc_wide_group_destroy(dyc_wide_group *g)
     if (g->hitems) (void)hipHostFree(g->hitems);
     if (g->items_free) (void)hipEventDestroy(g->items_free);
     for (void *p : {(void *)g->bk_ent, (void *)g->bk_ovf, (void *)g->bk_lcid, (void *)g->bk_partial,
-                    (void *)g->bk_chunks, (void *)g->bk_tabs,
-                    (void *)g->bk_ovfn, (void *)g->bk_blk, (void *)g->bk_btab})
+                    (void *)g->bk_chunks, (void *)g->bk_tabs, (void *)g->bk_items,
+                    (void *)g->bk_ovfn, (void *)g->bk_blk})
         if (p) (void)hipFree(p);
-    for (void *p : {(void *)g->bk_htabs, (void *)g->bk_hovfn, (void *)g->bk_hblk, (void *)g->bk_hbtab})
+    for (void *p : {(void *)g->bk_htabs, (void *)g->bk_hblk})
         if (p) (void)hipHostFree(p);
     delete g;
     return DYC_OK;
@@ -2417,12 +2316,12 @@ int dyc_wide_group_insert(dyc_wide_group *g, const uint64_t *keys, const uint64_
     rc = wg_reserve_pending(g, std::max<uint64_t>(65536, total / 16), s);
     if (rc) return rc;
     const uint64_t room = g->pend_cap - g->pend_n;
-    uint32_t n_tabs = 0;
+    bool filled = false;
     if (g->cfg.insert_order == 3) {
-        rc = wg_bulk_insert(g, keys, vals, offsets, zeroed, s, room, &n_tabs);
+        rc = wg_bulk_insert(g, keys, vals, offsets, zeroed, s, room, &filled);
         if (rc) return rc;
     }
-    if (!n_tabs) {
+    if (!filled) {
         uint32_t n_items = 0;
         rc = wg_upload_items(g, offsets, s, &n_items);
         if (rc) return rc;
@@ -2436,11 +2335,7 @@ int dyc_wide_group_insert(dyc_wide_group *g, const uint64_t *keys, const uint64_
     rc = wg_read_back(g, s);
     if (rc) return rc;
     const Counters &c = *g->hctr;
-    if (n_tabs) {
-        uint64_t left = 0;
-        for (uint32_t j = 0; j < n_tabs; ++j) left += g->bk_hovfn[j];
-        g->st.last_filled = total - c.rejected - left;
-    }
+    if (filled) g->st.last_filled = total - c.rejected - c.left;
     g->st.kicks += c.kicks;
     g->st.last_kicks = c.kicks;
     g->st.cas_retries += c.retries;

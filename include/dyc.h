@@ -105,8 +105,9 @@ typedef struct dyc_stats {
     uint32_t last_max_chain;    /* the longest eviction chain (exchanges) of the most recent insert call
                                    (32-bit tables; the maximum of the reference's iterator_count,
                                    api.cpp:219-243) */
-    uint64_t last_filled;       /* entries the most recent insert call placed by bucket fill
-                                   (insert_order 3); 0 when the eviction insert took the batch */
+    uint64_t last_filled;       /* entries the most recent insert call placed by bucket fill or in a
+                                   free slot of their other bucket (insert_order 3), so without
+                                   evicting; 0 when the eviction insert took the batch */
 } dyc_stats;
 
 /* Defaults (see field comments). */
