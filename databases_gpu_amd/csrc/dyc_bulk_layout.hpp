@@ -52,13 +52,12 @@ bool bulk_layout(uint32_t n_tables, const uint64_t *offsets, DescOf desc, BulkLa
 }
 
 // Find items laid out by XCD. Workgroups go to the device's XCDs in turn (workgroup b to XCD
-// b % kXcds) and a probe launch's wave w of workgroup b takes item slots b * 4 + w, then every
-// (grid * 4)-th slot after it, so slot i runs on XCD (i / 4) % kXcds (for a grid that is a
-// multiple of kXcds; any other grid only loses the layout's benefit). Each table goes whole to
-// one XCD (largest first, to the one with the fewest items), so the waves of an XCD probe a few
-// tables at a time and its L2 holds their lines, instead of every XCD reading every table the
-// launch has in flight. Slots an XCD has no item for hold empty items.
-constexpr uint32_t kXcds = 8, kProbeWavesPerBlock = 4;
+// b % kXcds) and a probe launch's workgroup b takes items b, b + grid, ..., so item i runs on XCD
+// i % kXcds (for a grid that is a multiple of kXcds; any other grid only loses the layout's
+// benefit). Each table goes whole to one XCD (largest first, to the one with the fewest items), so
+// the waves of an XCD probe a few tables at a time and its L2 holds their lines, instead of every
+// XCD reading every table the launch has in flight. Places an XCD has no item for hold empty items.
+constexpr uint32_t kXcds = 8;
 constexpr uint64_t kXcdLayoutKeys = 1ull << 22;  // eager finds of fewer keys keep the table order
 
 // The layout itself: n tables' batches (offsets, as the calls take them) cut into items of at
@@ -81,13 +80,9 @@ inline std::vector<GroupItem> items_by_xcd(const uint64_t *offsets, uint32_t n, 
     }
     size_t most = 0;
     for (const auto &q : seq) most = std::max(most, q.size());
-    const uint64_t rows = (most + kProbeWavesPerBlock - 1) / kProbeWavesPerBlock;  // slot groups per XCD
-    std::vector<GroupItem> items((size_t)(rows * kProbeWavesPerBlock * kXcds), GroupItem{0, 0, 0});
-    for (size_t i = 0; i < items.size(); ++i) {
-        const size_t x = (i / kProbeWavesPerBlock) % kXcds;
-        const size_t j = (i / (kProbeWavesPerBlock * kXcds)) * kProbeWavesPerBlock + i % kProbeWavesPerBlock;
-        if (j < seq[x].size()) items[i] = seq[x][j];
-    }
+    std::vector<GroupItem> items(most * kXcds, GroupItem{0, 0, 0});
+    for (size_t x = 0; x < kXcds; ++x)
+        for (size_t j = 0; j < seq[x].size(); ++j) items[j * kXcds + x] = seq[x][j];
     return items;
 }
 

@@ -184,7 +184,7 @@ int upload_segments(dyc_group *g, const std::vector<GroupItem> &segs, uint64_t p
 // Cut the batch into items (at most item_keys keys of one table) and upload them.
 int upload_items(dyc_group *g, const uint64_t *offsets, hipStream_t s, uint32_t *n_items)
 {
-    const uint64_t per = g->launch.item_keys ? g->launch.item_keys : kDefaultItemKeys;
+    const uint64_t per = group_item_keys(offsets[g->n], g->launch.item_keys);
     std::vector<GroupItem> segs;
     segs.reserve(g->n);
     for (uint32_t i = 0; i < g->n; ++i) {
@@ -197,11 +197,16 @@ int upload_items(dyc_group *g, const uint64_t *offsets, hipStream_t s, uint32_t 
 
 int upload_items_by_xcd(dyc_group *g, const uint64_t *offsets, hipStream_t s, uint32_t *n_items)
 {
-    const uint64_t per = g->launch.item_keys ? g->launch.item_keys : kDefaultItemKeys;
+    const uint64_t per = group_item_keys(offsets[g->n], g->launch.item_keys);
     for (uint32_t i = 0; i < g->n; ++i)
         if (offsets[i + 1] - offsets[i] > 0xffffffffull)
             return fail(DYC_ERR_INVALID, "table %u's batch is too large for 32-bit lengths", i);
     return upload_item_list(g, items_by_xcd(offsets, g->n, per), s, n_items);
+}
+
+int probe_grid(const dyc_group *g, uint64_t n, uint32_t n_items)
+{
+    return g->launch.find_blocks ? (int)g->launch.find_blocks : group_probe_grid(n, n_items);
 }
 
 int zero_and_run_prologue(dyc_group *g, hipStream_t s)
@@ -609,8 +614,7 @@ int dyc_group_find(dyc_group *g, const uint32_t *keys, const uint64_t *offsets, 
                                           : upload_items(g, offsets, s, &n_items);
     if (rc) return rc;
     Pool sp;
-    HIP_TRY(launch_group_find(g->ddir, g->ditems, n_items, keys, vals, hit,
-                              (int)g->launch.find_blocks, s, g->stash(sp), (int)g->launch.find_waves_per_eu));
+    HIP_TRY(launch_group_find(g->ddir, g->ditems, n_items, keys, vals, hit, probe_grid(g, offsets[g->n], n_items), s, g->stash(sp), (int)g->launch.find_waves_per_eu));
     return DYC_OK;
 }
 
@@ -628,8 +632,7 @@ int dyc_group_erase(dyc_group *g, const uint32_t *keys, const uint64_t *offsets,
     rc = zero_and_run_prologue(g, s);
     if (rc) return rc;
     Pool sp;
-    HIP_TRY(launch_group_erase(g->ddir, g->ditems, n_items, keys, deleted, g->tcounts,
-                               (int)g->launch.find_blocks, s, g->stash(sp), (int)g->launch.find_waves_per_eu));
+    HIP_TRY(launch_group_erase(g->ddir, g->ditems, n_items, keys, deleted, g->tcounts, probe_grid(g, offsets[g->n], n_items), s, g->stash(sp), (int)g->launch.find_waves_per_eu));
     rc = read_back(g, s);
     if (rc) return rc;
     for (uint32_t i = 0; i < g->n; ++i) g->count[i] -= std::min<uint64_t>(g->count[i], g->htcounts[i]);
@@ -780,7 +783,7 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
     rc = reserve_pending(g, std::max<uint64_t>(65536, ins_offsets[g->n] / 16), nullptr);
     if (rc) return rc;
     // the work items of both launches, cut and laid out as the eager calls do, uploaded once
-    const uint64_t per = g->launch.item_keys ? g->launch.item_keys : kDefaultItemKeys;
+    const uint64_t per = group_item_keys(ins_offsets[g->n], g->launch.item_keys);
     std::vector<GroupItem> items;
     for (uint32_t i = 0; i < g->n; ++i)
         for (uint64_t b = ins_offsets[i]; b < ins_offsets[i + 1]; b += per)
@@ -788,7 +791,7 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
     for (uint32_t i = 0; i < g->n; ++i)
         if (find_offsets[i + 1] - find_offsets[i] > 0xffffffffull)
             return fail(DYC_ERR_INVALID, "table %u's batch is too large for 32-bit lengths", i);
-    const std::vector<GroupItem> finds = items_by_xcd(find_offsets, g->n, per);
+    const std::vector<GroupItem> finds = items_by_xcd(find_offsets, g->n, group_item_keys(find_offsets[g->n], g->launch.item_keys));
     items.insert(items.end(), finds.begin(), finds.end());
     if (items.size() > 0xffffffffull) return fail(DYC_ERR_INVALID, "batch too large for 32-bit item indexes");
     dyc_group_plan *p = new dyc_group_plan();
@@ -870,7 +873,8 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
                                     (int)g->launch.insert_waves_per_eu);
         }
         if (k == hipSuccess)
-            k = launch_group_find(g->ddir, p->d_items + p->n_ins, p->n_find, lookups, vals_out, hit, (int)g->launch.find_blocks, cs, &stash,
+            k = launch_group_find(g->ddir, p->d_items + p->n_ins, p->n_find, lookups, vals_out, hit,
+                                  probe_grid(g, find_offsets[g->n], p->n_find), cs, &stash,
                                   (int)g->launch.find_waves_per_eu);
         if (k == hipSuccess)
             k = launch_copy(g->ctr, g->hctr, kCounterWords, g->tcounts, g->htcounts, g->n, cs);

@@ -401,6 +401,32 @@ __device__ inline uint32_t vote_slot(const Desc &D, const uint32_t (&k4)[4], uin
     return slot < (uint32_t)kSlots ? slot : (kicks & 15u);
 }
 
+// At most this many buckets: a wave's lanes meet in one bucket often (64 lanes over 128 buckets: 24
+// of them share one) and the insert ranks them. Above it the ranking costs every step 60
+// instructions for little (64 over 1024: 4 lanes).
+constexpr uint32_t kCrowdedBuckets = 1024;
+
+// A number that tells the buckets of a crowded table apart (12 bits; two buckets of one number only
+// make a lane skip an empty slot).
+__device__ inline uint32_t bucket_id(const Desc &D, uint64_t at, uint32_t t)
+{
+    const uint64_t base = (uint64_t)selt(t, D.sub);
+    return (t << 9) | ((uint32_t)((at - base) / kBucketBytes) & 511u);
+}
+
+// How many lower lanes of `act` hold the same 12-bit number.
+__device__ inline uint32_t rank_among_equals(uint64_t act, uint32_t id)
+{
+    uint64_t same = act;
+#pragma unroll
+    for (int b = 0; b < 12; ++b) {
+        const bool bit = (id >> b) & 1u;
+        const uint64_t m = __ballot(bit);
+        same &= bit ? m : ~m;
+    }
+    return (uint32_t)__popcll(same & lanemask_lt());
+}
+
 // One eviction-chain iteration of every active lane; all 64 lanes call it together.
 __device__ inline void insert_step(const Desc &D, Hand &h, const InsertPolicy &P, Counters *C, const PendSink &sink,
                                    uint32_t tag, InsertTally &tally)
@@ -419,30 +445,26 @@ __device__ inline void insert_step(const Desc &D, Hand &h, const InsertPolicy &P
         if (__builtin_amdgcn_inverse_ballot_w64((low << 4) - low)) e[kk] = load_quad_slots<false>(lo, hi);
         else e[kk].a = e[kk].b = u32x4{0u, 0u, 0u, 0u};
     });
-    // the first empty slot at or past h.from of the quad's four buckets, bucket kk's in lane kk
+    // the empty slots of the quad's four buckets, bucket kk's 16-bit mask in lane kk
     uint32_t c[4];
-    const bool some_from = __ballot(h.active && h.from) != 0;  // wave-uniform, rare
-    each_of_quad([&](auto q) {
-        constexpr int kk = decltype(q)::value;
-        const uint32_t b = s * 4u;
-        if (!some_from) {
-            c[kk] = e[kk].b.w == 0u ? b + 3u : 64u;
-            c[kk] = e[kk].b.y == 0u ? b + 2u : c[kk];
-            c[kk] = e[kk].a.w == 0u ? b + 1u : c[kk];
-            c[kk] = e[kk].a.y == 0u ? b : c[kk];
-        } else {
-            const uint32_t f = quad_bcast<kk>(h.from);
-            c[kk] = e[kk].b.w == 0u && b + 3u >= f ? b + 3u : 64u;
-            c[kk] = e[kk].b.y == 0u && b + 2u >= f ? b + 2u : c[kk];
-            c[kk] = e[kk].a.w == 0u && b + 1u >= f ? b + 1u : c[kk];
-            c[kk] = e[kk].a.y == 0u && b >= f ? b : c[kk];
-        }
-    });
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+        c[kk] = ((e[kk].a.y == 0u ? 1u : 0u) | (e[kk].a.w == 0u ? 2u : 0u) | (e[kk].b.y == 0u ? 4u : 0u) |
+                 (e[kk].b.w == 0u ? 8u : 0u))
+                << (4u * s);
     const bool odd = s & 1u, high = s & 2u;
-    const uint32_t c01 = min(odd ? c[1] : c[0], quad_swap<1>(odd ? c[0] : c[1]));
-    const uint32_t c23 = min(odd ? c[3] : c[2], quad_swap<1>(odd ? c[2] : c[3]));
-    uint32_t slot = min(high ? c23 : c01, quad_swap<2>(high ? c01 : c23));
-    const bool full = slot >= (uint32_t)kSlots;
+    const uint32_t c01 = (odd ? c[1] : c[0]) | quad_swap<1>(odd ? c[0] : c[1]);
+    const uint32_t c23 = (odd ? c[3] : c[2]) | quad_swap<1>(odd ? c[2] : c[3]);
+    const uint32_t open = ((high ? c23 : c01) | quad_swap<2>(high ? c01 : c23)) & (0xffffu << h.from);
+    const bool full = open == 0u;
+    uint32_t slot = (uint32_t)__builtin_ctz(open | 0x10000u);
+    if (D.nb[0] * D.d <= kCrowdedBuckets) {
+        // a table of few buckets: several lanes of the wave want the same bucket's first empty slot,
+        // and all but one would lose it; the r-th of them takes the r-th empty slot
+        const uint32_t r = rank_among_equals(act, bucket_id(D, at, t));
+        const uint32_t left = (uint32_t)__builtin_popcount(open);
+        if (r && left > 1u) slot = nth_set_bit16(open, r < left ? r : r % left);
+    }
     const bool place = h.active && !full;
     const bool swing = h.active && full && h.fresh && P.kick_bound == 0;
     const bool evict = h.active && full && !swing;
@@ -887,25 +909,41 @@ __global__ __launch_bounds__(256) void probe_count_kernel(Desc D, const uint32_t
 // wave-uniform), so the per-tile code is the single-table code with a different Desc.
 __device__ inline uint32_t wave_uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// The kGroupWaves waves of a workgroup share its items: wave w takes the tiles (64 keys) t of the
+// workgroup's r-th item with t % kGroupWaves == (w - r) % kGroupWaves, without waiting for the others;
+// turning by r spreads items of one tile over the waves. The keys that the waves of an XCD work on
+// at a time then span few tables, and its L2 holds their lines: with a whole 4096-key item per
+// wave, 2048 tables of 2^8..2^18 keys (77 M lookups) took 1897 us, 80 % of the lines missing L2;
+// shared by eight waves 1250 us. Small batches gain too: a table of 200 keys is four tiles at
+// once, not in turn.
+constexpr int kGroupWaves = kProbeWavesPerBlock;
+constexpr int kGroupThreads = kGroupWaves * kWave;
+
+// This wave's first tile of its workgroup's r-th item.
+__device__ inline uint32_t group_first_tile(uint32_t r)
+{
+    return (wave_uniform(threadIdx.x / kWave) - r) % (uint32_t)kGroupWaves;
+}
+
 // W: the least waves per SIMD the compiler must leave room for (1: its own choice); the group
 // launches take it as an occupancy knob, chosen by measurement.
 template <bool ERASE, int W>
-__global__ __launch_bounds__(256, W) void group_probe_kernel(const Desc *__restrict__ dir,
+__global__ __launch_bounds__(kGroupThreads, W) void group_probe_kernel(const Desc *__restrict__ dir,
                                                           const GroupItem *__restrict__ items, uint32_t n_items,
                                                           const uint32_t *__restrict__ keys,
                                                           uint32_t *__restrict__ vals, uint8_t *__restrict__ flags,
                                                           unsigned long long *__restrict__ table_counts, Pool pool)
 {
-    const uint32_t waves = gridDim.x * (blockDim.x / kWave);
     const uint64_t np = pool_size(pool);
-    for (uint32_t it = wave_uniform(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave); it < n_items;
-         it += waves) {
+    uint32_t r = 0;
+    for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x, ++r) {
         const GroupItem item = items[it];
-        if (item.len == 0) continue;  // wave-uniform: an empty slot of a layout by XCD
+        const uint32_t first = group_first_tile(r) * kWave;
+        if (first >= item.len) continue;  // wave-uniform: none of its tiles (or an empty slot of a layout by XCD)
         const Desc D = as_global(dir[item.table]);
         const uint64_t end = item.begin + item.len;
         unsigned long long nd = 0;
-        for (uint64_t base = item.begin; base < end; base += kWave) {
+        for (uint64_t base = item.begin + first; base < end; base += kGroupThreads) {
             uint32_t f = probe_tile<ERASE ? 1 : 0>(D, keys, vals, flags, base, end);
             if (np) f |= pool_probe_at<ERASE ? 1 : 0>(pool, np, keys, vals, flags, end, item.table, base, f);
             nd += f;
@@ -917,35 +955,54 @@ __global__ __launch_bounds__(256, W) void group_probe_kernel(const Desc *__restr
     }
 }
 
-// A wave takes an item's entries in chunks and moves on only when all its lanes have placed (or
-// pended) theirs. FROM_ENTRIES: the items index a bulk fill's overflow (packed entries) instead of
-// keys/vals, and there are *n_dev of them if that is less than n_items.
-template <int W, bool FROM_ENTRIES = false>
-__global__ __launch_bounds__(256, W) void group_insert_kernel(const Desc *__restrict__ dir,
+// The waves of a workgroup share its items as in the probe, chunk by chunk. A wave moves on only when
+// all its lanes have placed (or pended) their entries.
+template <int W>
+__global__ __launch_bounds__(kGroupThreads, W) void group_insert_kernel(const Desc *__restrict__ dir,
                                                            const GroupItem *__restrict__ items, uint32_t n_items,
                                                            const uint32_t *__restrict__ keys,
                                                            const uint32_t *__restrict__ vals, InsertPolicy P,
                                                            Counters *__restrict__ C, PendSink sink,
-                                                           unsigned long long *__restrict__ table_counts,
-                                                           const uint64_t *__restrict__ entries,
-                                                           const unsigned long long *__restrict__ n_dev)
+                                                           unsigned long long *__restrict__ table_counts)
+{
+    InsertTally tally;
+    uint32_t r = 0;
+    for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x, ++r) {
+        const GroupItem item = items[it];
+        const uint32_t first = group_first_tile(r);
+        if (first * kWave >= item.len) continue;  // wave-uniform
+        const Desc D = as_global(dir[item.table]);
+        const unsigned long long rej0 = tally.rejected;
+        InsertRange<false> in{keys, vals, nullptr, nullptr, kNoTable};
+        in.run(D, item.begin, item.begin + item.len, first, kGroupWaves, P, C, sink, item.table, tally);
+        const unsigned long long rej = tally.rejected - rej0;
+        if (__lane_id() == 0 && in.taken > rej) atomicAdd(&table_counts[item.table], in.taken - rej);
+    }
+    tally_out(C, tally);
+}
+
+// The overflow of a group's bulk fill: small items, each one wave's; there are *n_dev of them if
+// that is less than n_items.
+__global__ __launch_bounds__(256) void group_overflow_kernel(const Desc *__restrict__ dir,
+                                                             const GroupItem *__restrict__ items, uint32_t n_items,
+                                                             const unsigned long long *__restrict__ n_dev,
+                                                             const uint64_t *__restrict__ ovf, InsertPolicy P,
+                                                             Counters *__restrict__ C, PendSink sink,
+                                                             unsigned long long *__restrict__ table_counts)
 {
     InsertTally tally;
     unsigned long long taken = 0;
-    if constexpr (FROM_ENTRIES) n_items = (uint32_t)min((unsigned long long)n_items, *n_dev);
+    n_items = (uint32_t)min((unsigned long long)n_items, *n_dev);
     const uint32_t waves = gridDim.x * (blockDim.x / kWave);
     for (uint32_t it = wave_slot(); it < n_items; it += waves) {
         const GroupItem item = items[it];
         const Desc D = as_global(dir[item.table]);
-        const unsigned long long rej0 = tally.rejected;
-        InsertRange<FROM_ENTRIES> in{keys, vals, entries, nullptr, FROM_ENTRIES ? kAfterFill : kNoTable};
+        InsertRange<true> in{nullptr, nullptr, ovf, nullptr, kAfterFill};
         in.run(D, item.begin, item.begin + item.len, 0, 1, P, C, sink, item.table, tally);
         taken += in.taken;
-        const unsigned long long rej = tally.rejected - rej0;
-        if (__lane_id() == 0 && item.len > rej) atomicAdd(&table_counts[item.table], item.len - rej);
+        if (__lane_id() == 0) atomicAdd(&table_counts[item.table], (unsigned long long)item.len);
     }
-    if (FROM_ENTRIES && __lane_id() == 0 && taken > tally.direct)
-        tally_add(C, &C->left, taken - tally.direct, wave_slot());
+    if (__lane_id() == 0 && taken > tally.direct) tally_add(C, &C->left, taken - tally.direct, wave_slot());
     tally_out(C, tally);
 }
 
@@ -1531,6 +1588,7 @@ hipError_t launch_downsize(const uint64_t *old, uint32_t new_nb, uint64_t *dst, 
 }
 
 constexpr int kGroupDefaultBlocks = 2048;  // 8192 waves: 256 CUs x 32 resident waves
+constexpr uint32_t kGroupInsertBlocks = 1024;  // as many waves, eight to a workgroup
 
 template <bool ERASE>
 static void group_probe_w(int wpe, int grid, hipStream_t st, const Desc *dir, const GroupItem *items, uint32_t n_items,
@@ -1539,13 +1597,16 @@ static void group_probe_w(int wpe, int grid, hipStream_t st, const Desc *dir, co
 {
     switch (wpe) {
     case 6:
-        group_probe_kernel<ERASE, 6><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, flags, table_counts, p);
+        group_probe_kernel<ERASE, 6>
+            <<<grid, kGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, flags, table_counts, p);
         break;
     case 8:
-        group_probe_kernel<ERASE, 8><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, flags, table_counts, p);
+        group_probe_kernel<ERASE, 8>
+            <<<grid, kGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, flags, table_counts, p);
         break;
     default:
-        group_probe_kernel<ERASE, 1><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, flags, table_counts, p);
+        group_probe_kernel<ERASE, 1>
+            <<<grid, kGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, flags, table_counts, p);
         break;
     }
 }
@@ -1556,7 +1617,7 @@ hipError_t launch_group_find(const Desc *dir, const GroupItem *items, uint32_t n
 {
     const Pool p = pool ? *pool : Pool{};
     if (n_items == 0) return hipSuccess;
-    const int grid = blocks > 0 ? blocks : std::min<int>(kGroupDefaultBlocks, (int)((n_items + 3) / 4));
+    const int grid = blocks > 0 ? blocks : group_probe_grid(0, n_items);
     group_probe_w<false>(waves_per_eu, grid, st, dir, items, n_items, keys, vals, hit, nullptr, p);
     return hipGetLastError();
 }
@@ -1567,7 +1628,7 @@ hipError_t launch_group_erase(const Desc *dir, const GroupItem *items, uint32_t 
 {
     const Pool p = pool ? *pool : Pool{};
     if (n_items == 0) return hipSuccess;
-    const int grid = blocks > 0 ? blocks : std::min<int>(kGroupDefaultBlocks, (int)((n_items + 3) / 4));
+    const int grid = blocks > 0 ? blocks : group_probe_grid(0, n_items);
     group_probe_w<true>(waves_per_eu, grid, st, dir, items, n_items, keys, nullptr, deleted, table_counts, p);
     return hipGetLastError();
 }
@@ -1577,19 +1638,19 @@ hipError_t launch_group_insert(const Desc *dir, const GroupItem *items, uint32_t
                                unsigned long long *table_counts, hipStream_t st, int waves_per_eu)
 {
     if (n_items == 0) return hipSuccess;
-    const int grid = blocks > 0 ? blocks : std::min<int>(kGroupDefaultBlocks, (int)((n_items + 3) / 4));
+    const int grid = blocks > 0 ? blocks : (int)std::min<uint32_t>(kGroupInsertBlocks, n_items);
     switch (waves_per_eu) {
     case 6:
-        group_insert_kernel<6><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts,
-                                                       nullptr, nullptr);
+        group_insert_kernel<6>
+            <<<grid, kGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts);
         break;
     case 8:
-        group_insert_kernel<8><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts,
-                                                       nullptr, nullptr);
+        group_insert_kernel<8>
+            <<<grid, kGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts);
         break;
     default:
-        group_insert_kernel<1><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts,
-                                                       nullptr, nullptr);
+        group_insert_kernel<1>
+            <<<grid, kGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts);
         break;
     }
     return hipGetLastError();
@@ -1602,8 +1663,8 @@ hipError_t launch_group_insert_overflow(const Desc *dir, const GroupItem *items,
     if (max_items == 0) return hipSuccess;
     if (max_items > 0xffffffffull) return hipErrorInvalidValue;
     const int grid = blocks > 0 ? blocks : (int)std::min<uint64_t>(kGroupDefaultBlocks, (max_items + 3) / 4);
-    group_insert_kernel<1, true><<<grid, 256, 0, st>>>(dir, items, (uint32_t)max_items, nullptr, nullptr, pol, C, sink,
-                                                       table_counts, ovf, n_items);
+    group_overflow_kernel<<<grid, 256, 0, st>>>(dir, items, (uint32_t)max_items, n_items, ovf, pol, C, sink,
+                                                table_counts);
     return hipGetLastError();
 }
 

@@ -172,10 +172,31 @@ struct GroupItem {
     uint32_t table;
 };
 
-// Persistent launches over a directory of table descriptors: each wave takes items w, w + W, ...
+// Persistent launches over a directory of table descriptors: workgroup b takes items b, b + B, ...,
+// each shared by its kProbeWavesPerBlock waves.
+constexpr uint32_t kProbeWavesPerBlock = 8;
+// Default workgroups of a group probe over n keys in n_items items. From 2^24 keys two per CU: few
+// enough that the tables in flight on an XCD stay in its L2 (77 M lookups of 2048 tables: 512
+// workgroups 1250 us, 1024 1437, 2048 1390; 100 M of 400 tables of 2^14..2^20 keys 2081, 2304,
+// 2308); below it as many as the device holds (5.7 M lookups of 4096 tables 77, 71, 65 us).
+inline int group_probe_grid(uint64_t n, uint32_t n_items)
+{
+    const uint32_t most = n >= (1ull << 24) ? 512u : 2048u;
+    return (int)(n_items < most ? n_items : most);
+}
+// Keys per item of a group call of n keys whose launch shape allows at most `most` (0: 4096): enough
+// items for the device's CUs, none smaller than one tile per wave (64 tables of 2^6..2^14 keys,
+// 0.2 M lookups: 18 us with 4096 keys per item, 6.8 with 1024).
+inline uint64_t group_item_keys(uint64_t n, uint32_t most)
+{
+    const uint64_t cap = most ? most : 4096u, tile = 64ull * kProbeWavesPerBlock;
+    const uint64_t per = (n / 1024 + tile - 1) / tile * tile;
+    return per < tile ? (tile < cap ? tile : cap) : (per < cap ? per : cap);
+}
 // find: vals/hit may be null. erase: per-table deleted counts are added to table_counts.
 // pool (optional): misses of an item of table i also look in the pool's entries tagged i.
-// waves_per_eu: 6 or 8 builds the kernel for at least that many waves per SIMD (fewer
+// blocks: the grid (group_probe_grid's by default for probes; 0 for an insert: as many as fill the
+// device). waves_per_eu: 6 or 8 builds the kernel for at least that many waves per SIMD (fewer
 // registers); anything else leaves the register budget to the compiler.
 hipError_t launch_group_find(const Desc *dir, const GroupItem *items, uint32_t n_items, const uint32_t *keys,
                              uint32_t *vals, uint8_t *hit, int blocks, hipStream_t st,

@@ -413,8 +413,15 @@ __global__ __launch_bounds__(256) void wide_insert_kernel(WideDesc W, const uint
 // The group forms: one persistent launch over work items of one table each (GroupItem), the
 // table's descriptor read from a directory, the per-tile and per-chain code above unchanged.
 // Pending entries carry their table in sink.tags / stash.tags.
+// The waves of a probe's workgroup share its items tile by tile, as the 32-bit group's do.
+constexpr int kWideGroupThreads = kProbeWavesPerBlock * kWave;
+__device__ inline uint32_t wide_first_tile(uint32_t r)
+{
+    return (__builtin_amdgcn_readfirstlane(threadIdx.x / kWave) - r) % kProbeWavesPerBlock;
+}
+
 template <int MODE>
-__global__ __launch_bounds__(256) void wide_group_probe_kernel(const WideDesc *__restrict__ dir,
+__global__ __launch_bounds__(kWideGroupThreads) void wide_group_probe_kernel(const WideDesc *__restrict__ dir,
                                                                const GroupItem *__restrict__ items, uint32_t n_items,
                                                                const uint64_t *__restrict__ keys,
                                                                uint64_t *__restrict__ vals,
@@ -422,17 +429,17 @@ __global__ __launch_bounds__(256) void wide_group_probe_kernel(const WideDesc *_
                                                                unsigned long long *__restrict__ table_counts,
                                                                WideStash stash)
 {
-    const uint32_t waves = gridDim.x * (blockDim.x / kWave);
-    for (uint32_t it = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave);
-         it < n_items; it += waves) {
+    uint32_t r = 0;
+    for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x, ++r) {
         const GroupItem item = items[it];
-        if (item.len == 0) continue;  // wave-uniform: an empty slot of a layout by XCD
+        const uint32_t first = wide_first_tile(r) * kWave;
+        if (first >= item.len) continue;  // wave-uniform: none of its tiles (or an empty slot of a layout by XCD)
         const WideDesc W = as_global(dir[item.table]);
         WideStash st = stash;
         st.table = item.table;
         const uint64_t end = item.begin + item.len;
         unsigned long long nd = 0;
-        for (uint64_t base = item.begin; base < end; base += kWave)
+        for (uint64_t base = item.begin + first; base < end; base += kWideGroupThreads)
             nd += wide_probe_tile<MODE>(W, keys, vals, flags, base, end, st);
         if constexpr (MODE == 1) {
             nd = wave_sum(nd);
@@ -1004,11 +1011,13 @@ hipError_t launch_wide_group_probe(const WideDesc *dir, const GroupItem *items, 
                                    int blocks, const WideStash &stash, hipStream_t st)
 {
     if (n_items == 0) return hipSuccess;
-    const int grid = blocks > 0 ? blocks : std::min<int>(kWideGroupBlocks, (int)((n_items + 3) / 4));
+    const int grid = blocks;
     if (erase)
-        wide_group_probe_kernel<1><<<grid, 256, 0, st>>>(dir, items, n_items, keys, nullptr, flags, table_counts, stash);
+        wide_group_probe_kernel<1>
+            <<<grid, kWideGroupThreads, 0, st>>>(dir, items, n_items, keys, nullptr, flags, table_counts, stash);
     else
-        wide_group_probe_kernel<0><<<grid, 256, 0, st>>>(dir, items, n_items, keys, vals, flags, nullptr, stash);
+        wide_group_probe_kernel<0>
+            <<<grid, kWideGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, flags, nullptr, stash);
     return hipGetLastError();
 }
 
@@ -1944,7 +1953,7 @@ int wg_check_offsets(const dyc_wide_group *g, const uint64_t *offsets)
 // between), else the items in table order.
 int wg_upload_items(dyc_wide_group *g, const uint64_t *offsets, hipStream_t s, uint32_t *n_items, bool by_xcd = false)
 {
-    const uint64_t per = kWideGroupItemKeys;
+    const uint64_t per = group_item_keys(offsets[g->n], kWideGroupItemKeys);
     std::vector<GroupItem> laid;
     if (by_xcd) laid = dyc::host::items_by_xcd(offsets, g->n, per);
     uint64_t need = laid.size();
@@ -2010,6 +2019,11 @@ int wg_reserve_pending(dyc_wide_group *g, uint64_t extra, hipStream_t s)
     g->ptag = nt;
     g->pend_cap = cap;
     return DYC_OK;
+}
+
+int wg_probe_grid(const dyc_wide_group *g, uint64_t n, uint32_t n_items)
+{
+    return g->cfg.max_blocks ? (int)g->cfg.max_blocks : group_probe_grid(n, n_items);
 }
 
 int wg_prologue(dyc_wide_group *g, hipStream_t s)
@@ -2364,7 +2378,8 @@ int dyc_wide_group_find(dyc_wide_group *g, const uint64_t *keys, const uint64_t 
     uint32_t n_items = 0;
     rc = wg_upload_items(g, offsets, s, &n_items, offsets[g->n] >= dyc::host::kXcdLayoutKeys);
     if (rc) return rc;
-    HIP_TRY(launch_wide_group_probe(g->ddir, g->ditems, n_items, keys, vals, hit, false, nullptr, (int)g->cfg.max_blocks,
+    HIP_TRY(launch_wide_group_probe(g->ddir, g->ditems, n_items, keys, vals, hit, false, nullptr,
+                                    wg_probe_grid(g, offsets[g->n], n_items),
                                     g->stash(), s));
     return DYC_OK;
 }
@@ -2384,7 +2399,7 @@ int dyc_wide_group_erase(dyc_wide_group *g, const uint64_t *keys, const uint64_t
     rc = wg_prologue(g, s);
     if (rc) return rc;
     HIP_TRY(launch_wide_group_probe(g->ddir, g->ditems, n_items, keys, nullptr, deleted, true, g->tcounts,
-                                    (int)g->cfg.max_blocks, g->stash(), s));
+                                    wg_probe_grid(g, offsets[g->n], n_items), g->stash(), s));
     rc = wg_read_back(g, s);
     if (rc) return rc;
     for (uint32_t i = 0; i < g->n; ++i) g->count[i] -= std::min<uint64_t>(g->count[i], g->htcounts[i]);
