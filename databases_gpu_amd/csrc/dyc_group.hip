@@ -44,6 +44,7 @@ struct dyc_group {
     dyc_stats st{};
     // every slot of every table is zero: set at create and clear, dropped by every insert
     bool zeroed = false;
+    dyc::host::FirstBucketRules rules;  // of all tables together
     // bulk fill (cfg.insert_order 3), grown on demand and kept by the group. Shared by the eager
     // calls and the plans (a plan refuses to run once one of these moved): partitioned entries and
     // the overflow (8 B per key each), local chunk ids (1 B per key), per-block chunk counts, chunk
@@ -208,6 +209,12 @@ int probe_grid(const dyc_group *g, uint64_t n, uint32_t n_items)
 {
     return g->launch.find_blocks ? (int)g->launch.find_blocks : group_probe_grid(n, n_items);
 }
+
+// A find that relies on the first-bucket rule reads fewer buckets and takes a quarter more
+// instructions. It pays where lookups wait for lines from memory, so for tables of 1 MiB and more
+// on average (mean 1.4 MiB, 199 M lookups: 4697 -> 4083 us; 2.6 MiB, 101 M: 2159 -> 1938); an XCD's
+// L2 holds smaller ones (0.35 MiB, 75 M lookups: 1338 -> 1395).
+bool first_bucket_pays(const dyc_group *g) { return g->arena_bytes >= (uint64_t)g->n << 20; }
 
 int zero_and_run_prologue(dyc_group *g, hipStream_t s)
 {
@@ -417,6 +424,7 @@ int group_bulk_insert(dyc_group *g, const uint32_t *keys, const uint32_t *vals, 
     HIP_TRY(hipMemcpyAsync(g->bk_tabs, g->bk_htabs, J * sizeof(BulkTable), hipMemcpyHostToDevice, s));
     int rc = zero_and_run_prologue(g, s);
     if (rc) return rc;
+    g->rules.filled(FirstBucket::kFill);
     const BulkArrays A{g->bk_blk, g->bk_tabs, NB, J, L.chunks};
     HIP_TRY(enqueue_group_bulk(g, A, keys, vals, L.total, zeroed,
                                PendSink{g->pend + g->pend_n, g->pend_tag + g->pend_n, room, 0, 0, nullptr}, s));
@@ -511,6 +519,7 @@ int dyc_group_create(const dyc_config *cfg_in, uint32_t n_tables, const uint64_t
     rc = reserve_pending(g, 65536, nullptr);
     if (rc) return cleanup(rc);
     g->zeroed = true;
+    g->rules.emptied();
     *out = g;
     return DYC_OK;
 }
@@ -589,6 +598,7 @@ int dyc_group_insert(dyc_group *g, const uint32_t *keys, const uint32_t *vals, c
     if (rc) return rc;
     rc = zero_and_run_prologue(g, s);
     if (rc) return rc;
+    g->rules.filled(FirstBucket::kStart);
     HIP_TRY(launch_group_insert(g->ddir, g->ditems, n_items, keys, vals, g->policy(),
                                 (int)g->launch.insert_blocks, g->ctr,
                                 PendSink{g->pend + g->pend_n, g->pend_tag + g->pend_n, room, 0, 0, nullptr}, g->tcounts,
@@ -614,7 +624,10 @@ int dyc_group_find(dyc_group *g, const uint32_t *keys, const uint64_t *offsets, 
                                           : upload_items(g, offsets, s, &n_items);
     if (rc) return rc;
     Pool sp;
-    HIP_TRY(launch_group_find(g->ddir, g->ditems, n_items, keys, vals, hit, probe_grid(g, offsets[g->n], n_items), s, g->stash(sp), (int)g->launch.find_waves_per_eu));
+    HIP_TRY(g->rules.find(first_bucket_pays(g) ? offsets[g->n] : 0, s, [&](FirstBucket rule) {
+        return launch_group_find(g->ddir, g->ditems, n_items, keys, vals, hit, probe_grid(g, offsets[g->n], n_items), s,
+                                 g->stash(sp), (int)g->launch.find_waves_per_eu, rule);
+    }));
     return DYC_OK;
 }
 
@@ -629,6 +642,7 @@ int dyc_group_erase(dyc_group *g, const uint32_t *keys, const uint64_t *offsets,
     uint32_t n_items = 0;
     rc = upload_items(g, offsets, s, &n_items);
     if (rc) return rc;
+    HIP_TRY(g->rules.freeing(s));
     rc = zero_and_run_prologue(g, s);
     if (rc) return rc;
     Pool sp;
@@ -654,6 +668,7 @@ int dyc_group_insert_per_table(dyc_group *g, const uint32_t *keys, const uint32_
     if (rc) return rc;
     rc = zero_and_run_prologue(g, s);
     if (rc) return rc;
+    g->rules.filled(FirstBucket::kStart);
     const uint64_t room = g->pend_cap - g->pend_n;
     const LaunchShape sh{256, (int)g->launch.insert_blocks};
     // one launch per table; all share the counters, so pended entries append one after another
@@ -875,7 +890,10 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
         if (k == hipSuccess)
             k = launch_group_find(g->ddir, p->d_items + p->n_ins, p->n_find, lookups, vals_out, hit,
                                   probe_grid(g, find_offsets[g->n], p->n_find), cs, &stash,
-                                  (int)g->launch.find_waves_per_eu);
+                                  (int)g->launch.find_waves_per_eu,
+                                  !first_bucket_pays(g) ? FirstBucket::kNone
+                                  : p->bulk            ? FirstBucket::kFill
+                                                       : FirstBucket::kStart);
         if (k == hipSuccess)
             k = launch_copy(g->ctr, g->hctr, kCounterWords, g->tcounts, g->htcounts, g->n, cs);
         e = hipStreamEndCapture(cs, &p->graph);
@@ -905,6 +923,8 @@ int dyc_group_plan_run(dyc_group_plan *p, dyc_stream stream)
     hipStream_t s = (hipStream_t)stream;
     g->zeroed = false;
     g->st.last_filled = 0;
+    // the graph clears every table and fills it under one rule, which its own find relies on
+    g->rules.emptied_then(p->bulk ? FirstBucket::kFill : FirstBucket::kStart);
     HIP_TRY(hipGraphLaunch(p->exec, s));
     HIP_TRY(hipStreamSynchronize(s));
     fold_tallies(g->hctr);
@@ -923,6 +943,7 @@ int dyc_group_clear(dyc_group *g, dyc_stream stream)
     std::fill(g->count.begin(), g->count.end(), 0);
     g->pend_n = 0;
     g->st.pending = 0;
+    g->rules.emptied();
     g->zeroed = true;
     return DYC_OK;
 }

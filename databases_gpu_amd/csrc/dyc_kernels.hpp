@@ -80,9 +80,17 @@ struct InsertPolicy {
 };
 
 struct Pool;
+// The bucket of its pair that every stored key was first put to, where a table still keeps the rule:
+// a key is elsewhere only if that bucket had no free slot then, and none has become free since (no
+// erase, resize or load). kStart: the start rule of the eviction insert (odd keys pos2), kFill: the
+// bulk fill's fill_target.
+enum class FirstBucket : uint32_t { kNone = 0, kStart = 1, kFill = 2 };
+
 // find: vals/hit may be null. pool (optional): misses also look in the pool's entries of `table`.
+// rule: what the table keeps (kNone reads in the reference order).
 hipError_t launch_find(const Desc &D, const uint32_t *keys, uint32_t *vals, uint8_t *hit, uint64_t n, LaunchShape sh,
-                       hipStream_t st, const Pool *pool = nullptr, uint32_t table = 0);
+                       hipStream_t st, const Pool *pool = nullptr, uint32_t table = 0,
+                       FirstBucket rule = FirstBucket::kNone);
 // erase: deleted may be null; counts into C->deleted.
 hipError_t launch_erase(const Desc &D, const uint32_t *keys, uint8_t *deleted, uint64_t n, LaunchShape sh,
                         Counters *C, hipStream_t st, const Pool *pool = nullptr, uint32_t table = 0);
@@ -200,7 +208,8 @@ inline uint64_t group_item_keys(uint64_t n, uint32_t most)
 // registers); anything else leaves the register budget to the compiler.
 hipError_t launch_group_find(const Desc *dir, const GroupItem *items, uint32_t n_items, const uint32_t *keys,
                              uint32_t *vals, uint8_t *hit, int blocks, hipStream_t st,
-                             const Pool *pool = nullptr, int waves_per_eu = 0);
+                             const Pool *pool = nullptr, int waves_per_eu = 0,
+                             FirstBucket rule = FirstBucket::kNone);
 hipError_t launch_group_erase(const Desc *dir, const GroupItem *items, uint32_t n_items, const uint32_t *keys,
                               uint8_t *deleted, unsigned long long *table_counts, int blocks,
                               hipStream_t st, const Pool *pool = nullptr, int waves_per_eu = 0);

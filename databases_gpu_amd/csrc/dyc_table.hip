@@ -103,6 +103,7 @@ struct dyc_table {
     // every slot is zero: set when the table is created or cleared, dropped by every call that
     // may store an entry (a bulk fill into such a table need not read it)
     bool zeroed = false;
+    dyc::host::FirstBucketRules rules;  // see there
     uint64_t *part = nullptr;   // insert batch ordered by bucket region
     uint64_t part_cap = 0;
     unsigned long long *part_counts = nullptr;   // kMaxRegions counts, then kMaxRegions cursors
@@ -282,6 +283,7 @@ int alloc_slab(uint32_t d, const uint32_t *nb, uint8_t **base, uint64_t **sub)
 int install_slab(dyc_table *t, uint8_t *base, uint64_t *const *sub, const uint32_t *nb)
 {
     t->zeroed = false;  // new memory: only the caller knows what it holds
+    t->rules.lost();
     for (uint32_t i = 0; i < t->D.d; ++i) {
         const int rc = release_sub(t, i);
         if (rc) return rc;
@@ -332,6 +334,7 @@ int absorb_insert_counters(dyc_table *t, uint64_t room)
 int do_resize_up(dyc_table *t, hipStream_t s)
 {
     t->zeroed = false;
+    t->rules.lost();
     const uint32_t sub = choose_up(t->D.nb, t->D.d);
     const uint32_t old_nb = t->D.nb[sub];
     if ((uint64_t)old_nb * 2 >= kMaxBuckets) return fail(DYC_ERR_INVALID, "subtable %u cannot grow past 2^29 buckets", sub);
@@ -398,6 +401,7 @@ int place_pending(dyc_table *t, hipStream_t s, uint64_t before)
 int do_resize_down(dyc_table *t, hipStream_t s)
 {
     t->zeroed = false;
+    t->rules.lost();
     const uint64_t pend_before = t->pend_n;
     const uint32_t sub = choose_down(t->D.nb, t->D.d);
     const uint32_t old_nb = t->D.nb[sub];
@@ -995,6 +999,7 @@ int dyc_create(const dyc_config *cfg_in, uint64_t capacity_hint, dyc_table **out
     if (rc == DYC_OK) rc = reserve_pending(t, DYC_NOALLOC_MAX_KEYS, nullptr);
     if (rc == DYC_OK && hipStreamSynchronize(nullptr) != hipSuccess) rc = fail(DYC_ERR_HIP, "create sync failed");
     t->zeroed = rc == DYC_OK;
+    if (t->zeroed) t->rules.emptied();
     if (rc != DYC_OK) {
         char keep[sizeof g_err];
         memcpy(keep, g_err, sizeof keep);
@@ -1077,6 +1082,7 @@ int dyc_insert_counted(dyc_table *t, const uint32_t *keys, const uint32_t *vals,
             return rc;
         }
     }
+    t->rules.filled(bulk ? FirstBucket::kFill : FirstBucket::kStart);
     if (bulk) {
         rc = bulk_insert(t, keys, vals, n, zeroed, s);
         if (rc) return rc;
@@ -1119,6 +1125,7 @@ int dyc_insert_async(dyc_table *t, const uint32_t *keys, const uint32_t *vals, u
     t->zeroed = false;
     hipStream_t s = (hipStream_t)stream;
     if (n == 0) return DYC_OK;
+    t->rules.filled(FirstBucket::kStart);
     int rc;
     if (t->cfg.auto_resize &&
         (double)(t->count + t->async_keys + n) > t->cfg.upper_bound * (double)t->capacity()) {
@@ -1185,6 +1192,7 @@ int dyc_insert_noalloc(dyc_table *t, const uint32_t *keys, const uint32_t *vals,
     t->st.last_kicks = t->st.last_max_chain = 0;
     t->st.last_filled = 0;
     if (n == 0) return DYC_OK;
+    t->rules.filled(FirstBucket::kStart);
     Counters *C = nullptr;
     int rc = noalloc_counters(t->device, &C);
     if (rc) return rc;
@@ -1218,6 +1226,7 @@ int dyc_upsert(dyc_table *t, const uint32_t *keys, const uint32_t *vals, uint64_
     t->st.last_kicks = t->st.last_max_chain = 0;
     t->st.last_filled = 0;
     if (n == 0) return DYC_OK;
+    t->rules.filled(FirstBucket::kStart);
     int rc;
     if (t->cfg.auto_resize) {  // sized as if every key were new (api.cpp:360-369)
         while ((double)(t->count + n) > t->cfg.upper_bound * (double)t->capacity()) {
@@ -1268,8 +1277,10 @@ int dyc_find(dyc_table *t, const uint32_t *keys, uint32_t *vals, uint8_t *hit, u
     DeviceGuard dg(t->device);
     SETTLE(t);
     Pool sp;
-    HIP_TRY(launch_find(t->D, keys, vals, hit, n, t->shape(), (hipStream_t)stream,
-                        stash_of(t, sp)));
+    hipStream_t s = (hipStream_t)stream;
+    HIP_TRY(t->rules.find(n, s, [&](FirstBucket rule) {
+        return launch_find(t->D, keys, vals, hit, n, t->shape(), s, stash_of(t, sp), 0, rule);
+    }));
     return DYC_OK;
 }
 
@@ -1281,6 +1292,7 @@ int dyc_erase(dyc_table *t, const uint32_t *keys, uint8_t *deleted, uint64_t n, 
     SETTLE(t);
     hipStream_t s = (hipStream_t)stream;
     if (n == 0) return DYC_OK;
+    HIP_TRY(t->rules.freeing(s));
     int rc = zero_counters(t, s);
     if (rc) return rc;
     Pool sp;
@@ -1372,6 +1384,7 @@ int dyc_clear(dyc_table *t, dyc_stream stream)
     t->count = 0;
     t->pend_n = 0;
     t->st.pending = 0;
+    t->rules.emptied();
     t->zeroed = true;
     return DYC_OK;
 }
@@ -1472,6 +1485,7 @@ int dyc_insert_host(dyc_table *t, const uint32_t *keys, const uint32_t *vals, ui
     t->st.last_kicks = t->st.last_max_chain = 0;
     t->st.last_filled = 0;
     if (n == 0) return DYC_OK;
+    t->rules.filled(FirstBucket::kStart);
     int rc;
     if (t->cfg.auto_resize) {
         while ((double)(t->count + n) > t->cfg.upper_bound * (double)t->capacity()) {
@@ -1587,6 +1601,7 @@ int dyc_erase_host(dyc_table *t, const uint32_t *keys, uint8_t *deleted, uint64_
     DeviceGuard dg(t->device);
     SETTLE(t);
     hipStream_t s = (hipStream_t)stream;
+    HIP_TRY(t->rules.freeing(s));
     int rc = zero_counters(t, s);
     if (rc) return rc;
     rc = probe_host(t, keys, nullptr, deleted, n, s, true);
