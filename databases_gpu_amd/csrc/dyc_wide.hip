@@ -88,94 +88,170 @@ __device__ inline void store2(uint64_t *p, uint64_t a, uint64_t b)
 }
 
 // --------------------------------------------------------------------- find / erase / update
-// A wave owns 64 consecutive keys; groups of 8 lanes probe 8 keys each, lane s reading keys
-// 2s, 2s+1 of a bucket (one 128-byte line per group). The first bucket (pos1, then pos2) that
-// holds a key answers: find (MODE 0) takes the first matching slot's value (read by the key's
-// own lane from the value line), erase (MODE 1) CASes every matching key of that bucket to 0,
+// The narrow table's probe tile over key lines: a wave owns 64 consecutive keys, a quad reads the key
+// lines of its four keys, 32 bytes (four keys) a lane, and hands addresses and keys round by quad
+// permutes (eight lanes a line and LDS permutes took 1249 vector instructions a tile, this 470).
+// With the first-bucket rule 2^26 lookups at 50 % hits take 2.64 ms, in the reference order 2.92: 47 G
+// lines and value words a second, the device's rate of random accesses.
+struct WideKeys {
+    u32x4 a, b;
+};
+__device__ inline WideKeys load_wide_keys(uint32_t lo, uint32_t hi)
+{
+    const DYC_GLOBAL u32x4 *p = (const DYC_GLOBAL u32x4 *)((uint64_t)hi << 32 | lo);
+    return WideKeys{p[0], p[1]};
+}
+__device__ inline uint64_t wide_key(const WideKeys &e, int j)
+{
+    const uint32_t lo = j == 0 ? e.a.x : (j == 1 ? e.a.z : (j == 2 ? e.b.x : e.b.z));
+    const uint32_t hi = j == 0 ? e.a.y : (j == 1 ? e.a.w : (j == 2 ? e.b.y : e.b.w));
+    return (uint64_t)hi << 32 | lo;
+}
+__device__ inline bool keys_hold(const WideKeys &e, uint64_t k)
+{
+    return (wide_key(e, 0) == k) | (wide_key(e, 1) == k) | (wide_key(e, 2) == k) | (wide_key(e, 3) == k);
+}
+__device__ inline bool keys_hold_two(const WideKeys &e, uint64_t k)
+{
+    const bool a = wide_key(e, 0) == k, b = wide_key(e, 1) == k, c = wide_key(e, 2) == k, d = wide_key(e, 3) == k;
+    return (a & b) | (c & d) | ((a | b) & (c | d));
+}
+// 1 + the first of the lane's slots that holds k (slot numbers of the bucket; s: the lane's place in
+// its quad), or 0.
+__device__ inline uint32_t keys_slot(const WideKeys &e, uint64_t k, uint32_t s)
+{
+    uint32_t c = wide_key(e, 3) == k ? 4u * s + 4u : 0u;
+    c = wide_key(e, 2) == k ? 4u * s + 3u : c;
+    c = wide_key(e, 1) == k ? 4u * s + 2u : c;
+    return wide_key(e, 0) == k ? 4u * s + 1u : c;
+}
+
+// One wave probes keys [base, base + 64) clipped to n; returns this lane's flag (found, deleted
+// or updated), also written to flags. All 64 lanes call it together. The first bucket (pos1, then
+// pos2) that holds a key answers: find (MODE 0) takes the first matching slot's value (read by the
+// key's own lane from the value line), erase (MODE 1) CASes every matching key of that bucket to 0,
 // update (MODE 2) writes vals[i] to the value of every matching slot of that bucket. Keys
 // neither bucket holds are then looked up in the stash (erase and update act on every copy
 // there). Update: keys of one launch are distinct, so no two lanes write one value; the key word
-// is untouched, and the value is an agent-scope atomic store.
-// One wave probes keys [base, base + 64) clipped to n; returns this lane's flag (found, deleted
-// or updated), also written to flags. All 64 lanes call it together.
-template <int MODE>
+// is untouched, and the value is an agent-scope atomic store. rule (find): the first-bucket rule the
+// table keeps, which the find may rely on as the narrow table's does (find_tile_first).
+template <int MODE, bool FIRST = false>
 __device__ inline uint32_t wide_probe_tile(const WideDesc &W, const uint64_t *__restrict__ keys,
                                            uint64_t *__restrict__ vals, uint8_t *__restrict__ flags, uint64_t base,
-                                           uint64_t n, const WideStash &stash)
+                                           uint64_t n, const WideStash &stash, FirstBucket rule = FirstBucket::kNone)
 {
     constexpr bool ERASE = MODE == 1;
     constexpr bool UPDATE = MODE == 2;
-    constexpr int G = 8;
-    const int lane = __lane_id();
-    const int g = lane / G, s = lane % G;
+    const uint32_t lane = __lane_id(), s = lane & 3u;
     const uint64_t i = base + lane;
     const bool inb = i < n;
     const uint64_t k = inb ? keys[i] : 0ull;
     const uint64_t nv = (UPDATE && inb) ? vals[i] : 0ull;  // update: the new value
     const uint32_t f = fold64(k);
-    const uint32_t p = pair_of(W.D, f);
-    const uint32_t t1 = pos1(W.D, p), t2 = pos2(W.D, p);
-    const uint32_t loc1 = wide_loc(t1, bucket_of(W.D, f, t1));
-    const uint32_t loc2 = wide_loc(t2, bucket_of(W.D, f, t2));
-
-    uint64_t e[G][2];
-    uint64_t kk_key[G];
-    uint64_t kk_new[UPDATE ? G : 1];
-    bool kk_valid[G];
-    uint32_t kk_l[G];
-    uint32_t my_flag = 0, my_loc = 0, my_slot = 0, done = 0;
+    const uint32_t p = pair_of(W.D, f), ta = pos1(W.D, p), tb = pos2(W.D, p);
+    const bool from2 = FIRST && (rule == FirstBucket::kFill ? fill_target(W.D, (uint32_t)k, p) == tb : (k & 1u) != 0);
+    const uint32_t t1 = from2 ? tb : ta, t2 = from2 ? ta : tb;
+    const uint32_t loc1 = wide_loc(t1, bucket_of(W.D, f, t1)), loc2 = wide_loc(t2, bucket_of(W.D, f, t2));
+    const uint64_t a1 = (uint64_t)wide_keys_at(W, loc1), a2 = (uint64_t)wide_keys_at(W, loc2);
+    const uint64_t valid = __ballot(inb && !wide_reserved(k));
+    const uint64_t second = __ballot(from2);
+    const uint32_t off = s * 32u;
+    uint64_t key[4];
+    WideKeys e[4];
+    each_of_quad([&](auto q) {
+        constexpr int kk = decltype(q)::value;
+        key[kk] = (uint64_t)quad_bcast<kk>((uint32_t)(k >> 32)) << 32 | quad_bcast<kk>((uint32_t)k);
+        e[kk] = load_wide_keys(quad_bcast<kk>((uint32_t)a1) | off, quad_bcast<kk>((uint32_t)(a1 >> 32)));
+    });
+    uint64_t any[4], more[4];
+    uint32_t c[4];  // 1 + matching slot (find)
 #pragma unroll
-    for (int phase = 0; phase < 2; ++phase) {
-        const uint32_t lp = phase == 0 ? loc1 : loc2;
-#pragma unroll
-        for (int kk = 0; kk < G; ++kk) {
-            const int src = g * G + kk;
-            if (phase == 0) {
-                kk_key[kk] = shfl64(k, src);
-                kk_valid[kk] = !wide_reserved(kk_key[kk]);
-                if constexpr (UPDATE) kk_new[kk] = shfl64(nv, src);
-            }
-            kk_l[kk] = __shfl(lp, src);
-            e[kk][0] = e[kk][1] = 0;
-            if (kk_valid[kk] && !(done & (1u << kk))) load2(wide_keys_at(W, kk_l[kk]) + s * 2, e[kk]);
-        }
-#pragma unroll
-        for (int kk = 0; kk < G; ++kk) {
-            if (done & (1u << kk)) continue;  // group-uniform
-            const int first = e[kk][0] == kk_key[kk] ? 0 : (e[kk][1] == kk_key[kk] ? 1 : -1);
-            const uint32_t gm = (uint32_t)((__ballot(first >= 0 && kk_valid[kk]) >> (g * G)) & 0xffu);
-            if (!gm) continue;
-            done |= 1u << kk;
-            if constexpr (ERASE) {
-                int ok = 0;
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    if (kk_valid[kk] && e[kk][j] == kk_key[kk]) {
-                        uint64_t exp = e[kk][j];
-                        ok |= cas_slot(wide_keys_at(W, kk_l[kk]) + s * 2 + j, exp, 0ull);
-                    }
-                const uint32_t okm = (uint32_t)((__ballot(ok) >> (g * G)) & 0xffu);
-                if (kk == s) my_flag = okm != 0;
-            } else if constexpr (UPDATE) {
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    if (kk_valid[kk] && e[kk][j] == kk_key[kk])
-                        __hip_atomic_store(wide_vals_at(W, kk_l[kk]) + s * 2 + j, kk_new[UPDATE ? kk : 0],
-                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (kk == s) my_flag = 1;
-            } else {
-                const int w = __builtin_ctz(gm);
-                const int fj = __shfl(first, g * G + w);
-                if (kk == s) {
-                    my_flag = 1;
-                    my_loc = kk_l[kk];
-                    my_slot = (uint32_t)(w * 2 + fj);
-                }
-            }
+    for (int kk = 0; kk < 4; ++kk) {
+        const uint64_t m = __ballot(keys_hold(e[kk], key[kk]));
+        any[kk] = quad_any(m);
+        more[kk] = ~any[kk];
+        if constexpr (FIRST) {
+            c[kk] = first_of_quad(m, any[kk], keys_slot(e[kk], key[kk], s));
+            const uint64_t open = quad_any(__ballot(keys_hold(e[kk], 0ull)));
+            more[kk] = ~open & (~any[kk] | quad_of_key(second, kk));
         }
     }
+    each_of_quad([&](auto q) {
+        constexpr int kk = decltype(q)::value;
+        const uint32_t lo = quad_bcast<kk>((uint32_t)a2) | off, hi = quad_bcast<kk>((uint32_t)(a2 >> 32));
+        if (__builtin_amdgcn_inverse_ballot_w64(more[kk])) e[kk] = load_wide_keys(lo, hi);
+    });
+    uint64_t found = 0;
+    uint64_t in2 = 0;  // the keys whose answer is in their second bucket
+    if constexpr (MODE == 0) {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            const uint64_t m = __ballot(keys_hold(e[kk], key[kk])) & (FIRST ? more[kk] : ~0ull), there = quad_any(m);
+            const uint32_t c2 = first_of_quad(m, there, keys_slot(e[kk], key[kk], s));
+            if constexpr (FIRST) {
+                if (__builtin_amdgcn_inverse_ballot_w64(there)) c[kk] = c2;
+                in2 |= there & (kQuadLow << kk);
+            } else {
+                c[kk] = c2;
+                in2 |= more[kk] & (kQuadLow << kk);
+            }
+            found |= (any[kk] | there) & (kQuadLow << kk);
+        }
+    } else {
+        uint64_t got[4], m[4], at[4];
+        each_of_quad([&](auto q) {
+            constexpr int kk = decltype(q)::value;
+            const bool first = __builtin_amdgcn_inverse_ballot_w64(any[kk]);
+            const uint32_t slot = keys_slot(e[kk], key[kk], s);
+            m[kk] = __ballot(slot != 0u) & quad_of_key(valid, kk);
+            const uint32_t l1 = quad_bcast<kk>(loc1), l2 = quad_bcast<kk>(loc2);
+            const uint32_t l = first ? l1 : l2;
+            const uint64_t *const line = ERASE ? wide_keys_at(W, l) : wide_vals_at(W, l);
+            at[kk] = (uint64_t)line;
+            const uint64_t new_v = UPDATE ? (uint64_t)quad_bcast<kk>((uint32_t)(nv >> 32)) << 32 | quad_bcast<kk>((uint32_t)nv) : 0ull;
+            got[kk] = 0;
+            if (__builtin_amdgcn_inverse_ballot_w64(m[kk])) {
+                DYC_GLOBAL uint64_t *const x = (DYC_GLOBAL uint64_t *)(at[kk] + 8u * (slot - 1u));
+                if constexpr (ERASE) got[kk] = cas_old(x, key[kk], 0ull);
+                else __hip_atomic_store(x, new_v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        });
+        // as in the narrow tile: keeps the CASes of the four keys in flight together
+        if constexpr (ERASE)
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) asm volatile("" : "+v"(got[kk]));
+        each_of_quad([&](auto q) {
+            constexpr int kk = decltype(q)::value;
+            uint64_t ok = ERASE ? __ballot(got[kk] == key[kk]) & m[kk] : m[kk];
+            // copies of one key in several of a lane's slots: the rest, one at a time (uniform, rare)
+            if (__ballot(keys_hold_two(e[kk], key[kk])) & m[kk]) {
+                const uint64_t new_v = UPDATE ? (uint64_t)quad_bcast<kk>((uint32_t)(nv >> 32)) << 32 | quad_bcast<kk>((uint32_t)nv) : 0ull;
+                bool seen = false, deleted = false;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (wide_key(e[kk], j) != key[kk] || !__builtin_amdgcn_inverse_ballot_w64(m[kk])) continue;
+                    if (seen) {
+                        DYC_GLOBAL uint64_t *const x = (DYC_GLOBAL uint64_t *)(at[kk] + off + 8 * j);
+                        if constexpr (ERASE) deleted |= cas_old(x, key[kk], 0ull) == key[kk];
+                        else __hip_atomic_store(x, new_v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                    seen = true;
+                }
+                ok |= __ballot(deleted);
+            }
+            found |= quad_any(ok) & (kQuadLow << kk);
+        });
+    }
+    found &= valid;
+    uint32_t my_flag = __builtin_amdgcn_inverse_ballot_w64(found) ? 1u : 0u;
     uint64_t my_val = 0;
-    if (MODE == 0 && my_flag) my_val = wide_vals_at(W, my_loc)[my_slot];
+    if constexpr (MODE == 0) {
+        const uint32_t slot = quad_gather_or(c, s) - 1u;
+        if (my_flag) {
+            const uint32_t l = __builtin_amdgcn_inverse_ballot_w64(in2) ? loc2 : loc1;
+            my_val = *(const DYC_GLOBAL uint64_t *)((uint64_t)wide_vals_at(W, l) + 8u * slot);
+        }
+    }
     if (inb && !my_flag && stash.n && !wide_reserved(k)) {  // the stash counts as one more bucket
         for (uint64_t j = 0; j < stash.n; ++j) {
             const uint64_t sk = __hip_atomic_load(stash.keys + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -200,16 +276,16 @@ __device__ inline uint32_t wide_probe_tile(const WideDesc &W, const uint64_t *__
     return my_flag;
 }
 
-template <int MODE>
+template <int MODE, bool FIRST = false>
 __global__ __launch_bounds__(256) void wide_probe_kernel(WideDesc W, const uint64_t *__restrict__ keys,
                                                          uint64_t *__restrict__ vals, uint8_t *__restrict__ flags,
-                                                         uint64_t n, Counters *__restrict__ C, WideStash stash)
+                                                         uint64_t n, Counters *__restrict__ C, WideStash stash,
+                                                         FirstBucket rule)
 {
     const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x / kWave);
     unsigned long long ndel = 0;
-    for (uint64_t base = ((uint64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave) * kWave; base < n;
-         base += waves * kWave)
-        ndel += wide_probe_tile<MODE>(W, keys, vals, flags, base, n, stash);
+    for (uint64_t base = (uint64_t)wave_slot() * kWave; base < n; base += waves * kWave)
+        ndel += wide_probe_tile<MODE, FIRST>(W, keys, vals, flags, base, n, stash, rule);
     if constexpr (MODE == 1) wave_tally(C, &C->deleted, ndel);
     if constexpr (MODE == 2) wave_tally(C, &C->updated, ndel);
 }
@@ -420,14 +496,14 @@ __device__ inline uint32_t wide_first_tile(uint32_t r)
     return (__builtin_amdgcn_readfirstlane(threadIdx.x / kWave) - r) % kProbeWavesPerBlock;
 }
 
-template <int MODE>
+template <int MODE, bool FIRST = false>
 __global__ __launch_bounds__(kWideGroupThreads) void wide_group_probe_kernel(const WideDesc *__restrict__ dir,
                                                                const GroupItem *__restrict__ items, uint32_t n_items,
                                                                const uint64_t *__restrict__ keys,
                                                                uint64_t *__restrict__ vals,
                                                                uint8_t *__restrict__ flags,
                                                                unsigned long long *__restrict__ table_counts,
-                                                               WideStash stash)
+                                                               WideStash stash, FirstBucket rule)
 {
     uint32_t r = 0;
     for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x, ++r) {
@@ -440,7 +516,7 @@ __global__ __launch_bounds__(kWideGroupThreads) void wide_group_probe_kernel(con
         const uint64_t end = item.begin + item.len;
         unsigned long long nd = 0;
         for (uint64_t base = item.begin + first; base < end; base += kWideGroupThreads)
-            nd += wide_probe_tile<MODE>(W, keys, vals, flags, base, end, st);
+            nd += wide_probe_tile<MODE, FIRST>(W, keys, vals, flags, base, end, st, rule);
         if constexpr (MODE == 1) {
             nd = wave_sum(nd);
             if (__lane_id() == 0 && nd) atomicAdd(&table_counts[item.table], nd);
@@ -955,14 +1031,17 @@ __global__ __launch_bounds__(THREADS) void wide_group_bulk_fill_kernel(const Gro
 
 // ------------------------------------------------------------------------------ launchers
 hipError_t launch_wide_probe(const WideDesc &W, const uint64_t *keys, uint64_t *vals, uint8_t *flags, uint64_t n,
-                             bool erase, LaunchShape sh, Counters *C, const WideStash &stash, hipStream_t st)
+                             bool erase, LaunchShape sh, Counters *C, const WideStash &stash, hipStream_t st,
+                             FirstBucket rule = FirstBucket::kNone)
 {
     if (n == 0) return hipSuccess;
     const int grid = grid_for((n + kWave - 1) / kWave, sh);
     if (erase)
-        wide_probe_kernel<1><<<grid, sh.block_threads, 0, st>>>(W, keys, nullptr, flags, n, C, stash);
+        wide_probe_kernel<1><<<grid, sh.block_threads, 0, st>>>(W, keys, nullptr, flags, n, C, stash, rule);
+    else if (rule != FirstBucket::kNone)
+        wide_probe_kernel<0, true><<<grid, sh.block_threads, 0, st>>>(W, keys, vals, flags, n, C, stash, rule);
     else
-        wide_probe_kernel<0><<<grid, sh.block_threads, 0, st>>>(W, keys, vals, flags, n, C, stash);
+        wide_probe_kernel<0><<<grid, sh.block_threads, 0, st>>>(W, keys, vals, flags, n, C, stash, rule);
     return hipGetLastError();
 }
 
@@ -974,7 +1053,7 @@ hipError_t launch_wide_update(const WideDesc &W, const uint64_t *keys, const uin
     if (n == 0) return hipSuccess;
     const int grid = grid_for((n + kWave - 1) / kWave, sh);
     wide_probe_kernel<2><<<grid, sh.block_threads, 0, st>>>(W, keys, const_cast<uint64_t *>(vals), updated, n, C,
-                                                            stash);
+                                                            stash, FirstBucket::kNone);
     return hipGetLastError();
 }
 
@@ -1008,16 +1087,20 @@ constexpr int kWideGroupBlocks = 2048;
 
 hipError_t launch_wide_group_probe(const WideDesc *dir, const GroupItem *items, uint32_t n_items, const uint64_t *keys,
                                    uint64_t *vals, uint8_t *flags, bool erase, unsigned long long *table_counts,
-                                   int blocks, const WideStash &stash, hipStream_t st)
+                                   int blocks, const WideStash &stash, hipStream_t st,
+                                   FirstBucket rule = FirstBucket::kNone)
 {
     if (n_items == 0) return hipSuccess;
     const int grid = blocks;
     if (erase)
         wide_group_probe_kernel<1>
-            <<<grid, kWideGroupThreads, 0, st>>>(dir, items, n_items, keys, nullptr, flags, table_counts, stash);
+            <<<grid, kWideGroupThreads, 0, st>>>(dir, items, n_items, keys, nullptr, flags, table_counts, stash, rule);
+    else if (rule != FirstBucket::kNone)
+        wide_group_probe_kernel<0, true>
+            <<<grid, kWideGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, flags, nullptr, stash, rule);
     else
         wide_group_probe_kernel<0>
-            <<<grid, kWideGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, flags, nullptr, stash);
+            <<<grid, kWideGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, flags, nullptr, stash, rule);
     return hipGetLastError();
 }
 
@@ -1139,6 +1222,7 @@ struct dyc_wide {
     // every key and value word is zero: set when the table is created or cleared, dropped by
     // every call that may store an entry (a bulk fill into such a table need not read it)
     bool zeroed = false;
+    dyc::host::FirstBucketRules rules;  // see there
     uint8_t *live = nullptr;  // downsize: tile flags of the residual list
     uint64_t live_cap = 0;
     uint8_t *upd = nullptr;  // upsert: per-key "updated in place" flags
@@ -1259,6 +1343,7 @@ void wset(dyc_wide *t, uint32_t i, uint8_t *base, uint32_t nb)
 int winstall_slab(dyc_wide *t, const uint32_t *nb, bool zero, hipStream_t s, uint8_t **region)
 {
     t->zeroed = false;  // new memory: only the caller knows what it holds
+    t->rules.lost();
     const uint32_t d = t->W.D.d;
     size_t off[kMaxSubtables + 1] = {0};
     for (uint32_t i = 0; i < d; ++i) off[i + 1] = off[i] + ((2 * wide_bytes(nb[i]) + kWideAlign - 1) & ~(kWideAlign - 1));
@@ -1320,6 +1405,7 @@ int wabsorb(dyc_wide *t, uint64_t room)
 int wresize_up(dyc_wide *t, hipStream_t s)
 {
     t->zeroed = false;
+    t->rules.lost();
     const uint32_t sub = choose_up(t->W.D.nb, t->W.D.d);
     const uint32_t old_nb = t->W.D.nb[sub];
     if ((uint64_t)old_nb * 2 >= kMaxBuckets) return fail(DYC_ERR_INVALID, "subtable %u cannot grow past 2^29 buckets", sub);
@@ -1387,6 +1473,7 @@ int wplace_pending(dyc_wide *t, hipStream_t s, uint64_t before)
 int wresize_down(dyc_wide *t, hipStream_t s)
 {
     t->zeroed = false;
+    t->rules.lost();
     const uint64_t pend_before = t->pend_n;
     const uint32_t sub = choose_down(t->W.D.nb, t->W.D.d);
     const uint32_t old_nb = t->W.D.nb[sub];
@@ -1605,6 +1692,7 @@ int dyc_wide_create(const dyc_config *cfg_in, uint64_t capacity_hint, dyc_wide *
     if (rc == DYC_OK) rc = wreserve_pending(t, 1024, nullptr);
     if (rc == DYC_OK && hipStreamSynchronize(nullptr) != hipSuccess) rc = fail(DYC_ERR_HIP, "create sync failed");
     t->zeroed = rc == DYC_OK;
+    if (t->zeroed) t->rules.emptied();
     if (rc != DYC_OK) {
         char keep[512];
         strncpy(keep, dyc_last_error(), sizeof keep - 1);
@@ -1677,6 +1765,7 @@ int dyc_wide_insert(dyc_wide *t, const uint64_t *keys, const uint64_t *vals, uin
     }
     rc = wzero(t, s);
     if (rc) return rc;
+    t->rules.filled(bulk ? FirstBucket::kFill : FirstBucket::kStart);
     if (bulk) {
         rc = wbulk_insert(t, keys, vals, n, zeroed, s);
         if (rc) return rc;
@@ -1708,6 +1797,7 @@ int dyc_wide_upsert(dyc_wide *t, const uint64_t *keys, const uint64_t *vals, uin
     t->st.last_kicks = 0;
     t->st.last_filled = 0;
     if (n == 0) return DYC_OK;
+    t->rules.filled(FirstBucket::kStart);
     const uint64_t pend_before = t->pend_n;
     int rc;
     if (t->cfg.auto_resize) {  // sized as if every key were new
@@ -1756,7 +1846,10 @@ int dyc_wide_find(dyc_wide *t, const uint64_t *keys, uint64_t *vals, uint8_t *hi
     if (!t) return fail(DYC_ERR_INVALID, "null table");
     if (n && !keys) return fail(DYC_ERR_INVALID, "null keys");
     DeviceGuard dg(t->device);
-    HIP_TRY(launch_wide_probe(t->W, keys, vals, hit, n, false, t->shape(), t->ctr, t->stash(), (hipStream_t)stream));
+    hipStream_t s = (hipStream_t)stream;
+    HIP_TRY(t->rules.find(n, s, [&](FirstBucket rule) {
+        return launch_wide_probe(t->W, keys, vals, hit, n, false, t->shape(), t->ctr, t->stash(), s, rule);
+    }));
     return DYC_OK;
 }
 
@@ -1767,6 +1860,7 @@ int dyc_wide_erase(dyc_wide *t, const uint64_t *keys, uint8_t *deleted, uint64_t
     DeviceGuard dg(t->device);
     hipStream_t s = (hipStream_t)stream;
     if (n == 0) return DYC_OK;
+    HIP_TRY(t->rules.freeing(s));
     int rc = wzero(t, s);
     if (rc) return rc;
     HIP_TRY(launch_wide_probe(t->W, keys, nullptr, deleted, n, true, t->shape(), t->ctr, t->stash(), s));
@@ -1822,6 +1916,7 @@ int dyc_wide_clear(dyc_wide *t, dyc_stream stream)
     t->count = 0;
     t->pend_n = 0;
     t->st.pending = 0;
+    t->rules.emptied();
     t->zeroed = true;
     return DYC_OK;
 }
@@ -1914,6 +2009,7 @@ struct dyc_wide_group {
     // every key and value word of every table is zero: set at create and clear, dropped by every
     // insert
     bool zeroed = false;
+    dyc::host::FirstBucketRules rules;  // of all tables together
     // bulk fill (cfg.insert_order 3), grown on demand: partitioned entries and the overflow (16 B
     // per key each), local chunk ids, per-block chunk counts, chunk records, overflow counts and
     // items, and the block and table arrays (device, with pinned staging)
@@ -2025,6 +2121,9 @@ int wg_probe_grid(const dyc_wide_group *g, uint64_t n, uint32_t n_items)
 {
     return g->cfg.max_blocks ? (int)g->cfg.max_blocks : group_probe_grid(n, n_items);
 }
+
+// As first_bucket_pays in dyc_group.hip (the arena also holds the value lines).
+bool wg_first_bucket_pays(const dyc_wide_group *g) { return g->arena_bytes >= (uint64_t)g->n << 20; }
 
 int wg_prologue(dyc_wide_group *g, hipStream_t s)
 {
@@ -2205,6 +2304,7 @@ int wg_bulk_insert(dyc_wide_group *g, const uint64_t *keys, const uint64_t *vals
     HIP_TRY(hipMemcpyAsync(g->bk_tabs, g->bk_htabs, J * sizeof(BulkTable), hipMemcpyHostToDevice, s));
     const int rc = wg_prologue(g, s);
     if (rc) return rc;
+    g->rules.filled(FirstBucket::kFill);
     HIP_TRY(wg_enqueue_bulk(g, NB, J, L.chunks, keys, vals, L.total, zeroed,
                             WideSink{g->pk + g->pend_n, g->pv + g->pend_n, room, g->ptag + g->pend_n}, s));
     *filled = true;
@@ -2310,6 +2410,7 @@ int dyc_wide_group_create(const dyc_config *cfg_in, uint32_t n_tables, const uin
     int rc = wg_reserve_pending(g, 65536, nullptr);
     if (rc) return cleanup(rc);
     g->zeroed = true;
+    g->rules.emptied();
     *out = g;
     return DYC_OK;
 }
@@ -2341,6 +2442,7 @@ int dyc_wide_group_insert(dyc_wide_group *g, const uint64_t *keys, const uint64_
         if (rc) return rc;
         rc = wg_prologue(g, s);
         if (rc) return rc;
+        g->rules.filled(FirstBucket::kStart);
         HIP_TRY(launch_wide_group_insert(g->ddir, g->ditems, n_items, keys, vals, g->policy(),
                                          (int)g->cfg.insert_blocks, g->ctr,
                                          WideSink{g->pk + g->pend_n, g->pv + g->pend_n, room, g->ptag + g->pend_n},
@@ -2378,9 +2480,10 @@ int dyc_wide_group_find(dyc_wide_group *g, const uint64_t *keys, const uint64_t 
     uint32_t n_items = 0;
     rc = wg_upload_items(g, offsets, s, &n_items, offsets[g->n] >= dyc::host::kXcdLayoutKeys);
     if (rc) return rc;
-    HIP_TRY(launch_wide_group_probe(g->ddir, g->ditems, n_items, keys, vals, hit, false, nullptr,
-                                    wg_probe_grid(g, offsets[g->n], n_items),
-                                    g->stash(), s));
+    HIP_TRY(g->rules.find(wg_first_bucket_pays(g) ? offsets[g->n] : 0, s, [&](FirstBucket rule) {
+        return launch_wide_group_probe(g->ddir, g->ditems, n_items, keys, vals, hit, false, nullptr,
+                                       wg_probe_grid(g, offsets[g->n], n_items), g->stash(), s, rule);
+    }));
     return DYC_OK;
 }
 
@@ -2396,6 +2499,7 @@ int dyc_wide_group_erase(dyc_wide_group *g, const uint64_t *keys, const uint64_t
     uint32_t n_items = 0;
     rc = wg_upload_items(g, offsets, s, &n_items);
     if (rc) return rc;
+    HIP_TRY(g->rules.freeing(s));
     rc = wg_prologue(g, s);
     if (rc) return rc;
     HIP_TRY(launch_wide_group_probe(g->ddir, g->ditems, n_items, keys, nullptr, deleted, true, g->tcounts,
@@ -2418,6 +2522,7 @@ int dyc_wide_group_insert_per_table(dyc_wide_group *g, const uint64_t *keys, con
     DeviceGuard dg(g->device);
     hipStream_t s = (hipStream_t)stream;
     g->zeroed = false;
+    g->rules.filled(FirstBucket::kStart);
     g->st.last_filled = 0;
     rc = wg_reserve_pending(g, std::max<uint64_t>(65536, offsets[g->n] / 16), s);
     if (rc) return rc;
@@ -2530,6 +2635,7 @@ int dyc_wide_group_clear(dyc_wide_group *g, dyc_stream stream)
     std::fill(g->count.begin(), g->count.end(), 0);
     g->pend_n = 0;
     g->st.pending = 0;
+    g->rules.emptied();
     g->zeroed = true;
     return DYC_OK;
 }

@@ -85,6 +85,34 @@ def test_same_as_the_reference_order(D, order, d):
     t.close()
 
 
+@pytest.mark.parametrize("d", [2, 4])
+@pytest.mark.parametrize("order", [0, 3])
+def test_wide_tables(D, order, d):
+    print(f"\n[gpu-case] first-bucket rule, wide d={d} insert_order={order}", flush=True)
+    m = 1 << 19
+    t = D.DyCuckooWide(int(m / (0.6 if d == 2 else 0.75)), subtables=d, insert_order=order, kick_bound=0, auto_resize=0)
+    wide = lambda x: x.long() * 0x1_0000_0001 ^ 0x55  # noqa: E731
+    k = wide(keys(0, m))
+    q = torch.cat([wide(lookups(LARGE + 5, m, d)), torch.tensor([0, -1], device="cuda")])
+    _, h = both_ways(t, q)
+    assert not h.any()
+    t.insert(k, k ^ 1)
+    both_ways(t, q)
+    t.insert(k[: m // 16], k[: m // 16] ^ 2)
+    both_ways(t, q)
+    t.upsert(k[: m // 16], k[: m // 16] ^ 3)  # under the start rule
+    both_ways(t, q)
+    assert t.erase(k[: m // 2]).all()
+    both_ways(t, q)
+    t.clear()
+    t.insert(k, k ^ 4)
+    v, h = both_ways(t, q)
+    t.resize_up()
+    v2, h2 = both_ways(t, q)
+    assert torch.equal(h, h2) and torch.equal(v, v2)
+    t.close()
+
+
 def test_upsert_and_host_inserts_keep_the_start_rule(D):
     print("\n[gpu-case] first-bucket rule, upsert and host inserts", flush=True)
     m = 1 << 19

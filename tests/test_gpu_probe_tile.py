@@ -84,3 +84,40 @@ def test_find_erase_update_with_copies(D, d, n):
     assert np.array_equal(t.erase(dev(q)).cpu().numpy(), flags)
     assert all(np.array_equal(a, b) for a, b in zip(t.dump(), erased))
     t.close()
+
+
+@pytest.mark.parametrize("d", [2, 4])
+@pytest.mark.parametrize("n", [1, 64, 65, 601])
+def test_wide_find_erase_update_with_copies(D, d, n):
+    """The wide probe over the same images: keys below 2^32 live where the 32-bit table puts them."""
+    print(f"\n[gpu-case] wide probe tile d={d} n={n}", flush=True)
+    images, keys = images_with_copies(40 + d, d)
+    absent = distinct(900, 77)
+    absent = absent[~np.isin(absent, keys)][:200]
+    rng = np.random.default_rng(n)
+    q = np.concatenate([keys[:400], absent, np.array([0], dtype=np.uint32)])
+    q = rng.permutation(q)[:n] if n > 1 else keys[:1]
+    wide = lambda a: torch.from_numpy(a.astype(np.uint64).view(np.int64)).cuda()  # noqa: E731
+    lo = np.uint64(0xFFFFFFFF)
+    t = D.DyCuckooWide(1000, subtables=d, max_fail_rounds=0)
+    t.load([x >> np.uint64(32) for x in images], [x & lo for x in images])
+    v, h = t.find(wide(q))
+    want_v, want_h = on_oracle(images).find(q)
+    assert np.array_equal(h.cpu().numpy(), want_h)
+    assert np.array_equal(v.cpu().numpy().view(np.uint64), want_v.astype(np.uint64))
+    ref = on_oracle(images)
+    flags = ref.erase(q)
+    u = q[flags != 0]
+    if u.size:
+        new = u.astype(np.uint64) * np.uint64(0x100000001)
+        assert t.upsert(wide(u), torch.from_numpy(new.view(np.int64)).cuda()).cpu().numpy().all()
+        gk, gv = t.dump()
+        for k, val, old, gone in zip(gk, gv, images, ref.images()):
+            hit = old != gone
+            assert np.array_equal(k, old >> np.uint64(32))
+            assert np.array_equal(val, np.where(hit, (old >> np.uint64(32)) * np.uint64(0x100000001), old & lo))
+    # erase empties the key words of every copy in the bucket that find reads, and no other
+    assert np.array_equal(t.erase(wide(q)).cpu().numpy(), flags)
+    for k, gone in zip(t.dump()[0], ref.images()):
+        assert np.array_equal(k, gone >> np.uint64(32))
+    t.close()
