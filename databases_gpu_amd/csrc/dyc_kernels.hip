@@ -12,7 +12,6 @@
 #include "dyc_wave.hpp"
 
 #include <algorithm>
-#include <type_traits>
 
 namespace dyc {
 
@@ -82,41 +81,6 @@ __device__ inline void publish_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "m
 // of 2^23 5.2 us (7.6), of 2^23 keys 252 us (258: bound by the rate of random lines, 54 G/s), and
 // with 16 lanes 8.9, 10.8 and 316 us; so every probe takes this tile, whatever lanes per key the
 // caller set.
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-#define DYC_GLOBAL __attribute__((address_space(1)))
-
-// x of lane KK of each quad, in all of its lanes.
-template <int KK>
-__device__ inline uint32_t quad_bcast(uint32_t x)
-{
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, KK * 0x55, 0xf, 0xf, true);
-}
-// x of the quad lane whose number differs in bit 0 (XOR = 1) or bit 1 (XOR = 2).
-template <int XOR>
-__device__ inline uint32_t quad_swap(uint32_t x)
-{
-    static_assert(XOR == 1 || XOR == 2, "a quad permute");
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, XOR == 1 ? 0xb1 : 0x4e, 0xf, 0xf, true);
-}
-
-constexpr uint64_t kQuadLow = 0x1111111111111111ull;  // lane 0 of every quad
-// Every lane of each quad that has a lane in m.
-__device__ inline uint64_t quad_any(uint64_t m)
-{
-    m |= m >> 1;
-    m = (m | m >> 2) & kQuadLow;
-    return (m << 4) - m;
-}
-
-template <typename F>
-__device__ inline void each_of_quad(F f)
-{
-    f(std::integral_constant<int, 0>{});
-    f(std::integral_constant<int, 1>{});
-    f(std::integral_constant<int, 2>{});
-    f(std::integral_constant<int, 3>{});
-}
-
 // A lane's four slots (32 bytes) of a bucket. COH: read device-coherently (agent-scope relaxed
 // atomic loads, which skip lines another XCD's writes may have left stale in this XCD's L2), for
 // reads that must see exchanges made earlier in the same launch by other waves.
@@ -167,33 +131,6 @@ __device__ inline bool slots_hold_two(const QuadSlots &e, uint32_t k)
 {
     const bool a = e.a.y == k, b = e.a.w == k, c = e.b.y == k, d = e.b.w == k;
     return (a & b) | (c & d) | ((a | b) & (c | d));
-}
-
-// Clears v in the lanes whose slot is not the first match of its quad (copies of one key in slots of
-// several lanes: uniform, rare).
-__device__ inline uint32_t first_of_quad(uint64_t m, uint64_t any, uint32_t v)
-{
-    if (__popcll(m) * 4 != __popcll(any)) {
-        const uint64_t later = ((m << 1) & ~kQuadLow) | ((m << 2) & (kQuadLow * 0xc)) | ((m << 3) & (kQuadLow * 8));
-        if (__builtin_amdgcn_inverse_ballot_w64(later)) v = 0;
-    }
-    return v;
-}
-
-// The OR over the quad of key kk's word v[kk], in lane kk.
-__device__ inline uint32_t quad_gather_or(const uint32_t (&v)[4], uint32_t s)
-{
-    const bool odd = s & 1u, high = s & 2u;
-    const uint32_t v01 = (odd ? v[1] : v[0]) | quad_swap<1>(odd ? v[0] : v[1]);
-    const uint32_t v23 = (odd ? v[3] : v[2]) | quad_swap<1>(odd ? v[2] : v[3]);
-    return (high ? v23 : v01) | quad_swap<2>(high ? v01 : v23);
-}
-
-// The lanes of key kk's quads, of a mask of the keys' own lanes.
-__device__ inline uint64_t quad_of_key(uint64_t own, int kk)
-{
-    const uint64_t low = (own >> kk) & kQuadLow;
-    return (low << 4) - low;
 }
 
 // One wave probes the 64 keys keys[base, base + 64) clipped to n, in table D. Returns this
