@@ -340,22 +340,25 @@ Chunks make_chunks(const Desc &D)
 
 namespace {
 
-// The 8-byte entries' partition: 4096-entry tiles (256 threads), two blocks per CU.
-constexpr int kBulkSortThreads = 256;
-constexpr uint32_t kBulkSortTile = kBulkSortThreads * kSortItems;
+// Tiles of a whole CU's LDS (28 or 24 entries a thread; 20 with 4-byte chunk ids) write fewer
+// partial lines; 4096-entry tiles (8 a thread, three workgroups a CU) rank with three times the
+// waves and spread small batches over more CUs. First pass, small / large tiles: 2^22 entries
+// 17 / 24 us, 2^23 38 / 39, 2^24 79 / 75, 48 Mi 318 / 250, 2^28 2107 / 1626. Later passes, whose
+// ranking takes a ballot per digit bit: 2^24 75 / 89 us, 48 Mi 229 / 235, 2^28 1472 / 1257.
+constexpr uint64_t kLargeFirstTiles = 1ull << 24, kLargeLaterTiles = 1ull << 26;
 
-template <typename CidT>
+template <typename CidT, int ITEMS0, int ITEMS1>
 hipError_t bulk_partition(const Desc &D, const Chunks &Ch, const uint32_t *keys, const uint32_t *vals, uint64_t n,
-                          const BulkSpace &ws, uint32_t max_blocks, hipStream_t st, int *out)
+                          const BulkSpace &ws, hipStream_t st, int *out)
 {
     RadixPass P[kMaxRadixPasses];
     const uint32_t np = radix_passes(Ch.bits, P);
-    const PartGrid G = part_grid(n, max_blocks, kBulkSortTile);
+    const PartGrid G = part_grid<uint64_t, CidT, ITEMS0>(n);
     CidT *const cid[2] = {static_cast<CidT *>(ws.cid[0]), static_cast<CidT *>(ws.cid[1])};
     uint64_t *const ent[2] = {static_cast<uint64_t *>(ws.ent[0]), static_cast<uint64_t *>(ws.ent[1])};
     bulk_pack_kernel<CidT><<<G.blocks * G.sub, kCountThreads, 0, st>>>(D, Ch, keys, G, P[0], cid[0], ws.partial);
-    return partition_passes<uint64_t, KeyValSource, CidT, kBulkSortThreads>(
-        KeyValSource{keys, vals}, 0, ent, cid, G, P, np, ws.partial, ws.total, ws.start, Ch.total, st, out);
+    return partition_passes<uint64_t, KeyValSource, CidT, ITEMS0, ITEMS1>(
+        KeyValSource{keys, vals}, ent, cid, G, P, np, ws.partial, ws.total, ws.start, Ch.total, st, out);
 }
 
 }  // namespace
@@ -363,14 +366,19 @@ hipError_t bulk_partition(const Desc &D, const Chunks &Ch, const uint32_t *keys,
 size_t bulk_cid_bytes(const Chunks &Ch) { return Ch.total <= 65536u ? 2 : 4; }
 
 hipError_t launch_bulk_partition(const Desc &D, const Chunks &Ch, const uint32_t *keys, const uint32_t *vals,
-                                 uint64_t n, const BulkSpace &ws, uint32_t max_blocks, hipStream_t st, int *out)
+                                 uint64_t n, const BulkSpace &ws, hipStream_t st, int *out)
 {
     *out = 0;
     if (n == 0) return hipSuccess;
     if (n >= (1ull << 32) || Ch.total == 0 || Ch.bits > kMaxRadixPasses * kMaxRadixBits) return hipErrorInvalidValue;
-    if (bulk_cid_bytes(Ch) == 2)
-        return bulk_partition<uint16_t>(D, Ch, keys, vals, n, ws, max_blocks, st, out);
-    return bulk_partition<uint32_t>(D, Ch, keys, vals, n, ws, max_blocks, st, out);
+    if (bulk_cid_bytes(Ch) == 2) {
+        if (n < kLargeFirstTiles) return bulk_partition<uint16_t, 8, 8>(D, Ch, keys, vals, n, ws, st, out);
+        if (n < kLargeLaterTiles) return bulk_partition<uint16_t, 28, 8>(D, Ch, keys, vals, n, ws, st, out);
+        return bulk_partition<uint16_t, 28, 24>(D, Ch, keys, vals, n, ws, st, out);
+    }
+    if (n < kLargeFirstTiles) return bulk_partition<uint32_t, 8, 8>(D, Ch, keys, vals, n, ws, st, out);
+    if (n < kLargeLaterTiles) return bulk_partition<uint32_t, 20, 8>(D, Ch, keys, vals, n, ws, st, out);
+    return bulk_partition<uint32_t, 20, 20>(D, Ch, keys, vals, n, ws, st, out);
 }
 
 // ------------------------------------------------------------------------------ many tables
@@ -573,8 +581,8 @@ hipError_t launch_group_bulk_scatter(const GroupItem *blocks, uint32_t n_blocks,
     if (n >= (1ull << 32)) return hipErrorInvalidValue;
     const SegLayout lay{blocks, partial, n};
     uint8_t *const no_cid = nullptr;
-    part_scatter_kernel<uint64_t, KeyValSource, uint8_t, kBulkSortThreads, -1, SegLayout>
-        <<<n_blocks, kBulkSortThreads, 0, st>>>(KeyValSource{keys, vals}, lcid, lay, RadixPass{0, 8}, ent, no_cid);
+    part_scatter_kernel<uint64_t, KeyValSource, uint8_t, 8, -1, false, SegLayout>
+        <<<n_blocks, kSortThreads, 0, st>>>(KeyValSource{keys, vals}, lcid, lay, RadixPass{0, 8}, ent, no_cid);
     return hipGetLastError();
 }
 

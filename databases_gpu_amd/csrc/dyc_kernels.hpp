@@ -148,15 +148,11 @@ struct BulkSpace {
     uint32_t *start;
 };
 size_t bulk_cid_bytes(const Chunks &Ch);
-// Scatter blocks of a partition launch: two per CU on 256 CUs, of 4096-entry tiles. One per CU
-// (8192-entry tiles, or 4096) and three per CU measured slower.
-constexpr uint32_t kBulkSortBlocks = 512;
-constexpr uint32_t kWideSortBlocks = 512;
 // Group the n entries keys/vals (n < 2^32) by the chunk of each key's fill_target bucket (reserved
 // keys go to chunk 0). The sorted entries end in ws.ent[*out], and ws.start receives the first
 // index of every chunk.
 hipError_t launch_bulk_partition(const Desc &D, const Chunks &Ch, const uint32_t *keys, const uint32_t *vals,
-                                 uint64_t n, const BulkSpace &ws, uint32_t max_blocks, hipStream_t st, int *out);
+                                 uint64_t n, const BulkSpace &ws, hipStream_t st, int *out);
 // Fill free slots chunk by chunk from the partitioned entries (n < 2^32); start holds total + 1
 // words. Entries that do not fit are appended to ovf at C->overflow (ovf_cap >= n). Placements go
 // to the kick tally, reserved keys to the rejected tally. zeroed: every slot of the table is zero (a

@@ -22,13 +22,16 @@
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 
 #include "dyc_kernels.hpp"
 #include "dyc_wave.hpp"
 
 namespace dyc {
 
-constexpr int kSortItems = 16;  // entries per thread per scatter tile
+template <int V>
+using Int = std::integral_constant<int, V>;
+constexpr int kSortThreads = 512;  // threads of a scatter workgroup
 constexpr uint32_t kMaxRadixBits = 8;
 constexpr uint32_t kMaxRadix = 1u << kMaxRadixBits;
 constexpr uint32_t kMaxRadixPasses = 4;
@@ -58,10 +61,21 @@ struct PartGrid {
 };
 constexpr uint32_t kCountBlocks = 1024;  // counting blocks aimed for
 
-inline PartGrid part_grid(uint64_t n, uint32_t max_blocks, uint32_t tile)
+// Workgroups of a scatter that fit a CU: its LDS holds a tile's entries, their chunk ids and, at
+// most, 10 KiB of counters.
+__host__ __device__ constexpr uint32_t sort_blocks_per_cu(size_t entry_bytes, int items)
 {
+    return std::min<uint32_t>(4, 160 * 1024 / (uint32_t)(kSortThreads * items * entry_bytes + 11 * 1024));
+}
+
+template <typename Entry, typename CidT, int ITEMS>
+inline PartGrid part_grid(uint64_t n)
+{
+    constexpr uint32_t tile = kSortThreads * ITEMS;
+    constexpr uint32_t max_blocks = 256 * sort_blocks_per_cu(sizeof(Entry) + sizeof(CidT), ITEMS);
+    static_assert(max_blocks > 0 && max_blocks <= kMaxSortBlocks, "a tile fits a CU");
     const uint64_t tiles = (n + tile - 1) / tile;
-    uint32_t blocks = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(tiles, 1), std::min(max_blocks, kMaxSortBlocks));
+    uint32_t blocks = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(tiles, 1), max_blocks);
     const uint32_t per = (uint32_t)std::max<uint64_t>((tiles + blocks - 1) / blocks, 1);
     blocks = (uint32_t)std::max<uint64_t>((tiles + per - 1) / per, 1);  // no block without a tile
     uint32_t sub = std::max<uint32_t>(1, std::min(kCountBlocks, kMaxSortBlocks) / blocks);
@@ -101,19 +115,22 @@ __device__ inline uint64_t count_end(const PartGrid &G, uint64_t lo)
 }
 
 // Where a scatter pass reads its entries: an entry array, or the caller's key and value arrays
-// (the first pass of an insert batch).
+// (the first pass of an insert batch). from(i) is the source that starts at entry i.
 template <typename Entry>
 struct EntrySource {
     const Entry *e;
     __device__ Entry load(uint64_t i) const { return e[i]; }
+    __device__ EntrySource from(uint64_t i) const { return {e + i}; }
 };
 struct KeyValSource {
     const uint32_t *k, *v;
     __device__ uint64_t load(uint64_t i) const { return pack(k[i], v[i]); }
+    __device__ KeyValSource from(uint64_t i) const { return {k + i, v + i}; }
 };
 struct WideKeyValSource {
     const uint64_t *k, *v;
     __device__ WideEntry load(uint64_t i) const { return WideEntry{k[i], v[i]}; }
+    __device__ WideKeyValSource from(uint64_t i) const { return {k + i, v + i}; }
 };
 
 namespace {
@@ -297,14 +314,21 @@ __device__ inline uint64_t match_mask(uint64_t vm, uint32_t d, uint32_t bits)
 }
 
 // One pass: the entries of each block's range (from src, chunk ids from cid) go to their places
-// in ent_out (chunk ids to cid_out unless it is null), ordered by digit P. partial holds the
-// blocks' exclusive prefixes per digit and total the digits' totals (part_colscan_kernel). The
-// next tile's loads are issued before the current tile is ranked: a barrier here waits for LDS
-// operations only, so they stay in flight while the tile is placed and written out.
+// in ent_out (with CIDS chunk ids to cid_out), ordered by digit P. partial holds the blocks'
+// exclusive prefixes per digit and total the digits' totals (part_colscan_kernel).
+// What bounds it is how a tile's entries reach memory: a tile writes one run per digit, and the
+// first and last line of a run are written in part (4096-entry tiles, 16 entries a run: 35 % more
+// bytes than the entries and chunk ids have). So where the batch has tiles enough a tile takes a
+// CU's whole LDS, at 8 waves a CU (the caller chooses ITEMS, a thread's entries). The next tile's
+// loads are issued when the tile's entries have gone to LDS, ahead of the write-out's stores; all
+// of them, and a whole tile's stores, are issued without a branch, so every wait counts the
+// younger operations instead of draining the stores.
+// 2^28 entries of 8 bytes, first pass 2105 -> 1630 us (3.3 TB/s), last pass 1485 -> 1255 us
+// (3.8 TB/s); 2^26 entries of 16 bytes, 675 -> 620 us and 780 -> 505 us.
 // Ranking within a wave (BITS):
 //   > 0  stably (by digit, then index), with one ballot per digit bit; BITS = P.bits;
 //   0    the same with P.bits read at run time;
-//   < 0  not stably: each entry's rank is what its wave's LDS counter of the digit returned
+//   < 0  not stably: each entry's rank is what the workgroup's LDS counter of the digit returned
 //        when the entry added itself, in whatever order the lanes' atomics were applied. The
 //        first pass of a least-significant-digit partition may do this (its input order means
 //        nothing); every later pass must keep the order of the previous digits.
@@ -343,142 +367,163 @@ struct SegLayout {
     }
 };
 
-template <typename Entry, typename Src, typename CidT, int THREADS, int BITS, typename Layout = PassLayout>
-__global__ __launch_bounds__(THREADS) void part_scatter_kernel(Src src, const CidT *__restrict__ cid, Layout Lay,
-                                                               RadixPass P, Entry *__restrict__ ent_out,
-                                                               CidT *__restrict__ cid_out)
+template <typename Entry, typename Src, typename CidT, int ITEMS, int BITS, bool CIDS, typename Layout = PassLayout>
+__global__ __launch_bounds__(kSortThreads, 2) void part_scatter_kernel(
+    Src src, const CidT *__restrict__ cid, Layout Lay, RadixPass P, Entry *__restrict__ ent_out,
+    CidT *__restrict__ cid_out)
 {
-    constexpr int kWaves = THREADS / kWave;
-    constexpr uint32_t kTile = THREADS * kSortItems;
-    static_assert(THREADS >= (int)kMaxRadix && THREADS % kWave == 0, "one thread per digit");
+    constexpr int kWaves = kSortThreads / kWave;
+    constexpr uint32_t kTile = kSortThreads * ITEMS;
+    static_assert(kSortThreads >= (int)kMaxRadix && kSortThreads % kWave == 0, "one thread per digit");
     __shared__ Entry buf[kTile];
-    __shared__ CidT cbuf[kTile];
-    __shared__ uint32_t wcnt[kWaves][kMaxRadix];  // per-wave digit counts, then wave offsets
+    // what the write-out needs of a chunk id: all of it if it is passed on, else its digit
+    using Kept = std::conditional_t<CIDS, CidT, uint8_t>;
+    __shared__ Kept cbuf[kTile];
+    constexpr int kRows = BITS < 0 ? 1 : kWaves;  // counters: the workgroup's, or per wave
+    __shared__ uint32_t wcnt[kRows][kMaxRadix];   // digit counts, then first places in the tile
     __shared__ uint32_t gbase[kMaxRadix];         // global place of the block's next entry of d
     __shared__ uint32_t gdel[kMaxRadix];          // gbase[d] minus the tile's first place of d
-    __shared__ uint32_t loc[kMaxRadix];           // first place of digit d in the tile
     __shared__ uint32_t tmp[kScanWaves];
     const uint32_t R = 1u << P.bits;
-    const uint32_t tid = threadIdx.x, lane = __lane_id(), w = tid / kWave;
+    const uint32_t tid = threadIdx.x, lane = __lane_id(), w = __builtin_amdgcn_readfirstlane(tid / kWave);
     const uint64_t lo = Lay.begin(blockIdx.x);
     const uint64_t hi = Lay.end(blockIdx.x, lo);
-    if (lo >= hi) return;  // block-uniform: nothing to place (a clipped block of a fill's later round)
+    if (lo >= hi) return;  // block-uniform: nothing to place
     {
         const uint32_t b = Lay.base(blockIdx.x, tid, R, tmp);
         if (tid < R) gbase[tid] = b;
     }
     const uint64_t lanemask = lanemask_lt();
-    // wave w holds tile entries w * kSortItems * 64 + u * 64 + lane: stable ranking follows
+    // wave w holds tile entries w * ITEMS * 64 + u * 64 + lane: stable ranking follows
     // (u, lane) inside the wave, and the waves in order
-    const uint32_t wbase = w * kSortItems * kWave;
-    Entry e[kSortItems], en[kSortItems];
-    uint32_t c[kSortItems], cn[kSortItems];
-    auto load_tile = [&](uint64_t t0, Entry *ev, uint32_t *cv) {
+    const uint32_t wbase = w * ITEMS * kWave;
+    Entry e[ITEMS];
+    uint32_t c[ITEMS];
+    // entries past the range's end are read as its last one and not used
+    auto load_tile = [&](uint64_t t0) {
+        if (t0 + kTile <= hi) {
+            const Src ws = src.from(t0 + wbase);
+            const CidT *const wc = cid + t0 + wbase;
 #pragma unroll
-        for (int u = 0; u < kSortItems; ++u) {
-            const uint64_t i = t0 + wbase + u * kWave + lane;
-            if (i < hi) {
-                ev[u] = src.load(i);
-                cv[u] = (uint32_t)cid[i];
-            } else {
-                cv[u] = 0u;
+            for (int u = 0; u < ITEMS; ++u) {
+                e[u] = ws.load(u * kWave + lane);
+                c[u] = (uint32_t)wc[u * kWave + lane];
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < ITEMS; ++u) {
+                const uint64_t at = t0 + wbase + u * kWave + lane, i = at < hi ? at : hi - 1;
+                e[u] = src.load(i);
+                c[u] = (uint32_t)cid[i];
             }
         }
     };
-    if (lo < hi) load_tile(lo, e, c);
-    for (uint64_t t0 = lo; t0 < hi; t0 += kTile) {
-        const uint32_t tn = hi - t0 < kTile ? (uint32_t)(hi - t0) : kTile;
-        if (t0 + kTile < hi) load_tile(t0 + kTile, en, cn);
-        for (uint32_t x = tid; x < kWaves * kMaxRadix; x += THREADS) (&wcnt[0][0])[x] = 0;
+    auto tile = [&](uint64_t t0, auto whole) {
+        constexpr bool kWhole = decltype(whole)::value;
+        const uint32_t tn = kWhole ? kTile : (uint32_t)(hi - t0);
+        auto valid = [&](int u) { return kWhole || wbase + u * kWave + lane < tn; };
+        for (uint32_t x = tid; x < kRows * kMaxRadix; x += kSortThreads) (&wcnt[0][0])[x] = 0;
         __syncthreads();  // wcnt is zero; the previous tile's output is done with buf and gdel
-        uint32_t r[kSortItems];
+        uint32_t r[ITEMS];
         if constexpr (BITS < 0) {
 #pragma unroll
-            for (int u = 0; u < kSortItems; ++u)
-                r[u] = wbase + u * kWave + lane < tn ? atomicAdd(&wcnt[w][digit_of(c[u], P)], 1u) : 0u;
+            for (int u = 0; u < ITEMS; ++u) r[u] = valid(u) ? atomicAdd(&wcnt[0][digit_of(c[u], P)], 1u) : 0u;
         } else {
             // the lanes of one digit in an item (their match mask) take consecutive ranks in lane
             // order after the digit's count so far
             const uint32_t bits = P.bits;
 #pragma unroll
-            for (int u = 0; u < kSortItems; ++u) {
-                const bool valid = wbase + u * kWave + lane < tn;
+            for (int u = 0; u < ITEMS; ++u) {
                 const uint32_t d = digit_of(c[u], P);
-                const uint64_t m = match_mask<BITS>(__ballot(valid), d, bits);
+                const uint64_t m = match_mask<BITS>(__ballot(valid(u)), d, bits);
                 const uint32_t below = (uint32_t)__popcll(m & lanemask);
-                const uint32_t base = valid ? wcnt[w][d] : 0u;
+                const uint32_t base = valid(u) ? wcnt[w][d] : 0u;
                 r[u] = base + below;
-                if (valid && below == 0) wcnt[w][d] = base + (uint32_t)__popcll(m);
+                if (valid(u) && below == 0) wcnt[w][d] = base + (uint32_t)__popcll(m);
             }
         }
         __syncthreads();
-        // per digit: wave offsets (exclusive over the waves), the tile's first place, and the
-        // shift from a tile place to its global place
+        // per digit: the counters' first places in the tile (in their order), and the shift from
+        // a tile place to its global place
         {
-            uint32_t run = 0;
-            if (tid < R) {
+            uint32_t x[kRows], run = 0;
 #pragma unroll
-                for (int q = 0; q < kWaves; ++q) {
-                    const uint32_t x = wcnt[q][tid];
-                    wcnt[q][tid] = run;
-                    run += x;
-                }
+            for (int q = 0; q < kRows; ++q) {
+                x[q] = tid < R ? wcnt[q][tid] : 0u;
+                run += x[q];
             }
             uint32_t all;
-            const uint32_t first = block_exclusive_scan(tid < R ? run : 0u, tmp, &all);
+            uint32_t at = block_exclusive_scan(run, tmp, &all);
             if (tid < R) {
-                loc[tid] = first;
-                gdel[tid] = gbase[tid] - first;
+                gdel[tid] = gbase[tid] - at;
                 gbase[tid] += run;  // read again only after the next tile's offsets are made
-            }
-        }
-        __syncthreads();
 #pragma unroll
-        for (int u = 0; u < kSortItems; ++u) {
-            if (wbase + u * kWave + lane < tn) {
-                const uint32_t d = digit_of(c[u], P);
-                const uint32_t pos = loc[d] + wcnt[w][d] + r[u];  // < tn by construction
-                if (pos < kTile) {
-                    buf[pos] = e[u];
-                    cbuf[pos] = (CidT)c[u];
+                for (int q = 0; q < kRows; ++q) {
+                    wcnt[q][tid] = at;
+                    at += x[q];
                 }
             }
         }
         __syncthreads();
-#pragma unroll 4
-        for (uint32_t q = tid; q < tn; q += THREADS) {
-            const uint32_t cq = (uint32_t)cbuf[q];
-            const uint64_t g = (uint64_t)(uint32_t)(gdel[digit_of(cq, P)] + q);  // < n by construction
-            if (g < Lay.n) {
-                ent_out[g] = buf[q];
-                if (cid_out) cid_out[g] = (CidT)cq;
+#pragma unroll
+        for (int u = 0; u < ITEMS; ++u) {
+            if (valid(u)) {
+                const uint32_t d = digit_of(c[u], P);
+                const uint32_t pos = min(wcnt[BITS < 0 ? 0 : w][d] + r[u], kTile - 1);  // < tn by construction
+                buf[pos] = e[u];
+                cbuf[pos] = (Kept)(CIDS ? c[u] : d);
             }
         }
+        if constexpr (kWhole) load_tile(t0 + kTile);
+        __syncthreads();
+        auto put = [&](uint32_t q) {
+            const uint32_t cq = (uint32_t)cbuf[q];
+            const uint64_t g = (uint64_t)(uint32_t)(gdel[CIDS ? digit_of(cq, P) : cq] + q);  // < n by construction
+            return g < Lay.n ? g : Lay.n - 1;
+        };
+        if constexpr (kWhole) {
 #pragma unroll
-        for (int u = 0; u < kSortItems; ++u) {
-            e[u] = en[u];
-            c[u] = cn[u];
+            for (int u = 0; u < ITEMS; ++u) {
+                const uint32_t q = tid + u * kSortThreads;
+                const uint64_t g = put(q);
+                ent_out[g] = buf[q];
+                if constexpr (CIDS) cid_out[g] = cbuf[q];
+            }
+        } else {
+            for (uint32_t q = tid; q < tn; q += kSortThreads) {
+                const uint64_t g = put(q);
+                ent_out[g] = buf[q];
+                if constexpr (CIDS) cid_out[g] = cbuf[q];
+            }
         }
-    }
+    };
+    uint64_t t0 = lo;
+    load_tile(t0);
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), so the loop's waits count its own operations only
+    for (; t0 + kTile <= hi; t0 += kTile) tile(t0, std::true_type{});
+    if (t0 < hi) tile(t0, std::false_type{});
 }
 
 }  // namespace
 
 // The partition's launches after the pack, which has written the chunk ids of the n entries of
-// src0 to cid[0] and the counts of the first digit (passes P[0..np)) of the G.blocks * G.sub
-// counting blocks to partial. The first pass reads src0 and writes ent[first]; each later pass reads the entry
-// buffer the previous one wrote and writes the other. Chunk ids go from cid[p & 1] to
-// cid[(p + 1) & 1], except in the last pass. start (chunks + 1 words) receives the first index of
-// every chunk. Returns the entry buffer the sorted entries end in.
-template <typename Entry, typename Src, typename CidT, int THREADS>
-hipError_t partition_passes(Src src0, int first, Entry *const ent[2], CidT *const cid[2], const PartGrid &G,
-                            const RadixPass *P, uint32_t np, uint32_t *partial, uint32_t *total, uint32_t *start,
-                            uint32_t chunks, hipStream_t st, int *out)
+// src0 to cid[0] and the counts of the first digit (passes P[0..np)) of the counting blocks of
+// G0 = part_grid<Entry, CidT, ITEMS0>(n) to partial. The first pass (ITEMS0 entries a thread and
+// tile) reads src0 and writes ent[0]; each later one (ITEMS1) reads the entry buffer the previous
+// one wrote and writes the other. Chunk ids go from cid[p & 1] to cid[(p + 1) & 1], except in the
+// last pass. start (chunks + 1 words) receives the first index of every chunk. *out is the entry
+// buffer the sorted entries end in.
+template <typename Entry, typename Src, typename CidT, int ITEMS0, int ITEMS1>
+hipError_t partition_passes(Src src0, Entry *const ent[2], CidT *const cid[2], const PartGrid &G0, const RadixPass *P,
+                            uint32_t np, uint32_t *partial, uint32_t *total, uint32_t *start, uint32_t chunks,
+                            hipStream_t st, int *out)
 {
-    int e = first;
+    int e = 0;
+    const PartGrid G1 = part_grid<Entry, CidT, ITEMS1>(G0.n);
     for (uint32_t p = 0; p < np; ++p) {
         const uint32_t R = 1u << P[p].bits;
         const bool last = p + 1 == np;
+        const PartGrid &G = p == 0 ? G0 : G1;
         if (last) {  // the chunk counts gather in start[0, chunks) (zeroed as 8-byte words)
             const hipError_t z = launch_zero(reinterpret_cast<unsigned long long *>(start), (chunks + 1) / 2, st);
             if (z != hipSuccess) return z;
@@ -488,18 +533,25 @@ hipError_t partition_passes(Src src0, int first, Entry *const ent[2], CidT *cons
             part_count_kernel<CidT><<<G.blocks * G.sub, kCountThreads, 0, st>>>(cid[p & 1], G, P[p], partial,
                                                                                  last ? start : nullptr);
         part_colscan_kernel<<<R, 256, 0, st>>>(partial, G.blocks * G.sub, R, total);
-        CidT *const cout = last ? nullptr : cid[(p + 1) & 1];
-        // the first pass ranks by atomics; the later ones stably, 8-bit digits unrolled
+        CidT *const cout = cid[(p + 1) & 1];
         const PassLayout lay{G, partial, total, G.n};
-        if (p == 0)
-            part_scatter_kernel<Entry, Src, CidT, THREADS, -1>
-                <<<G.blocks, THREADS, 0, st>>>(src0, cid[0], lay, P[p], ent[e], cout);
-        else if (P[p].bits == kMaxRadixBits)
-            part_scatter_kernel<Entry, EntrySource<Entry>, CidT, THREADS, kMaxRadixBits><<<G.blocks, THREADS, 0, st>>>(
-                EntrySource<Entry>{ent[1 - e]}, cid[p & 1], lay, P[p], ent[e], cout);
-        else
-            part_scatter_kernel<Entry, EntrySource<Entry>, CidT, THREADS, 0><<<G.blocks, THREADS, 0, st>>>(
-                EntrySource<Entry>{ent[1 - e]}, cid[p & 1], lay, P[p], ent[e], cout);
+        const EntrySource<Entry> prev{ent[1 - e]};
+        auto scatter = [&](auto src, auto items, auto bits, auto cids) {
+            part_scatter_kernel<Entry, decltype(src), CidT, decltype(items)::value, decltype(bits)::value,
+                                decltype(cids)::value>
+                <<<G.blocks, kSortThreads, 0, st>>>(src, cid[p & 1], lay, P[p], ent[e], cout);
+        };
+        auto stable = [&](auto bits) { scatter(prev, Int<ITEMS1>{}, bits, std::false_type{}); };
+        // the first pass ranks by atomics; the later ones stably, the last one's digit bits unrolled
+        if (p == 0 && last) scatter(src0, Int<ITEMS0>{}, Int<-1>{}, std::false_type{});
+        else if (p == 0) scatter(src0, Int<ITEMS0>{}, Int<-1>{}, std::true_type{});
+        else if (!last) scatter(prev, Int<ITEMS1>{}, Int<0>{}, std::true_type{});
+        else if (P[p].bits == 4) stable(Int<4>{});
+        else if (P[p].bits == 5) stable(Int<5>{});
+        else if (P[p].bits == 6) stable(Int<6>{});
+        else if (P[p].bits == 7) stable(Int<7>{});
+        else if (P[p].bits == 8) stable(Int<8>{});
+        else stable(Int<0>{});
         if (!last) e = 1 - e;
     }
     const uint32_t nseg = (chunks + kScanSeg - 1) / kScanSeg;  // <= kPartialWords: partial is free now

@@ -590,7 +590,7 @@ int bulk_insert(dyc_table *t, const uint32_t *keys, const uint32_t *vals, uint64
     // created or cleared holds zeros only
     const bool zeroed = was_zeroed && t->count == 0 && t->pend_n == 0;
     int r = 0;
-    HIP_TRY(launch_bulk_partition(t->D, Ch, keys, vals, n, bulk_space(t), kBulkSortBlocks, s, &r));
+    HIP_TRY(launch_bulk_partition(t->D, Ch, keys, vals, n, bulk_space(t), s, &r));
     uint64_t *const ovf = t->bk_ent[1 - r];  // the buffer the partition did not end in
     HIP_TRY(launch_bulk_fill(t->D, Ch, t->bk_start, t->bk_ent[r], n, ovf, t->bk_cap, t->ctr, zeroed, s));
     HIP_TRY(launch_insert_overflow(t->D, ovf, n, t->policy(), t->insert_shape(), t->ctr, sink_at(t, t->pend_n), s));

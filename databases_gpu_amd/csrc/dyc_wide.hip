@@ -1130,34 +1130,33 @@ hipError_t launch_wide_group_insert_overflow(const WideDesc *dir, const GroupIte
     return hipGetLastError();
 }
 
-// Wide entries (16 bytes): 4096-entry tiles (256 threads), two blocks per CU.
-constexpr int kWideSortThreads = 256;
-constexpr uint32_t kWideSortTile = kWideSortThreads * kSortItems;
-
-template <typename CidT>
+// Tiles of a whole CU's LDS for every batch (16 entries a thread, 12 with 4-byte chunk ids): 8 a
+// thread are no faster in small batches (2^22 entries 64 us against 61, 2^24 271 against 261) and
+// slower in large ones (2^26: 1210 against 1123).
+template <typename CidT, int ITEMS0, int ITEMS1>
 hipError_t wide_partition(const WideDesc &W, const Chunks &Ch, const uint64_t *keys, const uint64_t *vals, uint64_t n,
-                          const BulkSpace &ws, uint32_t max_blocks, hipStream_t st, int *out)
+                          const BulkSpace &ws, hipStream_t st, int *out)
 {
     RadixPass P[kMaxRadixPasses];
     const uint32_t np = radix_passes(Ch.bits, P);
-    const PartGrid G = part_grid(n, max_blocks, kWideSortTile);
+    const PartGrid G = part_grid<WideEntry, CidT, ITEMS0>(n);
     CidT *const cid[2] = {static_cast<CidT *>(ws.cid[0]), static_cast<CidT *>(ws.cid[1])};
     WideEntry *const ent[2] = {static_cast<WideEntry *>(ws.ent[0]), static_cast<WideEntry *>(ws.ent[1])};
     wide_bulk_pack_kernel<CidT><<<G.blocks * G.sub, kCountThreads, 0, st>>>(W, Ch, keys, G, P[0], cid[0], ws.partial);
-    return partition_passes<WideEntry, WideKeyValSource, CidT, kWideSortThreads>(
-        WideKeyValSource{keys, vals}, 0, ent, cid, G, P, np, ws.partial, ws.total, ws.start, Ch.total, st, out);
+    return partition_passes<WideEntry, WideKeyValSource, CidT, ITEMS0, ITEMS1>(
+        WideKeyValSource{keys, vals}, ent, cid, G, P, np, ws.partial, ws.total, ws.start, Ch.total, st, out);
 }
 
 // Group n wide entries by chunk, as launch_bulk_partition does for the 32-bit table; the sorted
 // entries end in ws.ent[*out].
 hipError_t launch_wide_partition(const WideDesc &W, const Chunks &Ch, const uint64_t *keys, const uint64_t *vals,
-                                 uint64_t n, const BulkSpace &ws, uint32_t max_blocks, hipStream_t st, int *out)
+                                 uint64_t n, const BulkSpace &ws, hipStream_t st, int *out)
 {
     *out = 0;
     if (n == 0) return hipSuccess;
     if (n >= (1ull << 32) || Ch.total == 0 || Ch.bits > kMaxRadixPasses * kMaxRadixBits) return hipErrorInvalidValue;
-    if (bulk_cid_bytes(Ch) == 2) return wide_partition<uint16_t>(W, Ch, keys, vals, n, ws, max_blocks, st, out);
-    return wide_partition<uint32_t>(W, Ch, keys, vals, n, ws, max_blocks, st, out);
+    if (bulk_cid_bytes(Ch) == 2) return wide_partition<uint16_t, 16, 16>(W, Ch, keys, vals, n, ws, st, out);
+    return wide_partition<uint32_t, 12, 12>(W, Ch, keys, vals, n, ws, st, out);
 }
 
 hipError_t launch_wide_bulk_fill(const WideDesc &W, const Chunks &Ch, const uint32_t *start, const WideEntry *ent,
@@ -1641,7 +1640,7 @@ int wbulk_insert(dyc_wide *t, const uint64_t *keys, const uint64_t *vals, uint64
     const BulkSpace ws{{t->bk_ent[0], t->bk_ent[1]}, {t->bk_cid[0], t->bk_cid[1]}, t->bk_partial,
                        t->bk_partial + kPartialWords, t->bk_start};
     int r = 0;
-    HIP_TRY(launch_wide_partition(t->W, Ch, keys, vals, n, ws, kWideSortBlocks, s, &r));
+    HIP_TRY(launch_wide_partition(t->W, Ch, keys, vals, n, ws, s, &r));
     WideEntry *const ovf = t->bk_ent[1 - r];  // the buffer the partition did not end in
     HIP_TRY(launch_wide_bulk_fill(t->W, Ch, t->bk_start, t->bk_ent[r], n, ovf, t->bk_cap, t->ctr, zeroed, s));
     HIP_TRY(launch_wide_insert_overflow(t->W, ovf, n, t->policy(), t->insert_shape(), t->ctr, t->sink_at(t->pend_n), s));
@@ -2263,8 +2262,8 @@ hipError_t wg_enqueue_bulk(dyc_wide_group *g, uint32_t NB, uint32_t J, uint32_t 
     if ((e = hipGetLastError()) != hipSuccess ||
         (e = launch_group_bulk_scan(g->ddir, g->bk_tabs, J, g->bk_partial, g->bk_chunks, s)) != hipSuccess)
         return e;
-    part_scatter_kernel<WideEntry, WideKeyValSource, uint8_t, kWideSortThreads, -1, SegLayout>
-        <<<NB, kWideSortThreads, 0, s>>>(WideKeyValSource{keys, vals}, g->bk_lcid, lay, RadixPass{0, 8}, g->bk_ent,
+    part_scatter_kernel<WideEntry, WideKeyValSource, uint8_t, 8, -1, false, SegLayout>
+        <<<NB, kSortThreads, 0, s>>>(WideKeyValSource{keys, vals}, g->bk_lcid, lay, RadixPass{0, 8}, g->bk_ent,
                                          no_cid);
     if ((e = hipGetLastError()) != hipSuccess || (e = launch_zero(g->bk_ovfn, J + 1ull, s)) != hipSuccess) return e;
     wide_group_bulk_fill_kernel<1024><<<chunks, 1024, 0, s>>>(g->bk_chunks, g->bk_ent, g->bk_ovf, g->bk_ovfn,
