@@ -122,6 +122,7 @@ struct dyc_table {
     uint8_t *live = nullptr;  // downsize: tile flags of the residual list
     uint64_t live_cap = 0;
     Reclaimer reclaim;  // frees retired subtables off the calling thread
+    dyc::host::SpareBlock spare;  // the subtable storage the last resize replaced; see there
     AsyncSlot async[kAsyncSlots];
     uint64_t async_keys = 0;  // keys of the inserts in flight
     // Subtables created together (create, load, restore) share one allocation: the GPU's address
@@ -241,18 +242,29 @@ void release_workspace(dyc_table *t)
     t->part_cap = 0;
 }
 
-// hipMalloc for a resize; when it fails, wait for the frees still queued, release the idle
-// insert workspaces (up to 20-24 B per key of the largest bulk-filled batch) and try once more.
+// Storage for a resize: the block the last one left, or hipMalloc; when that fails, wait for the
+// frees still queued, release the kept block and the idle insert workspaces (up to 20-24 B per key
+// of the largest bulk-filled batch) and try once more.
 hipError_t resize_malloc(dyc_table *t, void **p, size_t bytes, hipStream_t s)
 {
+    if ((*p = t->spare.take(bytes))) return hipSuccess;
     if (hipMalloc(p, bytes) == hipSuccess) return hipSuccess;
     (void)hipGetLastError();
+    t->reclaim.defer(t->device, t->spare.give_back());
     t->reclaim.drain();
     if (hipStreamSynchronize(s) == hipSuccess) release_workspace(t);
     (void)hipGetLastError();
     const hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) (void)hipGetLastError();
     return e;
+}
+
+// Release the storage p of nb buckets that a resize on s replaced, having waited for s.
+int retire_block(dyc_table *t, uint64_t *p, bool in_slab, uint32_t nb, hipStream_t s)
+{
+    if (in_slab) return release_block(t, p, true);
+    t->spare.retire(t->reclaim, t->device, p, (size_t)nb * kBucketBytes, s);
+    return DYC_OK;
 }
 
 int release_sub(dyc_table *t, uint32_t i)
@@ -347,8 +359,9 @@ int do_resize_up(dyc_table *t, hipStream_t s)
     HIP_TRY(launch_upsize(t->D.sub[sub], old_nb, dst, sub, t->ctr, s));
     rc = read_counters(t, s);
     if (rc) return rc;
-    rc = release_sub(t, sub);
+    rc = retire_block(t, t->D.sub[sub], t->in_slab[sub], old_nb, s);
     if (rc) return rc;
+    t->in_slab[sub] = false;
     desc_set(t->D, (int)sub, dst, old_nb * 2);
     t->st.resizes_up++;
     if (t->hctr->misplaced)
@@ -467,7 +480,7 @@ int do_resize_down(dyc_table *t, hipStream_t s)
         (void)release_block(t, old, old_in_slab);
         return rc;
     }
-    rc = release_block(t, old, old_in_slab);  // freed once the device is idle
+    rc = retire_block(t, old, old_in_slab, old_nb, s);
     if (rc) return rc;
     if (t->pend_n > pend_before) return place_pending(t, s, pend_before);
     return DYC_OK;
@@ -1019,6 +1032,7 @@ int dyc_destroy(dyc_table *t)
     (void)hipDeviceSynchronize();
     async_free(t);
     for (uint32_t i = 0; i < t->D.d; ++i) (void)release_sub(t, i);
+    t->reclaim.defer(t->device, t->spare.give_back());
     t->reclaim.drain();  // every subtable is freed when this returns
     if (t->pend) (void)hipFree(t->pend);
     if (t->ctr) (void)hipFree(t->ctr);
@@ -1278,6 +1292,7 @@ int dyc_find(dyc_table *t, const uint32_t *keys, uint32_t *vals, uint8_t *hit, u
     SETTLE(t);
     Pool sp;
     hipStream_t s = (hipStream_t)stream;
+    t->spare.found_on(s);
     HIP_TRY(t->rules.find(n, s, [&](FirstBucket rule) {
         return launch_find(t->D, keys, vals, hit, n, t->shape(), s, stash_of(t, sp), 0, rule);
     }));

@@ -1236,6 +1236,7 @@ struct dyc_wide {
     uint64_t bk_start_cap = 0;
     uint32_t *bk_partial = nullptr;  // kPartialWords, then 256 digit totals
     Reclaimer reclaim;  // frees retired subtables off the calling thread
+    dyc::host::SpareBlock spare;  // the subtable storage the last resize replaced; see there
     dyc_stats st{};
 
     uint64_t capacity() const
@@ -1307,18 +1308,29 @@ void wrelease_workspace(dyc_wide *t)
     t->bk_start_cap = 0;
 }
 
-// hipMalloc for a resize; when it fails, wait for the frees still queued, release the idle
-// bulk-fill workspace (up to 36-40 B per key of the largest bulk-filled batch) and try once more.
+// Storage for a resize: the block the last one left, or hipMalloc; when that fails, wait for the
+// frees still queued, release the kept block and the idle bulk-fill workspace (up to 36-40 B per
+// key of the largest bulk-filled batch) and try once more.
 hipError_t wresize_malloc(dyc_wide *t, uint8_t **p, size_t bytes, hipStream_t s)
 {
+    if ((*p = static_cast<uint8_t *>(t->spare.take(bytes)))) return hipSuccess;
     if (hipMalloc(p, bytes) == hipSuccess) return hipSuccess;
     (void)hipGetLastError();
+    t->reclaim.defer(t->device, t->spare.give_back());
     t->reclaim.drain();
     if (hipStreamSynchronize(s) == hipSuccess) wrelease_workspace(t);
     (void)hipGetLastError();
     const hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) (void)hipGetLastError();
     return e;
+}
+
+// Release the storage of nb buckets that a resize on s replaced, having waited for s.
+int wretire_block(dyc_wide *t, uint8_t *own, uint32_t nb, hipStream_t s)
+{
+    if (!own) return wrelease_block(t, nullptr);
+    t->spare.retire(t->reclaim, t->device, own, 2 * wide_bytes(nb), s);
+    return DYC_OK;
 }
 
 int wrelease(dyc_wide *t, uint32_t i)
@@ -1417,7 +1429,7 @@ int wresize_up(dyc_wide *t, hipStream_t s)
                                reinterpret_cast<uint64_t *>(dst + wide_bytes(old_nb * 2)), sub, t->ctr, s));
     rc = wread(t, s);
     if (rc) return rc;
-    rc = wrelease(t, sub);
+    rc = wretire_block(t, t->own[sub], old_nb, s);
     if (rc) return rc;
     wset(t, sub, dst, old_nb * 2);
     t->own[sub] = dst;
@@ -1538,7 +1550,7 @@ int wresize_down(dyc_wide *t, hipStream_t s)
         (void)wrelease_block(t, old_own);
         return rc;
     }
-    rc = wrelease_block(t, old_own);  // freed once the device is idle
+    rc = wretire_block(t, old_own, old_nb, s);
     if (rc) return rc;
     if (t->pend_n > pend_before) return wplace_pending(t, s, pend_before);
     return DYC_OK;
@@ -1710,6 +1722,7 @@ int dyc_wide_destroy(dyc_wide *t)
     DeviceGuard dg(t->device);
     (void)hipDeviceSynchronize();
     for (uint32_t i = 0; i < t->W.D.d; ++i) (void)wrelease(t, i);
+    t->reclaim.defer(t->device, t->spare.give_back());
     t->reclaim.drain();  // every subtable is freed when this returns
     if (t->pk) (void)hipFree(t->pk);
     if (t->pv) (void)hipFree(t->pv);
@@ -1846,6 +1859,7 @@ int dyc_wide_find(dyc_wide *t, const uint64_t *keys, uint64_t *vals, uint8_t *hi
     if (n && !keys) return fail(DYC_ERR_INVALID, "null keys");
     DeviceGuard dg(t->device);
     hipStream_t s = (hipStream_t)stream;
+    t->spare.found_on(s);
     HIP_TRY(t->rules.find(n, s, [&](FirstBucket rule) {
         return launch_wide_probe(t->W, keys, vals, hit, n, false, t->shape(), t->ctr, t->stash(), s, rule);
     }));

@@ -199,7 +199,9 @@ int dyc_find(dyc_table *t, const uint32_t *keys, uint32_t *vals, uint8_t *hit, u
 int dyc_erase(dyc_table *t, const uint32_t *keys, uint8_t *deleted, uint64_t n, dyc_stream stream);
 
 /* Replaces hashAPI::resize_up (api.cpp:112-141) + GPU_cuckoo_resize_up (cuckoo.cu:731-758):
- * doubles the subtable chosen by api.cpp:116-122. Synchronous. */
+ * doubles the subtable chosen by api.cpp:116-122. Synchronous. A table keeps the storage that its
+ * last resize replaced for its next one (at most 256 MiB, and 1 GiB over all tables of the process)
+ * as long as its finds run on the resizes' stream; dyc_destroy frees it. */
 int dyc_resize_up(dyc_table *t, dyc_stream stream);
 
 /* Replaces hashAPI::resize_low (api.cpp:143-173) + GPU_cuckoo_resize_down (cuckoo.cu:762-788):
