@@ -171,7 +171,7 @@ struct Desc {
     uint32_t np;                   // pairs: d (d - 1) / 2, and 2 for d = 2
     uint32_t pm, psh;              // FastDiv of np (multiplier, s1 | s2 << 8)
     uint64_t p1, p2;               // pos1 / pos2 of pair p in bits [4p, 4p + 4)
-    uint32_t fr;                   // bulk fill, first round: bits [2p, 2p + 2) say where pair p's
+    uint32_t fr;                   // bulk fill: bits [2p, 2p + 2) say where pair p's
                                    // keys go (fill_target); 0 (the start rule) if never set
 };
 
@@ -335,7 +335,7 @@ inline bool pair_scheme(uint32_t d, uint32_t &np, uint64_t &p1, uint64_t &p2)
     return true;
 }
 
-// The bucket the bulk fill's first round sends key k of pair p to. The eviction insert starts a
+// The bucket the bulk fill sends key k of pair p to. The eviction insert starts a
 // key by the reference's start rule (odd keys in pos2, even ones in pos1, cuckoo.cu:336-341),
 // which gives every subtable the same share of the keys but puts only half of them in pos1, the
 // bucket a find reads first. Where the fill puts a key is its own choice: per pair, Desc::fr

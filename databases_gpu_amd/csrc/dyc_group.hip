@@ -879,7 +879,7 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
         if (k == hipSuccess) k = launch_zero(g->tcounts, g->n, cs);
         const PendSink sink{g->pend, g->pend_tag, g->pend_cap, 0, 0, nullptr};
         if (k == hipSuccess && p->bulk) {
-            // the graph clears every table first, so round 1 need not read them
+            // the graph clears every table first, so the fill need not read them
             const BulkArrays A{p->bk_blk, p->bk_tabs, (uint32_t)L.blocks.size(), p->bk_j, L.chunks};
             k = enqueue_group_bulk(g, A, keys, vals, p->total, true, sink, cs);
         } else if (k == hipSuccess) {

@@ -236,9 +236,9 @@ struct WideDesc {
     Desc D;                        // key arrays (D.sub), geometry and pair scheme
     uint64_t *val[kMaxSubtables];  // value arrays, slot for slot parallel to the key arrays
 };
-// One chunk of a group fill round with all that its workgroup reads before the entries, so the
+// One chunk of a group fill with all that its workgroup reads before the entries, so the
 // workgroup starts from a single load: a chain of chunk -> table -> directory loads, each
-// waiting behind the round's store traffic, kept the workgroups of a whole round idle for about
+// waiting behind the fill's store traffic, kept its workgroups idle for about
 // half their lifetime. Written by the scan.
 struct alignas(16) GroupChunk {
     SubRef S;          // the chunk's subtable

@@ -39,7 +39,7 @@ constexpr uint32_t kMaxSortBlocks = 2048;  // colscan gives each of its 256 thre
 static_assert(kPartialWords == (uint64_t)kMaxSortBlocks * kMaxRadix, "BulkSpace::partial holds every block's counts");
 static_assert(kMaxRadixWords == kMaxRadix, "BulkSpace::total holds every digit's total");
 // The counting launches (pack, count) stream their block's range with more waves per block
-// than the scatter, whose LDS limits it to one or two blocks per CU.
+// than the scatter, whose LDS limits it to one to three blocks per CU.
 constexpr int kCountThreads = 512;
 constexpr int kCountItems = 8;
 // Values of the bits below the last digit that one block of the last count bins in LDS; a

@@ -681,9 +681,9 @@ constexpr uint64_t kWideInsertBlocks = 16384;
 
 // ------------------------------------------------------------ bulk fill (insert_order 3)
 // The narrow table's bulk fill (dyc_bulk.hip) over fold(k): (chunk id, entry) pairs sorted by
-// chunk, one workgroup per chunk filling free slots, a second round in the other bucket, the
-// eviction insert for the rest. The dense round keeps the chunk's key lines and value lines in
-// LDS (2 x 64 KB), so one 1024-thread workgroup runs per CU.
+// chunk, one workgroup per chunk filling free slots, the eviction insert of the overflow into the
+// other buckets. The fill keeps the chunk's key lines and value lines in LDS (2 x 64 KB), so one
+// 1024-thread workgroup runs per CU.
 // Chunk ids of the batch in input order and each block's counts of the partition's first digit
 // (dyc_part.hpp), over fold(k), of the fill_target bucket (reserved keys go to chunk 0, whose fill
 // rejects them).

@@ -65,7 +65,8 @@ typedef struct dyc_config {
     uint32_t auto_resize;      /* 1: apply the fill bounds in dyc_insert / dyc_erase (default 0) */
     uint32_t find_lanes;       /* 4, 8 or 16 (default 8); checked, but every probe reads a bucket with
                                   four lanes, the fastest at every size */
-    uint32_t insert_lanes;     /* lanes per key for insert: 1, 2, 4, 8 or 16 (default 1) */
+    uint32_t insert_lanes;     /* 1, 2, 4, 8 or 16 (default 1); checked, but every insert carries an
+                                  entry with one lane, four of which read a bucket together */
     uint32_t block_threads;    /* threads per block, multiple of 64, <= 256 (default 256) */
     uint32_t max_blocks;       /* grid cap for find/erase, 0 = one wave per 64 keys up to 2^20 blocks */
     uint32_t insert_blocks;    /* grid of the insert kernel, 0 = default (65536 blocks) */
@@ -287,7 +288,7 @@ typedef struct dyc_group dyc_group;   /* opaque */
 /* Launch shape of a group's kernels; dyc_group_tune() picks these by measurement. */
 typedef struct dyc_group_launch {
     uint32_t find_lanes;     /* 4, 8 or 16 (checked; probes use four lanes a bucket) */
-    uint32_t insert_lanes;   /* 1, 2, 4, 8 or 16 */
+    uint32_t insert_lanes;   /* 1, 2, 4, 8 or 16 (checked; inserts use one lane an entry) */
     uint32_t find_blocks;    /* persistent grid for find/erase (0 = default) */
     uint32_t insert_blocks;  /* persistent grid for insert (0 = default) */
     uint32_t item_keys;      /* keys per work item (0 = default 4096) */
