@@ -545,13 +545,15 @@ hipError_t partition_passes(Src src0, Entry *const ent[2], CidT *const cid[2], c
         // the first pass ranks by atomics; the later ones stably, the last one's digit bits unrolled
         if (p == 0 && last) scatter(src0, Int<ITEMS0>{}, Int<-1>{}, std::false_type{});
         else if (p == 0) scatter(src0, Int<ITEMS0>{}, Int<-1>{}, std::true_type{});
-        else if (!last) scatter(prev, Int<ITEMS1>{}, Int<0>{}, std::true_type{});
-        else if (P[p].bits == 4) stable(Int<4>{});
+        else if (!last) {
+            if constexpr (sizeof(CidT) > 2) scatter(prev, Int<ITEMS1>{}, Int<0>{}, std::true_type{});
+            else return hipErrorInvalidValue;  // 2-byte chunk ids take at most two passes
+        } else if (P[p].bits == 4) stable(Int<4>{});
         else if (P[p].bits == 5) stable(Int<5>{});
         else if (P[p].bits == 6) stable(Int<6>{});
         else if (P[p].bits == 7) stable(Int<7>{});
         else if (P[p].bits == 8) stable(Int<8>{});
-        else stable(Int<0>{});
+        else return hipErrorInvalidValue;  // digits are spread evenly: 9 or more bits leave 4 to the last
         if (!last) e = 1 - e;
     }
     const uint32_t nseg = (chunks + kScanSeg - 1) / kScanSeg;  // <= kPartialWords: partial is free now
