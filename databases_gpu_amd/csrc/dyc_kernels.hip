@@ -242,7 +242,7 @@ __device__ inline uint32_t probe_tile(const Desc &D, const uint32_t *__restrict_
 // The find of a table that keeps a first-bucket rule (FirstBucket): a stored key is in its first
 // bucket, or that bucket had no free slot when the key went elsewhere and none since. So a first
 // bucket with a free slot answers alone, hit or miss, and a lookup reads fewer buckets: at fill 0.9
-// and 50 % hits 1.35 of them (1.68 in the reference order) over a bulk-filled table. The answer
+// and 50 % hits 1.40 of them (1.68 in the reference order) over a bulk-filled table. The answer
 // is the reference order's: a key whose first bucket is pos2 and full may have a copy in pos1,
 // which then counts. 2^28 uniform lookups 10.2 -> 8.65 ms, Zipf
 // 4.65 -> 4.28 ms.
