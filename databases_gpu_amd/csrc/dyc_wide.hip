@@ -134,7 +134,8 @@ __device__ inline uint32_t keys_slot(const WideKeys &e, uint64_t k, uint32_t s)
 // neither bucket holds are then looked up in the stash (erase and update act on every copy
 // there). Update: keys of one launch are distinct, so no two lanes write one value; the key word
 // is untouched, and the value is an agent-scope atomic store. rule (find): the first-bucket rule the
-// table keeps, which the find may rely on as the narrow table's does (find_tile_first).
+// table keeps, which the find may rely on as the narrow table's does (find_tile_first), with
+// nontemporal keys and results as there (2^26 keys and lookups 5.67 -> 5.59 ms in all).
 template <int MODE, bool FIRST = false>
 __device__ inline uint32_t wide_probe_tile(const WideDesc &W, const uint64_t *__restrict__ keys,
                                            uint64_t *__restrict__ vals, uint8_t *__restrict__ flags, uint64_t base,
@@ -145,7 +146,7 @@ __device__ inline uint32_t wide_probe_tile(const WideDesc &W, const uint64_t *__
     const uint32_t lane = __lane_id(), s = lane & 3u;
     const uint64_t i = base + lane;
     const bool inb = i < n;
-    const uint64_t k = inb ? keys[i] : 0ull;
+    const uint64_t k = !inb ? 0ull : FIRST ? __builtin_nontemporal_load(keys + i) : keys[i];
     const uint64_t nv = (UPDATE && inb) ? vals[i] : 0ull;  // update: the new value
     const uint32_t f = fold64(k);
     const uint32_t p = pair_of(W.D, f), ta = pos1(W.D, p), tb = pos2(W.D, p);
@@ -270,8 +271,13 @@ __device__ inline uint32_t wide_probe_tile(const WideDesc &W, const uint64_t *__
         }
     }
     if (inb) {
-        if (MODE == 0 && vals) vals[i] = my_val;
-        if (flags) flags[i] = (uint8_t)my_flag;
+        if constexpr (FIRST) {
+            if (vals) __builtin_nontemporal_store(my_val, vals + i);
+            if (flags) __builtin_nontemporal_store((uint8_t)my_flag, flags + i);
+        } else {
+            if (MODE == 0 && vals) vals[i] = my_val;
+            if (flags) flags[i] = (uint8_t)my_flag;
+        }
     }
     return my_flag;
 }
