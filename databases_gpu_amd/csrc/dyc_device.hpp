@@ -117,6 +117,24 @@ __host__ __device__ inline uint32_t nth_set_bit16(uint32_t m, uint32_t r)
     return pos + (r >= (m & 1u) ? 1u : 0u);
 }
 
+// Where an insert's chain puts its entry in the bucket it has come to, from the mask of the slots
+// that its (possibly old) view of the bucket shows empty. Finds may rely on a key's first bucket having
+// no free slot if the key is elsewhere, so a chain may take a bucket for full only when it knows of
+// every slot that it is taken: its view showed an entry there, or its own CAS found one (lost). Slots
+// that were merely passed over, for a lane of higher rank in a crowded table, stay open to it.
+struct BucketTries {
+    uint32_t lost = 0;  // slots of the bucket where another entry was found by a CAS
+    __host__ __device__ uint32_t open(uint32_t view) const { return view & ~lost; }
+    // The slot the r-th of the lanes that want this bucket aims at; 16 if none is open.
+    __host__ __device__ static uint32_t aim(uint32_t open, uint32_t r)
+    {
+        const uint32_t left = (uint32_t)__builtin_popcount(open);
+        if (r && left > 1u) return nth_set_bit16(open, r < left ? r : r % left);
+        return (uint32_t)__builtin_ctz(open | 0x10000u);
+    }
+    __host__ __device__ void lose(uint32_t slot) { lost |= 1u << slot; }
+};
+
 // ------------------------------------------------------------------ division by a runtime d
 // n % d for the per-subtable bucket count d without a hardware divide: Granlund & Montgomery,
 // "Division by Invariant Integers using Multiplication" (PLDI 1994), Fig. 4.1 (round-up

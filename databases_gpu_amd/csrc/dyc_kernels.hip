@@ -358,7 +358,7 @@ __global__ __launch_bounds__(256) void find_first_kernel(Desc D, FirstBucket rul
 // registers.
 // The buckets are read with plain vector loads. The view may be stale (another XCD's L2 may hold
 // a newer line), but no entry is lost or doubled by it: an empty slot is taken by CAS, and a slot
-// lost to another entry is not tried again (Hand::from; the bucket is read again, and the view
+// lost to another entry is not tried again (BucketTries; the bucket is read again, and the view
 // may still show the slot empty), so a bucket costs at most 16 lost races and an entry at most
 // max_retries before it is pended; a victim is exchanged, which cannot fail.
 //
@@ -371,7 +371,7 @@ struct Hand {
     uint32_t k, v;
     uint64_t idx;  // input index of the key that started the chain
     uint32_t pre, kicks, retries;
-    uint32_t from;  // the first slot of the current bucket still worth a CAS
+    BucketTries tries;  // in the current bucket
     bool fresh;     // not placed or carried yet: its other bucket is still to be tried
     bool active;
 };
@@ -431,8 +431,10 @@ __device__ inline uint32_t vote_slot(const Desc &D, const uint32_t (&k4)[4], uin
 // instructions for little (64 over 1024: 4 lanes).
 constexpr uint32_t kCrowdedBuckets = 1024;
 
-// A number that tells the buckets of a crowded table apart (12 bits; two buckets of one number only
-// make a lane skip an empty slot).
+// A number that tells the buckets of a crowded table apart (12 bits). Lanes of two buckets that share a
+// number are ranked together and may pass over an empty slot, which stays open to them. (The first
+// subtable stands for all in the choice of crowded tables. Resizes keep subtables within a factor of
+// two; loaded images need not, and then more buckets share a number.)
 __device__ inline uint32_t bucket_id(const Desc &D, uint64_t at, uint32_t t)
 {
     const uint64_t base = (uint64_t)selt(t, D.sub);
@@ -480,15 +482,13 @@ __device__ inline void insert_step(const Desc &D, Hand &h, const InsertPolicy &P
     const bool odd = s & 1u, high = s & 2u;
     const uint32_t c01 = (odd ? c[1] : c[0]) | quad_swap<1>(odd ? c[0] : c[1]);
     const uint32_t c23 = (odd ? c[3] : c[2]) | quad_swap<1>(odd ? c[2] : c[3]);
-    const uint32_t open = ((high ? c23 : c01) | quad_swap<2>(high ? c01 : c23)) & (0xffffu << h.from);
+    const uint32_t open = h.tries.open((high ? c23 : c01) | quad_swap<2>(high ? c01 : c23));
     const bool full = open == 0u;
-    uint32_t slot = (uint32_t)__builtin_ctz(open | 0x10000u);
+    uint32_t slot = BucketTries::aim(open, 0u);
     if (D.nb[0] * D.d <= kCrowdedBuckets) {
         // a table of few buckets: several lanes of the wave want the same bucket's first empty slot,
         // and all but one would lose it; the r-th of them takes the r-th empty slot
-        const uint32_t r = rank_among_equals(act, bucket_id(D, at, t));
-        const uint32_t left = (uint32_t)__builtin_popcount(open);
-        if (r && left > 1u) slot = nth_set_bit16(open, r < left ? r : r % left);
+        slot = BucketTries::aim(open, rank_among_equals(act, bucket_id(D, at, t)));
     }
     const bool place = h.active && !full;
     const bool swing = h.active && full && h.fresh && P.kick_bound == 0;
@@ -530,20 +530,20 @@ __device__ inline void insert_step(const Desc &D, Hand &h, const InsertPolicy &P
             h.v = val_of(out);
             h.pre = t;
             h.fresh = false;
-            h.from = 0;
+            h.tries = {};
             if (h.kicks >= P.kick_bound + P.rescue_kicks) give_up(h, C, sink, tag, tally);
         }
     }
     if (swing) {  // its other bucket next, with nothing exchanged
         h.pre = t;
         h.fresh = false;
-        h.from = 0;
+        h.tries = {};
     }
     const uint64_t losers = __ballot(lost);
     if (losers) {
         tally.retries += __popcll(losers);
         if (lost) {
-            h.from = slot + 1u;
+            h.tries.lose(slot);
             if (++h.retries > P.max_retries) give_up(h, C, sink, tag, tally);
         }
     }
@@ -640,7 +640,8 @@ struct InsertRange {
                     h.pre = pre_fixed == kAfterFill ? fill_target(D, k, pair_of(D, k)) : pre_fixed;
                     h.fresh = pre_fixed == kNoTable;
                     if (h.fresh && (k & 1u)) h.pre = kOddStart;
-                    h.kicks = h.retries = h.from = 0;
+                    h.kicks = h.retries = 0;
+                    h.tries = {};
                     h.active = true;
                 }
                 pos += take;

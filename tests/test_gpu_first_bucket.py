@@ -235,3 +235,27 @@ def test_plan_relies_on_its_own_fill(D):
             assert torch.equal(p.out_vals, torch.where(miss, torch.zeros_like(k), k ^ 7))
             g.erase(k, off)  # eager work between the replays
         g.close()
+
+
+@pytest.mark.parametrize("d", [2, 4])
+@pytest.mark.parametrize("kick_bound", [0, 15])
+def test_small_tables_looked_up_in_large_calls(D, kick_bound, d):
+    """Tables of at most 1024 buckets, whose inserts spread a wave's lanes over a bucket's empty slots:
+    each stored key is found by a find that stops at a first bucket with a free slot. The large
+    tables bring the group's mean to where its finds rely on the rule."""
+    from databases_gpu_amd.table import DyCuckooGroup
+
+    print(f"\n[gpu-case] first-bucket rule, small tables d={d} kick_bound={kick_bound}", flush=True)
+    sizes = np.concatenate([np.random.default_rng(d).integers(20, 3000, size=40), [1 << 21, (1 << 21) + 5, 1 << 21]])
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint64)
+    n = int(off[-1])
+    assert n > LARGE
+    g = DyCuckooGroup((sizes / (0.75 if d == 2 else 0.85)).astype(np.uint64) + 32, subtables=d, insert_order=0,
+                      kick_bound=kick_bound)
+    for seed in range(5):
+        k = keys(0, n, 11 + seed)
+        g.clear()
+        g.insert(k, k ^ seed, off)
+        v, h = g.find(k, off)
+        assert bool(h.all()) and torch.equal(v, k ^ seed)
+    g.close()
