@@ -924,9 +924,10 @@ int dyc_group_plan_run(dyc_group_plan *p, dyc_stream stream)
     g->zeroed = false;
     g->st.last_filled = 0;
     // the graph clears every table and fills it under one rule, which its own find relies on
-    g->rules.emptied_then(p->bulk ? FirstBucket::kFill : FirstBucket::kStart);
-    HIP_TRY(hipGraphLaunch(p->exec, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HIP_TRY(g->rules.refill(p->bulk ? FirstBucket::kFill : FirstBucket::kStart, [&] {
+        const hipError_t e = hipGraphLaunch(p->exec, s);
+        return e == hipSuccess ? hipStreamSynchronize(s) : e;
+    }));
     fold_tallies(g->hctr);
     // the step cleared every table: counts and the pending list start again from zero
     std::fill(g->count.begin(), g->count.end(), 0);

@@ -16,6 +16,7 @@
 
 #include "dyc.h"
 #include "dyc_device.hpp"
+#include "dyc_inflight.hpp"
 #include "dyc_kernels.hpp"
 #include "dyc_threads.hpp"
 
@@ -59,105 +60,31 @@ inline hipError_t await_post(const volatile unsigned long long *post, unsigned l
     return hipSuccess;
 }
 
-// Which first-bucket rules (FirstBucket) the entries of a table, or of a group's tables, keep, and
-// the finds in flight that rely on one. An empty table keeps both; an insert keeps its own; an
-// erase, which frees slots, keeps none. A find that relies on a rule marks its stream, and the erase
-// that drops the rule waits on its own stream for the marks, so it frees no slot under such a
-// find on another stream. Finds of fewer than kFirstBucketKeys keys read in the reference order
-// (the mark would cost them more than they save), as do finds being captured, which may be
-// replayed after an erase, finds on the per-thread stream (one handle for many streams), and those on
-// more than kMarks streams since the last erase or clear.
-constexpr uint64_t kFirstBucketKeys = 1ull << 22;
-class FirstBucketRules {
-  public:
-    FirstBucketRules() = default;
-    FirstBucketRules(const FirstBucketRules &) = delete;
-    FirstBucketRules &operator=(const FirstBucketRules &) = delete;
-    ~FirstBucketRules()
+// The HIP calls of the host state in dyc_inflight.hpp.
+struct HipRuntime {
+    using Stream = hipStream_t;
+    using Event = hipEvent_t;
+    using Error = hipError_t;
+    static constexpr Error kOk = hipSuccess;
+    static bool shared(Stream s) { return s == hipStreamPerThread; }
+    static bool capturing(Stream s)  // or it cannot be told
     {
-        for (Mark &m : marks_)
-            if (m.done) (void)hipEventDestroy(m.done);
-    }
-    // Cleared, or cleared and then filled under one rule. (A find still in flight would race with
-    // the clear itself, so there is nothing left to wait for.)
-    void emptied() { restart(kStartBit | kFillBit); }
-    void emptied_then(FirstBucket rule) { restart(bit(rule)); }
-    void filled(FirstBucket rule) { keep(bit(rule)); }  // entries are about to be stored under `rule`
-    void lost() { keep(0); }                            // resized or loaded
-    // Slots are about to be freed on s.
-    hipError_t freeing(hipStream_t s)
-    {
-        std::lock_guard<std::mutex> lk(mu_);
-        rules_ = 0;
-        for (Mark &m : marks_) {
-            if (!m.live) continue;
-            m.live = false;
-            if (m.stream == s) continue;
-            const hipError_t e = hipStreamWaitEvent(s, m.done, 0);
-            if (e != hipSuccess) return e;
-        }
-        return hipSuccess;
-    }
-    // Launch a find of n keys on s: launch(rule) with the rule it may rely on.
-    template <typename Launch>
-    hipError_t find(uint64_t n, hipStream_t s, Launch launch)
-    {
-        if (n < kFirstBucketKeys || s == hipStreamPerThread) return launch(FirstBucket::kNone);
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-            (void)hipGetLastError();
-            return launch(FirstBucket::kNone);
-        }
-        std::lock_guard<std::mutex> lk(mu_);
-        Mark *m = rules_ ? mark_for(s) : nullptr;
-        if (!m) return launch(FirstBucket::kNone);
-        hipError_t e = launch(rules_ & kFillBit ? FirstBucket::kFill : FirstBucket::kStart);
-        if (e == hipSuccess) e = hipEventRecord(m->done, s);
-        m->live = true;
-        return e;
+        const bool told = hipStreamIsCapturing(s, &cap) == hipSuccess;
+        if (!told) (void)hipGetLastError();
+        return !told || cap != hipStreamCaptureStatusNone;
     }
-
-  private:
-    static constexpr uint32_t kStartBit = 1u, kFillBit = 2u;
-    static constexpr int kMarks = 8;
-    struct Mark {
-        hipStream_t stream = nullptr;
-        hipEvent_t done = nullptr;
-        bool live = false;  // a find after the last erase relies on a rule
-    };
-    static uint32_t bit(FirstBucket r) { return r == FirstBucket::kFill ? kFillBit : (r == FirstBucket::kStart ? kStartBit : 0u); }
-    void keep(uint32_t bits)
+    static bool make(Event *e)
     {
-        std::lock_guard<std::mutex> lk(mu_);
-        rules_ &= bits;
+        if (hipEventCreateWithFlags(e, hipEventDisableTiming) == hipSuccess) return true;
+        (void)hipGetLastError();
+        return false;
     }
-    void restart(uint32_t bits)
-    {
-        std::lock_guard<std::mutex> lk(mu_);
-        rules_ = bits;
-        for (Mark &m : marks_) m.live = false;
-    }
-    // The mark of stream s: its own, or a free one; nullptr if there is none.
-    Mark *mark_for(hipStream_t s)
-    {
-        for (Mark &m : marks_)
-            if (m.live && m.stream == s) return &m;
-        for (Mark &m : marks_) {
-            if (m.live) continue;
-            if (!m.done && hipEventCreateWithFlags(&m.done, hipEventDisableTiming) != hipSuccess) {
-                (void)hipGetLastError();
-                m.done = nullptr;
-                return nullptr;
-            }
-            m.stream = s;
-            return &m;
-        }
-        return nullptr;
-    }
-    std::mutex mu_;
-    uint32_t rules_ = 0;
-    Mark marks_[kMarks];
+    static void drop(Event e) { (void)hipEventDestroy(e); }
+    static Error record(Event e, Stream s) { return hipEventRecord(e, s); }
+    static Error wait(Stream s, Event e) { return hipStreamWaitEvent(s, e, 0); }
 };
+using FirstBucketRules = FirstBucketRulesT<HipRuntime>;
 
 // Buckets per subtable of a d-subtable table for a slot-count hint (api.cpp:47-56, which
 // divides by TABLE_NUM * BUCKET_SIZE).

@@ -1,0 +1,129 @@
+// dyc_inflight.hpp -- host state about the device work a table may still have in flight, over the few
+// runtime calls it needs (Runtime), so that a host-only build can run it with a stand-in.
+#pragma once
+
+#include <stdint.h>
+
+#include <mutex>
+
+namespace dyc {
+
+// The bucket of its pair that every stored key was first put to, where a table still keeps the rule:
+// a key is elsewhere only if that bucket had no free slot then, and none has become free since (no
+// erase, resize or load). kStart: the start rule of the eviction insert (odd keys pos2), kFill: the
+// bulk fill's fill_target.
+enum class FirstBucket : uint32_t { kNone = 0, kStart = 1, kFill = 2 };
+
+namespace host {
+
+// Which first-bucket rules (FirstBucket) the entries of a table, or of a group's tables, keep, and
+// the finds in flight that rely on one. An empty table keeps both; an insert keeps its own; an
+// erase, which frees slots, keeps none. A find that relies on a rule marks its stream, and the erase
+// that drops the rule waits on its own stream for the marks, so it frees no slot under such a
+// find on another stream. Finds of fewer than kFirstBucketKeys keys read in the reference order
+// (the mark would cost them more than they save), as do finds being captured, which may be
+// replayed after an erase, finds on the per-thread stream (one handle for many streams), and those on
+// more than kMarks streams since the last erase or clear.
+constexpr uint64_t kFirstBucketKeys = 1ull << 22;
+template <typename Runtime>
+class FirstBucketRulesT {
+    using Stream = typename Runtime::Stream;
+    using Event = typename Runtime::Event;
+    using Error = typename Runtime::Error;
+
+  public:
+    FirstBucketRulesT() = default;
+    FirstBucketRulesT(const FirstBucketRulesT &) = delete;
+    FirstBucketRulesT &operator=(const FirstBucketRulesT &) = delete;
+    ~FirstBucketRulesT()
+    {
+        for (Mark &m : marks_)
+            if (m.made) Runtime::drop(m.done);
+    }
+    // Cleared. (A find still in flight would race with the clear itself, so there is nothing left to
+    // wait for.)
+    void emptied() { restart(kStartBit | kFillBit); }
+    // launch() clears the table and fills it under `rule`, and has waited for that when it returns. If
+    // it fails, the table may still hold what it held before: no rule then.
+    template <typename Launch>
+    Error refill(FirstBucket rule, Launch launch)
+    {
+        lost();
+        const Error e = launch();
+        if (e == Runtime::kOk) restart(bit(rule));
+        return e;
+    }
+    void filled(FirstBucket rule) { keep(bit(rule)); }  // entries are about to be stored under `rule`
+    void lost() { keep(0); }                            // resized or loaded
+    // Slots are about to be freed on s.
+    Error freeing(Stream s)
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        rules_ = 0;
+        for (Mark &m : marks_) {
+            if (!m.live) continue;
+            m.live = false;
+            if (m.stream == s) continue;
+            const Error e = Runtime::wait(s, m.done);
+            if (e != Runtime::kOk) return e;
+        }
+        return Runtime::kOk;
+    }
+    // Launch a find of n keys on s: launch(rule) with the rule it may rely on.
+    template <typename Launch>
+    Error find(uint64_t n, Stream s, Launch launch)
+    {
+        if (n < kFirstBucketKeys || Runtime::shared(s) || Runtime::capturing(s)) return launch(FirstBucket::kNone);
+        std::lock_guard<std::mutex> lk(mu_);
+        Mark *m = rules_ ? mark_for(s) : nullptr;
+        if (!m) return launch(FirstBucket::kNone);
+        Error e = launch(rules_ & kFillBit ? FirstBucket::kFill : FirstBucket::kStart);
+        if (e == Runtime::kOk) e = Runtime::record(m->done, s);
+        m->live = true;
+        return e;
+    }
+
+  private:
+    static constexpr uint32_t kStartBit = 1u, kFillBit = 2u;
+    static constexpr int kMarks = 8;
+    struct Mark {
+        Stream stream{};
+        Event done{};
+        bool made = false;  // done exists
+        bool live = false;  // a find after the last erase relies on a rule
+    };
+    static uint32_t bit(FirstBucket r)
+    {
+        return r == FirstBucket::kFill ? kFillBit : (r == FirstBucket::kStart ? kStartBit : 0u);
+    }
+    void keep(uint32_t bits)
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        rules_ &= bits;
+    }
+    void restart(uint32_t bits)
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        rules_ = bits;
+        for (Mark &m : marks_) m.live = false;
+    }
+    // The mark of stream s: its own, or a free one; nullptr if there is none.
+    Mark *mark_for(Stream s)
+    {
+        for (Mark &m : marks_)
+            if (m.live && m.stream == s) return &m;
+        for (Mark &m : marks_) {
+            if (m.live) continue;
+            if (!m.made && !(m.made = Runtime::make(&m.done))) return nullptr;
+            m.stream = s;
+            return &m;
+        }
+        return nullptr;
+    }
+    std::mutex mu_;
+    uint32_t rules_ = 0;
+    Mark marks_[kMarks];
+};
+
+}  // namespace host
+}  // namespace dyc

@@ -4,6 +4,7 @@
 #include <stddef.h>
 
 #include "dyc_device.hpp"
+#include "dyc_inflight.hpp"
 
 namespace dyc {
 
@@ -80,12 +81,6 @@ struct InsertPolicy {
 };
 
 struct Pool;
-// The bucket of its pair that every stored key was first put to, where a table still keeps the rule:
-// a key is elsewhere only if that bucket had no free slot then, and none has become free since (no
-// erase, resize or load). kStart: the start rule of the eviction insert (odd keys pos2), kFill: the
-// bulk fill's fill_target.
-enum class FirstBucket : uint32_t { kNone = 0, kStart = 1, kFill = 2 };
-
 // find: vals/hit may be null. pool (optional): misses also look in the pool's entries of `table`.
 // rule: what the table keeps (kNone reads in the reference order).
 hipError_t launch_find(const Desc &D, const uint32_t *keys, uint32_t *vals, uint8_t *hit, uint64_t n, LaunchShape sh,

@@ -1,0 +1,149 @@
+// Host check of dyc_inflight.hpp over a stand-in for the runtime: streams are sets of the work ordered
+// before what is next enqueued on them, events copy such a set. Prints "inflight ok".
+#include <cstdio>
+#include <cstdlib>
+#include <map>
+#include <set>
+
+#include "dyc_inflight.hpp"
+
+namespace {
+
+using Work = std::set<int>;
+struct Fake {
+    using Stream = int;  // a handle; 0 is the null stream
+    using Event = int;
+    using Error = int;
+    static constexpr Error kOk = 0;
+    static std::map<int, Work> streams, events;
+    static std::set<int> captured;
+    static int made, next;
+    static bool shared(Stream s) { return s == -1; }
+    static bool capturing(Stream s) { return captured.count(s) != 0; }
+    static bool make(Event *e)
+    {
+        *e = ++made;
+        return true;
+    }
+    static void drop(Event e) { events.erase(e); }
+    static Error record(Event e, Stream s)
+    {
+        events[e] = streams[s];
+        return kOk;
+    }
+    static Error wait(Stream s, Event e)
+    {
+        streams[s].insert(events[e].begin(), events[e].end());
+        return kOk;
+    }
+    // enqueue a piece of work on s
+    static int run(Stream s)
+    {
+        streams[s].insert(++next);
+        return next;
+    }
+    static bool before(int work, Stream s) { return streams[s].count(work) != 0; }
+    // the stream of this handle is destroyed and a new one gets the handle; its work may go on
+    static void reuse(Stream s) { streams[s].clear(); }
+};
+std::map<int, Work> Fake::streams, Fake::events;
+std::set<int> Fake::captured;
+int Fake::made = 0, Fake::next = 0;
+
+using dyc::FirstBucket;
+using Rules = dyc::host::FirstBucketRulesT<Fake>;
+constexpr uint64_t kMany = dyc::host::kFirstBucketKeys;
+
+int g_bad = 0;
+void check(bool ok, const char *what, int line)
+{
+    if (ok) return;
+    printf("line %d: %s\n", line, what);
+    ++g_bad;
+}
+#define CHECK(x) check((x), #x, __LINE__)
+
+// A find of n keys on s: the rule it was launched with; *work is its place in the stream.
+FirstBucket find(Rules &r, int s, int *work = nullptr, uint64_t n = kMany)
+{
+    FirstBucket used = FirstBucket::kNone;
+    const int e = r.find(n, s, [&](FirstBucket rule) {
+        used = rule;
+        const int w = Fake::run(s);
+        if (work) *work = w;
+        return Fake::kOk;
+    });
+    CHECK(e == Fake::kOk);
+    return used;
+}
+
+void rules_kept_and_dropped()
+{
+    Rules r;
+    CHECK(find(r, 1) == FirstBucket::kNone);  // nothing known of the table
+    r.emptied();
+    CHECK(find(r, 1) == FirstBucket::kFill);
+    r.filled(FirstBucket::kStart);
+    CHECK(find(r, 1) == FirstBucket::kStart);
+    CHECK(find(r, 1, nullptr, kMany - 1) == FirstBucket::kNone);
+    CHECK(find(r, -1) == FirstBucket::kNone);
+    Fake::captured = {1};
+    CHECK(find(r, 1) == FirstBucket::kNone);
+    Fake::captured.clear();
+    r.filled(FirstBucket::kFill);  // entries under both rules
+    CHECK(find(r, 1) == FirstBucket::kNone);
+    r.emptied();
+    r.lost();
+    CHECK(find(r, 1) == FirstBucket::kNone);
+}
+
+void refill_that_fails_leaves_no_rule()
+{
+    for (const bool had : {false, true}) {
+        Rules r;
+        r.emptied();
+        r.filled(FirstBucket::kStart);
+        if (!had) r.freeing(1);
+        CHECK(r.refill(FirstBucket::kFill, [] { return 7; }) == 7);
+        CHECK(find(r, 1) == FirstBucket::kNone);
+        FirstBucket during = FirstBucket::kFill;
+        CHECK(r.refill(FirstBucket::kFill, [&] {
+            during = find(r, 1);
+            return Fake::kOk;
+        }) == Fake::kOk);
+        CHECK(during == FirstBucket::kNone);
+        CHECK(find(r, 1) == FirstBucket::kFill);
+    }
+}
+
+void an_erase_comes_after_the_finds_that_rely_on_a_rule()
+{
+    Rules r;
+    r.emptied();
+    int a = 0, b = 0, c = 0;
+    CHECK(find(r, 1, &a) != FirstBucket::kNone && find(r, 2, &b) != FirstBucket::kNone);
+    CHECK(find(r, 2, &c) != FirstBucket::kNone);
+    CHECK(r.freeing(3) == Fake::kOk);
+    CHECK(Fake::before(a, 3) && Fake::before(b, 3) && Fake::before(c, 3));
+    CHECK(find(r, 1) == FirstBucket::kNone);
+    // more streams than marks: the rest read in the reference order
+    r.emptied();
+    int with = 0;
+    for (int s = 10; s < 30; ++s) {
+        int w = 0;
+        if (find(r, s, &w) == FirstBucket::kNone) continue;
+        ++with;
+    }
+    CHECK(with == 8);
+}
+
+}  // namespace
+
+int main()
+{
+    rules_kept_and_dropped();
+    refill_that_fails_leaves_no_rule();
+    an_erase_comes_after_the_finds_that_rely_on_a_rule();
+    if (!g_bad) printf("inflight ok\n");
+    return g_bad != 0;
+}
