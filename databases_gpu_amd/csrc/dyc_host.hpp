@@ -83,6 +83,7 @@ struct HipRuntime {
     static void drop(Event e) { (void)hipEventDestroy(e); }
     static Error record(Event e, Stream s) { return hipEventRecord(e, s); }
     static Error wait(Stream s, Event e) { return hipStreamWaitEvent(s, e, 0); }
+    static Error finish(Stream s) { return hipStreamSynchronize(s); }
 };
 using FirstBucketRules = FirstBucketRulesT<HipRuntime>;
 

@@ -18,9 +18,12 @@ namespace host {
 
 // Which first-bucket rules (FirstBucket) the entries of a table, or of a group's tables, keep, and
 // the finds in flight that rely on one. An empty table keeps both; an insert keeps its own; an
-// erase, which frees slots, keeps none. A find that relies on a rule marks its stream, and the erase
-// that drops the rule waits on its own stream for the marks, so it frees no slot under such a
-// find on another stream. Finds of fewer than kFirstBucketKeys keys read in the reference order
+// erase, which frees slots, keeps none. A find that relies on a rule records an event (a mark), and the
+// erase that drops the rule waits on its own stream for the marks, so it frees no slot under such a
+// find on another stream. A stream's handle says which mark its finds share and nothing more: the
+// handle may have been another stream's, destroyed with its finds still running. So every mark is
+// waited for, whatever its handle, and a mark is recorded again only after a wait for what it
+// stood for (both are nothing on the stream that recorded it). Finds of fewer than kFirstBucketKeys keys read in the reference order
 // (the mark would cost them more than they save), as do finds being captured, which may be
 // replayed after an erase, finds on the per-thread stream (one handle for many streams), and those on
 // more than kMarks streams since the last erase or clear.
@@ -62,10 +65,9 @@ class FirstBucketRulesT {
         rules_ = 0;
         for (Mark &m : marks_) {
             if (!m.live) continue;
-            m.live = false;
-            if (m.stream == s) continue;
             const Error e = Runtime::wait(s, m.done);
             if (e != Runtime::kOk) return e;
+            m.live = false;
         }
         return Runtime::kOk;
     }
@@ -76,9 +78,10 @@ class FirstBucketRulesT {
         if (n < kFirstBucketKeys || Runtime::shared(s) || Runtime::capturing(s)) return launch(FirstBucket::kNone);
         std::lock_guard<std::mutex> lk(mu_);
         Mark *m = rules_ ? mark_for(s) : nullptr;
-        if (!m) return launch(FirstBucket::kNone);
+        if (!m || (m->live && Runtime::wait(s, m->done) != Runtime::kOk)) return launch(FirstBucket::kNone);
         Error e = launch(rules_ & kFillBit ? FirstBucket::kFill : FirstBucket::kStart);
-        if (e == Runtime::kOk) e = Runtime::record(m->done, s);
+        if (e == Runtime::kOk && (e = Runtime::record(m->done, s)) != Runtime::kOk)
+            (void)Runtime::finish(s);  // no mark: nothing may be in flight
         m->live = true;
         return e;
     }

@@ -17,6 +17,8 @@ struct Fake {
     static constexpr Error kOk = 0;
     static std::map<int, Work> streams, events;
     static std::set<int> captured;
+    static Work finished;
+    static bool records_fail, waits_fail;
     static int made, next;
     static bool shared(Stream s) { return s == -1; }
     static bool capturing(Stream s) { return captured.count(s) != 0; }
@@ -28,12 +30,19 @@ struct Fake {
     static void drop(Event e) { events.erase(e); }
     static Error record(Event e, Stream s)
     {
+        if (records_fail) return 5;
         events[e] = streams[s];
         return kOk;
     }
     static Error wait(Stream s, Event e)
     {
+        if (waits_fail) return 6;
         streams[s].insert(events[e].begin(), events[e].end());
+        return kOk;
+    }
+    static Error finish(Stream s)
+    {
+        finished.insert(streams[s].begin(), streams[s].end());
         return kOk;
     }
     // enqueue a piece of work on s
@@ -42,12 +51,14 @@ struct Fake {
         streams[s].insert(++next);
         return next;
     }
-    static bool before(int work, Stream s) { return streams[s].count(work) != 0; }
+    static bool before(int work, Stream s) { return streams[s].count(work) != 0 || finished.count(work) != 0; }
     // the stream of this handle is destroyed and a new one gets the handle; its work may go on
     static void reuse(Stream s) { streams[s].clear(); }
 };
 std::map<int, Work> Fake::streams, Fake::events;
 std::set<int> Fake::captured;
+Work Fake::finished;
+bool Fake::records_fail = false, Fake::waits_fail = false;
 int Fake::made = 0, Fake::next = 0;
 
 using dyc::FirstBucket;
@@ -137,6 +148,41 @@ void an_erase_comes_after_the_finds_that_rely_on_a_rule()
     CHECK(with == 8);
 }
 
+// Streams 1 and 2 are destroyed with a find running; new streams get their handles.
+void a_handle_is_not_a_stream()
+{
+    Rules r;
+    r.emptied();
+    int a = 0, b = 0, c = 0;
+    CHECK(find(r, 1, &a) != FirstBucket::kNone && find(r, 2, &b) != FirstBucket::kNone);
+    Fake::reuse(1);
+    Fake::reuse(2);
+    CHECK(find(r, 2, &c) != FirstBucket::kNone);  // records stream 2's mark again
+    CHECK(r.freeing(1) == Fake::kOk);
+    CHECK(Fake::before(a, 1) && Fake::before(b, 1) && Fake::before(c, 1));
+}
+
+void runtime_errors()
+{
+    Rules r;
+    r.emptied();
+    int a = 0, b = 0;
+    CHECK(find(r, 1, &a) != FirstBucket::kNone);
+    Fake::waits_fail = true;
+    CHECK(r.freeing(2) == 6);  // the erase is not launched
+    Fake::waits_fail = false;
+    CHECK(find(r, 1) == FirstBucket::kNone);
+    CHECK(r.freeing(3) == Fake::kOk && Fake::before(a, 3));
+    r.emptied();
+    Fake::records_fail = true;
+    CHECK(r.find(kMany, 1, [&](FirstBucket) {
+        b = Fake::run(1);
+        return Fake::kOk;
+    }) == 5);
+    Fake::records_fail = false;
+    CHECK(r.freeing(4) == Fake::kOk && Fake::before(b, 4));
+}
+
 }  // namespace
 
 int main()
@@ -144,6 +190,8 @@ int main()
     rules_kept_and_dropped();
     refill_that_fails_leaves_no_rule();
     an_erase_comes_after_the_finds_that_rely_on_a_rule();
+    a_handle_is_not_a_stream();
+    runtime_errors();
     if (!g_bad) printf("inflight ok\n");
     return g_bad != 0;
 }
