@@ -84,6 +84,7 @@ struct HipRuntime {
     static Error record(Event e, Stream s) { return hipEventRecord(e, s); }
     static Error wait(Stream s, Event e) { return hipStreamWaitEvent(s, e, 0); }
     static Error finish(Stream s) { return hipStreamSynchronize(s); }
+    static bool null(Stream s) { return s == nullptr; }
 };
 using FirstBucketRules = FirstBucketRulesT<HipRuntime>;
 
@@ -129,71 +130,8 @@ struct HipFree {
 };
 using Reclaimer = ReclaimerT<HipFree>;
 
-// The storage a table's last resize replaced, kept for its next one: a table that grows and shrinks
-// around one fill takes the same two sizes in turn, and hipMalloc with the hipFree behind it cost
-// many times what the resize's kernels do (to 96 MB and back with a find after each: 3.0 ms, 0.18 ms
-// with this). Bounded to one block of at most kSpareBlock bytes a table (a downsize is there to give
-// memory back, and the larger the block the smaller hipMalloc's share) and to kSpareTotal in the
-// process; given back when the next resize leaves another one, when an allocation of the table's
-// resizes fails, and with the table.
-// hipFree waits for the device, so a replaced block could still be read by finds in flight; a
-// block kept must not be. A resize has waited for its own stream when it keeps one, so the table
-// notes the stream of its finds (every other call waits before it returns), and keeps nothing
-// once they ran on another one than the resize.
-constexpr size_t kSpareBlock = 256ull << 20, kSpareTotal = 1ull << 30;
-class SpareBlock {
-  public:
-    SpareBlock() = default;
-    SpareBlock(const SpareBlock &) = delete;
-    SpareBlock &operator=(const SpareBlock &) = delete;
-    // A find is about to be launched on s.
-    void found_on(hipStream_t s)
-    {
-        uintptr_t seen = kNoStream;
-        const uintptr_t now = s == hipStreamPerThread ? kManyStreams : reinterpret_cast<uintptr_t>(s);
-        if (!stream_.compare_exchange_strong(seen, now) && seen != now) stream_ = kManyStreams;
-    }
-    // The kept block if it has just `bytes` bytes, else nullptr.
-    void *take(size_t bytes)
-    {
-        return p_ && bytes_ == bytes ? give_back() : nullptr;
-    }
-    // p was replaced by a resize that has waited for s: keep it, and free the block kept before, or
-    // free it (on r's thread).
-    void retire(Reclaimer &r, int device, void *p, size_t bytes, hipStream_t s)
-    {
-        r.defer(device, give_back());
-        const uintptr_t on = stream_;
-        const bool done = on == kNoStream || (on == reinterpret_cast<uintptr_t>(s) && s != hipStreamPerThread);
-        if (done) stream_ = kNoStream;
-        if (!done || bytes > kSpareBlock || total().fetch_add(bytes) + bytes > kSpareTotal) {
-            if (done && bytes <= kSpareBlock) total() -= bytes;
-            r.defer(device, p);
-            return;
-        }
-        p_ = p;
-        bytes_ = bytes;
-    }
-    // The kept block, no longer kept (nullptr if there is none).
-    void *give_back()
-    {
-        void *const p = p_;
-        if (p) total() -= bytes_;
-        p_ = nullptr;
-        return p;
-    }
-
-  private:
-    static constexpr uintptr_t kNoStream = ~(uintptr_t)0, kManyStreams = kNoStream - 1;
-    static std::atomic<size_t> &total()
-    {
-        static std::atomic<size_t> bytes{0};
-        return bytes;
-    }
-    std::atomic<uintptr_t> stream_{kNoStream};
-    void *p_ = nullptr;
-    size_t bytes_ = 0;
-};
+// dyc_inflight.hpp
+using SpareBlock = SpareBlockT<HipRuntime>;
 
 struct DeviceGuard {
     int prev = -1;

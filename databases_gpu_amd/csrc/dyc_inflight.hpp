@@ -2,8 +2,10 @@
 // runtime calls it needs (Runtime), so that a host-only build can run it with a stand-in.
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <mutex>
 
 namespace dyc {
@@ -126,6 +128,75 @@ class FirstBucketRulesT {
     std::mutex mu_;
     uint32_t rules_ = 0;
     Mark marks_[kMarks];
+};
+
+// The storage a table's last resize replaced, kept for its next one: a table that grows and shrinks
+// around one fill takes the same two sizes in turn, and hipMalloc with the hipFree behind it cost
+// many times what the resize's kernels do (to 96 MB and back with a find after each: 3.0 ms, 0.18 ms
+// with this). A block fits only a resize to its very size, so a table that keeps growing never
+// uses it. Bounded to one block of at most kSpareBlock bytes a table (a downsize is there to give
+// memory back, and the larger the block the smaller hipMalloc's share) and to kSpareTotal in the
+// process; given back when the next resize leaves another one, when an allocation of the table's
+// resizes fails, and with the table.
+// hipFree waits for the device, so a replaced block could still be in use by finds and clears in
+// flight (every other call waits before it returns, or is waited for by the next one); a block kept
+// must not be. So those calls say where they run (used_on). What ran on the null stream has ended
+// when a resize on it has, which waits for it. No other handle says as much: the stream may be gone and
+// its handle another one's, and captured work is replayed anywhere. After a call on one of those
+// nothing is kept. (An event a call would tell, but costs a small find on such a stream 1.1 us of 6.)
+constexpr size_t kSpareBlock = 256ull << 20, kSpareTotal = 1ull << 30;
+template <typename Runtime>
+class SpareBlockT {
+    using Stream = typename Runtime::Stream;
+
+  public:
+    SpareBlockT() = default;
+    SpareBlockT(const SpareBlockT &) = delete;
+    SpareBlockT &operator=(const SpareBlockT &) = delete;
+    // Work that uses the table's blocks and is not waited for is about to be launched on s. can_keep: the
+    // table has a block that a resize could keep (storage that came with the table is never kept).
+    void used_on(Stream s, bool can_keep)
+    {
+        if (can_keep) (Runtime::null(s) ? on_null_ : elsewhere_) = true;
+    }
+    // The kept block if it has just `bytes` bytes, else nullptr.
+    void *take(size_t bytes) { return p_ && bytes_ == bytes ? give_back() : nullptr; }
+    // p was replaced by a resize that has waited for s: keep it, and free the block kept before, or
+    // free it (on r's thread).
+    template <typename Reclaimer>
+    void retire(Reclaimer &r, int device, void *p, size_t bytes, Stream s)
+    {
+        r.defer(device, give_back());
+        const bool idle = !elsewhere_ && (!on_null_ || Runtime::null(s));
+        if (idle) on_null_ = false;
+        if (!idle || bytes > kSpareBlock) return r.defer(device, p);
+        if (total().fetch_add(bytes) + bytes > kSpareTotal) {
+            total() -= bytes;
+            return r.defer(device, p);
+        }
+        p_ = p;
+        bytes_ = bytes;
+    }
+    // The kept block, no longer kept (nullptr if there is none).
+    void *give_back()
+    {
+        void *const p = p_;
+        if (p) total() -= bytes_;
+        p_ = nullptr;
+        return p;
+    }
+    size_t kept() const { return p_ ? bytes_ : 0; }
+
+  private:
+    static std::atomic<size_t> &total()
+    {
+        static std::atomic<size_t> bytes{0};
+        return bytes;
+    }
+    std::atomic<bool> on_null_{false};    // work on the null stream may not have ended
+    std::atomic<bool> elsewhere_{false};  // work on another stream, or captured: never known to have ended
+    void *p_ = nullptr;
+    size_t bytes_ = 0;
 };
 
 }  // namespace host

@@ -133,6 +133,12 @@ struct dyc_table {
     uint8_t *slab = nullptr;
     uint32_t slab_live = 0;
     bool in_slab[kMaxSubtables] = {};
+    bool has_own_block() const  // a subtable that a resize allocated
+    {
+        for (uint32_t i = 0; i < D.d; ++i)
+            if (!in_slab[i]) return true;
+        return false;
+    }
     dyc_stats st{};
 
     uint64_t capacity() const
@@ -1292,7 +1298,7 @@ int dyc_find(dyc_table *t, const uint32_t *keys, uint32_t *vals, uint8_t *hit, u
     SETTLE(t);
     Pool sp;
     hipStream_t s = (hipStream_t)stream;
-    t->spare.found_on(s);
+    t->spare.used_on(s, t->has_own_block());
     HIP_TRY(t->rules.find(n, s, [&](FirstBucket rule) {
         return launch_find(t->D, keys, vals, hit, n, t->shape(), s, stash_of(t, sp), 0, rule);
     }));
@@ -1394,6 +1400,7 @@ int dyc_clear(dyc_table *t, dyc_stream stream)
     DeviceGuard dg(t->device);
     SETTLE(t);
     hipStream_t s = (hipStream_t)stream;
+    t->spare.used_on(s, t->has_own_block());
     for (uint32_t i = 0; i < t->D.d; ++i)
         HIP_TRY(launch_zero(reinterpret_cast<unsigned long long *>(t->D.sub[i]), (uint64_t)t->D.nb[i] * kSlots, s));
     t->count = 0;

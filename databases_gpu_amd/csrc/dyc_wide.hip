@@ -1217,6 +1217,12 @@ struct dyc_wide {
     uint8_t *slab = nullptr;
     uint32_t slab_live = 0;
     uint8_t *own[kMaxSubtables] = {};
+    bool has_own_block() const  // a subtable that a resize allocated
+    {
+        for (uint32_t i = 0; i < W.D.d; ++i)
+            if (own[i]) return true;
+        return false;
+    }
     uint64_t count = 0;
     uint64_t *pk = nullptr, *pv = nullptr;  // pending keys / values [0, pend_n): the stash
     uint64_t pend_cap = 0, pend_n = 0;
@@ -1865,7 +1871,7 @@ int dyc_wide_find(dyc_wide *t, const uint64_t *keys, uint64_t *vals, uint8_t *hi
     if (n && !keys) return fail(DYC_ERR_INVALID, "null keys");
     DeviceGuard dg(t->device);
     hipStream_t s = (hipStream_t)stream;
-    t->spare.found_on(s);
+    t->spare.used_on(s, t->has_own_block());
     HIP_TRY(t->rules.find(n, s, [&](FirstBucket rule) {
         return launch_wide_probe(t->W, keys, vals, hit, n, false, t->shape(), t->ctr, t->stash(), s, rule);
     }));
@@ -1928,6 +1934,7 @@ int dyc_wide_clear(dyc_wide *t, dyc_stream stream)
     if (!t) return fail(DYC_ERR_INVALID, "null table");
     DeviceGuard dg(t->device);
     hipStream_t s = (hipStream_t)stream;
+    t->spare.used_on(s, t->has_own_block());
     for (uint32_t i = 0; i < t->W.D.d; ++i) {
         HIP_TRY(launch_zero(reinterpret_cast<unsigned long long *>(t->W.D.sub[i]), (uint64_t)t->W.D.nb[i] * kSlots, s));
         HIP_TRY(launch_zero(reinterpret_cast<unsigned long long *>(t->W.val[i]), (uint64_t)t->W.D.nb[i] * kSlots, s));

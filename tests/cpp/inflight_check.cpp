@@ -4,6 +4,7 @@
 #include <cstdlib>
 #include <map>
 #include <set>
+#include <vector>
 
 #include "dyc_inflight.hpp"
 
@@ -45,6 +46,7 @@ struct Fake {
         finished.insert(streams[s].begin(), streams[s].end());
         return kOk;
     }
+    static bool null(Stream s) { return s == 0; }
     // enqueue a piece of work on s
     static int run(Stream s)
     {
@@ -183,6 +185,71 @@ void runtime_errors()
     CHECK(r.freeing(4) == Fake::kOk && Fake::before(b, 4));
 }
 
+using Spare = dyc::host::SpareBlockT<Fake>;
+struct Freed {
+    std::set<void *> all;
+    void defer(int, void *p)
+    {
+        if (p) all.insert(p);
+    }
+};
+char g_block[4];
+
+// A resize on s replaces a block: whether it is kept (and then taken).
+bool resize_keeps(Spare &sp, int s, size_t bytes = 1 << 20)
+{
+    Freed r;
+    sp.retire(r, 0, g_block, bytes, s);
+    CHECK(sp.kept() == (r.all.empty() ? bytes : 0));
+    CHECK(sp.take(bytes + 1) == nullptr);
+    const bool kept = sp.take(bytes) == g_block;
+    CHECK(kept == r.all.empty());
+    return kept;
+}
+
+void a_block_is_kept_only_when_nothing_uses_it()
+{
+    for (int on : {0, 1, 2}) {  // nothing in flight
+        Spare sp;
+        CHECK(resize_keeps(sp, on));
+        sp.used_on(1, false);  // a find of a table whose blocks all came with it
+        CHECK(resize_keeps(sp, on));
+    }
+    {  // the null stream, which a resize on it has waited for
+        Spare sp;
+        sp.used_on(0, true);
+        CHECK(!resize_keeps(sp, 2));
+        CHECK(resize_keeps(sp, 0));
+        sp.used_on(0, true);
+        CHECK(resize_keeps(sp, 0));
+        CHECK(resize_keeps(sp, 2));
+    }
+    for (int on : {1, -1}) {  // a handle that may be another stream's by now, or many streams'
+        Spare sp;
+        sp.used_on(on, true);
+        CHECK(!resize_keeps(sp, on) && !resize_keeps(sp, 0) && !resize_keeps(sp, 2));
+    }
+}
+
+void kept_blocks_are_bounded()
+{
+    using dyc::host::kSpareBlock;
+    using dyc::host::kSpareTotal;
+    const size_t fit = kSpareTotal / kSpareBlock;
+    std::vector<Spare> sp(fit + 1);
+    Freed r;
+    CHECK(!resize_keeps(sp[0], 0, kSpareBlock + 1));
+    for (size_t i = 0; i < fit; ++i) sp[i].retire(r, 0, g_block, kSpareBlock, 0);
+    CHECK(r.all.empty());
+    CHECK(!resize_keeps(sp[fit], 0, 1));
+    // a table's next block takes the place of the one it kept, which is freed
+    sp[0].retire(r, 0, g_block + 1, kSpareBlock, 0);
+    CHECK(sp[0].kept() == kSpareBlock && r.all == std::set<void *>{g_block});
+    CHECK(sp[0].give_back() == g_block + 1 && sp[0].kept() == 0);
+    CHECK(resize_keeps(sp[fit], 0, 1));
+    for (Spare &x : sp) (void)x.give_back();
+}
+
 }  // namespace
 
 int main()
@@ -192,6 +259,8 @@ int main()
     an_erase_comes_after_the_finds_that_rely_on_a_rule();
     a_handle_is_not_a_stream();
     runtime_errors();
+    a_block_is_kept_only_when_nothing_uses_it();
+    kept_blocks_are_bounded();
     if (!g_bad) printf("inflight ok\n");
     return g_bad != 0;
 }
