@@ -944,7 +944,7 @@ int dyc_group_clear(dyc_group *g, dyc_stream stream)
     std::fill(g->count.begin(), g->count.end(), 0);
     g->pend_n = 0;
     g->st.pending = 0;
-    g->rules.emptied();
+    g->rules.cleared((hipStream_t)stream);
     g->zeroed = true;
     return DYC_OK;
 }

@@ -45,9 +45,14 @@ class FirstBucketRulesT {
         for (Mark &m : marks_)
             if (m.made) Runtime::drop(m.done);
     }
-    // Cleared. (A find still in flight would race with the clear itself, so there is nothing left to
-    // wait for.)
+    // Just created.
     void emptied() { restart(kStartBit | kFillBit); }
+    // Cleared on s. (A find still in flight would race with the clear itself, so there is nothing left
+    // to wait for.) A clear that is being captured empties nothing until it is replayed.
+    void cleared(Stream s)
+    {
+        if (!Runtime::capturing(s)) emptied();
+    }
     // launch() clears the table and fills it under `rule`, and has waited for that when it returns. If
     // it fails, the table may still hold what it held before: no rule then.
     template <typename Launch>

@@ -1406,7 +1406,7 @@ int dyc_clear(dyc_table *t, dyc_stream stream)
     t->count = 0;
     t->pend_n = 0;
     t->st.pending = 0;
-    t->rules.emptied();
+    t->rules.cleared(s);
     t->zeroed = true;
     return DYC_OK;
 }

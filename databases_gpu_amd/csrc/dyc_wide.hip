@@ -1942,7 +1942,7 @@ int dyc_wide_clear(dyc_wide *t, dyc_stream stream)
     t->count = 0;
     t->pend_n = 0;
     t->st.pending = 0;
-    t->rules.emptied();
+    t->rules.cleared(s);
     t->zeroed = true;
     return DYC_OK;
 }
@@ -2661,7 +2661,7 @@ int dyc_wide_group_clear(dyc_wide_group *g, dyc_stream stream)
     std::fill(g->count.begin(), g->count.end(), 0);
     g->pend_n = 0;
     g->st.pending = 0;
-    g->rules.emptied();
+    g->rules.cleared((hipStream_t)stream);
     g->zeroed = true;
     return DYC_OK;
 }

@@ -105,8 +105,13 @@ void rules_kept_and_dropped()
     Fake::captured.clear();
     r.filled(FirstBucket::kFill);  // entries under both rules
     CHECK(find(r, 1) == FirstBucket::kNone);
-    r.emptied();
+    r.cleared(1);
+    CHECK(find(r, 1) == FirstBucket::kFill);
     r.lost();
+    CHECK(find(r, 1) == FirstBucket::kNone);
+    Fake::captured = {2};
+    r.cleared(2);  // the table still holds its entries
+    Fake::captured.clear();
     CHECK(find(r, 1) == FirstBucket::kNone);
 }
 
