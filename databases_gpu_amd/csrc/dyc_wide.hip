@@ -1872,7 +1872,7 @@ int dyc_wide_find(dyc_wide *t, const uint64_t *keys, uint64_t *vals, uint8_t *hi
     DeviceGuard dg(t->device);
     hipStream_t s = (hipStream_t)stream;
     t->spare.used_on(s, t->has_own_block());
-    HIP_TRY(t->rules.find(n, s, [&](FirstBucket rule) {
+    HIP_TRY(t->rules.find(dyc::host::first_bucket_pays(t->capacity() * 16) ? n : 0, s, [&](FirstBucket rule) {
         return launch_wide_probe(t->W, keys, vals, hit, n, false, t->shape(), t->ctr, t->stash(), s, rule);
     }));
     return DYC_OK;

@@ -190,6 +190,14 @@ void runtime_errors()
     CHECK(r.freeing(4) == Fake::kOk && Fake::before(b, 4));
 }
 
+// Small tables read in the reference order, whatever the lookups.
+void tables_that_gain_from_a_rule()
+{
+    using dyc::host::first_bucket_pays;
+    CHECK(!first_bucket_pays(1 << 15) && !first_bucket_pays(4 << 20) && !first_bucket_pays((12 << 20) - 1));
+    CHECK(first_bucket_pays(12 << 20) && first_bucket_pays(1ull << 31));
+}
+
 using Spare = dyc::host::SpareBlockT<Fake>;
 struct Freed {
     std::set<void *> all;
@@ -264,6 +272,7 @@ int main()
     an_erase_comes_after_the_finds_that_rely_on_a_rule();
     a_handle_is_not_a_stream();
     runtime_errors();
+    tables_that_gain_from_a_rule();
     a_block_is_kept_only_when_nothing_uses_it();
     kept_blocks_are_bounded();
     if (!g_bad) printf("inflight ok\n");
