@@ -210,11 +210,10 @@ int probe_grid(const dyc_group *g, uint64_t n, uint32_t n_items)
     return g->launch.find_blocks ? (int)g->launch.find_blocks : group_probe_grid(n, n_items);
 }
 
-// A find that relies on the first-bucket rule reads fewer buckets and takes a quarter more
-// instructions. It pays where lookups wait for lines from memory, so for tables of 1 MiB and more
-// on average (mean 1.4 MiB, 199 M lookups: 4697 -> 4083 us; 2.6 MiB, 101 M: 2159 -> 1938); an XCD's
-// L2 holds smaller ones (0.35 MiB, 75 M lookups: 1338 -> 1395).
-bool first_bucket_pays(const dyc_group *g) { return g->arena_bytes >= (uint64_t)g->n << 20; }
+bool first_bucket_pays(const dyc_group *g, uint64_t n)
+{
+    return dyc::host::first_bucket_pays(g->arena_bytes, g->n, n);
+}
 
 int zero_and_run_prologue(dyc_group *g, hipStream_t s)
 {
@@ -624,7 +623,7 @@ int dyc_group_find(dyc_group *g, const uint32_t *keys, const uint64_t *offsets, 
                                           : upload_items(g, offsets, s, &n_items);
     if (rc) return rc;
     Pool sp;
-    HIP_TRY(g->rules.find(first_bucket_pays(g) ? offsets[g->n] : 0, s, [&](FirstBucket rule) {
+    HIP_TRY(g->rules.find(first_bucket_pays(g, offsets[g->n]) ? offsets[g->n] : 0, s, [&](FirstBucket rule) {
         return launch_group_find(g->ddir, g->ditems, n_items, keys, vals, hit, probe_grid(g, offsets[g->n], n_items), s,
                                  g->stash(sp), (int)g->launch.find_waves_per_eu, rule);
     }));
@@ -891,9 +890,9 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
             k = launch_group_find(g->ddir, p->d_items + p->n_ins, p->n_find, lookups, vals_out, hit,
                                   probe_grid(g, find_offsets[g->n], p->n_find), cs, &stash,
                                   (int)g->launch.find_waves_per_eu,
-                                  !first_bucket_pays(g) ? FirstBucket::kNone
-                                  : p->bulk            ? FirstBucket::kFill
-                                                       : FirstBucket::kStart);
+                                  !first_bucket_pays(g, find_offsets[g->n]) ? FirstBucket::kNone
+                                  : p->bulk                                ? FirstBucket::kFill
+                                                                           : FirstBucket::kStart);
         if (k == hipSuccess)
             k = launch_copy(g->ctr, g->hctr, kCounterWords, g->tcounts, g->htcounts, g->n, cs);
         e = hipStreamEndCapture(cs, &p->graph);

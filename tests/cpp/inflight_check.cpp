@@ -196,6 +196,13 @@ void tables_that_gain_from_a_rule()
     using dyc::host::first_bucket_pays;
     CHECK(!first_bucket_pays(1 << 15) && !first_bucket_pays(4 << 20) && !first_bucket_pays((12 << 20) - 1));
     CHECK(first_bucket_pays(12 << 20) && first_bucket_pays(1ull << 31));
+    // groups: by the tables' size on average and in all, and by the lookups
+    const uint64_t mib = 1 << 20, few = 1 << 22, many = 1 << 24;
+    CHECK(!first_bucket_pays(8 * mib, 4, few) && first_bucket_pays(16 * mib, 4, few));
+    CHECK(!first_bucket_pays(16 * mib, 16, many) && !first_bucket_pays(64 * mib, 64, many));
+    CHECK(first_bucket_pays(128 * mib, 16, many) && first_bucket_pays(256 * mib, 256, many));
+    CHECK(first_bucket_pays(32 * mib, 4, many) && !first_bucket_pays(16 * mib, 4, many));
+    CHECK(!first_bucket_pays(700 * mib, 2048, few) && !first_bucket_pays(700 * mib, 2048, many));
 }
 
 using Spare = dyc::host::SpareBlockT<Fake>;
