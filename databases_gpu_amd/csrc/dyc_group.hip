@@ -210,9 +210,10 @@ int probe_grid(const dyc_group *g, uint64_t n, uint32_t n_items)
     return g->launch.find_blocks ? (int)g->launch.find_blocks : group_probe_grid(n, n_items);
 }
 
-bool first_bucket_pays(const dyc_group *g, uint64_t n)
+bool first_bucket_pays(const dyc_group *g, const uint64_t *offsets)
 {
-    return dyc::host::first_bucket_pays(g->arena_bytes, g->n, n);
+    return dyc::host::first_bucket_pays(
+        g->n, offsets, [g](uint32_t i) { return (uint64_t)g->hdir[i].d * g->hdir[i].nb[0] * kBucketBytes; });
 }
 
 int zero_and_run_prologue(dyc_group *g, hipStream_t s)
@@ -623,7 +624,8 @@ int dyc_group_find(dyc_group *g, const uint32_t *keys, const uint64_t *offsets, 
                                           : upload_items(g, offsets, s, &n_items);
     if (rc) return rc;
     Pool sp;
-    HIP_TRY(g->rules.find(first_bucket_pays(g, offsets[g->n]) ? offsets[g->n] : 0, s, [&](FirstBucket rule) {
+    const bool first = offsets[g->n] >= dyc::host::kFirstBucketKeys && first_bucket_pays(g, offsets);
+    HIP_TRY(g->rules.find(first ? offsets[g->n] : 0, s, [&](FirstBucket rule) {
         return launch_group_find(g->ddir, g->ditems, n_items, keys, vals, hit, probe_grid(g, offsets[g->n], n_items), s,
                                  g->stash(sp), (int)g->launch.find_waves_per_eu, rule);
     }));
@@ -890,7 +892,7 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
             k = launch_group_find(g->ddir, p->d_items + p->n_ins, p->n_find, lookups, vals_out, hit,
                                   probe_grid(g, find_offsets[g->n], p->n_find), cs, &stash,
                                   (int)g->launch.find_waves_per_eu,
-                                  !first_bucket_pays(g, find_offsets[g->n]) ? FirstBucket::kNone
+                                  !first_bucket_pays(g, find_offsets) ? FirstBucket::kNone
                                   : p->bulk                                ? FirstBucket::kFill
                                                                            : FirstBucket::kStart);
         if (k == hipSuccess)

@@ -40,21 +40,37 @@ constexpr uint64_t kFirstBucketKeys = 1ull << 22;
 // in L2 longer: Zipf(0.99) 0.75 at 16 MiB, 0.85-0.95 at 64, 1.0-1.15 at 256.
 inline bool first_bucket_pays(uint64_t table_bytes) { return table_bytes >= (12ull << 20); }
 
-// Whether a group call of n lookups does. Finds lay whole tables out over the 8 XCDs, so 16 MiB in all
-// have 2 MiB of each L2; from 2^24 lookups on fewer tables are in flight at a time (group_probe_grid)
-// and each is read more often, so the L2s keep more of them. Time in the reference order over time with
-// the rule, lookups uniform in each table, half of them stored (32-bit keys; 64-bit ones within 0.05
-// up to 2^22 lookups, nearer to 1 above):
-//   2^22 lookups: 4 tables of 2 MiB 0.92-0.95, 4 of 4 MiB 1.1, 16 of 1 MiB 1.05, 16 of 2 MiB 1.1,
-//     256 of 1 MiB 1.2;
-//   2^24: 16 of 1 or 2 MiB 0.75-0.8, 64 of 1 MiB 0.8, 16 of 4 MiB 0.97-1.04, 64 of 2 MiB 1.03-1.07,
-//     16 of 8 MiB 1.2, 4 of 8 MiB 1.2, 256 of 1 MiB 1.14.
-// Many tables of less than 1 MiB on average pass through the L2s one after another (2048 of 0.35 MiB,
-// 75 M lookups: 1338 us in the reference order, 1395 with the rule; of 1.4 MiB, 199 M: 4697, 4083).
-inline bool first_bucket_pays(uint64_t bytes, uint64_t tables, uint64_t n)
+// Whether a group's lookups do: table i of tables_n has bytes(i) bytes and the lookups [offsets[i],
+// offsets[i + 1]). Large finds lay whole tables out over the 8 XCDs, so what counts is how much of the
+// tables an XCD's workgroups read at a time against its L2: the tables that the lookups in flight on it
+// span (about 2^18 of them in the grid taken from 2^24 lookups on, 2^19 in the larger one below), and
+// no more than its eighth of all. Time in the reference order over time with the rule, 32-bit keys,
+// lookups uniform in each table, half of them stored, by that span in MiB (weighted by lookups):
+//   2^22 and 2^23 lookups: 1-5 MiB 0.75-0.9, 7-9 0.85-1.15, 12 1.0-1.1, 16 and more 1.05-1.2;
+//   2^24 to 2^26: 1-2.5 MiB 0.72-0.95, 4.7 0.92-1.1, 9 and more 1.06-1.26;
+//   2^24 to 2^26, fewer than 8 tables (so fewer XCDs than all): 9 MiB 0.8-1.0, 18 1.13-1.2.
+// (100 M lookups of 400 tables of 2^14..2^20 keys, 5.2 MiB: 1.11.) 64-bit keys lie nearer to 1 on both
+// sides, with the same crossings. Where fewer lookups than two a line come, each line is read from
+// memory whatever the L2 holds. Groups of less than 1 MiB a table on average read in the reference
+// order at any size.
+template <typename Bytes>
+bool first_bucket_pays(uint32_t tables_n, const uint64_t *offsets, Bytes bytes)
 {
-    if (bytes < tables << 20) return false;
-    return bytes >= (n < (1ull << 24) ? 16ull << 20 : (8ull << 20) * (tables < 16 ? tables : 16));
+    const uint64_t n = offsets[tables_n];
+    const bool narrow_grid = n >= (1ull << 24);
+    const double flight = narrow_grid ? 1 << 18 : 1 << 19;
+    double all = 0, own = 0, span = 0;  // bytes; bytes of the lookup's own table, and of its span, over the lookups
+    for (uint32_t i = 0; i < tables_n; ++i) {
+        const double b = (double)bytes(i), m = (double)(offsets[i + 1] - offsets[i]);
+        all += b;
+        own += b * m;
+        span += m == 0 ? 0 : b * (m > flight ? m : flight);
+    }
+    if (n == 0 || all < tables_n * 1048576.0) return false;
+    if ((double)n * 64 <= all) return true;
+    const double most = own / (double)n > all / 8 ? own / (double)n : all / 8;
+    const double mib = (span / (double)n < most ? span / (double)n : most) / 1048576.0;
+    return mib >= (narrow_grid && tables_n >= 8 ? 5 : 10);
 }
 
 template <typename Runtime>

@@ -2148,9 +2148,10 @@ int wg_probe_grid(const dyc_wide_group *g, uint64_t n, uint32_t n_items)
     return g->cfg.max_blocks ? (int)g->cfg.max_blocks : group_probe_grid(n, n_items);
 }
 
-bool wg_first_bucket_pays(const dyc_wide_group *g, uint64_t n)
+bool wg_first_bucket_pays(const dyc_wide_group *g, const uint64_t *offsets)
 {
-    return dyc::host::first_bucket_pays(g->arena_bytes, g->n, n);
+    return dyc::host::first_bucket_pays(
+        g->n, offsets, [g](uint32_t i) { return 2ull * g->hdir[i].D.d * wide_bytes(g->hdir[i].D.nb[0]); });
 }
 
 int wg_prologue(dyc_wide_group *g, hipStream_t s)
@@ -2508,7 +2509,8 @@ int dyc_wide_group_find(dyc_wide_group *g, const uint64_t *keys, const uint64_t 
     uint32_t n_items = 0;
     rc = wg_upload_items(g, offsets, s, &n_items, offsets[g->n] >= dyc::host::kXcdLayoutKeys);
     if (rc) return rc;
-    HIP_TRY(g->rules.find(wg_first_bucket_pays(g, offsets[g->n]) ? offsets[g->n] : 0, s, [&](FirstBucket rule) {
+    const bool first = offsets[g->n] >= dyc::host::kFirstBucketKeys && wg_first_bucket_pays(g, offsets);
+    HIP_TRY(g->rules.find(first ? offsets[g->n] : 0, s, [&](FirstBucket rule) {
         return launch_wide_group_probe(g->ddir, g->ditems, n_items, keys, vals, hit, false, nullptr,
                                        wg_probe_grid(g, offsets[g->n], n_items), g->stash(), s, rule);
     }));

@@ -196,13 +196,25 @@ void tables_that_gain_from_a_rule()
     using dyc::host::first_bucket_pays;
     CHECK(!first_bucket_pays(1 << 15) && !first_bucket_pays(4 << 20) && !first_bucket_pays((12 << 20) - 1));
     CHECK(first_bucket_pays(12 << 20) && first_bucket_pays(1ull << 31));
-    // groups: by the tables' size on average and in all, and by the lookups
-    const uint64_t mib = 1 << 20, few = 1 << 22, many = 1 << 24;
-    CHECK(!first_bucket_pays(8 * mib, 4, few) && first_bucket_pays(16 * mib, 4, few));
-    CHECK(!first_bucket_pays(16 * mib, 16, many) && !first_bucket_pays(64 * mib, 64, many));
-    CHECK(first_bucket_pays(128 * mib, 16, many) && first_bucket_pays(256 * mib, 256, many));
-    CHECK(first_bucket_pays(32 * mib, 4, many) && !first_bucket_pays(16 * mib, 4, many));
-    CHECK(!first_bucket_pays(700 * mib, 2048, few) && !first_bucket_pays(700 * mib, 2048, many));
+    // groups of equal tables: what an XCD reads at a time
+    auto group = [](uint32_t tables, double mib, uint64_t n) {
+        std::vector<uint64_t> off(tables + 1);
+        for (uint32_t i = 0; i <= tables; ++i) off[i] = n * i / tables;
+        return first_bucket_pays(tables, off.data(), [mib](uint32_t) { return (uint64_t)(mib * (1 << 20)); });
+    };
+    const uint64_t few = 1 << 22, many = 1 << 24;
+    CHECK(!group(1, 8, few) && group(1, 16, few) && !group(1, 8, many) && group(1, 16, many));
+    CHECK(!group(4, 1, few) && !group(4, 4, few) && !group(4, 4, many) && group(4, 16, many));
+    CHECK(!group(16, 2, few) && group(16, 16, few) && !group(16, 4, many) && group(16, 8, many));
+    CHECK(!group(64, 1, few) && group(64, 2, few) && !group(64, 2, many) && group(64, 8, many));
+    CHECK(group(256, 1, few) && !group(256, 1, many) && group(256, 2, many) && !group(256, 2, 4 * many));
+    CHECK(group(512, 1, few) && group(512, 1, many) && !group(512, 1, 4 * many));
+    CHECK(!group(2048, 0.35, few) && !group(2048, 0.35, 4 * many));
+    CHECK(group(8, 4, 1 << 13) && group(8, 4, 1 << 17));  // a small captured step: each line once
+    CHECK(!group(8, 4, 0));
+    // one large table among small ones takes most lookups
+    const uint64_t off[4] = {0, 1000, 1000, 1u << 24};
+    CHECK(first_bucket_pays(3, off, [](uint32_t i) { return i == 2 ? 64ull << 20 : 1ull << 16; }));
 }
 
 using Spare = dyc::host::SpareBlockT<Fake>;
