@@ -627,7 +627,8 @@ int dyc_group_find(dyc_group *g, const uint32_t *keys, const uint64_t *offsets, 
     const bool first = offsets[g->n] >= dyc::host::kFirstBucketKeys && first_bucket_pays(g, offsets);
     HIP_TRY(g->rules.find(first ? offsets[g->n] : 0, s, [&](FirstBucket rule) {
         return launch_group_find(g->ddir, g->ditems, n_items, keys, vals, hit, probe_grid(g, offsets[g->n], n_items), s,
-                                 g->stash(sp), (int)g->launch.find_waves_per_eu, rule);
+                                 g->stash(sp), (int)g->launch.find_waves_per_eu,
+                                 dyc::host::narrow_rule(rule, g->cfg.subtables));
     }));
     return DYC_OK;
 }
@@ -892,9 +893,10 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
             k = launch_group_find(g->ddir, p->d_items + p->n_ins, p->n_find, lookups, vals_out, hit,
                                   probe_grid(g, find_offsets[g->n], p->n_find), cs, &stash,
                                   (int)g->launch.find_waves_per_eu,
-                                  !first_bucket_pays(g, find_offsets) ? FirstBucket::kNone
-                                  : p->bulk                                ? FirstBucket::kFill
-                                                                           : FirstBucket::kStart);
+                                  !first_bucket_pays(g, find_offsets)
+                                      ? FirstBucket::kNone
+                                      : dyc::host::narrow_rule(p->bulk ? FirstBucket::kFill : FirstBucket::kStart,
+                                                               g->cfg.subtables));
         if (k == hipSuccess)
             k = launch_copy(g->ctr, g->hctr, kCounterWords, g->tcounts, g->htcounts, g->n, cs);
         e = hipStreamEndCapture(cs, &p->graph);

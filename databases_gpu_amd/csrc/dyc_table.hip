@@ -1300,7 +1300,8 @@ int dyc_find(dyc_table *t, const uint32_t *keys, uint32_t *vals, uint8_t *hit, u
     hipStream_t s = (hipStream_t)stream;
     t->spare.used_on(s, t->has_own_block());
     HIP_TRY(t->rules.find(dyc::host::first_bucket_pays(t->capacity() * 8) ? n : 0, s, [&](FirstBucket rule) {
-        return launch_find(t->D, keys, vals, hit, n, t->shape(), s, stash_of(t, sp), 0, rule);
+        return launch_find(t->D, keys, vals, hit, n, t->shape(), s, stash_of(t, sp), 0,
+                           dyc::host::narrow_rule(rule, t->D.d));
     }));
     return DYC_OK;
 }

@@ -196,6 +196,10 @@ void tables_that_gain_from_a_rule()
     using dyc::host::first_bucket_pays;
     CHECK(!first_bucket_pays(1 << 15) && !first_bucket_pays(4 << 20) && !first_bucket_pays((12 << 20) - 1));
     CHECK(first_bucket_pays(12 << 20) && first_bucket_pays(1ull << 31));
+    using dyc::host::narrow_rule;
+    CHECK(narrow_rule(FirstBucket::kStart, 2) == FirstBucket::kNone);
+    CHECK(narrow_rule(FirstBucket::kFill, 2) == FirstBucket::kFill);
+    CHECK(narrow_rule(FirstBucket::kStart, 3) == FirstBucket::kStart);
     // groups of equal tables: what an XCD reads at a time
     auto group = [](uint32_t tables, double mib, uint64_t n) {
         std::vector<uint64_t> off(tables + 1);
