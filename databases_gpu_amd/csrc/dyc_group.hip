@@ -625,10 +625,9 @@ int dyc_group_find(dyc_group *g, const uint32_t *keys, const uint64_t *offsets, 
     if (rc) return rc;
     Pool sp;
     const bool first = offsets[g->n] >= dyc::host::kFirstBucketKeys && first_bucket_pays(g, offsets);
-    HIP_TRY(g->rules.find(first ? offsets[g->n] : 0, s, [&](FirstBucket rule) {
+    HIP_TRY(g->rules.find(first ? offsets[g->n] : 0, s, g->cfg.subtables, [&](FirstBucket rule) {
         return launch_group_find(g->ddir, g->ditems, n_items, keys, vals, hit, probe_grid(g, offsets[g->n], n_items), s,
-                                 g->stash(sp), (int)g->launch.find_waves_per_eu,
-                                 dyc::host::narrow_rule(rule, g->cfg.subtables));
+                                 g->stash(sp), (int)g->launch.find_waves_per_eu, rule);
     }));
     return DYC_OK;
 }
@@ -763,6 +762,7 @@ struct dyc_group_plan {
     // insert_order 3: the batch's own bulk-fill arrays, and the group's shared workspace the graph
     // uses (an eager insert that grows it moves these)
     bool bulk = false;
+    FirstBucket rule = FirstBucket::kNone;  // of the graph's find
     uint64_t total = 0;
     GroupItem *bk_blk = nullptr;
     BulkTable *bk_tabs = nullptr;
@@ -889,14 +889,12 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
                                     (int)g->launch.insert_blocks, g->ctr, sink, g->tcounts, cs,
                                     (int)g->launch.insert_waves_per_eu);
         }
+        if (first_bucket_pays(g, find_offsets))
+            p->rule = dyc::host::narrow_rule(p->bulk ? FirstBucket::kFill : FirstBucket::kStart, g->cfg.subtables);
         if (k == hipSuccess)
             k = launch_group_find(g->ddir, p->d_items + p->n_ins, p->n_find, lookups, vals_out, hit,
                                   probe_grid(g, find_offsets[g->n], p->n_find), cs, &stash,
-                                  (int)g->launch.find_waves_per_eu,
-                                  !first_bucket_pays(g, find_offsets)
-                                      ? FirstBucket::kNone
-                                      : dyc::host::narrow_rule(p->bulk ? FirstBucket::kFill : FirstBucket::kStart,
-                                                               g->cfg.subtables));
+                                  (int)g->launch.find_waves_per_eu, p->rule);
         if (k == hipSuccess)
             k = launch_copy(g->ctr, g->hctr, kCounterWords, g->tcounts, g->htcounts, g->n, cs);
         e = hipStreamEndCapture(cs, &p->graph);
@@ -951,5 +949,8 @@ int dyc_group_clear(dyc_group *g, dyc_stream stream)
     g->zeroed = true;
     return DYC_OK;
 }
+
+uint32_t dyc_internal_group_rule(const dyc_group *g) { return (uint32_t)g->rules.last(); }  // as dyc_internal_rule
+uint32_t dyc_internal_plan_rule(const dyc_group_plan *p) { return (uint32_t)p->rule; }
 
 }  // extern "C"

@@ -130,20 +130,28 @@ class FirstBucketRulesT {
         }
         return Runtime::kOk;
     }
-    // Launch a find of n keys on s: launch(rule) with the rule it may rely on.
+    // Launch a find of n keys on s: launch(rule) with the rule it may rely on. subtables: of tables of
+    // 32-bit keys, else 0.
     template <typename Launch>
-    Error find(uint64_t n, Stream s, Launch launch)
+    Error find(uint64_t n, Stream s, uint32_t subtables, Launch launch)
     {
+        last_ = FirstBucket::kNone;
         if (n < kFirstBucketKeys || Runtime::shared(s) || Runtime::capturing(s)) return launch(FirstBucket::kNone);
         std::lock_guard<std::mutex> lk(mu_);
-        Mark *m = rules_ ? mark_for(s) : nullptr;
+        const FirstBucket kept = rules_ & kFillBit ? FirstBucket::kFill : (rules_ ? FirstBucket::kStart : FirstBucket::kNone);
+        const FirstBucket rule = narrow_rule(kept, subtables);
+        Mark *m = rule != FirstBucket::kNone ? mark_for(s) : nullptr;
         if (!m || (m->live && Runtime::wait(s, m->done) != Runtime::kOk)) return launch(FirstBucket::kNone);
-        Error e = launch(rules_ & kFillBit ? FirstBucket::kFill : FirstBucket::kStart);
+        last_ = rule;
+        Error e = launch(rule);
         if (e == Runtime::kOk && (e = Runtime::record(m->done, s)) != Runtime::kOk)
             (void)Runtime::finish(s);  // no mark: nothing may be in flight
         m->live = true;
         return e;
     }
+
+    // The rule of the last find (tests).
+    FirstBucket last() const { return last_; }
 
   private:
     static constexpr uint32_t kStartBit = 1u, kFillBit = 2u;
@@ -183,6 +191,7 @@ class FirstBucketRulesT {
         return nullptr;
     }
     std::mutex mu_;
+    std::atomic<FirstBucket> last_{FirstBucket::kNone};
     uint32_t rules_ = 0;
     Mark marks_[kMarks];
 };

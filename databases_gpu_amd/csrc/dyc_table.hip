@@ -1299,9 +1299,9 @@ int dyc_find(dyc_table *t, const uint32_t *keys, uint32_t *vals, uint8_t *hit, u
     Pool sp;
     hipStream_t s = (hipStream_t)stream;
     t->spare.used_on(s, t->has_own_block());
-    HIP_TRY(t->rules.find(dyc::host::first_bucket_pays(t->capacity() * 8) ? n : 0, s, [&](FirstBucket rule) {
-        return launch_find(t->D, keys, vals, hit, n, t->shape(), s, stash_of(t, sp), 0,
-                           dyc::host::narrow_rule(rule, t->D.d));
+    const bool first = dyc::host::first_bucket_pays(t->capacity() * 8);
+    HIP_TRY(t->rules.find(first ? n : 0, s, t->D.d, [&](FirstBucket rule) {
+        return launch_find(t->D, keys, vals, hit, n, t->shape(), s, stash_of(t, sp), 0, rule);
     }));
     return DYC_OK;
 }
@@ -1742,5 +1742,10 @@ int dyc_checkpoint_read(const char *path, const dyc_config *cfg, dyc_table **out
     *out = t;
     return DYC_OK;
 }
+
+// For the library's tests (not in dyc.h): the first-bucket rule of the handle's last find, or of a
+// plan's (0 none, 1 start, 2 fill), and the bytes a table's last resize kept.
+uint32_t dyc_internal_rule(const dyc_table *t) { return (uint32_t)t->rules.last(); }
+uint64_t dyc_internal_kept(const dyc_table *t) { return t->spare.kept(); }
 
 }  // extern "C"

@@ -1872,7 +1872,8 @@ int dyc_wide_find(dyc_wide *t, const uint64_t *keys, uint64_t *vals, uint8_t *hi
     DeviceGuard dg(t->device);
     hipStream_t s = (hipStream_t)stream;
     t->spare.used_on(s, t->has_own_block());
-    HIP_TRY(t->rules.find(dyc::host::first_bucket_pays(t->capacity() * 16) ? n : 0, s, [&](FirstBucket rule) {
+    const bool first = dyc::host::first_bucket_pays(t->capacity() * 16);
+    HIP_TRY(t->rules.find(first ? n : 0, s, 0, [&](FirstBucket rule) {
         return launch_wide_probe(t->W, keys, vals, hit, n, false, t->shape(), t->ctr, t->stash(), s, rule);
     }));
     return DYC_OK;
@@ -2510,7 +2511,7 @@ int dyc_wide_group_find(dyc_wide_group *g, const uint64_t *keys, const uint64_t 
     rc = wg_upload_items(g, offsets, s, &n_items, offsets[g->n] >= dyc::host::kXcdLayoutKeys);
     if (rc) return rc;
     const bool first = offsets[g->n] >= dyc::host::kFirstBucketKeys && wg_first_bucket_pays(g, offsets);
-    HIP_TRY(g->rules.find(first ? offsets[g->n] : 0, s, [&](FirstBucket rule) {
+    HIP_TRY(g->rules.find(first ? offsets[g->n] : 0, s, 0, [&](FirstBucket rule) {
         return launch_wide_group_probe(g->ddir, g->ditems, n_items, keys, vals, hit, false, nullptr,
                                        wg_probe_grid(g, offsets[g->n], n_items), g->stash(), s, rule);
     }));
@@ -2669,5 +2670,9 @@ int dyc_wide_group_clear(dyc_wide_group *g, dyc_stream stream)
     g->zeroed = true;
     return DYC_OK;
 }
+
+uint32_t dyc_internal_wide_rule(const dyc_wide *t) { return (uint32_t)t->rules.last(); }  // as dyc_internal_rule
+uint64_t dyc_internal_wide_kept(const dyc_wide *t) { return t->spare.kept(); }
+uint32_t dyc_internal_wide_group_rule(const dyc_wide_group *g) { return (uint32_t)g->rules.last(); }
 
 }  // extern "C"

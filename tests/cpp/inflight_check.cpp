@@ -77,16 +77,16 @@ void check(bool ok, const char *what, int line)
 #define CHECK(x) check((x), #x, __LINE__)
 
 // A find of n keys on s: the rule it was launched with; *work is its place in the stream.
-FirstBucket find(Rules &r, int s, int *work = nullptr, uint64_t n = kMany)
+FirstBucket find(Rules &r, int s, int *work = nullptr, uint64_t n = kMany, uint32_t subtables = 4)
 {
     FirstBucket used = FirstBucket::kNone;
-    const int e = r.find(n, s, [&](FirstBucket rule) {
+    const int e = r.find(n, s, subtables, [&](FirstBucket rule) {
         used = rule;
         const int w = Fake::run(s);
         if (work) *work = w;
         return Fake::kOk;
     });
-    CHECK(e == Fake::kOk);
+    CHECK(e == Fake::kOk && r.last() == used);
     return used;
 }
 
@@ -99,6 +99,7 @@ void rules_kept_and_dropped()
     r.filled(FirstBucket::kStart);
     CHECK(find(r, 1) == FirstBucket::kStart);
     CHECK(find(r, 1, nullptr, kMany - 1) == FirstBucket::kNone);
+    CHECK(find(r, 1, nullptr, kMany, 2) == FirstBucket::kNone && find(r, 1, nullptr, kMany, 0) == FirstBucket::kStart);
     CHECK(find(r, -1) == FirstBucket::kNone);
     Fake::captured = {1};
     CHECK(find(r, 1) == FirstBucket::kNone);
@@ -182,7 +183,7 @@ void runtime_errors()
     CHECK(r.freeing(3) == Fake::kOk && Fake::before(a, 3));
     r.emptied();
     Fake::records_fail = true;
-    CHECK(r.find(kMany, 1, [&](FirstBucket) {
+    CHECK(r.find(kMany, 1, 4, [&](FirstBucket) {
         b = Fake::run(1);
         return Fake::kOk;
     }) == 5);

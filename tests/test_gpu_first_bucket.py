@@ -2,7 +2,10 @@
 erased from, resized or loaded since it was empty) against the same lookups in smaller calls, which
 read in the reference order: values and flags bit for bit, also for copies of one key in both its
 buckets, under each rule and under none, and where an erase on another stream, a captured find or
-a refill could leave the rule behind."""
+a refill could leave the rule behind. Each large find is checked to have taken the rule that the
+table keeps then (NONE where it keeps none, or is too small to gain)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -10,6 +13,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 LARGE = 1 << 22
+NONE, START, FILL = 0, 1, 2
 
 
 @pytest.fixture(scope="module")
@@ -36,10 +40,21 @@ def lookups(n, stored, seed=0):
     return pool[torch.randint(0, pool.numel(), (n,), generator=g, device="cuda")]
 
 
-def both_ways(t, q):
-    """The large find, checked against small ones."""
+def last_rule(t):
+    """The rule of the last find of a table, a group or a plan's graph."""
+    kind = {"DyCuckoo": "", "DyCuckooWide": "wide_", "DyCuckooGroup": "group_", "DyCuckooWideGroup": "wide_group_",
+            "GroupPlan": "plan_"}[type(t).__name__]
+    f = getattr((t.group if kind == "plan_" else t).lib, f"dyc_internal_{kind}rule")
+    f.restype, f.argtypes = ctypes.c_uint32, [ctypes.c_void_p]
+    return f(t.h)
+
+
+def both_ways(t, q, rule):
+    """The large find, which takes `rule`, checked against small ones."""
     v, h = t.find(q)
+    assert last_rule(t) == rule
     sv, sh = zip(*(t.find(x) for x in torch.split(q, LARGE - 1)))
+    assert last_rule(t) == NONE
     assert torch.equal(h, torch.cat(sh)) and torch.equal(v, torch.cat(sv))
     return v, h
 
@@ -48,40 +63,59 @@ def both_ways(t, q):
 @pytest.mark.parametrize("order", [0, 3])
 def test_same_as_the_reference_order(D, order, d):
     print(f"\n[gpu-case] first-bucket rule d={d} insert_order={order}", flush=True)
-    m = 1 << 19
-    t = D.DyCuckoo(int(m / (0.6 if d == 2 else 0.75)), subtables=d, insert_order=order, kick_bound=0, auto_resize=0)
+    m = 1 << 21
+    t = D.DyCuckoo(int(m / (0.6 if d == 2 else 0.65)), subtables=d, insert_order=order, kick_bound=0, auto_resize=0)
+    # 32-bit keys all start in one of two subtables, so no find relies on that
+    start = NONE if d == 2 else START
+    kept = FILL if order == 3 else start
     k = keys(0, m)
     q = lookups(LARGE + 77, m, d)
-    _, h = both_ways(t, q)  # empty
+    _, h = both_ways(t, q, FILL)  # empty
     assert not h.any()
     t.insert(k, k ^ 1)
-    _, h = both_ways(t, q)
-    # a second copy of some keys: where the first bucket is full, in the other one
-    t.insert(k[: m // 16], k[: m // 16] ^ 2)
-    both_ways(t, q)
-    # entries under the other rule (a bulk fill into an eviction-built table, or the reverse)
+    _, h = both_ways(t, q, kept)
+    # a second copy of some keys (enough of them for a bulk fill): where the first bucket is full, in the
+    # other one
+    t.insert(k[: m // 4], k[: m // 4] ^ 2)
+    both_ways(t, q, kept)
+    # entries under the other rule (too few for a bulk fill)
     t.configure(insert_order=3 - order)
     extra = keys(3 * m, 3 * m + m // 32)
     t.insert(extra, extra)
-    both_ways(t, torch.cat([q, extra]))
+    both_ways(t, torch.cat([q, extra]), NONE if order == 3 else start)
     # erased slots: the rule is gone
     gone = t.erase(k[: m // 2])
     assert gone.all()
-    _, h2 = both_ways(t, q)
+    _, h2 = both_ways(t, q, NONE)
     assert int(h2.sum()) < int(h.sum())
     t.insert(k[: m // 2], k[: m // 2] ^ 3)
-    both_ways(t, q)
+    both_ways(t, q, NONE)
     # emptied and filled again: the rule is back
     t.clear()
     t.insert(k, k ^ 4)
-    v, h = both_ways(t, q)
+    v, h = both_ways(t, q, start if order == 3 else FILL)
     t.resize_up()
-    v2, h2 = both_ways(t, q)
+    v2, h2 = both_ways(t, q, NONE)
     assert torch.equal(h, h2) and torch.equal(v, v2)
     assert t.resize_down()
-    both_ways(t, q)
+    both_ways(t, q, NONE)
     t.load(t.dump())
-    both_ways(t, q)
+    both_ways(t, q, NONE)
+    t.close()
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+def test_small_tables_read_in_the_reference_order(D, bits):
+    print(f"\n[gpu-case] first-bucket rule, small table of {bits}-bit keys", flush=True)
+    from databases_gpu_amd.workload import u32_to_i64
+
+    m = 1 << 18
+    t = (D.DyCuckoo if bits == 32 else D.DyCuckooWide)(int(m / 0.8), insert_order=3, kick_bound=0, auto_resize=0)
+    k, q = keys(0, m), lookups(LARGE, m)
+    if bits == 64:
+        k, q = u32_to_i64(k), u32_to_i64(q)
+    t.insert(k, k)
+    both_ways(t, q, NONE)
     t.close()
 
 
@@ -89,33 +123,34 @@ def test_same_as_the_reference_order(D, order, d):
 @pytest.mark.parametrize("order", [0, 3])
 def test_wide_tables(D, order, d):
     print(f"\n[gpu-case] first-bucket rule, wide d={d} insert_order={order}", flush=True)
-    m = 1 << 19
-    t = D.DyCuckooWide(int(m / (0.6 if d == 2 else 0.75)), subtables=d, insert_order=order, kick_bound=0, auto_resize=0)
+    m = 1 << 20
+    t = D.DyCuckooWide(int(m / (0.6 if d == 2 else 0.65)), subtables=d, insert_order=order, kick_bound=0, auto_resize=0)
     wide = lambda x: x.long() * 0x1_0000_0001 ^ 0x55  # noqa: E731
+    kept = FILL if order == 3 else START
     k = wide(keys(0, m))
     q = torch.cat([wide(lookups(LARGE + 5, m, d)), torch.tensor([0, -1], device="cuda")])
-    _, h = both_ways(t, q)
+    _, h = both_ways(t, q, FILL)
     assert not h.any()
     t.insert(k, k ^ 1)
-    both_ways(t, q)
-    t.insert(k[: m // 16], k[: m // 16] ^ 2)
-    both_ways(t, q)
+    both_ways(t, q, kept)
+    t.insert(k[: m // 4], k[: m // 4] ^ 2)
+    both_ways(t, q, kept)
     t.upsert(k[: m // 16], k[: m // 16] ^ 3)  # under the start rule
-    both_ways(t, q)
+    both_ways(t, q, NONE if order == 3 else START)
     assert t.erase(k[: m // 2]).all()
-    both_ways(t, q)
+    both_ways(t, q, NONE)
     t.clear()
     t.insert(k, k ^ 4)
-    v, h = both_ways(t, q)
+    v, h = both_ways(t, q, kept)
     t.resize_up()
-    v2, h2 = both_ways(t, q)
+    v2, h2 = both_ways(t, q, NONE)
     assert torch.equal(h, h2) and torch.equal(v, v2)
     t.close()
 
 
 def test_upsert_and_host_inserts_keep_the_start_rule(D):
     print("\n[gpu-case] first-bucket rule, upsert and host inserts", flush=True)
-    m = 1 << 19
+    m = 1 << 21
     t = D.DyCuckoo(int(m / 0.8), insert_order=0, kick_bound=15, auto_resize=0)
     k = keys(0, m)
     q = lookups(LARGE, m)
@@ -123,7 +158,7 @@ def test_upsert_and_host_inserts_keep_the_start_rule(D):
     t.insert_host(k[m // 4: m // 2].cpu().numpy(), k[m // 4: m // 2].cpu().numpy())
     t.insert_async(k[m // 2:], k[m // 2:])
     t.upsert(k[: m // 4], k[: m // 4] ^ 9)
-    both_ways(t, q)
+    both_ways(t, q, START)
     t.close()
 
 
@@ -143,17 +178,18 @@ def test_erase_on_another_stream_waits_for_the_find(D):
         t.insert(k, k ^ 5)
         torch.cuda.synchronize()
         v, h = t.find(q, stream=a)
+        assert last_rule(t) == FILL
         gone = t.erase(go, stream=b)
         torch.cuda.synchronize()
         assert gone.all() and h.all() and torch.equal(v, q ^ 5)
-        v, h = both_ways(t, k.repeat(4))
+        v, h = both_ways(t, k.repeat(4), NONE)
         assert torch.equal(h.view(4, m)[0].bool(), torch.arange(m, device="cuda") < m // 2)
     t.close()
 
 
 def test_captured_find_is_replayed_after_an_erase(D):
     print("\n[gpu-case] first-bucket rule, captured find", flush=True)
-    m = 1 << 19
+    m = 1 << 21
     k = keys(0, m)
     q = lookups(LARGE, m)
     t = D.DyCuckoo(int(m / 0.9), insert_order=3, kick_bound=0, auto_resize=0)
@@ -161,10 +197,12 @@ def test_captured_find_is_replayed_after_an_erase(D):
     v = torch.empty_like(q)
     h = torch.empty(q.numel(), dtype=torch.uint8, device="cuda")
     t.find(q, v, h)
+    assert last_rule(t) == FILL
     torch.cuda.synchronize()
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g):
         t.find(q, v, h)
+        assert last_rule(t) == NONE
     for part in torch.split(k, m // 3):
         t.erase(part)
         g.replay()
@@ -180,27 +218,31 @@ def test_groups(D, bits, order):
     from databases_gpu_amd.table import DyCuckooGroup, DyCuckooWideGroup
 
     print(f"\n[gpu-case] first-bucket rule, groups bits={bits} insert_order={order}", flush=True)
-    # a mean of 1 MiB and more a table, from which a group's finds rely on the rule
-    sizes = np.random.default_rng(1).integers(0, 400_000, size=24)
+    # one lookup for three keys: the tables in flight on an XCD are more than its L2 holds, so the group's
+    # finds rely on the rule
+    sizes = np.random.default_rng(1).integers(0, 1_300_000, size=24)
     off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint64)
     n = int(off[-1])
-    assert n > LARGE
     k = keys(0, n)
-    miss = torch.rand(n, device="cuda") < 0.5
-    q = torch.where(miss, keys(n, 2 * n), k)
+    pick = torch.cat([torch.arange(int(off[i]), int(off[i + 1]), 3, device="cuda") for i in range(sizes.size)])
+    fsizes = -(-sizes // 3)
+    foff = np.concatenate([[0], np.cumsum(fsizes)]).astype(np.uint64)
+    assert LARGE < pick.numel() == int(foff[-1]) < 1 << 24
+    q = torch.where(torch.rand(pick.numel(), device="cuda") < 0.5, keys(n, n + pick.numel()), k[pick])
     if bits == 64:
         k, q = k.long() * 0x9E3779B1 | 1, q.long() * 0x9E3779B1 | 1
     g = (DyCuckooGroup if bits == 32 else DyCuckooWideGroup)((sizes / 0.85).astype(np.uint64) + 128,
                                                              insert_order=order, kick_bound=0)
 
-    def halves():
-        cut = sizes.size // 2
-        zero = np.zeros(sizes.size - cut, dtype=np.uint64)
-        lo = np.concatenate([off[: cut + 1], off[cut] + zero])
-        hi = np.concatenate([np.zeros(cut, dtype=np.uint64), off[cut:] - off[cut]])
-        c = int(off[cut])
-        a, b = g.find(q[:c].contiguous(), lo), g.find(q[c:].contiguous(), hi)
-        return torch.cat([a[0], b[0]]), torch.cat([a[1], b[1]])
+    def parts():
+        out = []
+        for lo in range(0, sizes.size, 4):
+            some = np.where((np.arange(sizes.size) >= lo) & (np.arange(sizes.size) < lo + 4), fsizes, 0)
+            a, b = int(foff[lo]), int(foff[min(lo + 4, sizes.size)])
+            assert b - a < LARGE
+            out.append(g.find(q[a:b].contiguous(), np.concatenate([[0], np.cumsum(some)]).astype(np.uint64)))
+            assert last_rule(g) == NONE
+        return torch.cat([x[0] for x in out]), torch.cat([x[1] for x in out])
 
     for step in range(3):
         if step == 2:
@@ -210,8 +252,9 @@ def test_groups(D, bits, order):
         else:
             erased = torch.arange(n, device="cuda") % 3 == 0
             g.erase(torch.where(erased, k, torch.zeros_like(k)), off)
-        v, h = g.find(q, off)
-        sv, sh = halves()
+        v, h = g.find(q, foff)
+        assert last_rule(g) == (NONE if step == 1 else FILL if order == 3 else START)
+        sv, sh = parts()
         assert torch.equal(h, sh) and torch.equal(v, sv)
     g.close()
 
@@ -225,19 +268,24 @@ def test_plan_relies_on_its_own_fill(D):
         off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint64)
         n = int(off[-1])
         k = keys(0, n)
-        miss = torch.rand(n, device="cuda") < 0.4
-        q = torch.where(miss, keys(n, 2 * n), k)
-        g = DyCuckooGroup((sizes / 0.85).astype(np.uint64) + 128, insert_order=order, kick_bound=0)
-        p = g.plan(k, k ^ 7, off, q, off)
-        for _ in range(3):
-            p.run()
-            assert torch.equal(p.out_hit.bool(), ~miss)
-            assert torch.equal(p.out_vals, torch.where(miss, torch.zeros_like(k), k ^ 7))
-            g.erase(k, off)  # eager work between the replays
-        g.close()
+        # as many lookups as keys, which find the tables in L2, and few of them
+        for every, rule in ((1, NONE), (16, FILL if order == 3 else START)):
+            pick = torch.cat([torch.arange(int(off[i]), int(off[i + 1]), every, device="cuda") for i in range(9)])
+            foff = np.concatenate([[0], np.cumsum(-(-sizes // every))]).astype(np.uint64)
+            miss = torch.rand(pick.numel(), device="cuda") < 0.4
+            q = torch.where(miss, keys(n, n + pick.numel()), k[pick])
+            g = DyCuckooGroup((sizes / 0.85).astype(np.uint64) + 128, insert_order=order, kick_bound=0)
+            p = g.plan(k, k ^ 7, off, q, foff)
+            assert last_rule(p) == rule
+            for _ in range(3):
+                p.run()
+                assert torch.equal(p.out_hit.bool(), ~miss)
+                assert torch.equal(p.out_vals, torch.where(miss, torch.zeros_like(q), q ^ 7))
+                g.erase(k, off)  # eager work between the replays
+            g.close()
 
 
-@pytest.mark.parametrize("d", [2, 4])
+@pytest.mark.parametrize("d", [3, 4])
 @pytest.mark.parametrize("kick_bound", [0, 15])
 def test_small_tables_looked_up_in_large_calls(D, kick_bound, d):
     """Tables of at most 1024 buckets, whose inserts spread a wave's lanes over a bucket's empty slots:
@@ -250,12 +298,13 @@ def test_small_tables_looked_up_in_large_calls(D, kick_bound, d):
     off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint64)
     n = int(off[-1])
     assert n > LARGE
-    g = DyCuckooGroup((sizes / (0.75 if d == 2 else 0.85)).astype(np.uint64) + 32, subtables=d, insert_order=0,
+    g = DyCuckooGroup((sizes / 0.85).astype(np.uint64) + 32, subtables=d, insert_order=0,
                       kick_bound=kick_bound)
     for seed in range(5):
         k = keys(0, n, 11 + seed)
         g.clear()
         g.insert(k, k ^ seed, off)
         v, h = g.find(k, off)
+        assert last_rule(g) == START
         assert bool(h.all()) and torch.equal(v, k ^ seed)
     g.close()

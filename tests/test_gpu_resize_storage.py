@@ -1,6 +1,10 @@
 """Resizes that take the storage an earlier one left: up and down around one size, up twice (the kept
 block has the wrong size), finds on a second stream in between (nothing is kept then), and blocks
-above the bound; every key is found after each step and the memory in use stays bounded."""
+above the bound; every key is found after each step, what is kept is what should be, and the memory in
+use stays bounded."""
+import ctypes
+import time
+
 import pytest
 import torch
 
@@ -40,27 +44,122 @@ def check(t, k, q, stream):
     assert torch.equal(v[: k.numel()], k ^ 77)
 
 
+def kept(t):
+    """The bytes the table's last resize kept."""
+    f = getattr(t.lib, "dyc_internal_wide_kept" if type(t).__name__ == "DyCuckooWide" else "dyc_internal_kept")
+    f.restype, f.argtypes = ctypes.c_uint64, [ctypes.c_void_p]
+    return f(t.h)
+
+
+def settled(limit):
+    """The device memory in use, once replaced blocks are freed (on a helper thread) or after 10 s."""
+    end = time.monotonic() + 10
+    while True:
+        free, total = torch.cuda.mem_get_info()
+        if total - free <= limit or time.monotonic() > end:
+            return total - free
+        time.sleep(0.01)
+
+
+BOUND = 256 << 20
+
+
 @pytest.mark.parametrize("bits", [32, 64])
 @pytest.mark.parametrize("second_stream", [False, True])
 @pytest.mark.parametrize("capacity", [1 << 12, 3 << 18, 9 << 23])
 def test_resizes_in_turn(D, bits, second_stream, capacity):
     print(f"\n[gpu-case] resizes in turn, {bits} bits, {capacity} slots, second stream {second_stream}", flush=True)
-    t = table(D, bits, capacity)
     own = torch.cuda.current_stream()
+    assert own.cuda_stream == 0  # the null stream
     other = torch.cuda.Stream() if second_stream else own
     k, q = contents(bits, min(capacity // 2, 1 << 20))
+    torch.cuda.synchronize()
+    free, total = torch.cuda.mem_get_info()
+    before = total - free
+    t = table(D, bits, capacity)
     t.insert(k, k ^ 77)
     torch.cuda.synchronize()
-    size = t.stats()["capacity"] * bits // 4
-    used = []
-    for step in "ududuuddud":
+    slot = bits // 4
+    first = sum(t.buckets) * 16 * slot
+    ever = 0
+    for i, step in enumerate("ududuuddud"):
+        old = t.buckets
         if step == "u":
             t.resize_up()
         else:
             assert t.resize_down()
+        replaced = [a for a, b in zip(old, t.buckets) if a != b]
+        assert len(replaced) == 1
+        block = replaced[0] * 16 * slot
+        if kept(t):
+            assert kept(t) == block <= BOUND
+            ever += 1
+        elif not second_stream and step == "d":
+            # a downsize replaces storage that a resize allocated, so it is kept where it fits
+            assert block > BOUND
         check(t, k, q, other if step == "u" else own)
-        used.append(torch.cuda.mem_get_info()[0])
+        size = sum(t.buckets) * 16 * slot
+        # the table (its first storage is one allocation, held while any of it is in use), the kept
+        # block and what else was allocated meanwhile (torch's blocks, the library's lists)
+        limit = before + first + size + kept(t) + (192 << 20)
+        assert settled(limit) <= limit
+    assert (ever == 0) == (second_stream or capacity == 9 << 23 and bits == 64)
     assert t.stats()["count"] == k.numel()
-    # the table itself, at most one and a half times its first size, a kept block and frees not yet done
-    assert max(used) - min(used) < 2 * size + (512 << 20)
+    t.close()
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+def test_blocks_of_a_side_stream_are_not_kept(D, bits):
+    """A long find on a side stream is still running when resizes on the null stream replace the blocks it
+    reads and ask for more of their sizes. (A table of few keys: a downsize moves none of them to
+    another subtable, so the find's blocks stay as they were.)"""
+    print(f"\n[gpu-case] a side stream's find under resizes, {bits} bits", flush=True)
+    t = table(D, bits, 3 << 18)
+    k, q = contents(bits, 1 << 15)
+    t.insert(k, k ^ 77)
+    t.resize_up()
+    assert t.resize_down()
+    assert kept(t) > 0
+    t.resize_up()
+    reps = 4096
+    long = q.repeat(reps)  # 2^28 lookups: milliseconds
+    v, h = torch.empty_like(long), torch.empty(long.numel(), dtype=torch.uint8, device="cuda")
+    side, done = torch.cuda.Stream(), torch.cuda.Event()
+    torch.cuda.synchronize()
+    t.find(long, v, h, stream=side)
+    done.record(side)
+    running = 0
+    for _ in range(4):
+        assert t.resize_down()
+        assert kept(t) == 0
+        t.resize_up()
+        assert kept(t) == 0
+        running += not done.query()
+    torch.cuda.synchronize()
+    print(f"running after {running} of 4 pairs of resizes", flush=True)
+    want_h = (torch.arange(q.numel(), device="cuda") < k.numel()).to(torch.uint8)
+    want_v = torch.where(want_h.bool(), q ^ 77, torch.zeros_like(q))
+    assert torch.equal(h.view(reps, -1), want_h.expand(reps, -1))
+    assert torch.equal(v.view(reps, -1), want_v.expand(reps, -1))
+    check(t, k, q, torch.cuda.current_stream())
+    t.close()
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+def test_a_captured_find_keeps_nothing(D, bits):
+    print(f"\n[gpu-case] a captured find under resizes, {bits} bits", flush=True)
+    t = table(D, bits, 3 << 18)
+    k, q = contents(bits, 3 << 17)
+    t.insert(k, k ^ 77)
+    t.resize_up()
+    v, h = torch.empty_like(q), torch.empty(q.numel(), dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        t.find(q, v, h)
+    g.replay()
+    torch.cuda.synchronize()
+    assert int(h.sum()) == k.numel()
+    assert t.resize_down()
+    assert kept(t) == 0
     t.close()
