@@ -1,15 +1,15 @@
 """Launch-shape autotuner for DyCuckoo groups (and single tables).
 
-The kernels take their shape at run time: lanes per key ("bucket width": how many lanes share
-one 128-byte bucket read -- the bucket itself stays 16 slots), grid size (resident waves per
-CU), keys per work item, the eviction bound (iterations under the reference victim rule
-before the pseudo-random rescue takes over; results are the same, placement and speed differ),
-and, for groups, occupancy: the persistent kernels exist in builds for at least 6 or 8 waves
-per SIMD (fewer registers each) besides the compiler's own choice.
+The kernels take their shape at run time: grid size (resident waves per CU), keys per work item, the
+eviction bound (iterations under the reference victim rule before the pseudo-random rescue takes
+over; results are the same, placement and speed differ), and, for groups, occupancy: the
+persistent kernels exist in builds for at least 6 or 8 waves per SIMD (fewer registers each) besides
+the compiler's own choice. (The lanes per key of a configuration have no effect on the kernels, so
+they are left as they are.) Every space holds the library's own default (0).
 `tune_group` times every candidate on the caller's own batch (or a sample of its tables) with
 HIP events and installs the fastest insert shape and the fastest find shape (the occupancy
 builds are tried on the best shape of the grid). Results are cached in a JSON file keyed by
-device name and a workload signature.
+device name, the kernels' shape version and a workload signature.
 """
 from __future__ import annotations
 
@@ -23,16 +23,17 @@ import torch
 
 CACHE_PATH = os.environ.get("DYC_AUTOTUNE_CACHE", os.path.join(os.path.expanduser("~"), ".cache", "dyc_autotune.json"))
 
+# Part of every cache key: raise it when a change to the kernels changes what a shape means (the
+# workgroup of a group's kernels, how an item is shared), so that older shapes are not installed.
+SHAPES = 2
+
 INSERT_SPACE = {
-    "insert_lanes": (1, 2, 4),
-    "insert_blocks": (1024, 2048, 4096, 8192),
-    "item_keys": (2048, 8192),
+    "insert_blocks": (0, 1024, 2048, 4096, 8192),
+    "item_keys": (0, 2048, 8192),
     "kick_bound": (15, 0),
 }
-FIND_SPACE = {
-    "find_lanes": (4, 8, 16),
-    "find_blocks": (1024, 2048, 4096, 8192),
-    "item_keys": (2048, 8192),
+FIND_SPACE = {  # at the insert's item size: both launches read the one field
+    "find_blocks": (0, 512, 1024, 2048, 4096, 8192),
 }
 WAVES_PER_EU = (6, 8)  # occupancy builds tried on the best grid shape (0 = the compiler's own)
 
@@ -85,7 +86,7 @@ def tune_group(group, keys: torch.Tensor, vals: torch.Tensor, offsets, lookups: 
     # the insert order changes what the insert launch does (the whole batch, or the few keys the
     # bulk fill leaves), so shapes tuned under one order are not reused under another
     order = getattr(getattr(group, "cfg", None), "insert_order", 0)
-    key = f"{torch.cuda.get_device_name(group.device)}|group|{_signature(offsets)}|io{order}"
+    key = f"{torch.cuda.get_device_name(group.device)}|v{SHAPES}|group|{_signature(offsets)}|io{order}"
     cache = _load_cache() if use_cache else {}
     t0 = time.perf_counter()
     if key in cache:
@@ -153,24 +154,19 @@ def tune_group(group, keys: torch.Tensor, vals: torch.Tensor, offsets, lookups: 
         if use_cache:
             cache[key] = best
             _store_cache(cache)
-    # install: the find item size only matters for find, the insert one for insert; keep the
-    # insert's item size (both launches read the same field) unless find measured better with
-    # the same value
     shape = {k: v for k, v in best["insert"].items() if k != "ms"}
-    shape.update({k: v for k, v in best["find"].items() if k not in ("ms", "item_keys")})
+    shape.update({k: v for k, v in best["find"].items() if k != "ms"})
     group.set_launch(**shape)
     best = dict(best, seconds=round(time.perf_counter() - t0, 3), installed=shape)
     return best
 
 
 TABLE_INSERT_SPACE = {
-    "insert_lanes": (1, 2, 4),
-    "insert_blocks": (16384, 32768, 65536),
+    "insert_blocks": (0, 1024, 2048, 4096, 8192, 16384, 32768, 49152, 65536),
     "kick_bound": (15, 0),
 }
-TABLE_FIND_SPACE = {
-    "find_lanes": (4, 8, 16),
-}
+# The find's grid: the default (a wave for 64 keys), and the half and the eighth of it.
+TABLE_FIND_GRIDS = (1, 2, 8)
 
 
 def tune_table(table, keys: torch.Tensor, vals: torch.Tensor, lookups, reps: int = 2,
@@ -185,7 +181,7 @@ def tune_table(table, keys: torch.Tensor, vals: torch.Tensor, lookups, reps: int
     afterwards."""
     sets = [lookups] if isinstance(lookups, torch.Tensor) else list(lookups)
     space = dict(TABLE_INSERT_SPACE, kick_bound=tuple(kick_bounds))
-    key = (f"{torch.cuda.get_device_name(table.device)}|table|n{keys.numel()}|cap{table.capacity}"
+    key = (f"{torch.cuda.get_device_name(table.device)}|v{SHAPES}|table|n{keys.numel()}|cap{table.capacity}"
            f"|kb{'-'.join(map(str, space['kick_bound']))}|f{'-'.join(str(q.numel()) for q in sets)}")
     cache = _load_cache() if use_cache else {}
     t0 = time.perf_counter()
@@ -216,8 +212,12 @@ def tune_table(table, keys: torch.Tensor, vals: torch.Tensor, lookups, reps: int
         out_v = torch.empty(m, dtype=torch.int32, device=sets[0].device)
         out_h = torch.empty(m, dtype=torch.uint8, device=sets[0].device)
         find_best = (float("inf"), None)
-        for combo in itertools.product(*TABLE_FIND_SPACE.values()):
-            shape = dict(zip(TABLE_FIND_SPACE.keys(), combo))
+        cfg = table.config()
+        blocks = min(-(-m // cfg["block_threads"]), 1 << 20)
+        # a grid that the caller has capped stays so
+        caps = [cfg["max_blocks"]] if cfg["max_blocks"] else [0 if p == 1 else max(1, blocks // p) for p in TABLE_FIND_GRIDS]
+        for cap in caps:
+            shape = {"find_lanes": cfg["find_lanes"], "max_blocks": cap}
             table.configure(**shape)
             ms = sum(_time(lambda q=q: table.find(q, out_v[:q.numel()], out_h[:q.numel()]), reps) for q in sets)
             trials += 1
