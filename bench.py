@@ -11,10 +11,10 @@ launch shapes and the eviction bound are tuned on the batch (untimed; --no-tune 
 the library launches on. `value` is the step's operations (3 * 2^28) per second of step time, in
 Mops/s.
 
-Roofline: the algorithmic bytes per operation follow the reference algorithm and layout
-(128-byte buckets, pos1 then pos2): find = 4 (key) + 4 (value) + 1 (hit flag) + 128 * p, with
-p the exact mean number of buckets the find order reads (dyc_probe_count over the same lookups,
-outside the timed region); insert = 8 (key, value) + i * (128 + 8), with i the mean number of
+Roofline: the algorithmic bytes per operation follow the reference's layout (128-byte buckets): find = 4
+(key) + 4 (value) + 1 (hit flag) + 128 * p, with p the exact mean number of buckets the timed find's order
+reads (counted over the same lookups, outside the timed region; a find that relies on a first-bucket
+rule reads fewer than the reference's pos1 then pos2, which is reported beside it); insert = 8 (key, value) + i * (128 + 8), with i the mean number of
 bucket exchanges per key from the insert kernel's counter. Achieved GB/s = bytes / kernel time;
 peak = 8 TB/s.
 
@@ -191,6 +191,21 @@ def traffic_from_csv(paths, log2n: int, cfg: dict) -> dict:
             e["l2_hit_rate"] = round(d["TCC_HIT_sum"] / max(1.0, d["TCC_HIT_sum"] + d["TCC_MISS_sum"]), 4)
         out[name] = e
     return out
+
+
+def find_probes(t, keys) -> int:
+    """Buckets (64-bit keys: key lines) that the table's last find reads in its order for these keys."""
+    import ctypes
+
+    import torch
+
+    f = t.lib.dyc_internal_wide_probes if keys.dtype == torch.int64 else t.lib.dyc_internal_probes
+    vp, u64 = ctypes.c_void_p, ctypes.c_uint64
+    f.restype, f.argtypes = ctypes.c_int, [vp, vp, u64, ctypes.POINTER(u64), vp]
+    out = u64()
+    if f(t.h, keys.data_ptr(), keys.numel(), ctypes.byref(out), torch.cuda.current_stream().cuda_stream):
+        raise RuntimeError("counting a find's buckets failed")
+    return out.value
 
 
 def pct(xs, q):
@@ -580,7 +595,7 @@ def run_subtables(args, dev) -> int:
         st = t.stats()
         good = st["count"] == n and st["pending"] == 0 and st["lost"] == 0 and bool((out_h.bool() == present).all()) \
             and bool((out_v[present] == W.splitmix32(look[present])).all())
-        probes, _ = t.probe_count(look)
+        probes = find_probes(t, look)
         ok &= good
         i_ms, f_ms = float(np.median(ins)), float(np.median(fnd))
         per_d[str(d)] = {"insert_ms": round(i_ms, 3), "insert_mops": round(n / i_ms / 1e3, 1),
@@ -673,9 +688,7 @@ def run_wide(args, dev) -> int:
         and bool((out_v[~out_h.bool()] == 0).all())
     i_ms, f_ms = float(np.median(ins)), float(np.median(fnd))
     x = float(np.mean(kicks)) / n
-    # key lines per lookup: 2 per miss, 1.5 per hit (pos1 holds half the keys: the start rule sends
-    # odd keys to pos2 first), as dyc_probe_count measures on the 32-bit table (1.75 at 50 % hit)
-    p_ = 2.0 * (1.0 - args.hit) + 1.5 * args.hit
+    p_ = find_probes(t, look) / n  # key lines per lookup
     b_ins = (16 + x * (128 + 24)) * n
     b_find = (17 + 128 * p_ + 8 * args.hit) * n
 
@@ -695,7 +708,7 @@ def run_wide(args, dev) -> int:
         "insert": dict(roof(b_ins, i_ms), ms=round(i_ms, 3), mops=round(n / i_ms / 1e3, 1),
                        mean_exchanges=round(x, 4), bytes_per_op=round(b_ins / n, 1)),
         "find": dict(roof(b_find, f_ms), ms=round(f_ms, 3), mops=round(n / f_ms / 1e3, 1),
-                     bytes_per_op=round(b_find / n, 1)),
+                     bytes_per_op=round(b_find / n, 1), mean_key_lines=round(p_, 4)),
         "parity": "ok" if ok else "mismatch",
     }
     t.close()
@@ -1106,9 +1119,8 @@ def main() -> int:
     log(f"parity vs generator: {'ok' if parity_ok else 'MISMATCH'}")
 
     # ---- algorithmic bytes
-    probes_u, pos1_u = t.probe_count(look_u)
-    probes_z, pos1_z = t.probe_count(look_z)
-    p_u, p_z = probes_u / n, probes_z / n
+    p_u, p_z = (find_probes(t, q) / n for q in (look_u, look_z))  # of the finds above
+    ref_u, ref_z = (t.probe_count(q)[0] / n for q in (look_u, look_z))
     i_bar = float(np.mean(kicks)) / n
     bytes_find_u = (4 + 4 + 1 + 128 * p_u) * n
     bytes_find_z = (4 + 4 + 1 + 128 * p_z) * n
@@ -1128,10 +1140,10 @@ def main() -> int:
                        mean_exchanges=round(i_bar, 4)),
         "find_uniform": dict(roof(bytes_find_u, med("find_uniform")), ms=round(med("find_uniform"), 3),
                              mops=round(n / med("find_uniform") / 1e3, 1), bytes_per_op=round(bytes_find_u / n, 2),
-                             mean_probes=round(p_u, 5)),
+                             mean_probes=round(p_u, 5), reference_probes=round(ref_u, 5)),
         "find_zipf": dict(roof(bytes_find_z, med("find_zipf")), ms=round(med("find_zipf"), 3),
                           mops=round(n / med("find_zipf") / 1e3, 1), bytes_per_op=round(bytes_find_z / n, 2),
-                          mean_probes=round(p_z, 5)),
+                          mean_probes=round(p_z, 5), reference_probes=round(ref_z, 5)),
     }
     # Fields below that this run cannot measure come from committed files, and say so: HBM bytes
     # per launch need a rocprofv3 --pmc run of their own (profiles/traffic.json, bench.py
@@ -1194,9 +1206,7 @@ def main() -> int:
                                                 "achieved": round(ex / 1e9, 2), "frac": round(ex / rc_, 3),
                                                 "unit": "G/s", "source": src}
             rd = p_u * n / (med("find_uniform") * 1e-3)
-            # counted in the reference's order; a find that the first bucket's free slot ends reads
-            # fewer, so the fraction may pass 1
-            kernels["find_uniform"]["ceiling"] = {"kind": "random 128-B bucket reads/s, reference order",
+            kernels["find_uniform"]["ceiling"] = {"kind": "random 128-B bucket reads/s",
                                                   "rate": round(ms_["bucket_reads_per_s"] / 1e9, 2),
                                                   "achieved": round(rd / 1e9, 2),
                                                   "frac": round(rd / ms_["bucket_reads_per_s"], 3), "unit": "G/s",

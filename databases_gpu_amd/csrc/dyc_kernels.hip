@@ -908,24 +908,31 @@ __global__ __launch_bounds__(256) void downsize_kernel(const uint64_t *__restric
     wave_tally(C, &C->residuals, nres, slot);
 }
 
-// Buckets the reference find order reads per key: 1 if pos1 holds the key, else 2 (0 for
-// reserved keys). One thread per key; a diagnostic pass, not on the hot path.
-__global__ __launch_bounds__(256) void probe_count_kernel(Desc D, const uint32_t *__restrict__ keys, uint64_t n,
-                                                          Counters *__restrict__ C)
+// Buckets a find reads per key (0 for reserved keys): in the reference order 1 if pos1 holds the key, else
+// 2; under a first-bucket rule as find_tile_first. first_hits: keys that the first bucket read holds.
+// One thread per key; a diagnostic pass, not on the hot path.
+__global__ __launch_bounds__(256) void probe_count_kernel(Desc D, FirstBucket rule, const uint32_t *__restrict__ keys,
+                                                          uint64_t n, Counters *__restrict__ C)
 {
-    unsigned long long probes = 0, pos1_hits = 0;
+    unsigned long long probes = 0, first_hits = 0;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
         const uint32_t k = keys[i];
         if (reserved_key(k)) continue;
-        const uint64_t *b = bucket_ptr(D, k, pos1(D, pair_of(D, k)));
-        bool hit = false;
-        for (int j = 0; j < kSlots; ++j) hit |= key_of(b[j]) == k;
-        probes += hit ? 1 : 2;
-        pos1_hits += hit;
+        const uint32_t p = pair_of(D, k), tb = pos2(D, p);
+        const bool from2 = rule != FirstBucket::kNone &&
+                           (rule == FirstBucket::kFill ? fill_target(D, k, p) == tb : (k & 1u) != 0);
+        const uint64_t *b = bucket_ptr(D, k, from2 ? tb : pos1(D, p));
+        bool hit = false, open = false;
+        for (int j = 0; j < kSlots; ++j) {
+            hit |= key_of(b[j]) == k;
+            open |= key_of(b[j]) == 0;
+        }
+        probes += (rule != FirstBucket::kNone && open) || (hit && !from2) ? 1 : 2;
+        first_hits += hit;
     }
     wave_tally(C, &C->kicks, probes);
-    wave_tally(C, &C->occupied, pos1_hits);
+    wave_tally(C, &C->occupied, first_hits);
 }
 
 // ---------------------------------------------------------------------------- many tables
@@ -1848,12 +1855,13 @@ hipError_t launch_fold_post(Counters *C, unsigned long long *post, unsigned long
     return hipGetLastError();
 }
 
-hipError_t launch_probe_count(const Desc &D, const uint32_t *keys, uint64_t n, Counters *C, hipStream_t st)
+hipError_t launch_probe_count(const Desc &D, const uint32_t *keys, uint64_t n, Counters *C, hipStream_t st,
+                              FirstBucket rule)
 {
     if (n == 0) return hipSuccess;
     uint64_t blocks = (n + 255) / 256;
     if (blocks > 65536) blocks = 65536;
-    probe_count_kernel<<<(int)blocks, 256, 0, st>>>(D, keys, n, C);
+    probe_count_kernel<<<(int)blocks, 256, 0, st>>>(D, rule, keys, n, C);
     return hipGetLastError();
 }
 

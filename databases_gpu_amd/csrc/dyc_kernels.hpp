@@ -445,7 +445,8 @@ constexpr int kPostWords = 1 + (int)(sizeof(Counters) / sizeof(unsigned long lon
 hipError_t launch_copy(const void *src0, void *dst0, uint64_t words0, const void *src1, void *dst1, uint64_t words1,
                        hipStream_t st);
 // buckets the pos1-then-pos2 find order reads for keys -> C->kicks, pos1 hits -> C->occupied
-hipError_t launch_probe_count(const Desc &D, const uint32_t *keys, uint64_t n, Counters *C, hipStream_t st);
+hipError_t launch_probe_count(const Desc &D, const uint32_t *keys, uint64_t n, Counters *C, hipStream_t st,
+                              FirstBucket rule = FirstBucket::kNone);
 // count non-empty slots of one subtable into C->occupied
 hipError_t launch_count(const uint64_t *sub, uint64_t slots, Counters *C, hipStream_t st);
 

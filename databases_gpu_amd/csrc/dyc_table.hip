@@ -1412,21 +1412,26 @@ int dyc_clear(dyc_table *t, dyc_stream stream)
     return DYC_OK;
 }
 
-int dyc_probe_count(dyc_table *t, const uint32_t *keys, uint64_t n, uint64_t *probes, uint64_t *pos1_hits,
-                    dyc_stream stream)
+static int probe_count(dyc_table *t, const uint32_t *keys, uint64_t n, uint64_t *probes, uint64_t *first_hits,
+                       hipStream_t s, FirstBucket rule)
 {
     if (!t || (n && !keys)) return fail(DYC_ERR_INVALID, "null argument");
     DeviceGuard dg(t->device);
     SETTLE(t);
-    hipStream_t s = (hipStream_t)stream;
     int rc = zero_counters(t, s);
     if (rc) return rc;
-    HIP_TRY(launch_probe_count(t->D, keys, n, t->ctr, s));
+    HIP_TRY(launch_probe_count(t->D, keys, n, t->ctr, s, rule));
     rc = read_counters(t, s);
     if (rc) return rc;
     if (probes) *probes = t->hctr->kicks;
-    if (pos1_hits) *pos1_hits = t->hctr->occupied;
+    if (first_hits) *first_hits = t->hctr->occupied;
     return DYC_OK;
+}
+
+int dyc_probe_count(dyc_table *t, const uint32_t *keys, uint64_t n, uint64_t *probes, uint64_t *pos1_hits,
+                    dyc_stream stream)
+{
+    return probe_count(t, keys, n, probes, pos1_hits, (hipStream_t)stream, FirstBucket::kNone);
 }
 
 int dyc_dump(dyc_table *t, uint32_t sub, uint64_t *host_slots, uint64_t n_slots, dyc_stream stream)
@@ -1743,9 +1748,14 @@ int dyc_checkpoint_read(const char *path, const dyc_config *cfg, dyc_table **out
     return DYC_OK;
 }
 
-// For the library's tests (not in dyc.h): the first-bucket rule of the handle's last find, or of a
-// plan's (0 none, 1 start, 2 fill), and the bytes a table's last resize kept.
+// For the library's tests and its benchmark (not in dyc.h): the first-bucket rule of the handle's last
+// find, or of a plan's (0 none, 1 start, 2 fill), the buckets that find's order reads for keys, and the
+// bytes a table's last resize kept.
 uint32_t dyc_internal_rule(const dyc_table *t) { return (uint32_t)t->rules.last(); }
+int dyc_internal_probes(dyc_table *t, const uint32_t *keys, uint64_t n, uint64_t *probes, dyc_stream stream)
+{
+    return probe_count(t, keys, n, probes, nullptr, (hipStream_t)stream, t ? t->rules.last() : FirstBucket::kNone);
+}
 uint64_t dyc_internal_kept(const dyc_table *t) { return t->spare.kept(); }
 
 }  // extern "C"

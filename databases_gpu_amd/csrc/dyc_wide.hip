@@ -282,6 +282,30 @@ __device__ inline uint32_t wide_probe_tile(const WideDesc &W, const uint64_t *__
     return my_flag;
 }
 
+// Key lines a find reads per key, as probe_count_kernel counts buckets.
+__global__ __launch_bounds__(256) void wide_probe_count_kernel(WideDesc W, FirstBucket rule,
+                                                               const uint64_t *__restrict__ keys, uint64_t n,
+                                                               Counters *__restrict__ C)
+{
+    unsigned long long probes = 0;
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+        const uint64_t k = keys[i];
+        if (wide_reserved(k)) continue;
+        const uint32_t f = fold64(k), p = pair_of(W.D, f), tb = pos2(W.D, p);
+        const bool from2 = rule != FirstBucket::kNone &&
+                           (rule == FirstBucket::kFill ? fill_target(W.D, (uint32_t)k, p) == tb : (k & 1u) != 0);
+        const uint64_t *line = bucket_ptr(W.D, f, from2 ? tb : pos1(W.D, p));
+        bool hit = false, open = false;
+        for (int j = 0; j < kSlots; ++j) {
+            hit |= line[j] == k;
+            open |= line[j] == 0;
+        }
+        probes += (rule != FirstBucket::kNone && open) || (hit && !from2) ? 1 : 2;
+    }
+    wave_tally(C, &C->kicks, probes);
+}
+
 template <int MODE, bool FIRST = false>
 __global__ __launch_bounds__(256) void wide_probe_kernel(WideDesc W, const uint64_t *__restrict__ keys,
                                                          uint64_t *__restrict__ vals, uint8_t *__restrict__ flags,
@@ -2672,6 +2696,21 @@ int dyc_wide_group_clear(dyc_wide_group *g, dyc_stream stream)
 }
 
 uint32_t dyc_internal_wide_rule(const dyc_wide *t) { return (uint32_t)t->rules.last(); }  // as dyc_internal_rule
+int dyc_internal_wide_probes(dyc_wide *t, const uint64_t *keys, uint64_t n, uint64_t *probes, dyc_stream stream)
+{
+    if (!t || (n && !keys)) return fail(DYC_ERR_INVALID, "null argument");
+    DeviceGuard dg(t->device);
+    hipStream_t s = (hipStream_t)stream;
+    int rc = wzero(t, s);
+    if (rc) return rc;
+    const uint64_t blocks = std::min<uint64_t>((n + 255) / 256, 65536);
+    if (n) wide_probe_count_kernel<<<(int)blocks, 256, 0, s>>>(t->W, t->rules.last(), keys, n, t->ctr);
+    HIP_TRY(hipGetLastError());
+    rc = wread(t, s);
+    if (rc) return rc;
+    *probes = t->hctr->kicks;
+    return DYC_OK;
+}
 uint64_t dyc_internal_wide_kept(const dyc_wide *t) { return t->spare.kept(); }
 uint32_t dyc_internal_wide_group_rule(const dyc_wide_group *g) { return (uint32_t)g->rules.last(); }
 

@@ -104,6 +104,43 @@ def test_same_as_the_reference_order(D, order, d):
     t.close()
 
 
+def probes(t, q):
+    """Buckets the last find's order reads for q."""
+    f = t.lib.dyc_internal_wide_probes if q.dtype == torch.int64 else t.lib.dyc_internal_probes
+    f.restype, f.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint64,
+                                           ctypes.POINTER(ctypes.c_uint64), ctypes.c_void_p]
+    out = ctypes.c_uint64()
+    torch.cuda.synchronize()
+    assert f(t.h, q.data_ptr(), q.numel(), ctypes.byref(out), None) == 0
+    return out.value
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("order", [0, 3])
+def test_buckets_counted_are_those_the_find_reads(D, order, bits):
+    print(f"\n[gpu-case] buckets a find reads, {bits}-bit keys, insert_order={order}", flush=True)
+    from databases_gpu_amd.workload import u32_to_i64
+
+    m = 1 << 21
+    t = (D.DyCuckoo if bits == 32 else D.DyCuckooWide)(int(m / 0.8), insert_order=order, kick_bound=0, auto_resize=0)
+    k, q = keys(0, m), lookups(LARGE, m)
+    valid = int(((q != 0) & (q != -1)).sum())
+    if bits == 64:
+        k, q = u32_to_i64(k), u32_to_i64(q)  # 0xffffffff is no reserved 64-bit key
+        valid = int((q != 0).sum())
+    t.find(q)
+    assert last_rule(t) == FILL and probes(t, q) == valid  # empty: every first bucket ends the search
+    t.insert(k, k)
+    t.find(q[:5])
+    reference = probes(t, q)
+    t.find(q)
+    assert last_rule(t) == (FILL if order == 3 else START)
+    assert valid < probes(t, q) < reference < 2 * valid
+    if bits == 32:
+        assert reference == t.probe_count(q)[0]
+    t.close()
+
+
 @pytest.mark.parametrize("bits", [32, 64])
 def test_small_tables_read_in_the_reference_order(D, bits):
     print(f"\n[gpu-case] first-bucket rule, small table of {bits}-bit keys", flush=True)
