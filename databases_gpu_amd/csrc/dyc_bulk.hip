@@ -3,8 +3,8 @@
 // The eviction insert spends one random 64-bit CAS per exchange, and the device's CAS rate is
 // the insert's ceiling however local the accesses are. A large batch can place most of its keys
 // without any global atomic instead:
-//   1. pack: each key's target bucket (the start rule's table, cuckoo.cu:336-341) names a
-//      chunk of kChunkBuckets consecutive buckets of one subtable; write the chunk ids and count
+//   1. pack: each key's target bucket (fill_target: pos1 for as many keys as equal subtable
+//      shares allow) names a chunk of kChunkBuckets consecutive buckets of one subtable; write the chunk ids and count
 //      their lowest digit per block;
 //   2. partition the entries by chunk (dyc_part.hpp: a least-significant-digit radix partition,
 //      8 bits of chunk id per pass, with no wait between blocks), which also gives the first

@@ -18,21 +18,12 @@ namespace dyc {
 namespace {
 
 
-// Plain (non-atomic) read of SPL consecutive slots, 16-byte vector loads where possible.
-template <int SPL>
-__device__ inline void load_slots(const uint64_t *p, uint64_t (&e)[SPL])
+// Plain (non-atomic) read of two consecutive slots.
+__device__ inline void load_slots(const uint64_t *p, uint64_t (&e)[2])
 {
-    if constexpr (SPL == 1) {
-        uint2 v = *reinterpret_cast<const uint2 *>(p);
-        e[0] = ((uint64_t)v.y << 32) | v.x;
-    } else {
-#pragma unroll
-        for (int j = 0; j < SPL; j += 2) {
-            uint4 v = *reinterpret_cast<const uint4 *>(p + j);
-            e[j] = ((uint64_t)v.y << 32) | v.x;
-            e[j + 1] = ((uint64_t)v.w << 32) | v.z;
-        }
-    }
+    const uint4 v = *reinterpret_cast<const uint4 *>(p);
+    e[0] = ((uint64_t)v.y << 32) | v.x;
+    e[1] = ((uint64_t)v.w << 32) | v.z;
 }
 
 // An input word (key or value). COH: read device-coherently, for a launch that outlives the
@@ -831,7 +822,7 @@ __global__ __launch_bounds__(256) void upsize_kernel(const uint64_t *__restrict_
         const uint64_t j = tile + g;
         if (j >= old_nb) continue;
         uint64_t e[2];
-        load_slots<2>(old + j * kSlots + s * 2, e);
+        load_slots(old + j * kSlots + s * 2, e);
         uint64_t lo[2], hi[2];
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
@@ -882,9 +873,9 @@ __global__ __launch_bounds__(256) void downsize_kernel(const uint64_t *__restric
         const bool ok = j < new_nb;
         uint64_t e[2] = {0, 0}, c[2] = {0, 0};
         if (ok) {
-            load_slots<2>(old + j * kSlots + s * 2, e);
+            load_slots(old + j * kSlots + s * 2, e);
             uint64_t x[2];
-            load_slots<2>(old + (j + new_nb) * kSlots + (7 - s) * 2, x);
+            load_slots(old + (j + new_nb) * kSlots + (7 - s) * 2, x);
             c[0] = x[1];  // slot 15-2s
             c[1] = x[0];  // slot 14-2s
         }
@@ -1504,23 +1495,23 @@ __global__ __launch_bounds__(256) void count_kernel(const uint64_t *__restrict__
 // every kernel here loops grid-stride, so the grid is capped (default_cap when the caller set
 // no max_blocks); the rest of the work is taken by the resident waves as they finish.
 
-// Insert groups take their next key when they finish one, so a grid of a few times the resident
-// capacity (256 CUs x 2048 threads) keeps every CU busy without launching a block per key.
+// Waves hand their chunks' keys to lanes as these finish, and eviction chains vary in length, so a
+// grid whose lanes take one key each ends on a tail of late blocks. With no grid from the caller, a lane
+// gets at least kInsertKeysPerLane keys, in no fewer than kInsertFloorBlocks blocks (about what the
+// device holds) and no more than kInsertDefaultBlocks. Insert into a table at fill 0.8-0.85, by grid:
+// 1.7 M keys with eviction bound 15 144 us at 1024 blocks, 156 at 4096 and more (bound 0: 107, 105);
+// 2^24 keys 970 us at the default 8192, 974 at 1024, 957 at 65,536 (839, 838, 822); 2^26 keys 3.18 ms at
+// the default 32,768, 3.36 at 8192, 3.75 at a block for 256 keys (2.85, 2.91, 3.05). Not everywhere
+// the best: 2^22 keys into an empty table take 243 us at 512 blocks, 286 at the default 2048 (302, 352).
 constexpr uint64_t kInsertDefaultBlocks = 65536;
-
-// Eviction chains vary in length, so a grid whose groups each take one or two keys ends on a tail
-// of late blocks: a batch of 1.6 M keys inserts 18% faster as 1024 resident blocks that take about
-// eight keys per group than as one block per 256 keys. With no max_blocks from the caller, the
-// default grid gives each group at least kInsertKeysPerGroup keys, never below kInsertFloorBlocks
-// (enough to fill the device) unless the batch is smaller than that.
-constexpr uint64_t kInsertKeysPerGroup = 8;
+constexpr uint64_t kInsertKeysPerLane = 8;
 constexpr uint64_t kInsertFloorBlocks = 1024;
 
 inline uint64_t insert_default_cap(uint64_t work_waves, LaunchShape sh)
 {
     const uint64_t wpb = (uint64_t)sh.block_threads / kWave;
     const uint64_t work_blocks = (work_waves + wpb - 1) / wpb;
-    uint64_t cap = work_blocks / kInsertKeysPerGroup;
+    uint64_t cap = work_blocks / kInsertKeysPerLane;
     if (cap < kInsertFloorBlocks) cap = kInsertFloorBlocks;
     if (cap > kInsertDefaultBlocks) cap = kInsertDefaultBlocks;
     return cap;
@@ -1756,6 +1747,8 @@ hipError_t launch_serve_insert(const Desc *dir, const ServeItem *items, uint32_t
     return hipGetLastError();
 }
 
+// The lanes have no effect on the kernels; a server that was refused the tick or the loop for them
+// still is.
 bool serve_tick_supported(int insert_lanes, int find_lanes)
 {
     return (insert_lanes == 1 || insert_lanes == 2 || insert_lanes == 4) &&

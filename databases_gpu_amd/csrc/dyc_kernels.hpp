@@ -175,9 +175,12 @@ struct GroupItem {
 // each shared by its kProbeWavesPerBlock waves.
 constexpr uint32_t kProbeWavesPerBlock = 8;
 // Default workgroups of a group probe over n keys in n_items items. From 2^24 keys two per CU: few
-// enough that the tables in flight on an XCD stay in its L2 (77 M lookups of 2048 tables: 512
-// workgroups 1250 us, 1024 1437, 2048 1390; 100 M of 400 tables of 2^14..2^20 keys 2081, 2304,
-// 2308); below it as many as the device holds (5.7 M lookups of 4096 tables 77, 71, 65 us).
+// enough that the tables in flight on an XCD stay in its L2 (75 M lookups of 2048 tables of 2^8..2^18
+// keys: 512 workgroups 1430 us, 1024 1608, 2048 1583; 16.3 M of 64 tables of 2^14..2^20 keys 306, 346,
+// 332; 97 M of 400 such tables 1894, 1989, 1945); below it as many as the device holds (13.4 M
+// lookups of 2048 tables of 2^8..2^15 keys 312, 305, 276; 3.9 M of 1024 of 2^8..2^14 keys 101, 95, 84).
+// From 2^24 to 2^26 lookups of tables of at most 2^17 keys the two are within 3 % (23 M: 494, 517, 485;
+// 42 M: 794, 852, 779).
 inline int group_probe_grid(uint64_t n, uint32_t n_items)
 {
     const uint32_t most = n >= (1ull << 24) ? 512u : 2048u;
@@ -435,7 +438,7 @@ inline uint64_t res_tiles(uint32_t new_nb) { return (new_nb + kResTileBuckets - 
 hipError_t launch_downsize(const uint64_t *old, uint32_t new_nb, uint64_t *dst, Counters *C, uint64_t *res,
                            uint64_t res_cap, uint8_t *live, hipStream_t st);
 hipError_t launch_zero(unsigned long long *p, uint64_t words, hipStream_t st);
-// Read a counter block back: one wave folds the stripes into the 16 counter words, writes them to
+// Read a counter block back: one workgroup folds the stripes into the 16 counter words, writes them to
 // post[1..16] (host-pinned), then seq to post[0], and clears the whole block for the next launch
 // group. The host waits for post[0] == seq (await_post) instead of copying 16.6 KB and
 // synchronising the stream: 7 us against 20 us per read on MI355X.

@@ -202,7 +202,8 @@ int dyc_erase(dyc_table *t, const uint32_t *keys, uint8_t *deleted, uint64_t n, 
 /* Replaces hashAPI::resize_up (api.cpp:112-141) + GPU_cuckoo_resize_up (cuckoo.cu:731-758):
  * doubles the subtable chosen by api.cpp:116-122. Synchronous. A table keeps the storage that its
  * last resize replaced for its next one (at most 256 MiB, and 1 GiB over all tables of the process)
- * as long as its finds run on the resizes' stream; dyc_destroy frees it. */
+ * if that one asks for just its size, so not while it only grows, and unless its finds or clears ran
+ * on another stream than the null stream since a resize; dyc_destroy frees it. */
 int dyc_resize_up(dyc_table *t, dyc_stream stream);
 
 /* Replaces hashAPI::resize_low (api.cpp:143-173) + GPU_cuckoo_resize_down (cuckoo.cu:762-788):
