@@ -182,10 +182,9 @@ int upload_segments(dyc_group *g, const std::vector<GroupItem> &segs, uint64_t p
     return DYC_OK;
 }
 
-// Cut the batch into items (at most item_keys keys of one table) and upload them.
-int upload_items(dyc_group *g, const uint64_t *offsets, hipStream_t s, uint32_t *n_items)
+// Cut the batch into items (at most per keys of one table) and upload them.
+int upload_items(dyc_group *g, const uint64_t *offsets, uint64_t per, hipStream_t s, uint32_t *n_items)
 {
-    const uint64_t per = group_item_keys(offsets[g->n], g->launch.item_keys);
     std::vector<GroupItem> segs;
     segs.reserve(g->n);
     for (uint32_t i = 0; i < g->n; ++i) {
@@ -594,13 +593,13 @@ int dyc_group_insert(dyc_group *g, const uint32_t *keys, const uint32_t *vals, c
         }
     }
     uint32_t n_items = 0;
-    rc = upload_items(g, offsets, s, &n_items);
+    rc = upload_items(g, offsets, group_insert_item_keys(total, g->launch.item_keys), s, &n_items);
     if (rc) return rc;
     rc = zero_and_run_prologue(g, s);
     if (rc) return rc;
     g->rules.filled(FirstBucket::kStart);
     HIP_TRY(launch_group_insert(g->ddir, g->ditems, n_items, keys, vals, g->policy(),
-                                (int)g->launch.insert_blocks, g->ctr,
+                                (int)g->launch.insert_blocks, total < kSharedInsertKeys, g->ctr,
                                 PendSink{g->pend + g->pend_n, g->pend_tag + g->pend_n, room, 0, 0, nullptr}, g->tcounts,
                                 s, (int)g->launch.insert_waves_per_eu));
     rc = read_back(g, s);
@@ -621,7 +620,7 @@ int dyc_group_find(dyc_group *g, const uint32_t *keys, const uint64_t *offsets, 
     // the layout by XCD pays where the batch spans more than the L2s hold; below that its host
     // work (a sort of the tables) would be most of a small call
     rc = offsets[g->n] >= kXcdLayoutKeys ? upload_items_by_xcd(g, offsets, s, &n_items)
-                                          : upload_items(g, offsets, s, &n_items);
+                                          : upload_items(g, offsets, group_item_keys(offsets[g->n], g->launch.item_keys), s, &n_items);
     if (rc) return rc;
     Pool sp;
     const bool first = offsets[g->n] >= dyc::host::kFirstBucketKeys && first_bucket_pays(g, offsets);
@@ -641,7 +640,7 @@ int dyc_group_erase(dyc_group *g, const uint32_t *keys, const uint64_t *offsets,
     DeviceGuard dg(g->device);
     hipStream_t s = (hipStream_t)stream;
     uint32_t n_items = 0;
-    rc = upload_items(g, offsets, s, &n_items);
+    rc = upload_items(g, offsets, group_item_keys(offsets[g->n], g->launch.item_keys), s, &n_items);
     if (rc) return rc;
     HIP_TRY(g->rules.freeing(s));
     rc = zero_and_run_prologue(g, s);
@@ -800,7 +799,7 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
     rc = reserve_pending(g, std::max<uint64_t>(65536, ins_offsets[g->n] / 16), nullptr);
     if (rc) return rc;
     // the work items of both launches, cut and laid out as the eager calls do, uploaded once
-    const uint64_t per = group_item_keys(ins_offsets[g->n], g->launch.item_keys);
+    const uint64_t per = group_insert_item_keys(ins_offsets[g->n], g->launch.item_keys);
     std::vector<GroupItem> items;
     for (uint32_t i = 0; i < g->n; ++i)
         for (uint64_t b = ins_offsets[i]; b < ins_offsets[i + 1]; b += per)
@@ -886,7 +885,8 @@ int dyc_group_plan_create(dyc_group *g, const uint32_t *keys, const uint32_t *va
             k = enqueue_group_bulk(g, A, keys, vals, p->total, true, sink, cs);
         } else if (k == hipSuccess) {
             k = launch_group_insert(g->ddir, p->d_items, p->n_ins, keys, vals, g->policy(),
-                                    (int)g->launch.insert_blocks, g->ctr, sink, g->tcounts, cs,
+                                    (int)g->launch.insert_blocks, ins_offsets[g->n] < kSharedInsertKeys, g->ctr, sink,
+                                    g->tcounts, cs,
                                     (int)g->launch.insert_waves_per_eu);
         }
         if (first_bucket_pays(g, find_offsets))

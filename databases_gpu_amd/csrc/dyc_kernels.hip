@@ -983,26 +983,29 @@ __global__ __launch_bounds__(kGroupThreads, W) void group_probe_kernel(const Des
     }
 }
 
-// The waves of a workgroup share its items as in the probe, chunk by chunk. A wave moves on only when
-// all its lanes have placed (or pended) their entries.
+// shared: the waves of a workgroup share its items as in the probe, chunk by chunk; else each wave takes
+// items of its own (group_insert_item_keys says when). A wave moves on only when all its lanes have
+// placed (or pended) their entries.
 template <int W>
 __global__ __launch_bounds__(kGroupThreads, W) void group_insert_kernel(const Desc *__restrict__ dir,
                                                            const GroupItem *__restrict__ items, uint32_t n_items,
                                                            const uint32_t *__restrict__ keys,
                                                            const uint32_t *__restrict__ vals, InsertPolicy P,
                                                            Counters *__restrict__ C, PendSink sink,
-                                                           unsigned long long *__restrict__ table_counts)
+                                                           unsigned long long *__restrict__ table_counts,
+                                                           bool shared)
 {
     InsertTally tally;
     uint32_t r = 0;
-    for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x, ++r) {
+    const uint32_t step = shared ? gridDim.x : gridDim.x * kGroupWaves;
+    for (uint32_t it = shared ? blockIdx.x : wave_slot(); it < n_items; it += step, ++r) {
         const GroupItem item = items[it];
-        const uint32_t first = group_first_tile(r);
+        const uint32_t first = shared ? group_first_tile(r) : 0u;
         if (first * kWave >= item.len) continue;  // wave-uniform
         const Desc D = as_global(dir[item.table]);
         const unsigned long long rej0 = tally.rejected;
         InsertRange<false> in{keys, vals, nullptr, nullptr, kNoTable};
-        in.run(D, item.begin, item.begin + item.len, first, kGroupWaves, P, C, sink, item.table, tally);
+        in.run(D, item.begin, item.begin + item.len, first, shared ? kGroupWaves : 1, P, C, sink, item.table, tally);
         const unsigned long long rej = tally.rejected - rej0;
         if (__lane_id() == 0 && in.taken > rej) atomicAdd(&table_counts[item.table], in.taken - rej);
     }
@@ -1668,23 +1671,24 @@ hipError_t launch_group_erase(const Desc *dir, const GroupItem *items, uint32_t 
 }
 
 hipError_t launch_group_insert(const Desc *dir, const GroupItem *items, uint32_t n_items, const uint32_t *keys,
-                               const uint32_t *vals, InsertPolicy pol, int blocks, Counters *C, PendSink sink,
-                               unsigned long long *table_counts, hipStream_t st, int waves_per_eu)
+                               const uint32_t *vals, InsertPolicy pol, int blocks, bool shared, Counters *C,
+                               PendSink sink, unsigned long long *table_counts, hipStream_t st, int waves_per_eu)
 {
     if (n_items == 0) return hipSuccess;
-    const int grid = blocks > 0 ? blocks : (int)std::min<uint32_t>(kGroupInsertBlocks, n_items);
+    const uint32_t most = shared ? n_items : (n_items + kGroupWaves - 1) / kGroupWaves;
+    const int grid = blocks > 0 ? blocks : (int)std::min<uint32_t>(kGroupInsertBlocks, most);
     switch (waves_per_eu) {
     case 6:
         group_insert_kernel<6>
-            <<<grid, kGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts);
+            <<<grid, kGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts, shared);
         break;
     case 8:
         group_insert_kernel<8>
-            <<<grid, kGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts);
+            <<<grid, kGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts, shared);
         break;
     default:
         group_insert_kernel<1>
-            <<<grid, kGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts);
+            <<<grid, kGroupThreads, 0, st>>>(dir, items, n_items, keys, vals, pol, C, sink, table_counts, shared);
         break;
     }
     return hipGetLastError();

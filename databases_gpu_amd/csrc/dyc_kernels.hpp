@@ -195,6 +195,23 @@ inline uint64_t group_item_keys(uint64_t n, uint32_t most)
     const uint64_t per = (n / 1024 + tile - 1) / tile * tile;
     return per < tile ? (tile < cap ? tile : cap) : (per < cap ? per : cap);
 }
+// An eviction insert's items. A wave that leaves an item waits for the chains it has begun there, so where
+// the batch has enough keys each wave takes whole items (kSharedInsertKeys and more; `shared` false
+// below), large enough that about 1400 waves (6 a CU) have one each: with the items shared a wave
+// leaves one after an eighth of it, and more waves only meet in the atomics. Shared / whole items
+// of that size: 0.35 M keys in 1024 tables 99 / 79 us, 1.6 M in 16 256 / 170, 5.7 M in 64 491 / 345, 75 M in
+// 2048 4311 / 3640 (eviction bound 15: 5787 / 4221). Fewer keys are bound by the chain of steps a wave
+// goes through, and shared (22,000 keys in 256 tables 47.7 / 50.5 us, a whole step of clear, insert
+// and find; 43,000 in 1024 52 / 54; 86,000 in 256 70 / 65).
+constexpr uint64_t kSharedInsertKeys = 1ull << 16;
+inline uint64_t group_insert_item_keys(uint64_t n, uint32_t most)
+{
+    if (n < kSharedInsertKeys) return group_item_keys(n, most);
+    const uint64_t cap = most && most != 4096 ? most : 8192u;
+    uint64_t per = (n / 1400 + 63) / 64 * 64;
+    if (per < 256) per = 256;
+    return per < cap ? per : cap;
+}
 // find: vals/hit may be null. erase: per-table deleted counts are added to table_counts.
 // pool (optional): misses of an item of table i also look in the pool's entries tagged i.
 // blocks: the grid (group_probe_grid's by default for probes; 0 for an insert: as many as fill the
@@ -208,9 +225,10 @@ hipError_t launch_group_erase(const Desc *dir, const GroupItem *items, uint32_t 
                               uint8_t *deleted, unsigned long long *table_counts, int blocks,
                               hipStream_t st, const Pool *pool = nullptr, int waves_per_eu = 0);
 // insert: failures go to sink.pend with their table index in sink.tags; per-table inserted
-// counts (placed or pended, reserved keys excluded) are added to table_counts.
+// counts (placed or pended, reserved keys excluded) are added to table_counts. shared: a workgroup's
+// waves share each item, else each wave takes whole ones.
 hipError_t launch_group_insert(const Desc *dir, const GroupItem *items, uint32_t n_items, const uint32_t *keys,
-                               const uint32_t *vals, InsertPolicy pol, int blocks, Counters *C,
+                               const uint32_t *vals, InsertPolicy pol, int blocks, bool shared, Counters *C,
                                PendSink sink, unsigned long long *table_counts, hipStream_t st,
                                int waves_per_eu = 0);
 

@@ -292,7 +292,8 @@ typedef struct dyc_group_launch {
     uint32_t insert_lanes;   /* 1, 2, 4, 8 or 16 (checked; inserts use one lane an entry) */
     uint32_t find_blocks;    /* persistent grid for find/erase (0 = default) */
     uint32_t insert_blocks;  /* persistent grid for insert (0 = default) */
-    uint32_t item_keys;      /* keys per work item (0 = default 4096) */
+    uint32_t item_keys;      /* keys per work item, at most (0 and 4096, the default: by the batch, up to
+                                4096 for find/erase and 8192 for insert) */
     uint32_t kick_bound;     /* eviction iterations under the reference victim rule */
     uint32_t insert_waves_per_eu;  /* occupancy: 6 or 8 = the insert kernel built for at least that
                                       many waves per SIMD (fewer registers); 0 = the compiler's own */

@@ -82,6 +82,35 @@ def test_sizes_around_tiles(D, bits, item_keys):
     g.close()
 
 
+@pytest.mark.parametrize("kick_bound", [0, 15])
+@pytest.mark.parametrize("item_keys", [0, 64, 500])
+@pytest.mark.parametrize("n", [(1 << 16) - 1, 1 << 16, 400_000])
+def test_inserts_of_shared_and_of_whole_items(D, n, item_keys, kick_bound):
+    """Below 2^16 keys the waves of a workgroup share an insert's items, from there on each takes whole
+    ones: tables of sizes around a tile and around an item, full ones among them."""
+    from databases_gpu_amd.table import DyCuckooGroup
+    from databases_gpu_amd.workload import keys_range, splitmix32
+
+    print(f"\n[gpu-case] group insert of {n} keys, item_keys={item_keys} kick_bound={kick_bound}", flush=True)
+    sizes = np.array(SIZES * (n // sum(SIZES)) + [0], dtype=np.int64)
+    sizes[-1] = n - sizes.sum()
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint64)
+    dv = torch.device("cuda", 0)
+    k = keys_range(0, n, 21, dv)
+    g = DyCuckooGroup((sizes / 0.85).astype(np.uint64) + 32, insert_order=0, kick_bound=kick_bound)
+    g.set_launch(item_keys=item_keys)
+    miss = torch.rand(n, device=dv) < 0.4
+    q = torch.where(miss, keys_range(n, 2 * n, 21, dv), k)
+    for _ in range(2):
+        g.clear()
+        g.insert(k, splitmix32(k), off)
+        assert [g.table_stats(i)["count"] for i in range(sizes.size)] == sizes.tolist()
+        v, h = g.find(q, off)
+        assert torch.equal(h.bool(), ~miss)
+        assert torch.equal(v, torch.where(miss, torch.zeros_like(k), splitmix32(k)))
+    g.close()
+
+
 @pytest.mark.parametrize("order", [0, 3])
 def test_large_find_is_laid_out_by_xcd(D, order):
     """More than 2^22 lookups: items on their tables' XCDs, empty places among them."""
