@@ -349,12 +349,14 @@ __device__ inline void wide_give_up(WideCarry &c, const WideSink &sink, Counters
     c.active = false;
 }
 
-// Take entry (k, v) into the lane's hand; pr is its previous table (kNoTable for a fresh key,
-// kAfterFill for one the bulk fill found no slot for).
+// Take entry (k, v) into the lane's hand; pr is its previous table (kNoTable for a fresh key). AFTER_FILL:
+// the bulk fill found no slot for it, so its fill_target is. (Known when compiled: as a value of pr it
+// cost every insert some 200 instructions, and eviction chains 3-10 % of their time.)
+template <bool AFTER_FILL>
 __device__ inline void wide_take(WideCarry &c, const Desc &D, uint64_t k, uint64_t v, uint32_t pr)
 {
-    c.swing = pr == kNoTable;
-    if (pr == kAfterFill) pr = fill_target(D, (uint32_t)k, pair_of(D, fold64(k)));
+    c.swing = !AFTER_FILL && pr == kNoTable;
+    if constexpr (AFTER_FILL) pr = fill_target(D, (uint32_t)k, pair_of(D, fold64(k)));
     else if (pr == kNoTable && (k & 1u)) pr = pos1(D, pair_of(D, fold64(k)));  // odd keys start in pos2
     c.key = k;
     c.val = v;
@@ -500,7 +502,7 @@ __global__ __launch_bounds__(256) void wide_insert_kernel(WideDesc W, const uint
                 continue;
             }
             ++taken;
-            wide_take(c, W.D, e.k, e.v, pre_fixed);
+            wide_take<SRC == kWideOverflow>(c, W.D, e.k, e.v, SRC == kWideBatch ? kNoTable : pre_fixed);
         }
         if (!__any(c.active)) break;
         if (c.active) wide_step(c, W, P, C, sink, sink.tag, kicks, retries, direct);
@@ -590,7 +592,7 @@ __global__ __launch_bounds__(256) void wide_group_insert_kernel(const WideDesc *
                     continue;
                 }
                 ++taken;
-                wide_take(c, W.D, e.k, e.v, SRC == kWideOverflow ? kAfterFill : kNoTable);
+                wide_take<SRC == kWideOverflow>(c, W.D, e.k, e.v, kNoTable);
             }
             if (!__any(c.active)) break;
             if (c.active) wide_step(c, W, P, C, sink, item.table, kicks, retries, direct);
