@@ -25,10 +25,10 @@ namespace host {
 // find on another stream. A stream's handle says which mark its finds share and nothing more: the
 // handle may have been another stream's, destroyed with its finds still running. So every mark is
 // waited for, whatever its handle, and a mark is recorded again only after a wait for what it
-// stood for (both are nothing on the stream that recorded it). Finds of fewer than kFirstBucketKeys keys read in the reference order:
-// the mark, and two buckets' latencies in turn, cost small calls more than they save (with the mark, in
-// tables of 10 MiB and more: 2^18 lookups 0.8-1.1 times as fast, 2^20 0.95-1.2, 2^21 1.03-1.3, 2^22
-// 1.06-1.35). So do finds being captured, which may be replayed after an erase, finds on the per-thread
+// stood for (both are nothing on the stream that recorded it).
+// Finds of fewer than kFirstBucketKeys keys read in the reference order: the mark, and two buckets'
+// latencies in turn, cost small calls more than they save (with the mark, in tables of 10 MiB and more:
+// 2^18 lookups 0.8-1.1 times as fast, 2^20 0.95-1.2, 2^21 1.03-1.3, 2^22 1.06-1.35). So do finds being captured, which may be replayed after an erase, finds on the per-thread
 // stream (one handle for many streams), and those on more than kMarks streams since the last erase or
 // clear.
 constexpr uint64_t kFirstBucketKeys = 1ull << 22;
